@@ -3,7 +3,7 @@
 #include "mfma_decode.h"
 #include "mfma_decode_ring.h"
 #include "mfma_decode_resident.h"
-#include "mfma_pipelined.h"
+#include "pipe_tiles.h"
 #include "mfma_ragged.h"
 #include "mfma_skinny.h"
 #include "plan.h"
@@ -120,36 +120,43 @@ int compute_units() {
     return cus;
 }
 
-template <class Cfg>
-void launch_splitk(const void *A, const void *B, void *C, size_t M, size_t N, size_t K, int splits,
-                   const Workspace &ws) {
+template <class Cfg, bool EDGE>
+void launch_splitk_form(const void *A, const void *B, void *C, size_t M, size_t N, size_t K, int splits,
+                        const Workspace &ws) {
     static bool configured = [] {
-        HGEMM_CHECK_HIP_ERROR(hipFuncSetAttribute(reinterpret_cast<const void *>(&hgemm_skinny_kernel<Cfg, false>),
+        HGEMM_CHECK_HIP_ERROR(hipFuncSetAttribute(reinterpret_cast<const void *>(&hgemm_skinny_kernel<Cfg, false, EDGE>),
                                                   hipFuncAttributeMaxDynamicSharedMemorySize, Cfg::LDS_BYTES));
-        HGEMM_CHECK_HIP_ERROR(hipFuncSetAttribute(reinterpret_cast<const void *>(&hgemm_skinny_kernel<Cfg, true>),
+        HGEMM_CHECK_HIP_ERROR(hipFuncSetAttribute(reinterpret_cast<const void *>(&hgemm_skinny_kernel<Cfg, true, EDGE>),
                                                   hipFuncAttributeMaxDynamicSharedMemorySize, Cfg::LDS_BYTES));
         return true;
     }();
     (void)configured;
-    HGEMM_CHECK(N % Cfg::BN == 0);
-    HGEMM_CHECK(splits >= 1 && K % (size_t)Cfg::BK == 0 && K / (size_t)Cfg::BK >= (size_t)splits);
-    const size_t tiles_n = N / Cfg::BN, tiles = tiles_n * div_ceil(M, Cfg::BM);  // < 2^31 / (BM * BN)
+    HGEMM_CHECK(EDGE ? K % 8 == 0 && K >= 64 : N % Cfg::BN == 0 && K % (size_t)Cfg::BK == 0);
+    HGEMM_CHECK(splits >= 1 && div_ceil(K, (size_t)Cfg::BK) >= (size_t)splits);
+    const size_t tiles_n = div_ceil(N, (size_t)Cfg::BN), tiles = tiles_n * div_ceil(M, (size_t)Cfg::BM);  // < 2^31
     const dim3 grid((unsigned)tiles, (unsigned)splits);
     HGEMM_CHECK(splits <= 65535);
     float *partial = nullptr;
     if (splits > 1) {
-        HGEMM_CHECK(ws.partial != nullptr && ws.partial_bytes >= (size_t)splits * M * N * sizeof(float));
+        HGEMM_CHECK(ws.partial != nullptr && ws.partial_bytes >= (size_t)splits * M * partial_ld(N) * sizeof(float));
         partial = ws.partial;
     }
     // a B of 48 MB or more is streamed past the caches: +2-12 % from 64 MB up (N = 8192 ... 28672 at K = 4096),
     // 0-7 % slower at 32 MB (N = K = 4096), where the next call finds parts of B in the Infinity Cache otherwise
     const bool stream_b = div_ceil(M, Cfg::BM) == 1 && N * K >= ((size_t)24 << 20);
-    auto kernel = stream_b ? &hgemm_skinny_kernel<Cfg, true> : &hgemm_skinny_kernel<Cfg, false>;
+    auto kernel = stream_b ? &hgemm_skinny_kernel<Cfg, true, EDGE> : &hgemm_skinny_kernel<Cfg, false, EDGE>;
     kernel<<<grid, dim3(Cfg::THREADS), Cfg::LDS_BYTES, nullptr>>>(
         reinterpret_cast<const half_t *>(A), reinterpret_cast<const half_t *>(B), reinterpret_cast<half_t *>(C),
         partial, (int)M, (int)N, (int)K, splits, (int)tiles_n);
     HGEMM_CHECK_HIP_ERROR(hipGetLastError());
-    if (splits > 1) launch_splitk_reduce(partial, reinterpret_cast<half_t *>(C), M * N, splits);
+    if (splits > 1) launch_splitk_reduce(partial, reinterpret_cast<half_t *>(C), M, N, splits);
+}
+template <class Cfg>
+void launch_splitk(const void *A, const void *B, void *C, size_t M, size_t N, size_t K, int splits, const Workspace &ws) {
+    if (N % Cfg::BN == 0 && K % (size_t)Cfg::BK == 0)
+        launch_splitk_form<Cfg, false>(A, B, C, M, N, K, splits, ws);
+    else
+        launch_splitk_form<Cfg, true>(A, B, C, M, N, K, splits, ws);
 }
 
 //                             BM   BN  WM WN stages
@@ -159,19 +166,6 @@ using Split64x128 = SkinnyConfig<64, 128, 2, 2, 4>;
 using Split128x64 = SkinnyConfig<128, 64, 2, 2, 4>;
 using Split128x128 = SkinnyConfig<128, 128, 2, 2, 4>;
 
-// 256x256x64 tile on v_mfma_f32_16x16x32_f16, two B buffers and three A buffers (all 160 KB of LDS)
-using Big256 = PipeConfig<256, 256, 64, 2, 2, 2, 16, 1>;
-using Mid128 = PipeConfig<128, 128, 64, 2, 2, 5, 16>;
-// two LDS buffers (64 KB): two workgroups fit a CU, and one's C tile goes out while the other multiplies.  Pays where
-// a workgroup's K loop is shorter than its epilogue and C outgrows the Infinity Cache: 16384^2 x 256 201 -> 170 us.
-using Mid128S2 = PipeConfig<128, 128, 64, 2, 2, 2, 16>;
-using Small64 = PipeConfig<64, 64, 64, 1, 1, 3, 16>;
-// one row of tiles for M <= 64: four waves side by side, 64x32 each
-using Row64x128 = PipeConfig<64, 128, 64, 1, 4, 5, 16>;
-// one row of tiles for M = 129 ... 192: four stages of 24 + 16 KB are the whole LDS
-using Row192x128 = PipeConfig<192, 128, 64, 2, 2, 4, 16>;
-using Tile192 = PipeConfig<192, 192, 64, 2, 2, 3, 16>;
-using Rect256x128 = PipeConfig<256, 128, 64, 2, 2, 3, 16>;
 // 64x64x64 on four waves (one 32x32 MFMA tile each) with the ladder's kernel: a small tile whose chunk takes a quarter
 // of the one-wave tile's matrix-pipe time; for grids that give a CU at most one tile.  Three forms by the number of
 // chunks a workgroup walks: the plain 3-stage ring up to 4 (the look-ahead prologue costs more than it returns),
@@ -216,9 +210,36 @@ void launch_pipelined_plan(const void *A, const void *B, void *C, size_t M, size
         launch_pipelined<Cfg>(A, B, C, M, N, K, "hgemm_auto");
         return;
     }
-    HGEMM_CHECK(ws.partial != nullptr && ws.partial_bytes >= (size_t)splits * M * N * sizeof(float));
+    HGEMM_CHECK(ws.partial != nullptr && ws.partial_bytes >= (size_t)splits * M * partial_ld(N) * sizeof(float));
     launch_pipelined_split<Cfg>(A, B, ws.partial, M, N, K, splits, "hgemm_auto");
-    launch_splitk_reduce(ws.partial, reinterpret_cast<half_t *>(C), M * N, splits);
+    launch_splitk_reduce(ws.partial, reinterpret_cast<half_t *>(C), M, N, splits);
+}
+
+// The four-wave 64x64 tile in the form that suits the number of chunks a workgroup walks; EDGE: sizes that end inside a
+// tile or chunk.
+template <bool EDGE>
+void launch_small64_w4(const void *A, const void *B, void *C, size_t M, size_t N, size_t K, int splits, const Workspace &ws) {
+    const size_t chunks = div_ceil(K, (size_t)64) / (size_t)(splits > 1 ? splits : 1);
+    if (splits <= 1) {
+        if (chunks <= W4_SHORT_MAX_CHUNKS)
+            launch_tiled<Small64W4Short, EDGE>(A, B, C, M, N, K, "hgemm_auto");
+        else if (div_ceil(M, (size_t)64) * div_ceil(N, (size_t)64) > (size_t)compute_units())
+            launch_tiled<Small64W4Pair, EDGE>(A, B, C, M, N, K, "hgemm_auto");
+        else if (chunks < W4_DEEP_MIN_CHUNKS)
+            launch_tiled<Small64W4, EDGE>(A, B, C, M, N, K, "hgemm_auto");
+        else
+            launch_tiled<Small64W4Deep, EDGE>(A, B, C, M, N, K, "hgemm_auto");
+        return;
+    }
+    check_operands(A, B, C, M, N, K);
+    HGEMM_CHECK(ws.partial != nullptr && ws.partial_bytes >= (size_t)splits * M * partial_ld(N) * sizeof(float));
+    if (chunks <= W4_SHORT_MAX_CHUNKS)
+        launch_tiled_split<Small64W4Short, EDGE>(A, B, ws.partial, M, N, K, splits, "hgemm_auto");
+    else if (chunks < W4_DEEP_MIN_CHUNKS)
+        launch_tiled_split<Small64W4, EDGE>(A, B, ws.partial, M, N, K, splits, "hgemm_auto");
+    else
+        launch_tiled_split<Small64W4Deep, EDGE>(A, B, ws.partial, M, N, K, splits, "hgemm_auto");
+    launch_splitk_reduce(ws.partial, reinterpret_cast<half_t *>(C), M, N, splits);
 }
 
 // ---- cost model for the tile-aligned shapes.  A candidate is a tile (its kernel), how
@@ -262,9 +283,17 @@ double reduce_us(int slices, double elems) {
 }
 // extra cost of finishing a grid with a separate launch for its last round: in K slices / on smaller tiles
 constexpr double TAIL_US = 3.6, TAIL_SUB_US = 4.4;
+// K that is no multiple of 64: a 128-byte piece of a row straddles two cache lines, so the copies into LDS ask L2 for twice
+// the lines.  Chunk times grow by this factor (5112^3 269 us where 5120^3 takes 208; 1.18 ... 1.30 from 1000^3 to 8184^3), and from
+// about 4500^3 on it is cheaper to copy both operands first (5112^3 245 us, 8184^3 863 -> 802 us; 4000^2 x 4040 103 against 112).
+constexpr double OFF_LINE = 1.27;
+// that copy: fixed, and per byte read and written (20 us for 4095^2 twice)
+constexpr double COPY_US = 3.5, COPY_BYTES_PER_US = 5500e3;
 size_t padded_n(size_t N) { return (N + 7) / 8 * 8; }
 size_t padded_k(size_t K) { return (K + 63) / 64 * 64; }
-// A' (M x K'), B' (N' x K') and, when N grows, C' (M x N')
+// What a plan with copied operands reserves, and hgemm_auto_workspace_bytes reports: A' (M x K'), B' (N' x K') and, when N
+// is no multiple of 8, as much again as a C' (M x N') would take.  The copies are M + N rows of K'; the rest is a bound that
+// callers size their reservations by.
 size_t padded_bytes(size_t M, size_t N, size_t K) {
     const size_t Np = padded_n(N), Kp = padded_k(K);
     return ((M + Np) * Kp + (Np != N ? M * Np : 0)) * sizeof(half_t);
@@ -273,7 +302,7 @@ size_t padded_bytes(size_t M, size_t N, size_t K) {
 double predict_us(const Candidate &c, size_t M, size_t N, size_t K, int splits, size_t cus) {
     const size_t wgs = div_ceil(M, (size_t)c.bm) * div_ceil(N, (size_t)c.bn) * (size_t)splits;
     const size_t slots = cus * (size_t)c.per_cu;
-    const double chunks = (double)div_ceil(K / 64, (size_t)splits);  // the longest slice
+    const double chunks = (double)div_ceil(div_ceil(K, (size_t)64), (size_t)splits);  // the longest slice
     const size_t full = wgs / slots, rem = wgs % slots;
     double t = LAUNCH_US + (double)full * (c.fix + chunks * c.hi);
     if (rem) t += c.fix + chunks * (c.lo + (c.hi - c.lo) * (double)rem / (double)slots);
@@ -287,9 +316,9 @@ double predict_us(const Candidate &c, size_t M, size_t N, size_t K, int splits, 
 double predict_tail_us(const Candidate &c, size_t M, size_t N, size_t K, int ts, size_t cus) {
     const size_t wgs = div_ceil(M, (size_t)c.bm) * div_ceil(N, (size_t)c.bn), slots = cus * (size_t)c.per_cu;
     const size_t full = wgs / slots, rem = wgs % slots;
-    const double chunks = (double)(K / 64);
+    const double chunks = (double)div_ceil(K, (size_t)64);
     double t = LAUNCH_US + (double)full * (c.fix + chunks * c.hi);
-    t += LAUNCH_US + c.fix + (double)div_ceil(K / 64, (size_t)ts) * (c.lo + (c.hi - c.lo) * (double)(rem * ts) / (double)slots);
+    t += LAUNCH_US + c.fix + (double)div_ceil(div_ceil(K, (size_t)64), (size_t)ts) * (c.lo + (c.hi - c.lo) * (double)(rem * ts) / (double)slots);
     t += reduce_us(ts, (double)rem * c.bm * c.bn) + TAIL_US;
     return t;
 }
@@ -302,7 +331,7 @@ double predict_subtile_us(const Candidate &big, const Candidate &small, size_t M
     const size_t full = wgs / slots, rem = wgs % slots;
     const size_t parts = (size_t)(big.bm / small.bm) * (big.bn / small.bn);
     const size_t small_slots = cus * (size_t)small.per_cu, small_wgs = rem * parts;
-    const double chunks = (double)(K / 64);
+    const double chunks = (double)div_ceil(K, (size_t)64);
     double t = LAUNCH_US + (double)full * (big.fix + chunks * big.hi);
     t += LAUNCH_US + (double)(small_wgs / small_slots) * (small.fix + chunks * small.hi);
     if (small_wgs % small_slots)
@@ -329,7 +358,7 @@ int choose_splits(size_t tiles, size_t M, size_t N, size_t cus, size_t K, size_t
     double best_us = 0.0;
     const double stream_us = 2.0 * (double)N * (double)K / 5e6;
     for (int s = 1; s <= 16; ++s) {
-        if (s > 1 && (K % 64 != 0 || K / 64 / (size_t)s < min_chunks || (size_t)s * slice_bytes > limit)) break;
+        if (s > 1 && (K % 8 != 0 || div_ceil(K, (size_t)64) / (size_t)s < min_chunks || (size_t)s * slice_bytes > limit)) break;
         const size_t wgs = tiles * (size_t)s;
         const double balance = (double)wgs / (double)(div_ceil(wgs, cus) * cus);
         const double partials = s > 1 ? 8.0 * s * (double)M / (double)K : 0.0;
@@ -466,6 +495,22 @@ bool small_m_rule_covers(const SmallMRule &r, size_t M, size_t N, size_t K) {
     return true;
 }
 
+// Kernel that stands in for a row's on sizes its own kernel does not divide, 0 if it cannot run them either.  The ring
+// kernel's guarded form also stands in for the two decode kernels that have none.
+int small_m_edge_kernel(int kernel, size_t M, size_t N, size_t K) {
+    if (K % 8 != 0 || K < 64) return KERNEL_NONE;
+    const size_t chunks = div_ceil(K, (size_t)64);
+    switch (kernel) {
+        case KERNEL_DECODE_RING:
+        case KERNEL_DECODE_RESIDENT:
+        case KERNEL_DECODE_BN16: return decode_ring_edge_supports(M, N, K) ? (int)KERNEL_DECODE_RING_EDGE : (int)KERNEL_NONE;
+        case KERNEL_MID128:
+        case KERNEL_ROW64x128: return chunks >= 5 ? kernel : (int)KERNEL_NONE;
+        case KERNEL_T192: return chunks >= 3 ? kernel : (int)KERNEL_NONE;
+        default: return kernel;  // the split-K family
+    }
+}
+
 // shapes the kernel of a row can run at all (the row is skipped otherwise)
 bool small_m_kernel_supports(int kernel, size_t M, size_t N, size_t K) {
     switch (kernel) {
@@ -522,6 +567,21 @@ bool left_out(const PlanLimits &limits, int kernel, int splits, int tail_tiles =
     return left_out(limits, p);
 }
 
+// One pass that copies A and B with rows of whole 64-wide chunks, then the plan for that K (same products, same result);
+// no plan where the copies do not fit.
+Plan plan_on_copies(size_t M, size_t N, size_t K, const PlanLimits &limits) {
+    if (K < 192 || padded_bytes(M, N, K) > limits.operand_bytes) return Plan();
+    PlanLimits inner_limits;
+    inner_limits.partial_bytes = limits.partial_bytes;
+    inner_limits.operand_bytes = 0;
+    Plan p = plan_for(M, N, padded_k(K), inner_limits);
+    p.inner_kernel = p.kernel;
+    p.kernel = KERNEL_PADDED;
+    if (p.est_us > 0.0) p.est_us += COPY_US + 4.0 * (double)((M + N) * padded_k(K)) / COPY_BYTES_PER_US;
+    p.operand_bytes = padded_bytes(M, N, K);
+    return p;
+}
+
 // M <= 128: choices come from timing every candidate (tile x slices) on the specification's
 // decode shapes on an MI355X, operands rotated so small problems read HBM.  Larger,
 // tile-aligned shapes: the cheapest (tile, slices) pair under the cost model above.
@@ -529,16 +589,20 @@ Plan plan_for(size_t M, size_t N, size_t K, const PlanLimits &limits) {
     Plan p;
     if (M == 0 || N == 0 || K == 0) return p;
     const size_t cus = (size_t)compute_units();
-    const size_t slice_bytes = M * N * sizeof(float);  // fp32 partial sums of one K slice of the whole product
-    // M <= 128: the first row of the table above that covers the shape and whose kernel can run it
-    for (const SmallMRule &r : SMALL_M_RULES) {
-        if (M > 128) break;
+    const size_t slice_bytes = M * partial_ld(N) * sizeof(float);  // fp32 partial sums of one K slice of the whole product
+    // M <= 128: the first row of the table above that covers the shape and whose kernel can run it; where there is none
+    // (N or K that nothing divides), the first covering row whose kernel has a form with guarded edges
+    for (int at = 0; at < 2 * SMALL_M_RULE_COUNT && M <= 128; ++at) {
+        const SmallMRule &r = SMALL_M_RULES[at % SMALL_M_RULE_COUNT];
+        const bool edges = at >= SMALL_M_RULE_COUNT;
         if (limits.every_small_m_kernel ? (M < (size_t)r.m_lo || M > (size_t)r.m_hi) : !small_m_rule_covers(r, M, N, K)) continue;
-        if (!small_m_kernel_supports(r.kernel, M, N, K)) continue;
+        if (!edges && !small_m_kernel_supports(r.kernel, M, N, K)) continue;
         p = Plan();
-        p.kernel = r.kernel;
-        switch (r.kernel) {
+        p.kernel = edges ? small_m_edge_kernel(r.kernel, M, N, K) : r.kernel;
+        if (p.kernel == KERNEL_NONE) continue;
+        switch (p.kernel) {
             case KERNEL_DECODE_RING: p.splits = decode_ring_waves(M, N, K, cus); break;
+            case KERNEL_DECODE_RING_EDGE: p.splits = decode_ring_edge_waves(M, N, K, cus); break;
             case KERNEL_DECODE_RESIDENT: {
                 int chunks = 0;
                 p.splits = decode_resident_waves(M, K, &chunks);
@@ -566,7 +630,7 @@ Plan plan_for(size_t M, size_t N, size_t K, const PlanLimits &limits) {
             }
             default: {  // the split-K family: K slices across workgroups, then the ordered reduction
                 const size_t bn = (r.kernel == KERNEL_SPLIT_64x128 || r.kernel == KERNEL_SPLIT_128x128) ? 128 : 64;
-                p.splits = choose_splits(N / bn, M, N, cus, K, slice_bytes, limits.partial_bytes);
+                p.splits = choose_splits(div_ceil(N, bn), M, N, cus, K, slice_bytes, limits.partial_bytes);
                 if (p.splits > 1) p.partial_bytes = (size_t)p.splits * slice_bytes;
             }
         }
@@ -582,41 +646,45 @@ Plan plan_for(size_t M, size_t N, size_t K, const PlanLimits &limits) {
     // of B in flight per CU where the 192x192 tile's three stages keep two.
     {
         const size_t tiles = div_ceil(N, (size_t)128), last = tiles % cus;
-        if (M > 128 && M <= 192 && N % 8 == 0 && K % 64 == 0 && K >= 2048 && K <= 12288 && tiles >= 144 &&
+        if (M > 128 && M <= 192 && K % 8 == 0 && K >= 2048 && K <= 12288 && tiles >= 144 &&
             (last == 0 || last * 100 >= cus * 55) && !left_out(limits, KERNEL_ROW192x128, 1)) {
             p.kernel = KERNEL_ROW192x128;
             p.splits = 1;
             return p;
         }
     }
-    // Pipelined tiles: M and N may end inside a tile (guarded edges; the model charges whole
-    // tiles), as long as rows of C stay 16-byte aligned and K is a whole number of chunks.
+    // Pipelined tiles: M and N may end inside a tile and K inside a chunk (guarded edges; the model charges whole
+    // tiles and chunks), as long as rows of A and B stay 16-byte aligned.
+    // M and N that 64 does not divide while K does and rows of C are aligned: fitted on the one-wave tile, left to it
+    const bool one_wave = (M % 64 || N % 64) && N % 8 == 0 && K % 64 == 0;
     double best = 0.0;
-    for (const Candidate &c : CANDIDATES) {
-        if (N % 8) break;
-        const bool whole_tiles_only = c.kernel == KERNEL_SMALL64_W4;
-        if (whole_tiles_only && (M % c.bm || N % c.bn)) continue;
+    for (Candidate c : CANDIDATES) {
+        if (K % 8) break;
+        if (K % 64) c.lo *= OFF_LINE, c.hi *= OFF_LINE;
+        const bool w4 = c.kernel == KERNEL_SMALL64_W4;
+        const int kernel = w4 && (M % 64 || N % 64 || K % 64) ? (int)KERNEL_SMALL64_W4_EDGE : c.kernel;
+        if (w4 && one_wave) continue;
         for (int s = 1; s <= 32; ++s) {  // K slices: whole chunks, as even as that allows
-            if (whole_tiles_only) {
-                const size_t wgs = (M / c.bm) * (N / c.bn) * (size_t)s;
+            if (w4) {
+                const size_t wgs = div_ceil(M, (size_t)c.bm) * div_ceil(N, (size_t)c.bn) * (size_t)s;
                 if (wgs > cus * (size_t)c.per_cu) break;
-                if (c.per_cu == 2 && (wgs <= cus || s > 1 || K / 64 >= W4_DEEP_MIN_CHUNKS)) break;
+                if (c.per_cu == 2 && (wgs <= cus || s > 1 || div_ceil(K, (size_t)64) >= W4_DEEP_MIN_CHUNKS)) break;
                 // most CUs busy and a long walk per workgroup: the 128x128 tile in K slices moves half the bytes per
                 // flop into LDS and is ahead (1024^2 x 7168: 25.3 us here, 22.2 us in four slices of 128x128 tiles;
                 // level at K = 5120, behind at 4096)
                 if (wgs * 4 > cus * 3 && shortest_slice(K, 64, s) >= 64 * 96) continue;
             }
             if (c.kernel == KERNEL_MID128_S2 && (s > 1 || K > 256)) break;
-            // whole 64x64 tiles, at most one workgroup per CU: the four-wave tile is ahead of the one-wave tile on
+            // at most one workgroup of 64x64 tiles per CU: the four-wave tile is ahead of the one-wave tile on
             // every such grid that was measured (the model, fitted on larger grids, flatters the one-wave tile there)
-            if (c.kernel == KERNEL_SMALL64 && M % 64 == 0 && N % 64 == 0 && (M / 64) * (N / 64) * (size_t)s <= cus) continue;
-            if (K % 64 || shortest_slice(K, 64, s) < (size_t)64 * c.stages) break;
+            if (c.kernel == KERNEL_SMALL64 && !one_wave && div_ceil(M, (size_t)64) * div_ceil(N, (size_t)64) * (size_t)s <= cus) continue;
+            if (shortest_slice(K, 64, s) < (size_t)64 * c.stages) break;
             if (s > 1 && (size_t)s * slice_bytes > limits.partial_bytes) break;
-            if (left_out(limits, c.kernel, s)) continue;
+            if (left_out(limits, kernel, s)) continue;
             const double t = predict_us(c, M, N, K, s, cus);
             if (p.kernel == KERNEL_NONE || t < best) {
                 best = t;
-                p.kernel = c.kernel;
+                p.kernel = kernel;
                 p.splits = s;
                 p.est_us = t;
                 p.tail_tiles = 0;
@@ -628,9 +696,9 @@ Plan plan_for(size_t M, size_t N, size_t K, const PlanLimits &limits) {
         // a grid of whole rounds plus a few workgroups: run those few in K slices
         const size_t wgs = div_ceil(M, (size_t)c.bm) * div_ceil(N, (size_t)c.bn), slots = cus * (size_t)c.per_cu;
         const size_t rem = wgs % slots;
-        if (wgs > slots && rem > 0 && !whole_tiles_only && c.kernel != KERNEL_MID128_S2) {
+        if (wgs > slots && rem > 0 && !w4 && c.kernel != KERNEL_MID128_S2) {
             for (int ts = 2; ts <= 16; ++ts) {
-                if (K % 64 || shortest_slice(K, 64, ts) < (size_t)64 * c.stages || rem * ts > slots) break;
+                if (shortest_slice(K, 64, ts) < (size_t)64 * c.stages || rem * ts > slots) break;
                 if ((size_t)ts * rem * c.bm * c.bn * sizeof(float) > limits.partial_bytes) break;
                 if (left_out(limits, c.kernel, 1, (int)rem, ts)) continue;
                 const double t = predict_tail_us(c, M, N, K, ts, cus);
@@ -646,11 +714,12 @@ Plan plan_for(size_t M, size_t N, size_t K, const PlanLimits &limits) {
                 }
             }
             if (c.kernel == KERNEL_BIG256) {  // ... or on smaller tiles that divide this one
-                for (const Candidate &small : CANDIDATES) {
+                for (Candidate small : CANDIDATES) {
+                    if (K % 64) small.lo *= OFF_LINE, small.hi *= OFF_LINE;
                     if (small.kernel == KERNEL_BIG256 || small.kernel == KERNEL_SMALL64_W4 || small.kernel == KERNEL_MID128_S2 ||
                         c.bm % small.bm || c.bn % small.bn)
                         continue;
-                    if (K < (size_t)64 * small.stages || left_out(limits, c.kernel, 1, (int)rem, 1, small.kernel)) continue;
+                    if (div_ceil(K, (size_t)64) < (size_t)small.stages || left_out(limits, c.kernel, 1, (int)rem, 1, small.kernel)) continue;
                     const double t = predict_subtile_us(c, small, M, N, K, cus);
                     if (p.kernel != KERNEL_NONE && t < best) {
                         best = t;
@@ -666,95 +735,76 @@ Plan plan_for(size_t M, size_t N, size_t K, const PlanLimits &limits) {
             }
         }
     }
-    if (p.kernel != KERNEL_NONE) return p;
+    if (p.kernel != KERNEL_NONE) {
+        if (K % 64) {  // copied to rows of whole lines first?
+            Plan copied = plan_on_copies(M, N, K, limits);
+            if (copied.kernel != KERNEL_NONE && copied.est_us < p.est_us && !left_out(limits, copied)) return copied;
+        }
+        return p;
+    }
     if (limits.excluded_count > 0) return Plan();  // the tuner's question has no further answer
-    if (N % 64 == 0 && K % 64 == 0) {  // any M: rows beyond M are guarded
+    if (K % 8 == 0 && K >= 64) {  // K of one or two chunks; any M and N: guarded
         p.kernel = KERNEL_SPLIT_64x64;
-        p.splits = choose_splits(div_ceil(M, 64) * (N / 64), M, N, cus, K, slice_bytes, limits.partial_bytes);
+        p.splits = choose_splits(div_ceil(M, 64) * div_ceil(N, 64), M, N, cus, K, slice_bytes, limits.partial_bytes);
         if (p.splits > 1) p.partial_bytes = (size_t)p.splits * slice_bytes;
         return p;
     }
-    // Rows of C not 16-byte aligned (N % 8) or K not a whole number of chunks.  Large
-    // products are worth two extra passes over the operands: copy A and B zero-padded to a
-    // shape the pipelined kernels take and run that (same products, same result); the rest
-    // goes to the guarded kernel, which sustains about 80 TFLOP/s.
-    const size_t Np = padded_n(N), Kp = padded_k(K);
-    if (K >= 192 && padded_bytes(M, N, K) <= limits.operand_bytes) {
-        const Plan inner = plan_for(M, Np, Kp, limits);
-        const double inner_us = inner.est_us > 0.0 ? inner.est_us : 8.0 + (double)(Np * Kp * 2) / 4e6;
-        const double copy_us = 6.0 + 4.0 * (double)((M + Np) * Kp + (Np != N ? M * Np : 0)) / 3.5e6;
-        const double guarded_us = 5.0 + 2.0 * (double)M * (double)N * (double)K / 80e6;
-        if (inner.kernel != KERNEL_RAGGED && inner.kernel != KERNEL_PADDED && copy_us + inner_us < guarded_us) {
-            p.kernel = KERNEL_PADDED;
-            p.splits = inner.splits;
-            p.est_us = copy_us + inner_us;
-            p.partial_bytes = inner.partial_bytes;
-            p.operand_bytes = padded_bytes(M, N, K);
-            return p;
-        }
-    }
+    // Rows of A and B not 16-byte aligned: on copies from K = 192 on.  Below, and where the copies do not fit, the guarded
+    // kernel, which gathers such rows element by element (4 ... 5 us per 32 of K).
+    const Plan copied = plan_on_copies(M, N, K, limits);
+    if (copied.kernel != KERNEL_NONE) return copied;
     p.kernel = KERNEL_RAGGED;
     return p;
 }
 
-// dst[r][0..cols_dst) = src[r][0..cols_src) followed by zeros, for r < rows_src; rows
-// beyond rows_src are all zeros.  One thread per 8 halves of dst.
+// Rows of A and B that start on 2-byte boundaries (K % 8 != 0), copied so that they start on 128-byte ones: row r of A, then
+// row r - M of B, to dst[r][0 .. Kp), zeros from K on.  One wave per row and REALIGN_COLS columns; its loads are 16 bytes per lane
+// at the source's own alignment (which this part's vector memory takes at the price of one more cache line per 1 KB),
+// all issued before the first store.  Bound by memory: 4095^2 twice, 134 MB there and back.
+constexpr int REALIGN_UNROLL = 8, REALIGN_COLS = REALIGN_UNROLL * 64 * 8;
 __global__ void __launch_bounds__(256)
-    pad_copy_kernel(const half_t *__restrict__ src, half_t *__restrict__ dst, int rows_src, int cols_src, int rows_dst,
-                    int cols_dst) {
-    const size_t chunk = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int chunks_per_row = cols_dst / 8;
-    const size_t row = chunk / chunks_per_row;
-    if (row >= (size_t)rows_dst) return;
-    const int col = (int)(chunk % chunks_per_row) * 8;
-    half8 v;
+    realign_rows_kernel(const half_t *__restrict__ A, const half_t *__restrict__ B, half_t *__restrict__ dst, int M, int rows,
+                        int K, int Kp) {
+    const int lane = threadIdx.x & 63, row = (int)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (row >= rows) return;
+    const half_t *src = row < M ? A + (size_t)row * K : B + (size_t)(row - M) * K;
+    half_t *out = dst + (size_t)row * Kp;
+    const int block_col = (int)blockIdx.y * REALIGN_COLS, first = block_col + lane * 8;
+    // A piece that ends beyond K is loaded as the row's last eight elements and shifted down; one that starts beyond K is
+    // zero.  So every lane's loads are one instruction each, inside the row (K >= 8), and none waits for another.
+    u32x4 v[REALIGN_UNROLL];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) v[e] = (half_t)0.0f;
-    if (row < (size_t)rows_src && col < cols_src) {
-        const half_t *s = src + row * cols_src + col;
-        if ((cols_src & 7) == 0) {
-            v = *reinterpret_cast<const half8 *>(s);
-        } else {
-#pragma unroll
-            for (int e = 0; e < 8; ++e)
-                if (col + e < cols_src) v[e] = s[e];
+    for (int u = 0; u < REALIGN_UNROLL; ++u)
+        if (block_col + u * 512 < Kp) {
+            const int col = first + u * 512;
+            v[u] = *reinterpret_cast<const u32x4_any *>(src + (col + 8 <= K ? col : K - 8));
         }
-    }
-    *reinterpret_cast<half8 *>(dst + row * cols_dst + col) = v;
-}
-// dst[r][c] = src[r][c] for c < cols_dst <= cols_src (drops the padding columns of C).
-__global__ void __launch_bounds__(256)
-    unpad_copy_kernel(const half_t *__restrict__ src, half_t *__restrict__ dst, int rows, int cols_src, int cols_dst) {
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (size_t)rows * cols_dst) return;
-    const size_t r = i / cols_dst, c = i % cols_dst;
-    dst[i] = src[r * cols_src + c];
+    const int shift = 16 * (8 - (K & 7)) & 127;  // K % 8 == 0 has no such piece
+#pragma unroll
+    for (int u = 0; u < REALIGN_UNROLL; ++u)
+        if (block_col + u * 512 < Kp) {
+            const int col = first + u * 512;
+            unsigned __int128 bits = __builtin_bit_cast(unsigned __int128, v[u]);
+            bits = col + 8 <= K ? bits : col < K ? bits >> shift : (unsigned __int128)0;
+            if (col < Kp) *reinterpret_cast<u32x4 *>(out + col) = __builtin_bit_cast(u32x4, bits);
+        }
 }
 
 void run_padded(const Plan &p, const Workspace &ws, const void *A, const void *B, void *C, size_t M, size_t N,
                 size_t K) {
-    const size_t Np = padded_n(N), Kp = padded_k(K);
-    HGEMM_CHECK(ws.operands != nullptr && ws.operand_bytes >= padded_bytes(M, N, K));
-    half_t *Ap = reinterpret_cast<half_t *>(ws.operands), *Bp = Ap + M * Kp;
-    half_t *Cp = Np != N ? Bp + Np * Kp : reinterpret_cast<half_t *>(C);
-    pad_copy_kernel<<<dim3((unsigned)div_ceil(M * (Kp / 8), (size_t)256)), dim3(256), 0, nullptr>>>(
-        reinterpret_cast<const half_t *>(A), Ap, (int)M, (int)K, (int)M, (int)Kp);
-    pad_copy_kernel<<<dim3((unsigned)div_ceil(Np * (Kp / 8), (size_t)256)), dim3(256), 0, nullptr>>>(
-        reinterpret_cast<const half_t *>(B), Bp, (int)N, (int)K, (int)Np, (int)Kp);
+    const size_t Kp = padded_k(K), rows = M + N;
+    HGEMM_CHECK(ws.operands != nullptr && ws.operand_bytes >= rows * Kp * sizeof(half_t));
+    HGEMM_CHECK(div_ceil(Kp, (size_t)REALIGN_COLS) <= 65535);
+    half_t *copies = reinterpret_cast<half_t *>(ws.operands);
+    realign_rows_kernel<<<dim3((unsigned)div_ceil(rows, (size_t)4), (unsigned)div_ceil(Kp, (size_t)REALIGN_COLS)), dim3(256), 0, nullptr>>>(
+        reinterpret_cast<const half_t *>(A), reinterpret_cast<const half_t *>(B), copies, (int)M, (int)rows, (int)K, (int)Kp);
     HGEMM_CHECK_HIP_ERROR(hipGetLastError());
-    // The inner plan that plan_for sized p for: the best plan within a limit is still the best
-    // within the smaller limit of what it needs itself.
-    PlanLimits inner_limits;
-    inner_limits.partial_bytes = p.partial_bytes;
-    inner_limits.operand_bytes = 0;
-    const Plan inner = plan_for(M, Np, Kp, inner_limits);
-    HGEMM_CHECK(inner.kernel != KERNEL_PADDED && inner.kernel != KERNEL_RAGGED && inner.partial_bytes == p.partial_bytes);
-    run_plan(inner, ws, Ap, Bp, Cp, M, Np, Kp);
-    if (Np != N) {
-        unpad_copy_kernel<<<dim3((unsigned)div_ceil(M * N, (size_t)256)), dim3(256), 0, nullptr>>>(
-            Cp, reinterpret_cast<half_t *>(C), (int)M, (int)Np, (int)N);
-        HGEMM_CHECK_HIP_ERROR(hipGetLastError());
-    }
+    Plan inner = p;
+    inner.kernel = p.inner_kernel;
+    inner.inner_kernel = KERNEL_NONE;
+    inner.operand_bytes = 0;
+    HGEMM_CHECK(inner.kernel != KERNEL_PADDED && inner.kernel != KERNEL_RAGGED);
+    run_plan(inner, ws, copies, copies + M * Kp, C, M, N, Kp);
 }
 
 void run_plan(const Plan &p, const Workspace &ws, const void *A, const void *B, void *C, size_t M, size_t N,
@@ -768,30 +818,8 @@ void run_plan(const Plan &p, const Workspace &ws, const void *A, const void *B, 
         case KERNEL_ROW64x128: launch_pipelined_plan<Row64x128>(A, B, C, M, N, K, p, ws); break;
         case KERNEL_ROW192x128: launch_pipelined_plan<Row192x128>(A, B, C, M, N, K, p, ws); break;
         case KERNEL_SMALL64: launch_pipelined_plan<Small64>(A, B, C, M, N, K, p, ws); break;
-        case KERNEL_SMALL64_W4: {
-            const size_t chunks = K / 64 / (size_t)(p.splits > 1 ? p.splits : 1);
-            if (p.splits <= 1) {
-                if (chunks <= W4_SHORT_MAX_CHUNKS)
-                    launch_tiled<Small64W4Short>(A, B, C, M, N, K, "hgemm_auto");
-                else if ((M / 64) * (N / 64) > (size_t)compute_units())
-                    launch_tiled<Small64W4Pair>(A, B, C, M, N, K, "hgemm_auto");
-                else if (chunks < W4_DEEP_MIN_CHUNKS)
-                    launch_tiled<Small64W4>(A, B, C, M, N, K, "hgemm_auto");
-                else
-                    launch_tiled<Small64W4Deep>(A, B, C, M, N, K, "hgemm_auto");
-            } else {
-                check_operands(A, B, C, M, N, K);
-                HGEMM_CHECK(ws.partial != nullptr && ws.partial_bytes >= (size_t)p.splits * M * N * sizeof(float));
-                if (chunks <= W4_SHORT_MAX_CHUNKS)
-                    launch_tiled_split<Small64W4Short>(A, B, ws.partial, M, N, K, p.splits, "hgemm_auto");
-                else if (chunks < W4_DEEP_MIN_CHUNKS)
-                    launch_tiled_split<Small64W4>(A, B, ws.partial, M, N, K, p.splits, "hgemm_auto");
-                else
-                    launch_tiled_split<Small64W4Deep>(A, B, ws.partial, M, N, K, p.splits, "hgemm_auto");
-                launch_splitk_reduce(ws.partial, reinterpret_cast<half_t *>(C), M * N, p.splits);
-            }
-            break;
-        }
+        case KERNEL_SMALL64_W4: launch_small64_w4<false>(A, B, C, M, N, K, p.splits, ws); break;
+        case KERNEL_SMALL64_W4_EDGE: launch_small64_w4<true>(A, B, C, M, N, K, p.splits, ws); break;
         case KERNEL_SPLIT_32x64: launch_splitk<Split32x64>(A, B, C, M, N, K, p.splits, ws); break;
         case KERNEL_SPLIT_64x64: launch_splitk<Split64x64>(A, B, C, M, N, K, p.splits, ws); break;
         case KERNEL_SPLIT_64x128: launch_splitk<Split64x128>(A, B, C, M, N, K, p.splits, ws); break;
@@ -800,6 +828,7 @@ void run_plan(const Plan &p, const Workspace &ws, const void *A, const void *B, 
         case KERNEL_DECODE_BN16: launch_decode(A, B, C, M, N, K, 16, p.splits); break;
         case KERNEL_DECODE_BN32: launch_decode(A, B, C, M, N, K, 32, p.splits); break;
         case KERNEL_DECODE_RING: launch_decode_ring(A, B, C, M, N, K, p.splits); break;
+        case KERNEL_DECODE_RING_EDGE: launch_decode_ring_edge(A, B, C, M, N, K, p.splits); break;
         case KERNEL_DECODE_RESIDENT: launch_decode_resident(A, B, C, M, N, K, compute_units()); break;
         case KERNEL_RAGGED: launch_ragged(A, B, C, M, N, K); break;
         case KERNEL_PADDED: run_padded(p, ws, A, B, C, M, N, K); break;
@@ -1089,6 +1118,10 @@ extern "C" int hgemm_auto_plan_is_tuned(size_t M, size_t N, size_t K) {
 #define HGEMM_DEFINE_PIPELINED_VARIANT(symbol, Cfg, which)                                                   \
     extern "C" void symbol(const hgemm_half *A, const hgemm_half *B, hgemm_half *C, size_t M, size_t N,      \
                            size_t K) {                                                                       \
+        check_operands(A, B, C, M, N, K);                                                                    \
+        HGEMM_CHECK_MSG(pipelined_supports_edges<Cfg>(M, N, K),                                              \
+                        "%s needs N %% 8 == 0, K %% %d == 0, K >= %d (got M=%zu N=%zu K=%zu)", #symbol,      \
+                        Cfg::BK, Cfg::BK * Cfg::STAGES, M, N, K);                                            \
         launch_pipelined<Cfg>(A, B, C, M, N, K, #symbol, which);                                             \
     }                                                                                                        \
     extern "C" int symbol##_supports(size_t M, size_t N, size_t K) {                                         \
@@ -1211,6 +1244,7 @@ extern "C" const char *hgemm_kernel_name(int kernel) {
         case KERNEL_ROW192x128: return "pipelined 192x128x64, 4 waves, 4-stage ring";
         case KERNEL_SMALL64: return "pipelined 64x64x64, 1 wave, 3-stage ring";
         case KERNEL_SMALL64_W4: return "tiled 64x64x64, 4 waves of 32x32, look-ahead ring";
+        case KERNEL_SMALL64_W4_EDGE: return "edge-guarded 64x64x64, 4 waves of 32x32, look-ahead ring";
         case KERNEL_T192: return "pipelined 192x192x64, 4 waves, 3-stage ring";
         case KERNEL_R256x128: return "pipelined 256x128x64, 4 waves, 3-stage ring";
         case KERNEL_SPLIT_32x64: return "split-K 32x64x64, 2 waves, 4-stage ring";
@@ -1221,9 +1255,10 @@ extern "C" const char *hgemm_kernel_name(int kernel) {
         case KERNEL_DECODE_BN16: return "streaming decode, 16 columns per workgroup, one wave per K slice";
         case KERNEL_DECODE_BN32: return "streaming decode, 32 columns per workgroup, one wave per K slice";
         case KERNEL_DECODE_RING: return "streaming decode, 16 columns per workgroup, one wave and one LDS ring per K slice";
+        case KERNEL_DECODE_RING_EDGE: return "streaming decode, 16 columns per workgroup, per-wave LDS rings, guarded edges";
         case KERNEL_DECODE_RESIDENT: return "decode with A in registers, persistent workgroups over 16-column tiles, one wave per K slice";
         case KERNEL_RAGGED: return "guarded 128x128x32, 4 waves, any shape";
-        case KERNEL_PADDED: return "zero-padded operand copies + pipelined kernel of the padded shape";
+        case KERNEL_PADDED: return "zero-padded operand copies + kernel of the padded shape";
         case KERNEL_SIMT: return "scalar fallback";
         default: return "none";
     }

@@ -74,7 +74,7 @@ HGEMM_FOR_EACH_ACC_TILE(X)
 // consecutive n of one row m = lane % 16 of each tile): each wave parks 16 rows of its tile
 // in a private strip and reads them back row-contiguous, 16 bytes per lane, so a global
 // store instruction writes whole 128-byte lines.  Tile (i, j) of the wave is AccTile<j * TM + i>.
-// EDGE: rows >= M and 8-column pieces at or beyond N (N % 8 == 0) are not stored.
+// EDGE: rows >= M and columns >= N are not stored.
 template <class Cfg, bool EDGE = false>
 __device__ __forceinline__ void store_chained_tile(unsigned char *lds, half_t *__restrict__ C, int M, int N, int row0,
                                                 int col0, int wave, int lane) {
@@ -106,8 +106,11 @@ __device__ __forceinline__ void store_chained_tile(unsigned char *lds, half_t *_
         for (int it = 0; it < READS; ++it) {
             if (EXACT || (rd_row < ROWS_PER_READ && it * ROWS_PER_READ + rd_row < MI)) {
                 const u32x4 v = *reinterpret_cast<const u32x4 *>(rd + it * ROWS_PER_READ * STRIP_ROW_BYTES);
-                if (!EDGE || (row0 + rd_row + i * MI + it * ROWS_PER_READ < M && col0 + rd_col * 8 < N))
-                    store_streaming(reinterpret_cast<u32x4 *>(cp + (size_t)(i * MI + it * ROWS_PER_READ) * N), v);
+                half_t *dst = cp + (size_t)(i * MI + it * ROWS_PER_READ) * N;
+                if constexpr (!EDGE)
+                    store_streaming(reinterpret_cast<u32x4 *>(dst), v);
+                else if (row0 + rd_row + i * MI + it * ROWS_PER_READ < M)
+                    store_piece_edge(dst, v, col0 + rd_col * 8, N);
             }
         }
         wave_lds_exchange_point();
@@ -258,8 +261,10 @@ __global__ void __launch_bounds__(Cfg::THREADS)
             dma_load16_sv<(d - B_DMA) * Cfg::WAVES * 1024>(a_src, voff[d - B_DMA], dst_a);
     };
     const int last_chunk = num_k - 1;
-    auto a_chunk = [&](int c) { return a_base + (c < last_chunk ? c : last_chunk) * (BK * 2); };
-    auto b_chunk = [&](int c) { return b_base + (c < last_chunk ? c : last_chunk) * (BK * 2); };
+    const uint32_t last_off = frame.last_off;
+    auto clamped = [&](int c) { return (uint32_t)c * (uint32_t)(BK * 2) < last_off ? (uint32_t)c * (uint32_t)(BK * 2) : last_off; };
+    auto a_chunk = [&](int c) { return a_base + clamped(c); };
+    auto b_chunk = [&](int c) { return b_base + clamped(c); };
 
     // ---- prologue: A(0 .. SA-1) and B(0 .. SB-2) in that interleaved order; B(SB-1) and A(SA)
     // belong to the window before iteration 0.
@@ -300,8 +305,6 @@ __global__ void __launch_bounds__(Cfg::THREADS)
 
     // Sources of the copies, kept as byte offsets of K chunks so that "the last chunk again" is
     // one s_min: A(kt+SA) / B(kt-1+SB) finish window kt-1, A(kt+1+SA) / B(kt+SB) start window kt.
-    const uint32_t last_off = (uint32_t)last_chunk * (BK * 2);
-    auto clamped = [&](int c) { return (uint32_t)(c < last_chunk ? c : last_chunk) * (uint32_t)(BK * 2); };
     uint32_t a_off_far = clamped(SA), b_off_far = clamped(SB - 1);  // furthest chunk with a pointer so far
     const unsigned char *a_pre = a_base + a_off_far, *b_pre = b_base + b_off_far, *a_post = a_pre, *b_post = b_pre;
 
@@ -317,6 +320,15 @@ __global__ void __launch_bounds__(Cfg::THREADS)
         const uint32_t pre_dst_a = cp_lds + CUR_A * A_BYTES, pre_dst_b = cp_lds + B_REGION + PRV_B * B_BYTES;
         const uint32_t post_dst_a = cp_lds + NXT_A * A_BYTES, post_dst_b = cp_lds + B_REGION + CUR_B * B_BYTES;
         const uint32_t src_a_next = NXT_A * A_BYTES, src_b_cur = CUR_B * B_BYTES, src_b_next = NXT_B * B_BYTES;
+        if constexpr (EDGE && FINAL) {  // all A fragments of the last chunk and its first column's B fragments have landed
+            if (frame.tail_dup > 0) {
+                static_for<KSTEPS>([&](auto kk_c) {
+                    static_for<TM>([&](auto t) { frame.drop_counted(a_frag[AB][decltype(kk_c)::value][decltype(t)::value], kk_c); });
+                    frame.drop_counted(b_frag[0][decltype(kk_c)::value], kk_c);
+                });
+                frame.dropped();
+            }
+        }
         static_for<TN>([&](auto j_c) {
             constexpr int j = decltype(j_c)::value;
             constexpr bool last = (j + 1 == TN);
@@ -381,6 +393,12 @@ __global__ void __launch_bounds__(Cfg::THREADS)
                     __builtin_amdgcn_s_waitcnt((0x3f & 0xf) | ((0x3f >> 4) << 14) | (0x7 << 4) | (n_a << 8));
                 }
                 static_for<KSTEPS>([&](auto kk_c) { lds_landed(b_frag[(j + 1) & 1][decltype(kk_c)::value]); });
+                if constexpr (EDGE && FINAL) {
+                    if (frame.tail_dup > 0) {
+                        static_for<KSTEPS>([&](auto kk_c) { frame.drop_counted(b_frag[(j + 1) & 1][decltype(kk_c)::value], kk_c); });
+                        frame.dropped();
+                    }
+                }
             }
             if constexpr (j == TN - 2 && !FINAL) {
                 static_for<KSTEPS>([&](auto kk_c) {
@@ -442,9 +460,11 @@ __global__ void __launch_bounds__(Cfg::THREADS)
             store_wave_tile_f32<Cfg, false>(get, lds, partial + ((size_t)slice * tail_tiles + slot) * (BM * BN) +
                                                           (size_t)(wm * Cfg::WM) * BN + wn * Cfg::WN,
                                             BN, BM, BN, wave, lane_late);
-        else
-            store_wave_tile_f32<Cfg, EDGE>(get, lds, partial + ((size_t)slice * M + row0) * N + col0, N, M - row0,
-                                           N - col0, wave, lane_late);
+        else {
+            const int ld = EDGE ? (int)partial_ld(N) : N;
+            store_wave_tile_f32<Cfg, EDGE>(get, lds, partial + ((size_t)slice * M + row0) * ld + col0, ld, M - row0,
+                                           ld - col0, wave, lane_late);
+        }
     } else {
         (void)partial;
         __syncthreads();

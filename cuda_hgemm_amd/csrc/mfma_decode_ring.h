@@ -46,7 +46,10 @@ struct RingConfig {
 
 // STREAM_B: B's copies carry the non-temporal hint (every byte of B is read once; the launcher sets it from 48 MB of B on,
 // the threshold the split-K kernel uses for the same hint).
-template <int TM, int STAGES, bool STREAM_B = false>
+// EDGE: N ends anywhere inside a workgroup's 16 columns (rows of B beyond the last are copied from it, columns beyond N
+// are not stored), K % 8 == 0 is dealt to the waves in whole chunks that need not come out even, the last one treated as
+// `tail_pieces` says.
+template <int TM, int STAGES, bool STREAM_B = false, bool EDGE = false>
 __global__ void __launch_bounds__(RING_MAX_WAVES * 64)
     hgemm_decode_ring_kernel(const half_t *__restrict__ A, const half_t *__restrict__ B, half_t *__restrict__ C, int M,
                              int N, int K, int k_per_wave) {
@@ -57,7 +60,13 @@ __global__ void __launch_bounds__(RING_MAX_WAVES * 64)
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), waves = blockDim.x >> 6;
     const int n0 = blockIdx.x * 16;
-    const int k_begin = wave * k_per_wave;
+    int k_begin = wave * k_per_wave, num_k = k_per_wave / 64;
+    if constexpr (EDGE) {
+        slice_of_k((K + 63) / 64, waves, wave, k_begin, num_k);
+        k_begin *= 64;
+    }
+    const int tail_dup = EDGE && wave == waves - 1 ? tail_pieces(K, 64) : 0;
+    const int last_koff = (num_k - 1) * 64 - tail_dup * 8;  // where the wave's last chunk is read from, relative to k_begin
 
     // ---- copies: lane l of instruction h fetches piece (l % 8) ^ swizzle of row 8h + l / 8; rows of A beyond M are
     // redirected to row M-1 and never stored
@@ -69,19 +78,23 @@ __global__ void __launch_bounds__(RING_MAX_WAVES * 64)
         const int piece = copy_pos ^ ((r >> 1) & 7);
         const int m = r < M ? r : M - 1;
         a_src[h] = A + (size_t)m * K + k_begin + piece * 8;
-        if (h < 2) b_src[h] = B + (size_t)(n0 + r) * K + k_begin + piece * 8;
+        if (h < 2) {
+            const int n = EDGE && n0 + r >= N ? N - 1 : n0 + r;
+            b_src[h] = B + (size_t)n * K + k_begin + piece * 8;
+        }
     }
     const uint32_t ring_addr = (uint32_t)(uintptr_t)lds + wave * RING_BYTES;
     auto fetch = [&](int kt, int slot) {
         const uint32_t base = ring_addr + slot * RING_CHUNK_BYTES;
+        const int koff = EDGE && kt == num_k - 1 ? last_koff : kt * 64;
 #pragma unroll
-        for (int h = 0; h < 2 * TM; ++h) dma_load16(a_src[h] + kt * 64, base + h * 1024);
+        for (int h = 0; h < 2 * TM; ++h) dma_load16(a_src[h] + koff, base + h * 1024);
         if constexpr (STREAM_B) {
-            dma_load16_streaming(b_src[0] + kt * 64, base + A_BYTES);
-            dma_load16_streaming(b_src[1] + kt * 64, base + A_BYTES + 1024);
+            dma_load16_streaming(b_src[0] + koff, base + A_BYTES);
+            dma_load16_streaming(b_src[1] + koff, base + A_BYTES + 1024);
         } else {
-            dma_load16(b_src[0] + kt * 64, base + A_BYTES);
-            dma_load16(b_src[1] + kt * 64, base + A_BYTES + 1024);
+            dma_load16(b_src[0] + koff, base + A_BYTES);
+            dma_load16(b_src[1] + koff, base + A_BYTES + 1024);
         }
     };
 
@@ -94,7 +107,6 @@ __global__ void __launch_bounds__(RING_MAX_WAVES * 64)
     floatx4 acc[TM];
 #pragma unroll
     for (int i = 0; i < TM; ++i) acc[i] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
-    const int num_k = k_per_wave / 64;
 #pragma unroll
     for (int s = 0; s < STAGES - 1; ++s)
         if (s < num_k) fetch(s, s);
@@ -112,12 +124,23 @@ __global__ void __launch_bounds__(RING_MAX_WAVES * 64)
             a0[i] = *reinterpret_cast<const half8 *>(chunk + i * 2048 + step0);
             a1[i] = *reinterpret_cast<const half8 *>(chunk + i * 2048 + step1);
         }
-        const half8 b0 = *reinterpret_cast<const half8 *>(chunk + A_BYTES + step0);
-        const half8 b1 = *reinterpret_cast<const half8 *>(chunk + A_BYTES + step1);
+        half8 b0 = *reinterpret_cast<const half8 *>(chunk + A_BYTES + step0);
+        half8 b1 = *reinterpret_cast<const half8 *>(chunk + A_BYTES + step1);
         // the slot refilled next is the one read in the previous iteration; with this iteration's reads returned too,
         // no read of this wave is outstanding when the copy is issued
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         if (kt + STAGES - 1 < num_k) fetch(kt + STAGES - 1, fill);
+        if constexpr (EDGE) {
+            if (tail_dup > 0 && kt == num_k - 1) {
+                b0 = keep_or_zero(b0, quarter >= tail_dup);
+                b1 = keep_or_zero(b1, 4 + quarter >= tail_dup);
+#pragma unroll
+                for (int i = 0; i < TM; ++i) {
+                    a0[i] = keep_or_zero(a0[i], quarter >= tail_dup);
+                    a1[i] = keep_or_zero(a1[i], 4 + quarter >= tail_dup);
+                }
+            }
+        }
 #pragma unroll
         for (int i = 0; i < TM; ++i) {
             acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(b0, a0[i], acc[i], 0, 0, 0);
@@ -143,13 +166,21 @@ __global__ void __launch_bounds__(RING_MAX_WAVES * 64)
         half4 v;
 #pragma unroll
         for (int r = 0; r < 4; ++r) v[r] = (half_t)s[r];
-        *reinterpret_cast<half4 *>(C + (size_t)m * N + n0 + c) = v;
+        if constexpr (EDGE)
+            store_quad_edge(C + (size_t)m * N + n0 + c, v, n0 + c, N);
+        else
+            *reinterpret_cast<half4 *>(C + (size_t)m * N + n0 + c) = v;
     }
 }
 
 // M <= 128, N a multiple of 16, K a multiple of 128 (two waves get whole 64-wide chunks).
 inline bool decode_ring_supports(size_t M, size_t N, size_t K) {
     return M >= 1 && M <= 128 && N > 0 && N % 16 == 0 && K > 0 && K % 128 == 0 && N <= ((size_t)1 << 31) / 16;
+}
+// what the EDGE form runs: any N, K a multiple of 8 and at least 256 (up to four waves with a chunk each, see
+// decode_ring_edge_waves; a wave whose only chunk is the last reads from K - 64 on)
+inline bool decode_ring_edge_supports(size_t M, size_t N, size_t K) {
+    return M >= 1 && M <= 128 && N > 0 && K >= 256 && K % 8 == 0;
 }
 
 inline int decode_ring_max_waves(size_t M);
@@ -166,21 +197,30 @@ inline int decode_ring_waves(size_t M, size_t N, size_t K, size_t cus) {
     return w;
 }
 
-template <int TM, int STAGES>
+// The same rule without its divisibility conditions: chunks are dealt to the waves as evenly as they go.
+inline int decode_ring_edge_waves(size_t M, size_t N, size_t K, size_t cus) {
+    if (M > 64) return div_ceil(N, (size_t)16) <= cus ? 2 : 1;
+    int w = 2;
+    while (w < decode_ring_max_waves(M) && K / (size_t)w > 1280) w *= 2;
+    if (w < 4 && div_ceil(N, (size_t)16) < 2 * cus) w = 4;
+    return w;
+}
+
+template <int TM, int STAGES, bool EDGE>
 void launch_decode_ring_tile(const void *A, const void *B, void *C, size_t M, size_t N, size_t K, int waves) {
     using Cfg = RingConfig<TM, STAGES>;
     HGEMM_CHECK((size_t)waves * Cfg::RING_BYTES <= 160 * 1024);
     static bool configured = [] {
-        HGEMM_CHECK_HIP_ERROR(hipFuncSetAttribute(reinterpret_cast<const void *>(&hgemm_decode_ring_kernel<TM, STAGES, false>),
+        HGEMM_CHECK_HIP_ERROR(hipFuncSetAttribute(reinterpret_cast<const void *>(&hgemm_decode_ring_kernel<TM, STAGES, false, EDGE>),
                                                   hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
-        HGEMM_CHECK_HIP_ERROR(hipFuncSetAttribute(reinterpret_cast<const void *>(&hgemm_decode_ring_kernel<TM, STAGES, true>),
+        HGEMM_CHECK_HIP_ERROR(hipFuncSetAttribute(reinterpret_cast<const void *>(&hgemm_decode_ring_kernel<TM, STAGES, true, EDGE>),
                                                   hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
         return true;
     }();
     (void)configured;
-    auto kernel = N * K >= ((size_t)24 << 20) ? &hgemm_decode_ring_kernel<TM, STAGES, true>
-                                              : &hgemm_decode_ring_kernel<TM, STAGES, false>;
-    kernel<<<dim3((unsigned)(N / 16)), dim3(waves * 64), (size_t)waves * Cfg::RING_BYTES, nullptr>>>(
+    auto kernel = N * K >= ((size_t)24 << 20) ? &hgemm_decode_ring_kernel<TM, STAGES, true, EDGE>
+                                              : &hgemm_decode_ring_kernel<TM, STAGES, false, EDGE>;
+    kernel<<<dim3((unsigned)div_ceil(N, (size_t)16)), dim3(waves * 64), (size_t)waves * Cfg::RING_BYTES, nullptr>>>(
         reinterpret_cast<const half_t *>(A), reinterpret_cast<const half_t *>(B), reinterpret_cast<half_t *>(C), (int)M,
         (int)N, (int)K, (int)(K / (size_t)waves));
     HGEMM_CHECK_HIP_ERROR(hipGetLastError());
@@ -190,19 +230,30 @@ void launch_decode_ring_tile(const void *A, const void *B, void *C, size_t M, si
 // 54 KB): up to eight, four, four and two waves fit the 160 KB of a CU.
 inline int decode_ring_max_waves(size_t M) { return M <= 16 ? RING_MAX_WAVES : M <= 64 ? 4 : 2; }
 
+template <bool EDGE>
+void launch_decode_ring_m(const void *A, const void *B, void *C, size_t M, size_t N, size_t K, int waves) {
+    if (M <= 16)
+        launch_decode_ring_tile<1, 4, EDGE>(A, B, C, M, N, K, waves);
+    else if (M <= 32)
+        launch_decode_ring_tile<2, 4, EDGE>(A, B, C, M, N, K, waves);
+    else if (M <= 64)
+        launch_decode_ring_tile<4, 3, EDGE>(A, B, C, M, N, K, waves);
+    else
+        launch_decode_ring_tile<8, 3, EDGE>(A, B, C, M, N, K, waves);
+}
+
 inline void launch_decode_ring(const void *A, const void *B, void *C, size_t M, size_t N, size_t K, int waves) {
     check_operands(A, B, C, M, N, K);
     HGEMM_CHECK_MSG(decode_ring_supports(M, N, K), "ring decode kernel needs M <= 128, N %% 16 == 0, K %% 128 == 0 (got M=%zu N=%zu K=%zu)",
                     M, N, K);
     HGEMM_CHECK(waves >= 1 && waves <= decode_ring_max_waves(M) && K % ((size_t)waves * 64) == 0);
-    if (M <= 16)
-        launch_decode_ring_tile<1, 4>(A, B, C, M, N, K, waves);
-    else if (M <= 32)
-        launch_decode_ring_tile<2, 4>(A, B, C, M, N, K, waves);
-    else if (M <= 64)
-        launch_decode_ring_tile<4, 3>(A, B, C, M, N, K, waves);
-    else
-        launch_decode_ring_tile<8, 3>(A, B, C, M, N, K, waves);
+    launch_decode_ring_m<false>(A, B, C, M, N, K, waves);
+}
+inline void launch_decode_ring_edge(const void *A, const void *B, void *C, size_t M, size_t N, size_t K, int waves) {
+    check_operands(A, B, C, M, N, K);
+    HGEMM_CHECK(decode_ring_edge_supports(M, N, K) && waves >= 1 && waves <= decode_ring_max_waves(M) &&
+                div_ceil(K, (size_t)64) >= (size_t)waves);
+    launch_decode_ring_m<true>(A, B, C, M, N, K, waves);
 }
 
 }  // namespace hgemm

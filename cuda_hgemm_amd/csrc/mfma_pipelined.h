@@ -197,7 +197,7 @@ __device__ __forceinline__ void dma_load16_sv(const void *sbase, uint32_t voff, 
 // holds groups of four consecutive n of one row m = lane % MI): each wave parks MI rows of
 // its tile in a private strip and reads them back row-contiguous, 16 bytes per lane, so a
 // global store instruction writes whole 128-byte lines.
-// EDGE: rows >= M and 8-column pieces at or beyond N (N % 8 == 0) are not stored.
+// EDGE: rows >= M and columns >= N are not stored.
 template <class Cfg, class Acc, bool EDGE = false>
 __device__ __forceinline__ void store_wave_tile(const Acc (&acc)[Cfg::PTM][Cfg::PTN], unsigned char *lds,
                                                 half_t *__restrict__ C, int M, int N, int row0, int col0, int wave,
@@ -232,8 +232,11 @@ __device__ __forceinline__ void store_wave_tile(const Acc (&acc)[Cfg::PTM][Cfg::
         for (int it = 0; it < READS; ++it) {
             if (EXACT || (rd_row < ROWS_PER_READ && it * ROWS_PER_READ + rd_row < MI)) {
                 const u32x4 v = *reinterpret_cast<const u32x4 *>(rd + it * ROWS_PER_READ * STRIP_ROW_BYTES);
-                if (!EDGE || (row0 + rd_row + i * MI + it * ROWS_PER_READ < M && col0 + rd_col * 8 < N))
-                    store_streaming(reinterpret_cast<u32x4 *>(cp + (size_t)(i * MI + it * ROWS_PER_READ) * N), v);
+                half_t *dst = cp + (size_t)(i * MI + it * ROWS_PER_READ) * N;
+                if constexpr (!EDGE)
+                    store_streaming(reinterpret_cast<u32x4 *>(dst), v);
+                else if (row0 + rd_row + i * MI + it * ROWS_PER_READ < M)
+                    store_piece_edge(dst, v, col0 + rd_col * 8, N);
             }
         }
         wave_lds_exchange_point();
@@ -284,9 +287,10 @@ __device__ __forceinline__ void store_wave_tile_f32(Get get, unsigned char *lds,
 // What both tuned kernels (interleaved below, chained in mfma_chained.h) set up before their loops: which tile
 // and K slice the workgroup computes, the per-lane global offsets of its direct-to-LDS copies, and the LDS
 // addresses its lanes read MFMA operands from.
-// EDGE: M and N need not be multiples of the tile (N % 8 == 0 still, for aligned rows of
-// C).  Copies of rows beyond the matrix are redirected to its last row -- valid memory,
-// products never stored -- which costs nothing inside the loop; only the stores are guarded.
+// EDGE: M and N end anywhere inside a tile, K % 8 == 0 anywhere inside a chunk.  Copies of rows
+// beyond the matrix are redirected to its last row -- valid memory, products never stored --
+// which costs nothing inside the loop; only the stores are guarded.  The last chunk is treated
+// as `tail_pieces` says: one scalar minimum per chunk, and the masks in the last iteration.
 template <class Cfg, bool SPLIT, bool EDGE>
 struct PipeFrame {
     static constexpr int BM = Cfg::BM, BN = Cfg::BN, BK = Cfg::BK, MI = Cfg::MI;
@@ -305,6 +309,8 @@ struct PipeFrame {
     int tile_m, tile_n;      // the workgroup's tile (wave-uniform)
     int slot, slice;         // its position among the launch's tiles and, in a K-sliced launch, its slice
     int num_k;               // chunks it walks
+    int tail_dup;            // 16-byte pieces at the start of the last chunk that must not count (EDGE)
+    uint32_t last_off;       // byte offset of the last chunk from a_base / b_base
     const unsigned char *a_base, *b_base;  // first chunk of the tile's rows of A and of B
     uint32_t voff[L];        // per-lane byte offset of copy instruction i from a_base (i < A_DMA) or b_base
     uint32_t cp_lds;         // LDS address the wave's copy instruction 0 fills, without the ring-buffer offset
@@ -347,8 +353,11 @@ struct PipeFrame {
         tile_m = __builtin_amdgcn_readfirstlane(tile_m);  // wave-uniform by construction: keep them in SGPRs
         tile_n = __builtin_amdgcn_readfirstlane(tile_n);
         int first_chunk;
-        slice_of_k(K / BK, slices, slice, first_chunk, num_k);
+        const int chunks = EDGE ? (K + BK - 1) / BK : K / BK;
+        slice_of_k(chunks, slices, slice, first_chunk, num_k);
         const int k_begin = first_chunk * BK;
+        tail_dup = EDGE && first_chunk + num_k == chunks ? tail_pieces(K, BK) : 0;
+        last_off = (uint32_t)((num_k - 1) * (BK * 2) - tail_dup * 16);
 
         // ---- copies: wave w, instruction i fills LDS rows [(i*WAVES + w)*ROWS_PER_DMA, +ROWS_PER_DMA)
         a_base = reinterpret_cast<const unsigned char *>(A + (size_t)tile_m * BM * K + k_begin);
@@ -404,6 +413,20 @@ struct PipeFrame {
         constexpr int t = TC::value, kk = KC::value;
         return lds_read16<t * MI * ROW_BYTES>(b_addr[kk][ODD_FLIP ? (t & 1) : 0] + stage_bytes);
     }
+
+    // byte offset of chunk c from a_base / b_base
+    __device__ __forceinline__ uint32_t chunk_off(int c) const {
+        const uint32_t off = (uint32_t)c * (uint32_t)(BK * 2);
+        return EDGE && off > last_off ? last_off : off;
+    }
+    // clears what of a fragment of step kk of the last chunk must not count; a landed operand register, not one in flight
+    template <class KC>
+    __device__ __forceinline__ void drop_counted(half8 &f, KC) const {
+        f = keep_or_zero(f, (int)KC::value * CPS + lane / MI >= tail_dup);
+        lds_landed(f);  // the MFMAs are issued from assembly: keeps the selects in front of the wait states
+    }
+    // between the last of those selects and the first MFMA that reads one
+    static __device__ __forceinline__ void dropped() { asm volatile("s_nop 7" ::: "memory"); }
 };
 
 // STREAM_B: B's copies carry the non-temporal hint.  For one row of tiles against a B that outgrows the Infinity
@@ -541,7 +564,7 @@ __global__ void __launch_bounds__(Cfg::THREADS)
     static_for<AHEAD>([&](auto s_c) {
         constexpr int st = decltype(s_c)::value;
         static_for<L>([&](auto idx_c) {
-            dma_one(idx_c, a_base + st * BK * 2, b_base + st * BK * 2, cp_lds + st * A_BYTES,
+            dma_one(idx_c, a_base + frame.chunk_off(st), b_base + frame.chunk_off(st), cp_lds + st * A_BYTES,
                     cp_lds + B_REGION + st * B_BYTES);
         });
     });
@@ -556,6 +579,7 @@ __global__ void __launch_bounds__(Cfg::THREADS)
     wait_operands(std::integral_constant<int, 0>{});
 
     const unsigned char *a_next = a_base + AHEAD * BK * 2, *b_next = b_base + AHEAD * BK * 2;
+    uint32_t next_off = frame.chunk_off(AHEAD);  // EDGE: the same as an offset, so that the last chunk is one s_min away
     // One iteration = one K chunk.  ISSUE: chunk kt+AHEAD exists and is copied now.
     // NEXT: chunk kt+1 exists (the barrier is needed and its operands are prefetched).
     // cur_a / cur_b (ring buffers holding chunk kt) are plain ints or, in the unrolled steady
@@ -566,16 +590,25 @@ __global__ void __launch_bounds__(Cfg::THREADS)
         const int nxt_a = (cur_a + 1 == SA) ? 0 : cur_a + 1;
         const int nxt_b = (cur_b + 1 == SB) ? 0 : cur_b + 1;
         const int fill_a = (cur_a + FILL_OFF_A) % SA, fill_b = (cur_b + FILL_OFF_B) % SB;
-        const unsigned char *a_src = a_next, *b_src = b_next;  // chunk kt + AHEAD
+        const unsigned char *a_src = EDGE ? a_base + next_off : a_next, *b_src = EDGE ? b_base + next_off : b_next;  // chunk kt + AHEAD
         if constexpr (ISSUE) {
             a_next += BK * 2;
             b_next += BK * 2;
+            if constexpr (EDGE) next_off = next_off + BK * 2 < frame.last_off ? next_off + BK * 2 : frame.last_off;
         }
         const uint32_t dst_a = cp_lds + fill_a * A_BYTES, dst_b = cp_lds + B_REGION + fill_b * B_BYTES;
         static_for<KSTEPS>([&](auto kk_c) {
             constexpr int kk = decltype(kk_c)::value;
             constexpr int fb = kk & 1, nb = fb ^ 1;  // an even number of steps: step 0 always uses buffer 0
             constexpr bool last = (kk + 1 == KSTEPS);
+            if constexpr (EDGE && !NEXT) {  // the last chunk: its operands of this step have landed
+                if (frame.tail_dup > 0) {
+                    static_for<TM>([&](auto t) { frame.drop_counted(a_frag[fb][decltype(t)::value], kk_c); });
+                    static_for<NSB>([&](auto t) { frame.drop_counted(b_frag[decltype(t)::value], kk_c); });
+                    static_for<NDB>([&](auto t) { frame.drop_counted(b_last[fb][decltype(t)::value], kk_c); });
+                    frame.dropped();
+                }
+            }
             if constexpr (last && NEXT) {
                 if constexpr (ISSUE)
                     wait_vmcnt<STEADY_VMCNT>();
@@ -665,9 +698,11 @@ __global__ void __launch_bounds__(Cfg::THREADS)
             store_wave_tile_f32<Cfg, false>(get, lds, partial + ((size_t)slice * tail_tiles + slot) * (BM * BN) +
                                                           (size_t)(wm * Cfg::WM) * BN + wn * Cfg::WN,
                                             BN, BM, BN, wave, lane);
-        else
-            store_wave_tile_f32<Cfg, EDGE>(get, lds, partial + ((size_t)slice * M + row0) * N + col0, N, M - row0,
-                                           N - col0, wave, lane);
+        else {
+            const int ld = EDGE ? (int)partial_ld(N) : N;
+            store_wave_tile_f32<Cfg, EDGE>(get, lds, partial + ((size_t)slice * M + row0) * ld + col0, ld, M - row0,
+                                           ld - col0, wave, lane);
+        }
     } else {
         (void)partial;
         __syncthreads();
@@ -676,15 +711,20 @@ __global__ void __launch_bounds__(Cfg::THREADS)
     }
 }
 
-// Shapes a pipelined kernel accepts with guarded edges: any M, N a multiple of 8 (rows of C
-// stay 16-byte aligned), K a whole number of chunks and at least the ring depth.
+// Shapes the named entry points accept: any M, N a multiple of 8, K a whole number of chunks and at least the ring depth.
 template <class Cfg>
 bool pipelined_supports_edges(size_t M, size_t N, size_t K) {
     return M > 0 && N > 0 && N % 8 == 0 && K % Cfg::BK == 0 && K >= (size_t)Cfg::BK * Cfg::STAGES;
 }
+// Shapes the kernel runs: M and N end anywhere, K a multiple of 8 (rows of A and B start on 16-byte boundaries) with at
+// least as many chunks, the last one counted in full, as the ring is deep.
+template <class Cfg>
+bool pipelined_runs(size_t M, size_t N, size_t K) {
+    return M > 0 && N > 0 && K % 8 == 0 && div_ceil(K, (size_t)Cfg::BK) >= (size_t)Cfg::STAGES;
+}
 
 // C[tile of workgroup id first_block + t] = fp16(sum over slices of partial[slice][t][BM][BN]),
-// slices added in order; rows and 8-column pieces outside the matrix are skipped.
+// slices added in order; rows and columns outside the matrix are skipped.
 template <class Cfg>
 __global__ void __launch_bounds__(256)
     tail_reduce_kernel(const float *__restrict__ partial, half_t *__restrict__ C, int M, int N, int K, int tiles_m,
@@ -711,7 +751,10 @@ __global__ void __launch_bounds__(256)
             v[e] = (half_t)s0[e];
             v[4 + e] = (half_t)s1[e];
         }
-        store_streaming(reinterpret_cast<half8 *>(C + (size_t)row * N + col), v);
+        if ((N & 7) == 0)
+            store_streaming(reinterpret_cast<half8 *>(C + (size_t)row * N + col), v);
+        else
+            store_piece_edge(C + (size_t)row * N + col, __builtin_bit_cast(u32x4, v), col, N);
     }
 }
 
@@ -817,10 +860,10 @@ void launch_pipelined_with_tail(const void *A, const void *B, void *C, float *pa
     check_operands(A, B, C, M, N, K);
     const int tiles_m = (int)div_ceil(M, (size_t)Cfg::BM), tiles_n = (int)div_ceil(N, (size_t)Cfg::BN);
     const int total = tiles_m * tiles_n, head = total - tail_tiles;
-    HGEMM_CHECK(partial != nullptr && tail_tiles >= 1 && head >= 1 && tail_splits >= 2 && K % (size_t)Cfg::BK == 0);
-    HGEMM_CHECK_MSG(pipelined_supports_edges<Cfg>(M, N, shortest_slice(K, Cfg::BK, tail_splits)),
-                    "%s (tail in %d K slices) needs N %% 8 == 0, K %% %d == 0, shortest slice >= %d (got M=%zu N=%zu K=%zu)",
-                    name, tail_splits, Cfg::BK, Cfg::BK * Cfg::STAGES, M, N, K);
+    HGEMM_CHECK(partial != nullptr && tail_tiles >= 1 && head >= 1 && tail_splits >= 2);
+    HGEMM_CHECK_MSG(K % 8 == 0 && pipelined_runs<Cfg>(M, N, shortest_slice(K, Cfg::BK, tail_splits)),
+                    "%s (tail in %d K slices) needs K %% 8 == 0, shortest slice >= %d (got M=%zu N=%zu K=%zu)",
+                    name, tail_splits, Cfg::BK * Cfg::STAGES, M, N, K);
     if (Cfg::supports(M, N, K)) {
         launch_pipelined_impl<Cfg, false, false>(A, B, C, nullptr, M, N, K, 1, 0, head);
         launch_pipelined_impl<Cfg, true, false>(A, B, nullptr, partial, M, N, K, tail_splits, head, tail_tiles,
@@ -844,26 +887,25 @@ void launch_pipelined(const void *A, const void *B, void *C, size_t M, size_t N,
         launch_pipelined_impl<Cfg, false, false>(A, B, C, nullptr, M, N, K, 1, 0, -1, 0, which);
         return;
     }
-    HGEMM_CHECK_MSG(pipelined_supports_edges<Cfg>(M, N, K),
-                    "%s needs N %% 8 == 0, K %% %d == 0, K >= %d (got M=%zu N=%zu K=%zu)", name, Cfg::BK,
-                    Cfg::BK * Cfg::STAGES, M, N, K);
+    HGEMM_CHECK_MSG(pipelined_runs<Cfg>(M, N, K), "%s needs K %% 8 == 0, K > %d (got M=%zu N=%zu K=%zu)", name,
+                    Cfg::BK * (Cfg::STAGES - 1), M, N, K);
     launch_pipelined_impl<Cfg, false, true>(A, B, C, nullptr, M, N, K, 1, 0, -1, 0, which);
 }
 
-// K split into `splits` slices: fp32 partial sums of slice s go to partial[s][M][N] (the
-// caller provides splits * M * N floats and runs the reduction afterwards).
+// K split into `splits` slices: fp32 partial sums of slice s go to partial[s][M][partial_ld(N)] (the
+// caller provides that many floats and runs the reduction afterwards).
 template <class Cfg>
 void launch_pipelined_split(const void *A, const void *B, float *partial, size_t M, size_t N, size_t K, int splits,
                             const char *name) {
-    HGEMM_CHECK(splits >= 1 && K % (size_t)Cfg::BK == 0 && partial != nullptr);
+    HGEMM_CHECK(splits >= 1 && partial != nullptr);
     const size_t k_len = shortest_slice(K, Cfg::BK, splits);
-    if (k_len > 0 && Cfg::supports(M, N, k_len)) {
+    if (K % (size_t)Cfg::BK == 0 && k_len > 0 && Cfg::supports(M, N, k_len)) {
         launch_pipelined_impl<Cfg, true, false>(A, B, nullptr, partial, M, N, K, splits);
         return;
     }
-    HGEMM_CHECK_MSG(k_len > 0 && pipelined_supports_edges<Cfg>(M, N, k_len),
-                    "%s (K in %d slices) needs N %% 8 == 0, K %% %d == 0, shortest slice >= %d (got M=%zu N=%zu K=%zu)",
-                    name, splits, Cfg::BK, Cfg::BK * Cfg::STAGES, M, N, K);
+    HGEMM_CHECK_MSG(k_len > 0 && K % 8 == 0 && pipelined_runs<Cfg>(M, N, k_len),
+                    "%s (K in %d slices) needs K %% 8 == 0, shortest slice >= %d (got M=%zu N=%zu K=%zu)",
+                    name, splits, Cfg::BK * Cfg::STAGES, M, N, K);
     launch_pipelined_impl<Cfg, true, true>(A, B, nullptr, partial, M, N, K, splits);
 }
 
@@ -881,9 +923,9 @@ void launch_pipelined_with_subtiles(const void *A, const void *B, void *C, size_
     const int tiles_m = (int)div_ceil(M, (size_t)Parent::BM), tiles_n = (int)div_ceil(N, (size_t)Parent::BN);
     const int head = tiles_m * tiles_n - tail_tiles;
     HGEMM_CHECK(tail_tiles >= 1 && head >= 1);
-    HGEMM_CHECK_MSG(pipelined_supports_edges<Parent>(M, N, K) && pipelined_supports_edges<Child>(M, N, K),
-                    "%s needs N %% 8 == 0, K %% 64 == 0, K >= %d (got M=%zu N=%zu K=%zu)", name,
-                    64 * (Parent::STAGES > Child::STAGES ? Parent::STAGES : Child::STAGES), M, N, K);
+    HGEMM_CHECK_MSG(pipelined_runs<Parent>(M, N, K) && pipelined_runs<Child>(M, N, K),
+                    "%s needs K %% 8 == 0, K > %d (got M=%zu N=%zu K=%zu)", name,
+                    64 * ((Parent::STAGES > Child::STAGES ? Parent::STAGES : Child::STAGES) - 1), M, N, K);
     if (Parent::supports(M, N, K))
         launch_pipelined_impl<Parent, false, false>(A, B, C, nullptr, M, N, K, 1, 0, head);
     else

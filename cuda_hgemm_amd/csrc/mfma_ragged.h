@@ -1,4 +1,5 @@
-// MFMA kernel for shapes nothing else tiles: any M, N, K >= 1.
+// MFMA kernel for shapes nothing else runs: any M, N, K >= 1.  (hgemm_auto comes here for K that is no multiple of 8 and
+// below 192, for K below 64, and where device memory for aligned copies cannot be had.)
 //
 // 128x128x32 tile, 4 waves (2x2), 64x64 wave tiles on v_mfma_f32_32x32x16_f16, operands
 // staged global -> registers -> LDS so that every element can be guarded: rows beyond the

@@ -25,7 +25,9 @@ struct SkinnyConfig : TileConfig<BM_, BN_, 64, WAVES_M_, WAVES_N_, STAGES_, LOAD
 // STREAM_B: B is copied with the non-temporal hint.  Every byte of B is read once; when B is larger than the
 // Infinity Cache keeps (N = 28672, K = 4096: 235 MB) the hint is worth 11-12 % (M = 16 ... 64: 64.5 -> 72.6 %, 63.6 ->
 // 70.5 %, 57.6 -> 64.7 % of 8 TB/s), when B fits (N = K = 4096) it costs up to 7 %, so the launcher decides by size.
-template <class Cfg, bool STREAM_B = false>
+// EDGE: N ends anywhere inside a tile and K % 8 == 0 anywhere inside a chunk: rows of B beyond the last are copied from
+// it, columns beyond N are not stored, the last chunk is treated as `tail_pieces` says.
+template <class Cfg, bool STREAM_B = false, bool EDGE = false>
 __global__ void __launch_bounds__(Cfg::THREADS)
     hgemm_skinny_kernel(const half_t *__restrict__ A, const half_t *__restrict__ B, half_t *__restrict__ C,
                         float *__restrict__ partial, int M, int N, int K, int splits, int tiles_n) {
@@ -45,8 +47,11 @@ __global__ void __launch_bounds__(Cfg::THREADS)
     const int tile_n = (int)blockIdx.x % tiles_n, tile_m = (int)blockIdx.x / tiles_n, split = blockIdx.y;
     const int m0 = tile_m * BM;
     int first_chunk, num_k;  // K's chunks are dealt to the slices as evenly as whole chunks allow
-    slice_of_k(K / BK, splits, split, first_chunk, num_k);
+    const int chunks = EDGE ? (K + BK - 1) / BK : K / BK;
+    slice_of_k(chunks, splits, split, first_chunk, num_k);
     const int k_begin = first_chunk * BK;
+    const int tail_dup = EDGE && first_chunk + num_k == chunks ? tail_pieces(K, BK) : 0;
+    const int last_koff = (num_k - 1) * BK - tail_dup * 8;  // where the last chunk is read from, relative to k_begin
 
     // ---- copy set-up (rows of A clamped to the last valid row)
     constexpr int DMA_ROW_STEP = Cfg::WAVES * Cfg::ROWS_PER_DMA;
@@ -61,12 +66,15 @@ __global__ void __launch_bounds__(Cfg::THREADS)
         a_src[it] = A + (size_t)r * K + k_begin + cp_ch * 8;
     }
 #pragma unroll
-    for (int it = 0; it < Cfg::B_DMA; ++it)
-        b_src[it] = B + (size_t)(tile_n * BN + cp_row + it * DMA_ROW_STEP) * K + k_begin + cp_ch * 8;
+    for (int it = 0; it < Cfg::B_DMA; ++it) {
+        int r = tile_n * BN + cp_row + it * DMA_ROW_STEP;
+        if constexpr (EDGE) r = r < N ? r : N - 1;
+        b_src[it] = B + (size_t)r * K + k_begin + cp_ch * 8;
+    }
     const uint32_t cp_lds = (uint32_t)(uintptr_t)lds + wave * 1024;
 
     auto dma_fetch = [&](int kt, int stage) {
-        const int koff = kt * BK;
+        const int koff = EDGE && kt == num_k - 1 ? last_koff : kt * BK;
         const uint32_t base = cp_lds + stage * Cfg::STAGE_BYTES;
 #pragma unroll
         for (int it = 0; it < Cfg::A_DMA; ++it) dma_load16(a_src[it] + koff, base + it * Cfg::WAVES * 1024);
@@ -92,7 +100,8 @@ __global__ void __launch_bounds__(Cfg::THREADS)
 #pragma unroll
             for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
 
-    auto compute_stage = [&](int stage) {
+    // drop: 16-byte pieces at the start of the chunk that must not count (EDGE, last chunk)
+    auto compute_stage = [&](int stage, int drop) {
         const unsigned char *s = lds + stage * Cfg::STAGE_BYTES;
 #pragma unroll
         for (int kk = 0; kk < KSTEPS; ++kk) {
@@ -104,6 +113,15 @@ __global__ void __launch_bounds__(Cfg::THREADS)
 #pragma unroll
             for (int j = 0; j < TN; ++j)
                 bf[j] = *reinterpret_cast<const half8 *>(s + b_frag_off + j * 32 * ROW_BYTES + chunk);
+            if constexpr (EDGE) {
+                if (drop > 0) {
+                    const bool keep = kk * 2 + (lane >> 5) >= drop;
+#pragma unroll
+                    for (int i = 0; i < TM; ++i) af[i] = keep_or_zero(af[i], keep);
+#pragma unroll
+                    for (int j = 0; j < TN; ++j) bf[j] = keep_or_zero(bf[j], keep);
+                }
+            }
 #pragma unroll
             for (int i = 0; i < TM; ++i)
 #pragma unroll
@@ -124,7 +142,7 @@ __global__ void __launch_bounds__(Cfg::THREADS)
             wait_vmcnt<0>();
         __syncthreads();
         if (kt + STAGES - 1 < num_k) dma_fetch(kt + STAGES - 1, fill);
-        compute_stage(cur);
+        compute_stage(cur, kt == num_k - 1 ? tail_dup : 0);
         cur = (cur + 1 == STAGES) ? 0 : cur + 1;
         fill = (fill + 1 == STAGES) ? 0 : fill + 1;
     }
@@ -133,6 +151,7 @@ __global__ void __launch_bounds__(Cfg::THREADS)
     // register group: 8 bytes of fp16, or 16 bytes of an fp32 partial sum.
     const int row_in_wave = lane & 31;
     const int col_in_tile = (lane >> 5) << 2;
+    const size_t ld = EDGE ? partial_ld(N) : (size_t)N;
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
         const int m = m0 + wm * Cfg::WM + i * 32 + row_in_wave;
@@ -146,12 +165,16 @@ __global__ void __launch_bounds__(Cfg::THREADS)
                     floatx4 v;
 #pragma unroll
                     for (int r = 0; r < 4; ++r) v[r] = acc[i][j][g * 4 + r];
-                    *reinterpret_cast<floatx4 *>(partial + ((size_t)split * M + m) * N + n + g * 8) = v;
+                    if (!EDGE || (size_t)(n + g * 8) < ld)
+                        *reinterpret_cast<floatx4 *>(partial + ((size_t)split * M + m) * ld + n + g * 8) = v;
                 } else {
                     half4 v;
 #pragma unroll
                     for (int r = 0; r < 4; ++r) v[r] = (half_t)acc[i][j][g * 4 + r];
-                    *reinterpret_cast<half4 *>(C + (size_t)m * N + n + g * 8) = v;
+                    if constexpr (EDGE)
+                        store_quad_edge(C + (size_t)m * N + n + g * 8, v, n + g * 8, N);
+                    else
+                        *reinterpret_cast<half4 *>(C + (size_t)m * N + n + g * 8) = v;
                 }
             }
         }
@@ -162,9 +185,11 @@ __global__ void __launch_bounds__(Cfg::THREADS)
 // outputs per thread.  The loads of four slices are issued together before their adds, so
 // the kernel is not one memory round trip per slice; small outputs use a small VEC so the
 // reduction still spreads over the chip.
-template <int VEC>
+// EDGE: N is no multiple of 8: rows of the partial sums are partial_ld(N) apart (`elems` counts them so), rows of C
+// start anywhere.
+template <int VEC, bool EDGE = false>
 __global__ void __launch_bounds__(256)
-    splitk_reduce_kernel(const float *__restrict__ partial, half_t *__restrict__ C, size_t elems, int splits) {
+    splitk_reduce_kernel(const float *__restrict__ partial, half_t *__restrict__ C, size_t elems, int splits, int N) {
     typedef float vec_t __attribute__((ext_vector_type(VEC)));
     typedef half_t hvec_t __attribute__((ext_vector_type(VEC)));
     const size_t i = ((size_t)blockIdx.x * blockDim.x + threadIdx.x) * VEC;
@@ -186,21 +211,45 @@ __global__ void __launch_bounds__(256)
     hvec_t out;
 #pragma unroll
     for (int r = 0; r < VEC; ++r) out[r] = (half_t)acc[r];
-    store_streaming(reinterpret_cast<hvec_t *>(C + i), out);
+    if constexpr (EDGE) {
+        // 32 bits hold the index: the launcher checks
+        const uint32_t ld = (uint32_t)partial_ld(N), row = (uint32_t)i / ld;
+        const int col = (int)((uint32_t)i - row * ld);
+        half_t *dst = C + (size_t)row * N + col;
+        typedef hvec_t hvec_any __attribute__((aligned(2)));
+        if (col + VEC <= N) {
+            *reinterpret_cast<hvec_any *>(dst) = out;
+        } else {
+#pragma unroll
+            for (int r = 0; r < VEC; ++r)
+                if (col + r < N) dst[r] = out[r];
+        }
+    } else {
+        (void)N;
+        store_streaming(reinterpret_cast<hvec_t *>(C + i), out);
+    }
 }
 
-// elems must be a multiple of 8 (every tile dimension is).
-inline void launch_splitk_reduce(const float *partial, half_t *C, size_t elems, int splits) {
-    if (elems >= (size_t)2 << 20)
-        splitk_reduce_kernel<8><<<dim3((unsigned)div_ceil(elems / 8, 256)), dim3(256), 0, nullptr>>>(partial, C, elems,
-                                                                                                    splits);
-    else if (elems >= (size_t)512 << 10)
-        splitk_reduce_kernel<4><<<dim3((unsigned)div_ceil(elems / 4, 256)), dim3(256), 0, nullptr>>>(partial, C, elems,
-                                                                                                    splits);
+template <int VEC>
+void launch_splitk_reduce_vec(const float *partial, half_t *C, size_t M, size_t N, int splits) {
+    const size_t elems = M * partial_ld(N);
+    const dim3 grid((unsigned)div_ceil(elems / VEC, 256)), block(256);
+    if (N % 8 == 0)
+        splitk_reduce_kernel<VEC, false><<<grid, block, 0, nullptr>>>(partial, C, elems, splits, (int)N);
     else
-        splitk_reduce_kernel<2><<<dim3((unsigned)div_ceil(elems / 2, 256)), dim3(256), 0, nullptr>>>(partial, C, elems,
-                                                                                                    splits);
+        splitk_reduce_kernel<VEC, true><<<grid, block, 0, nullptr>>>(partial, C, elems, splits, (int)N);
     HGEMM_CHECK_HIP_ERROR(hipGetLastError());
+}
+// partial: [splits][M][partial_ld(N)]
+inline void launch_splitk_reduce(const float *partial, half_t *C, size_t M, size_t N, int splits) {
+    const size_t elems = M * partial_ld(N);
+    HGEMM_CHECK(elems < ((size_t)1 << 32));
+    if (elems >= (size_t)2 << 20)
+        launch_splitk_reduce_vec<8>(partial, C, M, N, splits);
+    else if (elems >= (size_t)512 << 10)
+        launch_splitk_reduce_vec<4>(partial, C, M, N, splits);
+    else
+        launch_splitk_reduce_vec<2>(partial, C, M, N, splits);
 }
 
 }  // namespace hgemm

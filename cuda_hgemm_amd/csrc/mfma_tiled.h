@@ -95,8 +95,26 @@ __host__ __device__ __forceinline__ void slice_of_k(int chunks, int slices, int 
     first = slice * base + (slice < longer ? slice : longer);
     count = base + (slice < longer ? 1 : 0);
 }
-// the length of the shortest of `splits` such slices of K (chunks of `bk`), which is what a kernel's minimum K applies to
-inline size_t shortest_slice(size_t K, int bk, int splits) { return K / (size_t)bk / (size_t)splits * (size_t)bk; }
+// the length of the shortest of `splits` such slices of K (chunks of `bk`, the last one perhaps not full), in whole
+// chunks: what a kernel's minimum K applies to
+inline size_t shortest_slice(size_t K, int bk, int splits) { return div_ceil(K, (size_t)bk) / (size_t)splits * (size_t)bk; }
+
+// ---- K that ends inside a chunk (K % 8 == 0, so rows still start on 16-byte boundaries).  The last chunk is read from
+// K - 64 on instead of from its own beginning: every copy stays inside the matrix and as aligned as the others, and
+// only a wave-uniform base address changes.  The chunk then starts with `tail_dup` 16-byte pieces that the chunk
+// before it has already multiplied; both operands' registers of those pieces are cleared before the last chunk's MFMAs
+// (both, because a product of a cleared and an infinite element would be NaN).  Padding the operands instead cost two
+// launches and 4 (M + N) K bytes: 1000^3 16.4 -> 7.8 us.
+__device__ __forceinline__ int tail_pieces(int K, int bk) { return ((K + bk - 1) / bk * bk - K) >> 3; }
+__device__ __forceinline__ half8 keep_or_zero(half8 v, bool keep) {
+    u32x4 bits = __builtin_bit_cast(u32x4, v);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) bits[r] = keep ? bits[r] : 0u;
+    return __builtin_bit_cast(half8, bits);
+}
+
+// Columns of the fp32 partial sums of one K slice: N rounded up so that rows start on 16-byte boundaries whatever N is.
+__host__ __device__ __forceinline__ size_t partial_ld(size_t N) { return (N + 7) / 8 * 8; }
 
 // s_waitcnt vmcnt(n) only (expcnt / lgkmcnt left at "do not wait"); gfx9 encoding.
 template <int N>
@@ -167,6 +185,32 @@ __device__ __forceinline__ void store_streaming(T *dst, const T &value) {
     __builtin_nontemporal_store(value, dst);
 }
 
+// Eight halves (or what of them lies left of column N) of a row of C whose rows start anywhere: 16-byte stores need no
+// more than the element's own alignment on this part.
+typedef u32x4 u32x4_any __attribute__((aligned(2)));
+__device__ __forceinline__ void store_piece_edge(half_t *dst, const u32x4 &value, int col, int N) {
+    if (col + 8 <= N) {
+        __builtin_nontemporal_store((u32x4_any)value, reinterpret_cast<u32x4_any *>(dst));
+    } else if (col < N) {
+        const half8 v = __builtin_bit_cast(half8, value);
+#pragma unroll
+        for (int e = 0; e < 7; ++e)
+            if (col + e < N) dst[e] = v[e];
+    }
+}
+
+// The same for four halves.
+__device__ __forceinline__ void store_quad_edge(half_t *dst, const half4 &v, int col, int N) {
+    typedef half4 half4_any __attribute__((aligned(2)));
+    if (col + 4 <= N) {
+        *reinterpret_cast<half4_any *>(dst) = v;
+    } else {
+#pragma unroll
+        for (int r = 0; r < 3; ++r)
+            if (col + r < N) dst[r] = v[r];
+    }
+}
+
 // Epilogue shared by the tiled kernels: accumulators -> fp16 -> C, staged through LDS.
 // A lane of the (operand-swapped) accumulator holds four consecutive n of one row; stored
 // straight to global memory that is 16 useful bytes per 32 rows per instruction, i.e. a
@@ -175,9 +219,10 @@ __device__ __forceinline__ void store_streaming(T *dst, const T &value) {
 // every global store instruction writes whole 128-byte lines, 16 bytes per lane.
 // The caller must have passed a workgroup barrier after the last operand read, because
 // the strips reuse the operand buffers.
-template <class Cfg>
+// EDGE: rows and columns beyond M and N are not stored.
+template <class Cfg, bool EDGE = false>
 __device__ __forceinline__ void store_tile_via_lds(const floatx16 (&acc)[Cfg::TM][Cfg::TN], unsigned char *lds,
-                                                   half_t *__restrict__ C, int N, int row0, int col0, int wave,
+                                                   half_t *__restrict__ C, int M, int N, int row0, int col0, int wave,
                                                    int lane) {
     constexpr int TM = Cfg::TM, TN = Cfg::TN, WN = Cfg::WN;
     constexpr int STRIP_ROW_BYTES = WN * 2 + 16;
@@ -206,7 +251,11 @@ __device__ __forceinline__ void store_tile_via_lds(const floatx16 (&acc)[Cfg::TM
 #pragma unroll
         for (int it = 0; it < READS; ++it) {
             const u32x4 v = *reinterpret_cast<const u32x4 *>(rd + it * ROWS_PER_READ * STRIP_ROW_BYTES);
-            store_streaming(reinterpret_cast<u32x4 *>(cp + (size_t)(i * 32 + it * ROWS_PER_READ) * N), v);
+            half_t *dst = cp + (size_t)(i * 32 + it * ROWS_PER_READ) * N;
+            if constexpr (!EDGE)
+                store_streaming(reinterpret_cast<u32x4 *>(dst), v);
+            else if (row0 + rd_row + i * 32 + it * ROWS_PER_READ < M)
+                store_piece_edge(dst, v, col0 + rd_col * 8, N);
         }
         wave_lds_exchange_point();
     }
@@ -215,13 +264,16 @@ __device__ __forceinline__ void store_tile_via_lds(const floatx16 (&acc)[Cfg::TM
 // SPLIT: a one-dimensional launch of tiles x slices workgroups; each computes one K slice of one tile and leaves
 // fp32 partial sums in partial[slice][M][N] for the ordered reduction; otherwise slices == 1 and C is written.
 // The K / BK chunks are dealt to the slices as evenly as whole chunks allow (`slice_of_k`).
-template <class Cfg, bool SPLIT = false>
+// EDGE (direct-to-LDS loader): M, N end anywhere inside a tile and K % 8 == 0 anywhere inside a chunk.  Copies of rows
+// beyond the matrix are redirected to its last row, stores are guarded, the last chunk is treated as `tail_pieces` says.
+template <class Cfg, bool SPLIT = false, bool EDGE = false>
 __global__ void __launch_bounds__(Cfg::THREADS)
     hgemm_tiled_kernel(const half_t *__restrict__ A, const half_t *__restrict__ B, half_t *__restrict__ C,
                        float *__restrict__ partial, int M, int N, int K, int slices, int tiles_m, int tiles_n) {
     constexpr int BM = Cfg::BM, BN = Cfg::BN, BK = Cfg::BK;
     constexpr int TM = Cfg::TM, TN = Cfg::TN, KSTEPS = Cfg::KSTEPS, CPR = Cfg::CPR;
     constexpr int ROW_BYTES = Cfg::ROW_BYTES, STAGES = Cfg::STAGES, THREADS = Cfg::THREADS;
+    static_assert(!EDGE || (Cfg::LOADER == LOAD_DMA && STAGES > 1), "guarded edges are written for the direct-to-LDS ring");
     (void)M;
 
     extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
@@ -242,8 +294,11 @@ __global__ void __launch_bounds__(Cfg::THREADS)
     }
 
     int first_chunk, num_k;
-    slice_of_k(K / BK, slices, slice, first_chunk, num_k);
+    const int chunks = EDGE ? (K + BK - 1) / BK : K / BK;
+    slice_of_k(chunks, slices, slice, first_chunk, num_k);
     const int k_begin = first_chunk * BK;
+    const int tail_dup = EDGE && first_chunk + num_k == chunks ? tail_pieces(K, BK) : 0;
+    const int last_koff = (num_k - 1) * BK - tail_dup * 8;  // where the last chunk is read from, relative to k_begin
     const half_t *Ag = A + (size_t)tile_m * BM * K + k_begin;
     const half_t *Bg = B + (size_t)tile_n * BN * K + k_begin;
 
@@ -269,6 +324,22 @@ __global__ void __launch_bounds__(Cfg::THREADS)
     }
     constexpr int REG_ROW_STEP = THREADS / CPR;                    // rows between a thread's REG chunks
     constexpr int DMA_ROW_STEP = Cfg::WAVES * Cfg::ROWS_PER_DMA;   // rows between a wave's DMA instructions
+    // EDGE: element offset of copy instruction `it` from a_src / b_src, its row clamped to the matrix
+    ptrdiff_t a_row_off[EDGE ? Cfg::A_DMA : 1], b_row_off[EDGE ? Cfg::B_DMA : 1];
+    if constexpr (EDGE) {
+        const int row = wave * Cfg::ROWS_PER_DMA + lane / CPR;
+        const int last_a = M - 1 - tile_m * BM, last_b = N - 1 - tile_n * BN;  // last valid row of the tile
+#pragma unroll
+        for (int it = 0; it < Cfg::A_DMA; ++it) {
+            const int r = row + it * DMA_ROW_STEP;
+            a_row_off[it] = (ptrdiff_t)((r < last_a ? r : last_a) - row) * K;
+        }
+#pragma unroll
+        for (int it = 0; it < Cfg::B_DMA; ++it) {
+            const int r = row + it * DMA_ROW_STEP;
+            b_row_off[it] = (ptrdiff_t)((r < last_b ? r : last_b) - row) * K;
+        }
+    }
 
     u32x4 ra[Cfg::LOADER == LOAD_REG ? Cfg::A_ITERS : 1];
     u32x4 rb[Cfg::LOADER == LOAD_REG ? Cfg::B_ITERS : 1];
@@ -293,15 +364,16 @@ __global__ void __launch_bounds__(Cfg::THREADS)
             *reinterpret_cast<u32x4 *>(sb + it * REG_ROW_STEP * ROW_BYTES) = rb[it];
     };
     auto dma_fetch = [&](int kt, int stage) {  // DMA loader: global -> LDS
-        const int koff = kt * BK;
+        const int koff = EDGE && kt == num_k - 1 ? last_koff : kt * BK;
         const uint32_t base =
             (uint32_t)(uintptr_t)(lds) + (uint32_t)(stage * Cfg::STAGE_BYTES) + cp_lds_off;
 #pragma unroll
         for (int it = 0; it < Cfg::A_DMA; ++it)
-            dma_load16(a_src + (size_t)it * DMA_ROW_STEP * K + koff, base + it * Cfg::WAVES * 1024);
+            dma_load16(a_src + (EDGE ? a_row_off[EDGE ? it : 0] : (ptrdiff_t)it * DMA_ROW_STEP * K) + koff,
+                       base + it * Cfg::WAVES * 1024);
 #pragma unroll
         for (int it = 0; it < Cfg::B_DMA; ++it)
-            dma_load16(b_src + (size_t)it * DMA_ROW_STEP * K + koff,
+            dma_load16(b_src + (EDGE ? b_row_off[EDGE ? it : 0] : (ptrdiff_t)it * DMA_ROW_STEP * K) + koff,
                        base + Cfg::A_BYTES + it * Cfg::WAVES * 1024);
     };
 
@@ -319,7 +391,8 @@ __global__ void __launch_bounds__(Cfg::THREADS)
 #pragma unroll
             for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
 
-    auto load_frags = [&](int stage, int kk, half8 (&af)[TM], half8 (&bf)[TN]) {
+    // drop: 16-byte pieces at the start of the chunk that must not count (EDGE, last chunk)
+    auto load_frags = [&](int stage, int kk, half8 (&af)[TM], half8 (&bf)[TN], int drop) {
         const unsigned char *s = lds + stage * Cfg::STAGE_BYTES;
         const uint32_t chunk = (uint32_t)((kk * 2) ^ frag_x) << 4;
 #pragma unroll
@@ -328,6 +401,15 @@ __global__ void __launch_bounds__(Cfg::THREADS)
 #pragma unroll
         for (int j = 0; j < TN; ++j)
             bf[j] = *reinterpret_cast<const half8 *>(s + b_frag_off + j * 32 * ROW_BYTES + chunk);
+        if constexpr (EDGE) {
+            if (drop > 0) {
+                const bool keep = kk * 2 + (lane >> 5) >= drop;
+#pragma unroll
+                for (int i = 0; i < TM; ++i) af[i] = keep_or_zero(af[i], keep);
+#pragma unroll
+                for (int j = 0; j < TN; ++j) bf[j] = keep_or_zero(bf[j], keep);
+            }
+        }
     };
     auto mma_step = [&](const half8 (&af)[TM], const half8 (&bf)[TN]) {
 #pragma unroll
@@ -338,20 +420,20 @@ __global__ void __launch_bounds__(Cfg::THREADS)
                 acc[i][jj] = __builtin_amdgcn_mfma_f32_32x32x16_f16(bf[jj], af[i], acc[i][jj], 0, 0, 0);
             }
     };
-    auto compute_stage = [&](int stage) {
+    auto compute_stage = [&](int stage, int drop = 0) {
         if constexpr (Cfg::FRAG_PREFETCH) {
             half8 af[2][TM], bf[2][TN];
-            load_frags(stage, 0, af[0], bf[0]);
+            load_frags(stage, 0, af[0], bf[0], drop);
 #pragma unroll
             for (int kk = 0; kk < KSTEPS; ++kk) {
-                if (kk + 1 < KSTEPS) load_frags(stage, kk + 1, af[(kk + 1) & 1], bf[(kk + 1) & 1]);
+                if (kk + 1 < KSTEPS) load_frags(stage, kk + 1, af[(kk + 1) & 1], bf[(kk + 1) & 1], drop);
                 mma_step(af[kk & 1], bf[kk & 1]);
             }
         } else {
             half8 af[TM], bf[TN];
 #pragma unroll
             for (int kk = 0; kk < KSTEPS; ++kk) {
-                load_frags(stage, kk, af, bf);
+                load_frags(stage, kk, af, bf, drop);
                 mma_step(af, bf);
             }
         }
@@ -403,11 +485,11 @@ __global__ void __launch_bounds__(Cfg::THREADS)
             wait_vmcnt<(STAGES - 2) * L>();
             __syncthreads();
             half8 af[2][KSTEPS][TM], bf[2][KSTEPS][TN];
-            auto load_chunk = [&](int stage, half8 (&a)[KSTEPS][TM], half8 (&b)[KSTEPS][TN]) {
+            auto load_chunk = [&](int stage, half8 (&a)[KSTEPS][TM], half8 (&b)[KSTEPS][TN], int drop) {
 #pragma unroll
-                for (int kk = 0; kk < KSTEPS; ++kk) load_frags(stage, kk, a[kk], b[kk]);
+                for (int kk = 0; kk < KSTEPS; ++kk) load_frags(stage, kk, a[kk], b[kk], drop);
             };
-            load_chunk(0, af[0], bf[0]);
+            load_chunk(0, af[0], bf[0], 0);  // never the last chunk: there are at least STAGES - 1
             int cur = 0, fill = STAGES - 1;
             // STEADY: the copy of chunk kt+STAGES-1 exists (so does chunk kt+1, and the wait count is the full one);
             // the last iterations (the odd one left by the unrolled pairs and those after the last copy) take their
@@ -428,7 +510,7 @@ __global__ void __launch_bounds__(Cfg::THREADS)
                     // consumed by MFMAs already issued)
                     __builtin_amdgcn_sched_barrier(0);  // the MFMAs of chunk kt-1 (and their waits) stay in front
                     asm volatile("s_barrier" ::: "memory");
-                    load_chunk(nxt, na, nb);
+                    load_chunk(nxt, na, nb, !STEADY && kt + 1 == num_k - 1 ? tail_dup : 0);
                 }
                 if (STEADY || kt + STAGES - 1 < num_k) dma_fetch(kt + STAGES - 1, fill);
                 __builtin_amdgcn_sched_barrier(0);
@@ -464,7 +546,7 @@ __global__ void __launch_bounds__(Cfg::THREADS)
                 }
                 __syncthreads();
                 if (kt + STAGES - 1 < num_k) dma_fetch(kt + STAGES - 1, fill);
-                compute_stage(cur);
+                compute_stage(cur, kt == num_k - 1 ? tail_dup : 0);
                 cur = (cur + 1 == STAGES) ? 0 : cur + 1;
                 fill = (fill + 1 == STAGES) ? 0 : fill + 1;
             }
@@ -474,8 +556,9 @@ __global__ void __launch_bounds__(Cfg::THREADS)
     if constexpr (SPLIT) {
         // Lane l holds row l % 32 of each 32x32 tile and, per register group g, four consecutive n at
         // 8 g + 4 (l / 32): 16 bytes of an fp32 partial sum.
-        float *dst = partial + ((size_t)slice * M + tile_m * BM + wm * Cfg::WM + (lane & 31)) * N + tile_n * BN +
-                     wn * Cfg::WN + ((lane >> 5) << 2);
+        const size_t ld = EDGE ? partial_ld(N) : (size_t)N;
+        const int row = tile_m * BM + wm * Cfg::WM + (lane & 31), col = tile_n * BN + wn * Cfg::WN + ((lane >> 5) << 2);
+        float *dst = partial + ((size_t)slice * M + row) * ld + col;
 #pragma unroll
         for (int i = 0; i < TM; ++i)
 #pragma unroll
@@ -485,57 +568,72 @@ __global__ void __launch_bounds__(Cfg::THREADS)
                     floatx4 v;
 #pragma unroll
                     for (int r = 0; r < 4; ++r) v[r] = acc[i][j][g * 4 + r];
-                    *reinterpret_cast<floatx4 *>(dst + (size_t)(i * 32) * N + j * 32 + g * 8) = v;
+                    if (!EDGE || (row + i * 32 < M && (size_t)(col + j * 32 + g * 8) < ld))
+                        *reinterpret_cast<floatx4 *>(dst + (size_t)(i * 32) * ld + j * 32 + g * 8) = v;
                 }
         return;
     }
     // ---------------- epilogue: accumulators -> fp16 -> C ----------------
     __syncthreads();
-    store_tile_via_lds<Cfg>(acc, lds, C, N, tile_m * BM + wm * Cfg::WM, tile_n * BN + wn * Cfg::WN, wave, lane);
+    store_tile_via_lds<Cfg, EDGE>(acc, lds, C, M, N, tile_m * BM + wm * Cfg::WM, tile_n * BN + wn * Cfg::WN, wave, lane);
+}
+
+// Shapes the EDGE form takes: any M and N; K a multiple of 8, long enough that the prologue's chunks exist.
+template <class Cfg>
+bool tiled_supports_edges(size_t M, size_t N, size_t K) {
+    return M > 0 && N > 0 && K % 8 == 0 && div_ceil(K, (size_t)Cfg::BK) >= (size_t)(Cfg::STAGES > 2 ? Cfg::STAGES - 1 : 2);
 }
 
 // Host launcher shared by every tiled entry point.  Sets the dynamic-LDS limit once per
 // instantiation (counterpart of the reference's one-time cudaFuncSetAttribute,
 // src/mma/mma_async_stage4.cu:619-635), checks the launch, does not synchronise.
-template <class Cfg>
+template <class Cfg, bool EDGE = false>
 void launch_tiled(const void *A, const void *B, void *C, size_t M, size_t N, size_t K, const char *name) {
     check_operands(A, B, C, M, N, K);
-    HGEMM_CHECK_MSG(Cfg::supports(M, N, K),
-                    "%s needs M %% %d == 0, N %% %d == 0, K %% %d == 0, K >= %d (got M=%zu N=%zu K=%zu)", name,
-                    Cfg::BM, Cfg::BN, Cfg::BK, Cfg::BK * (Cfg::STAGES > 1 ? Cfg::STAGES - 1 : 1), M, N, K);
+    if constexpr (EDGE)
+        HGEMM_CHECK(tiled_supports_edges<Cfg>(M, N, K));
+    else
+        HGEMM_CHECK_MSG(Cfg::supports(M, N, K),
+                        "%s needs M %% %d == 0, N %% %d == 0, K %% %d == 0, K >= %d (got M=%zu N=%zu K=%zu)", name,
+                        Cfg::BM, Cfg::BN, Cfg::BK, Cfg::BK * (Cfg::STAGES > 1 ? Cfg::STAGES - 1 : 1), M, N, K);
     static bool configured = [] {
-        HGEMM_CHECK_HIP_ERROR(hipFuncSetAttribute(reinterpret_cast<const void *>(&hgemm_tiled_kernel<Cfg>),
+        HGEMM_CHECK_HIP_ERROR(hipFuncSetAttribute(reinterpret_cast<const void *>(&hgemm_tiled_kernel<Cfg, false, EDGE>),
                                                   hipFuncAttributeMaxDynamicSharedMemorySize, Cfg::LDS_BYTES));
         return true;
     }();
     (void)configured;
-    const int tiles_m = (int)(M / Cfg::BM), tiles_n = (int)(N / Cfg::BN);
-    hgemm_tiled_kernel<Cfg><<<dim3(tiles_m * tiles_n), dim3(Cfg::THREADS), Cfg::LDS_BYTES, nullptr>>>(
+    const size_t tiles_m = div_ceil(M, (size_t)Cfg::BM), tiles_n = div_ceil(N, (size_t)Cfg::BN);
+    HGEMM_CHECK(tiles_m * tiles_n < ((size_t)1 << 31));
+    hgemm_tiled_kernel<Cfg, false, EDGE><<<dim3((unsigned)(tiles_m * tiles_n)), dim3(Cfg::THREADS), Cfg::LDS_BYTES, nullptr>>>(
         reinterpret_cast<const half_t *>(A), reinterpret_cast<const half_t *>(B), reinterpret_cast<half_t *>(C), nullptr,
-        (int)M, (int)N, (int)K, 1, tiles_m, tiles_n);
+        (int)M, (int)N, (int)K, 1, (int)tiles_m, (int)tiles_n);
     HGEMM_CHECK_HIP_ERROR(hipGetLastError());
 }
 
-// K in `splits` slices: fp32 partial sums of slice s go to partial[s][M][N]; the caller runs the ordered reduction.
-template <class Cfg>
+// K in `splits` slices: fp32 partial sums of slice s go to partial[s][M][partial_ld(N)]; the caller runs the ordered
+// reduction.
+template <class Cfg, bool EDGE = false>
 void launch_tiled_split(const void *A, const void *B, float *partial, size_t M, size_t N, size_t K, int splits,
                         const char *name) {
-    HGEMM_CHECK(splits >= 1 && K % (size_t)Cfg::BK == 0 && partial != nullptr && splits <= 65535);
+    HGEMM_CHECK(splits >= 1 && partial != nullptr && splits <= 65535);
     const size_t k_len = shortest_slice(K, Cfg::BK, splits);
-    HGEMM_CHECK_MSG(k_len > 0 && Cfg::supports(M, N, k_len),
-                    "%s (K in %d slices) needs M %% %d == 0, N %% %d == 0, K %% %d == 0, shortest slice >= %d (got M=%zu N=%zu K=%zu)",
-                    name, splits, Cfg::BM, Cfg::BN, Cfg::BK, Cfg::BK * (Cfg::STAGES > 1 ? Cfg::STAGES - 1 : 1), M, N, K);
+    if constexpr (EDGE)
+        HGEMM_CHECK(K % 8 == 0 && tiled_supports_edges<Cfg>(M, N, k_len));
+    else
+        HGEMM_CHECK_MSG(K % (size_t)Cfg::BK == 0 && k_len > 0 && Cfg::supports(M, N, k_len),
+                        "%s (K in %d slices) needs M %% %d == 0, N %% %d == 0, K %% %d == 0, shortest slice >= %d (got M=%zu N=%zu K=%zu)",
+                        name, splits, Cfg::BM, Cfg::BN, Cfg::BK, Cfg::BK * (Cfg::STAGES > 1 ? Cfg::STAGES - 1 : 1), M, N, K);
     static bool configured = [] {
-        HGEMM_CHECK_HIP_ERROR(hipFuncSetAttribute(reinterpret_cast<const void *>(&hgemm_tiled_kernel<Cfg, true>),
+        HGEMM_CHECK_HIP_ERROR(hipFuncSetAttribute(reinterpret_cast<const void *>(&hgemm_tiled_kernel<Cfg, true, EDGE>),
                                                   hipFuncAttributeMaxDynamicSharedMemorySize, Cfg::LDS_BYTES));
         return true;
     }();
     (void)configured;
-    const int tiles_m = (int)(M / Cfg::BM), tiles_n = (int)(N / Cfg::BN);
-    HGEMM_CHECK((size_t)tiles_m * tiles_n * (size_t)splits < ((size_t)1 << 31));
-    hgemm_tiled_kernel<Cfg, true><<<dim3(tiles_m * tiles_n * splits), dim3(Cfg::THREADS), Cfg::LDS_BYTES, nullptr>>>(
+    const size_t tiles_m = div_ceil(M, (size_t)Cfg::BM), tiles_n = div_ceil(N, (size_t)Cfg::BN);
+    HGEMM_CHECK(tiles_m * tiles_n * (size_t)splits < ((size_t)1 << 31));
+    hgemm_tiled_kernel<Cfg, true, EDGE><<<dim3((unsigned)(tiles_m * tiles_n * (size_t)splits)), dim3(Cfg::THREADS), Cfg::LDS_BYTES, nullptr>>>(
         reinterpret_cast<const half_t *>(A), reinterpret_cast<const half_t *>(B), nullptr, partial, (int)M, (int)N, (int)K,
-        splits, tiles_m, tiles_n);
+        splits, (int)tiles_m, (int)tiles_n);
     HGEMM_CHECK_HIP_ERROR(hipGetLastError());
 }
 

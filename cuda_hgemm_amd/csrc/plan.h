@@ -24,10 +24,12 @@ enum KernelId {
     KERNEL_SMALL64_W4,  // 64x64x64 tile on four waves of 32x32 (the ladder's kernel): grids of at most one tile per CU
     KERNEL_MID128_S2,   // pipelined 128x128x64, 4 waves, 2-stage ring: two workgroups per CU, for K of at most four chunks
     KERNEL_DECODE_RING, // decode kernel for M <= 128 whose waves stage operands through LDS rings of their own; `splits` waves over K
-    KERNEL_PADDED,      // operands copied zero-padded to N % 8 == 0, K % 64 == 0, then the plan for that shape
+    KERNEL_PADDED,      // operands copied with rows of whole 64-wide chunks, then the plan for that K (`inner_kernel`)
     KERNEL_ROW64x128,   // pipelined 64x128x64, 4 waves side by side, 5-stage ring: one row of tiles for M <= 64 against many columns
     KERNEL_DECODE_RESIDENT,  // decode kernel for M <= 32 with A in registers: persistent workgroups walk over 16-column tiles; `splits` waves over K
     KERNEL_ROW192x128,  // pipelined 192x128x64, 4 waves, 4-stage ring: one row of tiles for M = 129 ... 192 against many columns
+    KERNEL_SMALL64_W4_EDGE,  // KERNEL_SMALL64_W4 with guarded edges: M, N end inside a tile, K (K % 8 == 0) inside a chunk
+    KERNEL_DECODE_RING_EDGE, // KERNEL_DECODE_RING with guarded edges: any N, K % 8 == 0 dealt to the waves unevenly
 };
 
 struct Plan {
@@ -40,6 +42,7 @@ struct Plan {
     // pipelined kernels only: the last tail_tiles workgroup ids of the grid run in tail_splits K slices, or
     // (tail_kernel != KERNEL_NONE, 256x256 tiles only) divided among workgroups of that smaller tile
     int tail_tiles = 0, tail_splits = 1, tail_kernel = KERNEL_NONE;
+    int inner_kernel = KERNEL_NONE;  // KERNEL_PADDED only: what runs on the copies (the fields above are its)
 };
 
 // Device memory handed to run_plan; a plan is only run with at least what it asks for.

@@ -115,9 +115,9 @@ HGEMM_FUNC(hgemm_mfma_chained_192x192);
 HGEMM_FUNC(hgemm_skinny);
 
 /* Dispatcher: picks tile, kernel and number of K slices for the shape from a cost model
- * fitted to measurements; accepts every shape.  N % 8 == 0 and K % 64 == 0 run on the
- * pipelined kernels (M and N may end inside a tile: edges are guarded), anything else on a
- * fully guarded MFMA kernel.  This is the entry point the benchmark measures. */
+ * fitted to measurements; accepts every shape.  M and N may end anywhere inside a tile and K,
+ * a multiple of 8, anywhere inside a chunk (edges are guarded); other K from 192 on run on
+ * copies of A and B whose rows are aligned, shorter ones on a fully guarded MFMA kernel.  This is the entry point the benchmark measures. */
 HGEMM_FUNC(hgemm_auto);
 
 /* Kernel hgemm_auto would pick for a shape (an id for hgemm_kernel_name) and, through
@@ -168,8 +168,8 @@ int hgemm_auto_plan_is_tuned(size_t M, size_t N, size_t K);
 int hgemm_small_m_rule(int index, size_t *bounds, int *flags);
 
 /* ---- workspace of hgemm_auto / hgemm_skinny.  Plans that cut K into slices keep fp32
- * partial sums in device memory, and large shapes with N % 8 != 0 or K % 64 != 0 run on
- * zero-padded copies of A and B.  Both buffers belong to the library, one pair per device,
+ * partial sums in device memory, and shapes with K % 8 != 0 (large ones with K % 64 != 0 too)
+ * run on zero-padded copies of A and B.  Both buffers belong to the library, one pair per device,
  * and live until hgemm_release_workspace or the end of the process (the reference keeps its
  * vendor handle the same way, src/cublas_tensor_op.cu:18).  Each is allocated ONCE, at its
  * cap (512 MiB of partial sums, 1 GiB of operand copies), by the first call that needs it:

@@ -1,0 +1,66 @@
+"""hgemm_auto on sizes that end inside a tile and inside a 64-wide K chunk: every kernel with guarded edges, at K one, four
+and seven 8-element pieces into its last chunk, N odd, with and without K slices."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+GUARD, POISON = 4096, 0x7E5A   # elements around C (keeps it 16-byte aligned); a NaN no kernel produces
+
+# shape -> start of the kernel's name; together every kernel that has guarded edges, sliced and not
+CASES = [
+    ((313, 5, 184), "edge-guarded"), ((157, 1, 5104), "edge-guarded"),            # plain ring, alone and in slices
+    ((147, 4, 680), "edge-guarded"), ((168, 2, 5120), "edge-guarded"),            # look-ahead ring
+    ((2777, 131, 2912), "edge-guarded"), ((2420, 66, 7840), "edge-guarded"),      # its deep form
+    ((2358, 397, 360), "edge-guarded"), ((1000, 1000, 1000), "edge-guarded"),     # two workgroups per CU; one
+    ((147, 20, 72), "pipelined 128x128"), ((2813, 77, 5520), "pipelined 128x128"),
+    ((130, 3768, 6744), "pipelined 192x192"), ((48, 34155, 200), "pipelined 192x192"),
+    ((266, 13721, 4424), "pipelined 192x192"), ((131, 19105, 2072), "pipelined 192x128"),
+    ((137, 25461, 264), "pipelined 256x128"), ((2816, 259, 6240), "pipelined 256x128"),
+    ((432, 9491, 4072), "pipelined 256x128"), ((519, 18759, 272), "pipelined 256x256"),
+    ((199, 11317, 6312), "pipelined 256x256"), ((259, 26010, 1752), "pipelined 256x256"),
+    ((408, 36824, 288), "pipelined 256x256"), ((646, 26708, 616), "pipelined 256x256"),   # last round on smaller tiles
+    ((230, 16622, 4152), "pipelined 128x128"), ((258, 25173, 2096), "pipelined 192x192"),  # ... in K slices
+    ((36, 19412, 400), "pipelined 64x128"), ((41, 9311, 8208), "pipelined 64x128"), ((17, 35153, 3392), "pipelined 64x128"),
+    ((492, 2108, 136), "pipelined 64x64"), ((2574, 1, 3112), "pipelined 64x64"),
+    ((7, 20, 72), "split-K 32x64"), ((11, 5, 2792), "split-K 32x64"), ((39, 2, 176), "split-K 64x64"),
+    ((34, 2, 7416), "split-K 64x64"), ((38, 18838, 96), "split-K 64x128"), ((38, 17733, 2136), "split-K 64x128"),
+    ((67, 1, 216), "split-K 128x64"), ((76, 2, 6272), "split-K 128x64"), ((69, 23286, 88), "split-K 128x128"),
+    ((74, 17395, 3824), "split-K 128x128"),
+    ((1, 9, 312), "streaming decode"), ((4, 1475, 14528), "streaming decode"), ((18, 220, 288), "streaming decode"),
+    ((56, 81, 312), "streaming decode"), ((67, 4295, 272), "streaming decode"), ((67, 146, 280), "streaming decode"),
+    ((511, 511, 511), "zero-padded"), ((296, 299, 2113), "zero-padded"), ((3, 1001, 4099), "zero-padded"),
+    ((1027, 520, 193), "zero-padded"), ((2591, 11875, 1833), "zero-padded"),
+]
+
+
+def _gpu_bits(bits, gpu):
+    import torch
+    return torch.from_numpy(bits.view(np.int16)).to(gpu).view(torch.float16)
+
+
+@pytest.mark.parametrize("shape,kernel", CASES)
+def test_sizes_inside_tiles_and_chunks(oracle, hgemm_lib, gpu, shape, kernel):
+    """Exact on ternary inputs (sums are integers below 2048) inside a guard band; then with an infinity in one row of A, at
+    the k that the last chunk and the one before it both read: that row is infinite with B's sign, no other changes."""
+    import torch
+    M, N, K = shape
+    plan = hgemm_lib.auto_plan(M, N, K)
+    assert plan["kernel"].startswith(kernel), plan
+    A, B = oracle.fill((M, K), 31, 1, oracle.TERNARY, 0, 1), oracle.fill((N, K), 31, 2, oracle.TERNARY, 0, 1)
+    expect = oracle.hgemm(A, B)
+    assert np.abs(expect.view(np.float16).astype(np.float32)).max() < 2048
+    buf = torch.full((GUARD + M * N + GUARD,), POISON, dtype=torch.int16, device=gpu)
+    C = buf[GUARD:GUARD + M * N].view(torch.float16).view(M, N)
+    Ad, Bd = _gpu_bits(A, gpu), _gpu_bits(B, gpu)
+    print(f"[gpu] hgemm_auto M={M} N={N} K={K} {plan['kernel']} x{plan['splits']} tail {plan['tail_tiles']}", flush=True)
+    hgemm_lib.call("hgemm_auto", Ad, Bd, C, M, N, K)
+    host = buf.cpu().numpy().view(np.uint16)
+    assert np.all(host[:GUARD] == POISON) and np.all(host[GUARD + M * N:] == POISON)
+    assert np.array_equal(host[GUARD:GUARD + M * N].reshape(M, N), expect)
+    row, k = M - 1, K - 60 if K >= 64 else 0
+    Bd[:, k] = torch.where(torch.arange(N, device=gpu) % 2 == 0, 1.0, -1.0).half()
+    Ad[row, k] = float("inf")
+    hgemm_lib.call("hgemm_auto", Ad, Bd, C, M, N, K)
+    assert torch.equal(C[row], torch.where(torch.arange(N, device=gpu) % 2 == 0, float("inf"), float("-inf")).half())
+    assert M == 1 or bool(torch.isfinite(C[:row]).all())
