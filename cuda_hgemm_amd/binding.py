@@ -46,6 +46,7 @@ HELPER_SYMBOLS = [
     "hgemm_auto_plan", "hgemm_auto_plan_tail", "hgemm_auto_plan_tail_kernel", "hgemm_auto_plan_chained", "hgemm_kernel_name",
     "hgemm_small_m_rule", "hgemm_variant_count", "hgemm_variant_name", "hgemm_variant_symbol",
     "hgemm_variant_fn", "hgemm_variant_find", "hgemm_variant_supports", "hgemm_variant_in_default_run",
+    "hgemm_variant_run",
     "hgemm_profile_ms", "hgemm_profile_rotating_ms", "hgemm_clock_mark", "hgemm_clock_between_marks_mhz",
     "hgemm_tflops", "hgemm_bytes", "hgemm_version",
     "hgemm_reserve_workspace", "hgemm_release_workspace", "hgemm_auto_workspace_bytes",
@@ -68,7 +69,22 @@ def _share_hip_runtime_with_torch() -> None:
         pass  # a caller without torch brings its own device pointers and the system runtime
 
 
+# torch.Tensor and torch.float16 from the first tensor on; a process without torch keeps the empty tuple, which nothing
+# is an instance of
+_Tensor, _float16 = (), None
+
+
 def _tensor_ptr(t, rows: int, cols: int, what: str) -> int:
+    # An operand that is as it should be passes in one expression (0.6 us; a call has three, and 8.5 us of a call used to
+    # pass in Python before the launch); whatever does not is told why below.
+    if (isinstance(t, _Tensor) and t.dtype is _float16 and t.is_cuda and t.shape == (rows, cols) and t.is_contiguous()
+            and not t.data_ptr() % 16):
+        return t.data_ptr()
+    return _checked_ptr(t, rows, cols, what)
+
+
+def _checked_ptr(t, rows: int, cols: int, what: str) -> int:
+    global _Tensor, _float16
     from .hipmem import DeviceArray
     if isinstance(t, DeviceArray):
         if tuple(t.shape) != (rows, cols):
@@ -77,6 +93,7 @@ def _tensor_ptr(t, rows: int, cols: int, what: str) -> int:
             raise ValueError(f"{what}: the buffer has been freed")
         return t.ptr
     import torch
+    _Tensor, _float16 = torch.Tensor, torch.float16
     if not isinstance(t, torch.Tensor):
         raise TypeError(f"{what}: expected a torch.Tensor or a hipmem.DeviceArray, got {type(t).__name__}")
     if t.dtype != torch.float16:
@@ -133,6 +150,9 @@ class HgemmLibrary:
         d.hgemm_variant_find.argtypes, d.hgemm_variant_find.restype = [C.c_char_p], C.c_int
         d.hgemm_variant_supports.argtypes, d.hgemm_variant_supports.restype = [C.c_int, _SZ, _SZ, _SZ], C.c_int
         d.hgemm_variant_in_default_run.argtypes, d.hgemm_variant_in_default_run.restype = [C.c_int], C.c_int
+        d.hgemm_variant_run.argtypes, d.hgemm_variant_run.restype = [C.c_int] + _HGEMM_ARGS, C.c_int
+        self._run = d.hgemm_variant_run
+        self._indices = {}  # variant names seen by call() -> their indices
         d.hgemm_profile_ms.argtypes = [HGEMM_FN, _PTR, _PTR, _PTR, _SZ, _SZ, _SZ, _SZ, _SZ]
         d.hgemm_profile_ms.restype = C.c_double
         d.hgemm_profile_rotating_ms.argtypes = [HGEMM_FN, C.POINTER(_PTR), C.POINTER(_PTR), C.POINTER(_PTR), _SZ, _SZ,
@@ -253,9 +273,12 @@ class HgemmLibrary:
         a = _tensor_ptr(A, M, K, "A")
         b = _tensor_ptr(B, N, K, "B (stored as N rows of K)")
         c = _tensor_ptr(C_out, M, N, "C")
-        if not self.supports(name, M, N, K):
+        index = self._indices.get(name)
+        if index is None:
+            index = self._indices[name] = self.find(name)
+        # looks the variant up, asks whether it takes the shape and launches it: one call across the boundary
+        if not self._run(index, a, b, c, M, N, K):
             raise ValueError(f"variant {name!r} cannot run M={M} N={N} K={K}")
-        self.fn(name)(a, b, c, M, N, K)
 
     def profile_ms(self, name: str, A, B, C_out, M: int, N: int, K: int, warmup: int, iterations: int) -> float:
         """Average milliseconds per call of ``iterations`` back-to-back calls after ``warmup``
@@ -363,5 +386,5 @@ def hgemm(A, B, variant: str = "hgemm_auto", out=None):
     N = B.shape[0]
     if out is None:
         out = torch.empty((M, N), dtype=torch.float16, device=A.device)
-    library().call(variant, A, B, out, M, N, K)
+    (_library or library()).call(variant, A, B, out, M, N, K)
     return out

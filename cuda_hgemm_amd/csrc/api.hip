@@ -107,6 +107,14 @@ extern "C" int hgemm_variant_supports(int index, size_t M, size_t N, size_t K) {
     return variant_at(index)->supports(M, N, K);
 }
 
+// The question above and the launch in one call; 0 if the variant cannot run the shape (nothing is launched then).
+extern "C" int hgemm_variant_run(int index, const hgemm_half *A, const hgemm_half *B, hgemm_half *C, size_t M, size_t N,
+                                 size_t K) {
+    if (!hgemm_variant_supports(index, M, N, K)) return 0;
+    variant_at(index)->fn(A, B, C, M, N, K);
+    return 1;
+}
+
 // Timing loop of Tester::profile (reference src/common/tester.h:89-97) with the event
 // handling of CudaTimer (reference src/common/cuda_timer.h:32-42): events on the null
 // stream, no synchronisation between the timed calls.

@@ -227,6 +227,8 @@ hgemm_fn hgemm_variant_fn(int index);
 int hgemm_variant_find(const char *name);
 /* 1 if variant `index` can run the shape, 0 otherwise (no side effects). */
 int hgemm_variant_supports(int index, size_t M, size_t N, size_t K);
+/* Runs variant `index` if it can run the shape: returns 1, or 0 with nothing launched. */
+int hgemm_variant_run(int index, const hgemm_half *A, const hgemm_half *B, hgemm_half *C, size_t M, size_t N, size_t K);
 /* 1 if the variant belongs to the default run (reference src/main.cu:100-123 comments the
  * slow ones out), 0 otherwise. */
 int hgemm_variant_in_default_run(int index);

@@ -64,3 +64,23 @@ def test_sizes_inside_tiles_and_chunks(oracle, hgemm_lib, gpu, shape, kernel):
     hgemm_lib.call("hgemm_auto", Ad, Bd, C, M, N, K)
     assert torch.equal(C[row], torch.where(torch.arange(N, device=gpu) % 2 == 0, float("inf"), float("-inf")).half())
     assert M == 1 or bool(torch.isfinite(C[:row]).all())
+
+
+def test_call_refuses_what_it_refused_before_on_every_call(hgemm_lib, gpu):
+    """Operands pass the binding's one-expression check or are told why not, also after calls that were in order."""
+    import torch
+    A, B = torch.ones((48, 64), dtype=torch.float16, device=gpu), torch.ones((40, 64), dtype=torch.float16, device=gpu)
+    C = torch.empty((48, 40), dtype=torch.float16, device=gpu)
+    for _ in range(2):
+        hgemm_lib.call("hgemm_auto", torch.nn.Parameter(A, requires_grad=False), B, C, 48, 40, 64)  # a Tensor's subclass
+        assert bool((C == 64).all())
+        shifted = torch.ones(48 * 64 + 1, dtype=torch.float16, device=gpu)[1:].view(48, 64)
+        for bad, error, needle in [(A.float(), TypeError, "float16"), (A.cpu(), ValueError, "GPU"), (A[:, :32], ValueError, "shape"),
+                                   (A.t().contiguous().t(), ValueError, "contiguous"), (shifted, ValueError, "16-byte"),
+                                   (A.bfloat16(), TypeError, "float16"), ([1.0], TypeError, "list")]:
+            with pytest.raises(error, match=needle):
+                hgemm_lib.call("hgemm_auto", bad, B, C, 48, 40, 64)
+        with pytest.raises(ValueError, match="cannot run"):
+            hgemm_lib.call("hgemm_mfma_base", A, B, C, 48, 40, 64)
+        with pytest.raises(KeyError, match="no such"):
+            hgemm_lib.call("no such", A, B, C, 48, 40, 64)
