@@ -30,7 +30,7 @@ DEVICE_FLAGS = ["--offload-arch=" + ARCH, "-Xclang", "-target-feature", "-Xclang
 CXXFLAGS = ["-O3", "-std=c++17", "-fPIC", "-Wall", "-Wextra", "-Wno-unused-parameter", "-I" + INCLUDE]
 
 LIB_SOURCES = ["basic_kernels.hip", "ladder_sync.hip", "ladder_async.hip", "ladder_stages.hip", "tiles_256.hip",
-               "tiles_192.hip", "tiles_128.hip", "tiles_64.hip", "dispatch.hip", "api.hip"]
+               "tiles_224.hip", "tiles_192.hip", "tiles_160.hip", "tiles_128.hip", "tiles_64.hip", "dispatch.hip", "api.hip"]
 VENDOR_SOURCES = ["vendor_hipblaslt.cpp"]
 DRIVER_SOURCES = ["driver/main.cpp"]
 
@@ -69,8 +69,8 @@ def _run(cmd):
 NO_SPILL_KERNELS = ("hgemm_pipelined_kernel", "hgemm_chained_kernel", "hgemm_decode_resident_kernel")
 # sources that must contain such kernels: a remark format the parser no longer understands
 # must not turn the guard into a no-op
-MUST_CHECK = {"dispatch.hip": NO_SPILL_KERNELS, "tiles_256.hip": NO_SPILL_KERNELS[:2], "tiles_192.hip": NO_SPILL_KERNELS[:2],
-              "tiles_128.hip": NO_SPILL_KERNELS[:1], "tiles_64.hip": NO_SPILL_KERNELS[:1]}
+MUST_CHECK = {"dispatch.hip": NO_SPILL_KERNELS, "tiles_256.hip": NO_SPILL_KERNELS[:2], "tiles_224.hip": NO_SPILL_KERNELS[:2], "tiles_192.hip": NO_SPILL_KERNELS[:2],
+              "tiles_160.hip": NO_SPILL_KERNELS[:2], "tiles_128.hip": NO_SPILL_KERNELS[:1], "tiles_64.hip": NO_SPILL_KERNELS[:1]}
 
 
 def _chained_accumulator_registers(mangled):

@@ -35,6 +35,7 @@ __global__ void __launch_bounds__(Cfg::THREADS)
     constexpr int TM = Cfg::TM, TN = Cfg::TN, KSTEPS = Cfg::KSTEPS, CPR = Cfg::CPR;
     constexpr int ROW_BYTES = Cfg::ROW_BYTES, STAGES = Cfg::STAGES;
     constexpr int L = Cfg::A_DMA + Cfg::B_DMA;
+    static_assert(Cfg::WM % 32 == 0 && Cfg::WN % 32 == 0, "wave tile must be a multiple of the 32x32 MFMA tile");
 
     extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
 

@@ -72,7 +72,7 @@ struct TileConfig {
     static constexpr int LOADS_PER_STAGE = (LOADER == LOAD_DMA) ? (A_DMA + B_DMA) : (A_ITERS + B_ITERS);
 
     static_assert(BK == 32 || BK == 64, "K chunk must be 32 or 64 halves");
-    static_assert(WM % 32 == 0 && WN % 32 == 0, "wave tile must be a multiple of the 32x32 MFMA tile");
+    static_assert(WM % 16 == 0 && WN % 16 == 0, "wave tile must be a multiple of an MFMA tile");
     static_assert((BM * CPR) % THREADS == 0 && (BN * CPR) % THREADS == 0, "tile copy must divide evenly");
     static_assert(LOADER == LOAD_REG || LAYOUT != LDS_PADDED, "direct-to-LDS rows are contiguous: no padding");
     static_assert(LOADER == LOAD_REG || (A_BYTES % (1024 * WAVES) == 0 && B_BYTES % (1024 * WAVES) == 0),
@@ -273,6 +273,7 @@ __global__ void __launch_bounds__(Cfg::THREADS)
     constexpr int BM = Cfg::BM, BN = Cfg::BN, BK = Cfg::BK;
     constexpr int TM = Cfg::TM, TN = Cfg::TN, KSTEPS = Cfg::KSTEPS, CPR = Cfg::CPR;
     constexpr int ROW_BYTES = Cfg::ROW_BYTES, STAGES = Cfg::STAGES, THREADS = Cfg::THREADS;
+    static_assert(Cfg::WM % 32 == 0 && Cfg::WN % 32 == 0, "wave tile must be a multiple of the 32x32 MFMA tile");
     static_assert(!EDGE || (Cfg::LOADER == LOAD_DMA && STAGES > 1), "guarded edges are written for the direct-to-LDS ring");
     (void)M;
 

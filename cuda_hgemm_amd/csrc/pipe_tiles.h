@@ -19,6 +19,14 @@ using Row64x128 = PipeConfig<64, 128, 64, 1, 4, 5, 16>;
 using Row192x128 = PipeConfig<192, 128, 64, 2, 2, 4, 16>;
 using Tile192 = PipeConfig<192, 192, 64, 2, 2, 3, 16>;
 using Rect256x128 = PipeConfig<256, 128, 64, 2, 2, 3, 16>;
+// Sizes between those, for products whose tiles of the sizes above leave part of the chip idle in their last round or run
+// past M: 600 x 14336 x 4096 is 168 tiles of 256x256 (78.4 us), 224 of 160x256 (61.8 us).  Wave tiles are any multiple
+// of the 16x16 MFMA tile.  The rings are as deep as 160 KB allow (192 and 224 rows: two B buffers, three A buffers).
+using Tile160x128 = PipeConfig<160, 128, 64, 2, 2, 4, 16>;
+using Tile160x160 = PipeConfig<160, 160, 64, 2, 2, 4, 16>;
+using Tile160x256 = PipeConfig<160, 256, 64, 2, 2, 3, 16>;
+using Tile192x256 = PipeConfig<192, 256, 64, 2, 2, 2, 16, 1>;
+using Tile224x256 = PipeConfig<224, 256, 64, 2, 2, 2, 16, 1>;
 
 #define HGEMM_PIPE_LAUNCHERS(LINKAGE, Cfg)                                                                              \
     LINKAGE template void launch_pipelined<Cfg>(const void *, const void *, void *, size_t, size_t, size_t, const char *, \
@@ -27,6 +35,9 @@ using Rect256x128 = PipeConfig<256, 128, 64, 2, 2, 3, 16>;
                                                       const char *);                                                    \
     LINKAGE template void launch_pipelined_with_tail<Cfg>(const void *, const void *, void *, float *, size_t, size_t,    \
                                                           size_t, int, int, const char *);
+#define HGEMM_WHOLE_K_LAUNCHER(LINKAGE, Cfg)                                                                            \
+    LINKAGE template void launch_pipelined<Cfg>(const void *, const void *, void *, size_t, size_t, size_t, const char *, \
+                                                PipeKernel);
 #define HGEMM_SUBTILE_LAUNCHER(LINKAGE, Child)                                                                          \
     LINKAGE template void launch_pipelined_with_subtiles<Big256, Child>(const void *, const void *, void *, size_t, size_t, \
                                                                         size_t, int, const char *);
@@ -35,9 +46,14 @@ HGEMM_PIPE_LAUNCHERS(extern, Big256)        // tiles_256.hip
 HGEMM_PIPE_LAUNCHERS(extern, Tile192)       // tiles_192.hip
 HGEMM_PIPE_LAUNCHERS(extern, Row192x128)
 HGEMM_PIPE_LAUNCHERS(extern, Mid128)        // tiles_128.hip
-extern template void launch_pipelined<Mid128S2>(const void *, const void *, void *, size_t, size_t, size_t, const char *, PipeKernel);
+HGEMM_WHOLE_K_LAUNCHER(extern, Mid128S2)
 HGEMM_PIPE_LAUNCHERS(extern, Small64)       // tiles_64.hip
 HGEMM_PIPE_LAUNCHERS(extern, Row64x128)
+HGEMM_WHOLE_K_LAUNCHER(extern, Tile160x128)  // tiles_160.hip
+HGEMM_WHOLE_K_LAUNCHER(extern, Tile160x160)
+HGEMM_WHOLE_K_LAUNCHER(extern, Tile160x256)
+HGEMM_WHOLE_K_LAUNCHER(extern, Tile192x256)  // tiles_224.hip
+HGEMM_WHOLE_K_LAUNCHER(extern, Tile224x256)
 HGEMM_SUBTILE_LAUNCHER(extern, Rect256x128)  // tiles_256.hip
 HGEMM_SUBTILE_LAUNCHER(extern, Mid128)
 HGEMM_SUBTILE_LAUNCHER(extern, Small64)

@@ -30,6 +30,11 @@ enum KernelId {
     KERNEL_ROW192x128,  // pipelined 192x128x64, 4 waves, 4-stage ring: one row of tiles for M = 129 ... 192 against many columns
     KERNEL_SMALL64_W4_EDGE,  // KERNEL_SMALL64_W4 with guarded edges: M, N end inside a tile, K (K % 8 == 0) inside a chunk
     KERNEL_DECODE_RING_EDGE, // KERNEL_DECODE_RING with guarded edges: any N, K % 8 == 0 dealt to the waves unevenly
+    KERNEL_T160x128,    // pipelined tiles between the sizes above, where they fill the last round better; never sliced
+    KERNEL_T160x160,
+    KERNEL_T160x256,
+    KERNEL_T192x256,
+    KERNEL_T224x256,
 };
 
 struct Plan {

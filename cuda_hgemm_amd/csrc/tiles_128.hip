@@ -4,6 +4,6 @@
 namespace hgemm {
 
 HGEMM_PIPE_LAUNCHERS(, Mid128)
-template void launch_pipelined<Mid128S2>(const void *, const void *, void *, size_t, size_t, size_t, const char *, PipeKernel);
+HGEMM_WHOLE_K_LAUNCHER(, Mid128S2)
 
 }  // namespace hgemm

@@ -15,12 +15,17 @@ CASES = [
     ((2358, 397, 360), "edge-guarded"), ((1000, 1000, 1000), "edge-guarded"),     # two workgroups per CU; one
     ((147, 20, 72), "pipelined 128x128"), ((2813, 77, 5520), "pipelined 128x128"),
     ((130, 3768, 6744), "pipelined 192x192"), ((48, 34155, 200), "pipelined 192x192"),
-    ((266, 13721, 4424), "pipelined 192x192"), ((131, 19105, 2072), "pipelined 192x128"),
-    ((137, 25461, 264), "pipelined 256x128"), ((2816, 259, 6240), "pipelined 256x128"),
-    ((432, 9491, 4072), "pipelined 256x128"), ((519, 18759, 272), "pipelined 256x256"),
-    ((199, 11317, 6312), "pipelined 256x256"), ((259, 26010, 1752), "pipelined 256x256"),
+    ((186, 8157, 4984), "pipelined 192x192"), ((131, 19105, 2072), "pipelined 192x128"),
+    ((1003, 7001, 616), "pipelined 256x128"), ((2816, 259, 6240), "pipelined 256x128"),
+    ((1262, 5671, 1112), "pipelined 256x128"), ((950, 13327, 336), "pipelined 256x256"),
+    ((199, 11317, 6312), "pipelined 256x256"), ((2807, 5289, 312), "pipelined 256x256"),
     ((408, 36824, 288), "pipelined 256x256"), ((646, 26708, 616), "pipelined 256x256"),   # last round on smaller tiles
     ((230, 16622, 4152), "pipelined 128x128"), ((258, 25173, 2096), "pipelined 192x192"),  # ... in K slices
+    ((463, 9095, 1048), "160x128x64"), ((260, 13347, 1664), "160x128x64"), ((905, 6175, 1128), "160x160x64"),
+    ((443, 11908, 768), "160x160x64"), ((2154, 4499, 800), "160x256x64"), ((2233, 4257, 704), "160x256x64"),
+    ((517, 16923, 312), "192x256x64"), ((723, 15154, 704), "192x256x64"), ((2911, 4675, 584), "224x256x64"),
+    ((2282, 5454, 384), "224x256x64"), ((264, 23283, 4136), "160x256x64"),                 # the last three: chained
+    ((655, 13125, 4104), "192x256x64"), ((387, 21799, 4112), "224x256x64"),
     ((36, 19412, 400), "pipelined 64x128"), ((41, 9311, 8208), "pipelined 64x128"), ((17, 35153, 3392), "pipelined 64x128"),
     ((492, 2108, 136), "pipelined 64x64"), ((2574, 1, 3112), "pipelined 64x64"),
     ((7, 20, 72), "split-K 32x64"), ((11, 5, 2792), "split-K 32x64"), ((39, 2, 176), "split-K 64x64"),
