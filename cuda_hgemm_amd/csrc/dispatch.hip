@@ -613,7 +613,17 @@ Plan plan_for(size_t M, size_t N, size_t K, const PlanLimits &limits) {
         p.kernel = edges ? small_m_edge_kernel(r.kernel, M, N, K) : r.kernel;
         if (p.kernel == KERNEL_NONE) continue;
         switch (p.kernel) {
-            case KERNEL_DECODE_RING: p.splits = decode_ring_waves(M, N, K, cus); break;
+            case KERNEL_DECODE_RING: {
+                p.splits = decode_ring_waves(M, N, K, cus);
+                // Chunks that do not come out even over the waves the rule asks for: dealt unevenly rather than to half as
+                // many waves, where those would walk more than 1024 of K each and a CU has one workgroup at most
+                // (N = 1216 ... 4096, K = 2176 ... 15744: 0.99 ... 1.68x, median 1.25x; 1 x 1984 x 9600 18.4 -> 11.5 us on
+                // eight waves for two).  A shorter walk is latency either way (0.98 ... 1.11x), and with more workgroups
+                // they hide the difference and the even form is ahead (N = 5184 ... 46592: 0.84 ... 1.07x).
+                const int uneven = decode_ring_edge_waves(M, N, K, cus);
+                if (uneven > p.splits && N / 16 <= cus && K > 1024 * (size_t)p.splits) p.kernel = KERNEL_DECODE_RING_EDGE, p.splits = uneven;
+                break;
+            }
             case KERNEL_DECODE_RING_EDGE: p.splits = decode_ring_edge_waves(M, N, K, cus); break;
             case KERNEL_DECODE_RESIDENT: {
                 int chunks = 0;
