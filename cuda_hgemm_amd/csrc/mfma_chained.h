@@ -75,7 +75,7 @@ HGEMM_FOR_EACH_ACC_TILE(X)
 // in a private strip and reads them back row-contiguous, 16 bytes per lane, so a global
 // store instruction writes whole 128-byte lines.  Tile (i, j) of the wave is AccTile<j * TM + i>.
 // EDGE: rows >= M and columns >= N are not stored.
-template <class Cfg, bool EDGE = false>
+template <class Cfg, int EDGE = EDGE_NONE>
 __device__ __forceinline__ void store_chained_tile(unsigned char *lds, half_t *__restrict__ C, int M, int N, int row0,
                                                 int col0, int wave, int lane) {
     constexpr int MI = Cfg::MI, TM = Cfg::PTM, TN = Cfg::PTN, WN = Cfg::WN;
@@ -110,7 +110,7 @@ __device__ __forceinline__ void store_chained_tile(unsigned char *lds, half_t *_
                 if constexpr (!EDGE)
                     store_streaming(reinterpret_cast<u32x4 *>(dst), v);
                 else if (row0 + rd_row + i * MI + it * ROWS_PER_READ < M)
-                    store_piece_edge(dst, v, col0 + rd_col * 8, N);
+                    store_piece_guarded<EDGE>(dst, v, col0 + rd_col * 8, N);
             }
         }
         wave_lds_exchange_point();
@@ -119,7 +119,7 @@ __device__ __forceinline__ void store_chained_tile(unsigned char *lds, half_t *_
 
 // Tile, K slice, copy offsets and operand addresses come from PipeFrame (mfma_pipelined.h), as in the interleaved
 // kernel; EDGE as there.
-template <class Cfg, bool SPLIT = false, bool EDGE = false>
+template <class Cfg, bool SPLIT = false, int EDGE = EDGE_NONE>
 __global__ void __launch_bounds__(Cfg::THREADS)
     hgemm_chained_kernel(const half_t *__restrict__ A, const half_t *__restrict__ B, half_t *__restrict__ C,
                            float *__restrict__ partial, int M, int N, int K, int slices, int tiles_m, int tiles_n,
@@ -320,7 +320,7 @@ __global__ void __launch_bounds__(Cfg::THREADS)
         const uint32_t pre_dst_a = cp_lds + CUR_A * A_BYTES, pre_dst_b = cp_lds + B_REGION + PRV_B * B_BYTES;
         const uint32_t post_dst_a = cp_lds + NXT_A * A_BYTES, post_dst_b = cp_lds + B_REGION + CUR_B * B_BYTES;
         const uint32_t src_a_next = NXT_A * A_BYTES, src_b_cur = CUR_B * B_BYTES, src_b_next = NXT_B * B_BYTES;
-        if constexpr (EDGE && FINAL) {  // all A fragments of the last chunk and its first column's B fragments have landed
+        if constexpr (EDGE == EDGE_ANY && FINAL) {  // all A fragments of the last chunk and its first column's B fragments have landed
             if (frame.tail_dup > 0) {
                 static_for<KSTEPS>([&](auto kk_c) {
                     static_for<TM>([&](auto t) { frame.drop_counted(a_frag[AB][decltype(kk_c)::value][decltype(t)::value], kk_c); });
@@ -393,7 +393,7 @@ __global__ void __launch_bounds__(Cfg::THREADS)
                     __builtin_amdgcn_s_waitcnt((0x3f & 0xf) | ((0x3f >> 4) << 14) | (0x7 << 4) | (n_a << 8));
                 }
                 static_for<KSTEPS>([&](auto kk_c) { lds_landed(b_frag[(j + 1) & 1][decltype(kk_c)::value]); });
-                if constexpr (EDGE && FINAL) {
+                if constexpr (EDGE == EDGE_ANY && FINAL) {
                     if (frame.tail_dup > 0) {
                         static_for<KSTEPS>([&](auto kk_c) { frame.drop_counted(b_frag[(j + 1) & 1][decltype(kk_c)::value], kk_c); });
                         frame.dropped();
@@ -461,8 +461,8 @@ __global__ void __launch_bounds__(Cfg::THREADS)
                                                           (size_t)(wm * Cfg::WM) * BN + wn * Cfg::WN,
                                             BN, BM, BN, wave, lane_late);
         else {
-            const int ld = EDGE ? (int)partial_ld(N) : N;
-            store_wave_tile_f32<Cfg, EDGE>(get, lds, partial + ((size_t)slice * M + row0) * ld + col0, ld, M - row0,
+            const int ld = EDGE == EDGE_ANY ? (int)partial_ld(N) : N;
+            store_wave_tile_f32<Cfg, EDGE != EDGE_NONE>(get, lds, partial + ((size_t)slice * M + row0) * ld + col0, ld, M - row0,
                                            ld - col0, wave, lane_late);
         }
     } else {

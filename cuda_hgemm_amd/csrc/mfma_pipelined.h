@@ -21,6 +21,9 @@
 
 namespace hgemm {
 
+// how much of a product may end inside a tile or chunk (see PipeFrame)
+enum { EDGE_NONE = 0, EDGE_TILE, EDGE_ANY };
+
 template <int BM_, int BN_, int BK_, int WAVES_M_, int WAVES_N_, int STAGES_, int MI_ = 16, int EXTRA_A_ = 0>
 struct PipeConfig : TileConfig<BM_, BN_, BK_, WAVES_M_, WAVES_N_, STAGES_, LOAD_DMA, LDS_SWIZZLE, true> {
     using Base = TileConfig<BM_, BN_, BK_, WAVES_M_, WAVES_N_, STAGES_, LOAD_DMA, LDS_SWIZZLE, true>;
@@ -193,12 +196,21 @@ __device__ __forceinline__ void dma_load16_sv(const void *sbase, uint32_t voff, 
             : "memory", "scc");
 }
 
+// Eight halves of a row of C that may end before them.
+template <int EDGE>
+__device__ __forceinline__ void store_piece_guarded(half_t *dst, const u32x4 &v, int col, int N) {
+    if constexpr (EDGE == EDGE_ANY)
+        store_piece_edge(dst, v, col, N);
+    else if (col < N)
+        store_streaming(reinterpret_cast<u32x4 *>(dst), v);
+}
+
 // Accumulators -> fp16 -> C through LDS for either MFMA shape (operands swapped, so a lane
 // holds groups of four consecutive n of one row m = lane % MI): each wave parks MI rows of
 // its tile in a private strip and reads them back row-contiguous, 16 bytes per lane, so a
 // global store instruction writes whole 128-byte lines.
 // EDGE: rows >= M and columns >= N are not stored.
-template <class Cfg, class Acc, bool EDGE = false>
+template <class Cfg, class Acc, int EDGE = EDGE_NONE>
 __device__ __forceinline__ void store_wave_tile(const Acc (&acc)[Cfg::PTM][Cfg::PTN], unsigned char *lds,
                                                 half_t *__restrict__ C, int M, int N, int row0, int col0, int wave,
                                                 int lane) {
@@ -236,7 +248,7 @@ __device__ __forceinline__ void store_wave_tile(const Acc (&acc)[Cfg::PTM][Cfg::
                 if constexpr (!EDGE)
                     store_streaming(reinterpret_cast<u32x4 *>(dst), v);
                 else if (row0 + rd_row + i * MI + it * ROWS_PER_READ < M)
-                    store_piece_edge(dst, v, col0 + rd_col * 8, N);
+                    store_piece_guarded<EDGE>(dst, v, col0 + rd_col * 8, N);
             }
         }
         wave_lds_exchange_point();
@@ -287,11 +299,12 @@ __device__ __forceinline__ void store_wave_tile_f32(Get get, unsigned char *lds,
 // What both tuned kernels (interleaved below, chained in mfma_chained.h) set up before their loops: which tile
 // and K slice the workgroup computes, the per-lane global offsets of its direct-to-LDS copies, and the LDS
 // addresses its lanes read MFMA operands from.
-// EDGE: M and N end anywhere inside a tile, K % 8 == 0 anywhere inside a chunk.  Copies of rows
-// beyond the matrix are redirected to its last row -- valid memory, products never stored --
+// EDGE_TILE: M and N end inside a tile, N % 8 == 0 and K is whole chunks; EDGE_ANY: N ends anywhere, K % 8 == 0 anywhere
+// inside a chunk (a form of its own: on whole chunks its masks and unaligned stores cost 1 ... 3 %; 2944 x 1344 x 1088
+// 11.4 -> 11.7 us).  Copies of rows beyond the matrix are redirected to its last row -- valid memory, products never stored --
 // which costs nothing inside the loop; only the stores are guarded.  The last chunk is treated
 // as `tail_pieces` says: one scalar minimum per chunk, and the masks in the last iteration.
-template <class Cfg, bool SPLIT, bool EDGE>
+template <class Cfg, bool SPLIT, int EDGE>
 struct PipeFrame {
     static constexpr int BM = Cfg::BM, BN = Cfg::BN, BK = Cfg::BK, MI = Cfg::MI;
     static constexpr int KSTEPS = Cfg::PKSTEPS, CPR = Cfg::CPR, CPS = Cfg::CPS, ROW_BYTES = Cfg::ROW_BYTES;
@@ -309,7 +322,7 @@ struct PipeFrame {
     int tile_m, tile_n;      // the workgroup's tile (wave-uniform)
     int slot, slice;         // its position among the launch's tiles and, in a K-sliced launch, its slice
     int num_k;               // chunks it walks
-    int tail_dup;            // 16-byte pieces at the start of the last chunk that must not count (EDGE)
+    int tail_dup;            // 16-byte pieces at the start of the last chunk that must not count (EDGE_ANY)
     uint32_t last_off;       // byte offset of the last chunk from a_base / b_base
     const unsigned char *a_base, *b_base;  // first chunk of the tile's rows of A and of B
     uint32_t voff[L];        // per-lane byte offset of copy instruction i from a_base (i < A_DMA) or b_base
@@ -353,10 +366,10 @@ struct PipeFrame {
         tile_m = __builtin_amdgcn_readfirstlane(tile_m);  // wave-uniform by construction: keep them in SGPRs
         tile_n = __builtin_amdgcn_readfirstlane(tile_n);
         int first_chunk;
-        const int chunks = EDGE ? (K + BK - 1) / BK : K / BK;
+        const int chunks = EDGE == EDGE_ANY ? (K + BK - 1) / BK : K / BK;
         slice_of_k(chunks, slices, slice, first_chunk, num_k);
         const int k_begin = first_chunk * BK;
-        tail_dup = EDGE && first_chunk + num_k == chunks ? tail_pieces(K, BK) : 0;
+        tail_dup = EDGE == EDGE_ANY && first_chunk + num_k == chunks ? tail_pieces(K, BK) : 0;
         last_off = (uint32_t)((num_k - 1) * (BK * 2) - tail_dup * 16);
 
         // ---- copies: wave w, instruction i fills LDS rows [(i*WAVES + w)*ROWS_PER_DMA, +ROWS_PER_DMA)
@@ -417,7 +430,7 @@ struct PipeFrame {
     // byte offset of chunk c from a_base / b_base
     __device__ __forceinline__ uint32_t chunk_off(int c) const {
         const uint32_t off = (uint32_t)c * (uint32_t)(BK * 2);
-        return EDGE && off > last_off ? last_off : off;
+        return EDGE == EDGE_ANY && off > last_off ? last_off : off;
     }
     // clears what of a fragment of step kk of the last chunk must not count; a landed operand register, not one in flight
     template <class KC>
@@ -432,7 +445,7 @@ struct PipeFrame {
 // STREAM_B: B's copies carry the non-temporal hint.  For one row of tiles against a B that outgrows the Infinity
 // Cache: every byte of B is read once, and as an ordinary read it pushes the A panel every workgroup shares out of
 // L2 and the Infinity Cache.
-template <class Cfg, bool SPLIT = false, bool EDGE = false, bool STREAM_B = false>
+template <class Cfg, bool SPLIT = false, int EDGE = EDGE_NONE, bool STREAM_B = false>
 __global__ void __launch_bounds__(Cfg::THREADS)
     hgemm_pipelined_kernel(const half_t *__restrict__ A, const half_t *__restrict__ B, half_t *__restrict__ C,
                            float *__restrict__ partial, int M, int N, int K, int slices, int tiles_m, int tiles_n,
@@ -579,7 +592,7 @@ __global__ void __launch_bounds__(Cfg::THREADS)
     wait_operands(std::integral_constant<int, 0>{});
 
     const unsigned char *a_next = a_base + AHEAD * BK * 2, *b_next = b_base + AHEAD * BK * 2;
-    uint32_t next_off = frame.chunk_off(AHEAD);  // EDGE: the same as an offset, so that the last chunk is one s_min away
+    uint32_t next_off = frame.chunk_off(AHEAD);  // EDGE_ANY: the same as an offset, so that the last chunk is one s_min away
     // One iteration = one K chunk.  ISSUE: chunk kt+AHEAD exists and is copied now.
     // NEXT: chunk kt+1 exists (the barrier is needed and its operands are prefetched).
     // cur_a / cur_b (ring buffers holding chunk kt) are plain ints or, in the unrolled steady
@@ -590,18 +603,19 @@ __global__ void __launch_bounds__(Cfg::THREADS)
         const int nxt_a = (cur_a + 1 == SA) ? 0 : cur_a + 1;
         const int nxt_b = (cur_b + 1 == SB) ? 0 : cur_b + 1;
         const int fill_a = (cur_a + FILL_OFF_A) % SA, fill_b = (cur_b + FILL_OFF_B) % SB;
-        const unsigned char *a_src = EDGE ? a_base + next_off : a_next, *b_src = EDGE ? b_base + next_off : b_next;  // chunk kt + AHEAD
+        const unsigned char *a_src = EDGE == EDGE_ANY ? a_base + next_off : a_next;  // chunk kt + AHEAD
+        const unsigned char *b_src = EDGE == EDGE_ANY ? b_base + next_off : b_next;
         if constexpr (ISSUE) {
             a_next += BK * 2;
             b_next += BK * 2;
-            if constexpr (EDGE) next_off = next_off + BK * 2 < frame.last_off ? next_off + BK * 2 : frame.last_off;
+            if constexpr (EDGE == EDGE_ANY) next_off = next_off + BK * 2 < frame.last_off ? next_off + BK * 2 : frame.last_off;
         }
         const uint32_t dst_a = cp_lds + fill_a * A_BYTES, dst_b = cp_lds + B_REGION + fill_b * B_BYTES;
         static_for<KSTEPS>([&](auto kk_c) {
             constexpr int kk = decltype(kk_c)::value;
             constexpr int fb = kk & 1, nb = fb ^ 1;  // an even number of steps: step 0 always uses buffer 0
             constexpr bool last = (kk + 1 == KSTEPS);
-            if constexpr (EDGE && !NEXT) {  // the last chunk: its operands of this step have landed
+            if constexpr (EDGE == EDGE_ANY && !NEXT) {  // the last chunk: its operands of this step have landed
                 if (frame.tail_dup > 0) {
                     static_for<TM>([&](auto t) { frame.drop_counted(a_frag[fb][decltype(t)::value], kk_c); });
                     static_for<NSB>([&](auto t) { frame.drop_counted(b_frag[decltype(t)::value], kk_c); });
@@ -699,8 +713,8 @@ __global__ void __launch_bounds__(Cfg::THREADS)
                                                           (size_t)(wm * Cfg::WM) * BN + wn * Cfg::WN,
                                             BN, BM, BN, wave, lane);
         else {
-            const int ld = EDGE ? (int)partial_ld(N) : N;
-            store_wave_tile_f32<Cfg, EDGE>(get, lds, partial + ((size_t)slice * M + row0) * ld + col0, ld, M - row0,
+            const int ld = EDGE == EDGE_ANY ? (int)partial_ld(N) : N;
+            store_wave_tile_f32<Cfg, EDGE != EDGE_NONE>(get, lds, partial + ((size_t)slice * M + row0) * ld + col0, ld, M - row0,
                                            ld - col0, wave, lane);
         }
     } else {
@@ -799,9 +813,25 @@ constexpr bool stream_b_available() {
 }
 inline bool stream_b_pays(int tiles_m, size_t N, size_t K) { return tiles_m == 1 && N * K >= ((size_t)24 << 20); }
 
+// The form of the kernel a product needs (shapes that pipelined_runs admits).
+template <class Cfg>
+int edge_form(size_t M, size_t N, size_t K) {
+    if (K % (size_t)Cfg::BK || N % 8) return EDGE_ANY;
+    return M % Cfg::BM || N % Cfg::BN ? EDGE_TILE : EDGE_NONE;
+}
+
+template <class F>
+void with_edge_form(int form, F &&f) {
+    switch (form) {
+        case EDGE_NONE: f(std::integral_constant<int, EDGE_NONE>{}); break;
+        case EDGE_TILE: f(std::integral_constant<int, EDGE_TILE>{}); break;
+        default: f(std::integral_constant<int, EDGE_ANY>{});
+    }
+}
+
 // Launches workgroup ids [first_block, first_block + blocks) of the tile grid; tail_tiles
 // as in the kernel.
-template <class Cfg, bool SPLIT, bool EDGE>
+template <class Cfg, bool SPLIT, int EDGE>
 void launch_pipelined_impl(const void *A, const void *B, void *C, float *partial, size_t M, size_t N, size_t K,
                            int splits, int first_block = 0, int blocks = -1, int tail_tiles = 0,
                            PipeKernel which = PipeKernel::Auto) {
@@ -864,15 +894,10 @@ void launch_pipelined_with_tail(const void *A, const void *B, void *C, float *pa
     HGEMM_CHECK_MSG(K % 8 == 0 && pipelined_runs<Cfg>(M, N, shortest_slice(K, Cfg::BK, tail_splits)),
                     "%s (tail in %d K slices) needs K %% 8 == 0, shortest slice >= %d (got M=%zu N=%zu K=%zu)",
                     name, tail_splits, Cfg::BK * Cfg::STAGES, M, N, K);
-    if (Cfg::supports(M, N, K)) {
-        launch_pipelined_impl<Cfg, false, false>(A, B, C, nullptr, M, N, K, 1, 0, head);
-        launch_pipelined_impl<Cfg, true, false>(A, B, nullptr, partial, M, N, K, tail_splits, head, tail_tiles,
-                                                tail_tiles);
-    } else {
-        launch_pipelined_impl<Cfg, false, true>(A, B, C, nullptr, M, N, K, 1, 0, head);
-        launch_pipelined_impl<Cfg, true, true>(A, B, nullptr, partial, M, N, K, tail_splits, head, tail_tiles,
-                                               tail_tiles);
-    }
+    with_edge_form(edge_form<Cfg>(M, N, K), [&](auto edge) {
+        launch_pipelined_impl<Cfg, false, decltype(edge)::value>(A, B, C, nullptr, M, N, K, 1, 0, head);
+        launch_pipelined_impl<Cfg, true, decltype(edge)::value>(A, B, nullptr, partial, M, N, K, tail_splits, head, tail_tiles, tail_tiles);
+    });
     constexpr int PIECES = Cfg::BM * Cfg::BN / 8;
     tail_reduce_kernel<Cfg><<<dim3(PIECES / 256 > 8 ? 8 : (PIECES + 255) / 256, tail_tiles), dim3(256), 0, nullptr>>>(
         partial, reinterpret_cast<half_t *>(C), (int)M, (int)N, (int)K, tiles_m, tiles_n, head, tail_tiles, tail_splits);
@@ -883,13 +908,11 @@ template <class Cfg>
 void launch_pipelined(const void *A, const void *B, void *C, size_t M, size_t N, size_t K, const char *name,
                       PipeKernel which = PipeKernel::Auto) {
     check_operands(A, B, C, M, N, K);
-    if (Cfg::supports(M, N, K)) {
-        launch_pipelined_impl<Cfg, false, false>(A, B, C, nullptr, M, N, K, 1, 0, -1, 0, which);
-        return;
-    }
     HGEMM_CHECK_MSG(pipelined_runs<Cfg>(M, N, K), "%s needs K %% 8 == 0, K > %d (got M=%zu N=%zu K=%zu)", name,
                     Cfg::BK * (Cfg::STAGES - 1), M, N, K);
-    launch_pipelined_impl<Cfg, false, true>(A, B, C, nullptr, M, N, K, 1, 0, -1, 0, which);
+    with_edge_form(edge_form<Cfg>(M, N, K), [&](auto edge) {
+        launch_pipelined_impl<Cfg, false, decltype(edge)::value>(A, B, C, nullptr, M, N, K, 1, 0, -1, 0, which);
+    });
 }
 
 // K split into `splits` slices: fp32 partial sums of slice s go to partial[s][M][partial_ld(N)] (the
@@ -899,14 +922,12 @@ void launch_pipelined_split(const void *A, const void *B, float *partial, size_t
                             const char *name) {
     HGEMM_CHECK(splits >= 1 && partial != nullptr);
     const size_t k_len = shortest_slice(K, Cfg::BK, splits);
-    if (K % (size_t)Cfg::BK == 0 && k_len > 0 && Cfg::supports(M, N, k_len)) {
-        launch_pipelined_impl<Cfg, true, false>(A, B, nullptr, partial, M, N, K, splits);
-        return;
-    }
     HGEMM_CHECK_MSG(k_len > 0 && K % 8 == 0 && pipelined_runs<Cfg>(M, N, k_len),
                     "%s (K in %d slices) needs K %% 8 == 0, shortest slice >= %d (got M=%zu N=%zu K=%zu)",
                     name, splits, Cfg::BK * Cfg::STAGES, M, N, K);
-    launch_pipelined_impl<Cfg, true, true>(A, B, nullptr, partial, M, N, K, splits);
+    with_edge_form(edge_form<Cfg>(M, N, K), [&](auto edge) {
+        launch_pipelined_impl<Cfg, true, decltype(edge)::value>(A, B, nullptr, partial, M, N, K, splits);
+    });
 }
 
 // Whole rounds of workgroups on the Parent tile, the last `tail_tiles` workgroup ids of its
@@ -926,23 +947,21 @@ void launch_pipelined_with_subtiles(const void *A, const void *B, void *C, size_
     HGEMM_CHECK_MSG(pipelined_runs<Parent>(M, N, K) && pipelined_runs<Child>(M, N, K),
                     "%s needs K %% 8 == 0, K > %d (got M=%zu N=%zu K=%zu)", name,
                     64 * ((Parent::STAGES > Child::STAGES ? Parent::STAGES : Child::STAGES) - 1), M, N, K);
-    if (Parent::supports(M, N, K))
-        launch_pipelined_impl<Parent, false, false>(A, B, C, nullptr, M, N, K, 1, 0, head);
-    else
-        launch_pipelined_impl<Parent, false, true>(A, B, C, nullptr, M, N, K, 1, 0, head);
-    const bool edge = !Child::supports(M, N, K);
-    auto kernel = edge ? &hgemm_pipelined_kernel<Child, false, true> : &hgemm_pipelined_kernel<Child, false, false>;
-    static bool configured = [] {
-        HGEMM_CHECK_HIP_ERROR(hipFuncSetAttribute(reinterpret_cast<const void *>(&hgemm_pipelined_kernel<Child, false, true>),
-                                                  hipFuncAttributeMaxDynamicSharedMemorySize, Child::LDS_BYTES));
-        HGEMM_CHECK_HIP_ERROR(hipFuncSetAttribute(reinterpret_cast<const void *>(&hgemm_pipelined_kernel<Child, false, false>),
-                                                  hipFuncAttributeMaxDynamicSharedMemorySize, Child::LDS_BYTES));
-        return true;
-    }();
-    (void)configured;
-    kernel<<<dim3(tail_tiles * sub_m * sub_n), dim3(Child::THREADS), Child::LDS_BYTES, nullptr>>>(
-        reinterpret_cast<const half_t *>(A), reinterpret_cast<const half_t *>(B), reinterpret_cast<half_t *>(C), nullptr,
-        (int)M, (int)N, (int)K, 1, tiles_m, tiles_n, head, 0, (sub_m << 8) | sub_n);
+    with_edge_form(edge_form<Parent>(M, N, K), [&](auto edge) {
+        launch_pipelined_impl<Parent, false, decltype(edge)::value>(A, B, C, nullptr, M, N, K, 1, 0, head);
+    });
+    with_edge_form(edge_form<Child>(M, N, K), [&](auto edge) {
+        auto kernel = &hgemm_pipelined_kernel<Child, false, decltype(edge)::value>;
+        static bool configured = [&] {
+            HGEMM_CHECK_HIP_ERROR(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
+                                                      hipFuncAttributeMaxDynamicSharedMemorySize, Child::LDS_BYTES));
+            return true;
+        }();
+        (void)configured;
+        kernel<<<dim3(tail_tiles * sub_m * sub_n), dim3(Child::THREADS), Child::LDS_BYTES, nullptr>>>(
+            reinterpret_cast<const half_t *>(A), reinterpret_cast<const half_t *>(B), reinterpret_cast<half_t *>(C), nullptr,
+            (int)M, (int)N, (int)K, 1, tiles_m, tiles_n, head, 0, (sub_m << 8) | sub_n);
+    });
     HGEMM_CHECK_HIP_ERROR(hipGetLastError());
 }
 

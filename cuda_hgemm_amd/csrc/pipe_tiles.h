@@ -35,7 +35,7 @@ using Tile224x256 = PipeConfig<224, 256, 64, 2, 2, 2, 16, 1>;
                                                       const char *);                                                    \
     LINKAGE template void launch_pipelined_with_tail<Cfg>(const void *, const void *, void *, float *, size_t, size_t,    \
                                                           size_t, int, int, const char *);
-#define HGEMM_WHOLE_K_LAUNCHER(LINKAGE, Cfg)                                                                            \
+#define HGEMM_WHOLE_K_LAUNCHER(LINKAGE, Cfg)                                                                              \
     LINKAGE template void launch_pipelined<Cfg>(const void *, const void *, void *, size_t, size_t, size_t, const char *, \
                                                 PipeKernel);
 #define HGEMM_SUBTILE_LAUNCHER(LINKAGE, Child)                                                                          \
