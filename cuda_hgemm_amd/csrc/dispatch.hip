@@ -523,6 +523,16 @@ int small_m_edge_kernel(int kernel, size_t M, size_t N, size_t K) {
     }
 }
 
+// An odd number of whole chunks, which no two waves share evenly: on rows of the ring kernel its guarded form instead of the
+// split-K family with its second launch.  M = 1 ... 8, N = 1024 ... 28672, K = 1088 ... 4032: 1.08 ... 1.74x (1 x 1984 x 1344
+// 5.9 -> 3.5 us, 8 x 28672 x 3008 32.6 -> 27.7); M = 9 ... 16 up to N = 8192: 1.06 ... 1.30x; from K = 6000 on mixed (0.93 ...
+// 1.11x).  On rows of the streaming kernel, which such a K shuts out too, below 48 MB of B (17728 x 1088: 1.25 ... 1.35x;
+// 24000 x 1856: 0.96 ... 0.98x).  Below N = 1024 few workgroups share the chip and K slices across them stay.
+bool odd_chunks_on_ring(int kernel, size_t N, size_t K) {
+    if (N % 16 != 0 || N < 1024 || K % 128 != 64 || K < 1024 || K > 4096) return false;
+    return kernel == KERNEL_DECODE_RING || (kernel == KERNEL_DECODE_BN16 && N * K < ((size_t)24 << 20));
+}
+
 // shapes the kernel of a row can run at all (the row is skipped otherwise)
 bool small_m_kernel_supports(int kernel, size_t M, size_t N, size_t K) {
     switch (kernel) {
@@ -608,9 +618,10 @@ Plan plan_for(size_t M, size_t N, size_t K, const PlanLimits &limits) {
         const SmallMRule &r = SMALL_M_RULES[at % SMALL_M_RULE_COUNT];
         const bool edges = at >= SMALL_M_RULE_COUNT;
         if (limits.every_small_m_kernel ? (M < (size_t)r.m_lo || M > (size_t)r.m_hi) : !small_m_rule_covers(r, M, N, K)) continue;
-        if (!edges && !small_m_kernel_supports(r.kernel, M, N, K)) continue;
+        const bool odd_chunks = !edges && !small_m_kernel_supports(r.kernel, M, N, K) && odd_chunks_on_ring(r.kernel, N, K);
+        if (!edges && !odd_chunks && !small_m_kernel_supports(r.kernel, M, N, K)) continue;
         p = Plan();
-        p.kernel = edges ? small_m_edge_kernel(r.kernel, M, N, K) : r.kernel;
+        p.kernel = edges || odd_chunks ? small_m_edge_kernel(r.kernel, M, N, K) : r.kernel;
         if (p.kernel == KERNEL_NONE) continue;
         switch (p.kernel) {
             case KERNEL_DECODE_RING: {

@@ -36,6 +36,9 @@ CASES = [
     ((56, 81, 312), "streaming decode"), ((67, 4295, 272), "streaming decode"), ((67, 146, 280), "streaming decode"),
     ((1, 1984, 9600), "streaming decode, 16 columns per workgroup, per-wave"),             # N and K even, the waves' shares not
     ((18, 4096, 2688), "streaming decode, 16 columns per workgroup, per-wave"),
+    ((3, 1984, 1344), "streaming decode, 16 columns per workgroup, per-wave"),             # an odd number of whole chunks
+    ((16, 1024, 4032), "streaming decode, 16 columns per workgroup, per-wave"),
+    ((8, 17728, 1088), "streaming decode, 16 columns per workgroup, per-wave"),
     ((511, 511, 511), "zero-padded"), ((296, 299, 2113), "zero-padded"), ((3, 1001, 4099), "zero-padded"),
     ((1027, 520, 193), "zero-padded"), ((2591, 11875, 1833), "zero-padded"),
 ]
