@@ -1204,17 +1204,43 @@ extern "C" void hgemm_release_workspace(void) {
     g_heap[dev] = HeapState();
 }
 
+static bool fits_static_workspace(const Plan &p) {
+    return (p.partial_bytes + 255) / 256 * 256 + p.operand_bytes <= STATIC_WORKSPACE_BYTES;
+}
+
+// What hgemm_auto_static_workspace does with a shape whose plan needs more than its array: true, the best plan without a
+// workspace; false, it says so and launches nothing.  Products in whole chunks with aligned rows of C are refused (their plan
+// is too many K slices of a large C).  Others run a kernel with guarded edges; where that is the gather kernel (K % 8 != 0),
+// up to twice the time of the copies it does without, at the rates that kernel was once chosen by (80 TFLOP/s against
+// passes at 3.5 TB/s and 4 TB/s for a B that is only streamed): decode shapes, 16 x 8192 x 4097, but not 4095^3, 1.7 ms of
+// gathering for 0.12 ms.  Copies of more than the heap workspace ever holds leave no other way.
+static bool runs_unaided(size_t M, size_t N, size_t K) {
+    if (N % 8 == 0 && K % 64 == 0) return false;
+    if (cached_plan(M, N, K, true).kernel != KERNEL_RAGGED || padded_bytes(M, N, K) > MAX_PADDED_BYTES) return true;
+    const size_t Np = padded_n(N), Kp = padded_k(K);
+    PlanLimits inner_limits;
+    inner_limits.operand_bytes = 0;
+    const Plan inner = plan_for(M, Np, Kp, inner_limits);
+    const double inner_us = inner.est_us > 0.0 ? inner.est_us : 8.0 + (double)(Np * Kp * 2) / 4e6;
+    const double copies_us = 6.0 + 4.0 * (double)((M + Np) * Kp + (Np != N ? M * Np : 0)) / 3.5e6;
+    return 5.0 + 2.0 * (double)M * (double)N * (double)K / 80e6 <= 2.0 * (copies_us + inner_us);
+}
+
 extern "C" int hgemm_auto_static_workspace(const hgemm_half *A, const hgemm_half *B, hgemm_half *C, size_t M, size_t N,
                                            size_t K) {
     check_operands(A, B, C, M, N, K);
-    const Plan &p = cached_plan(M, N, K);  // the plan hgemm_auto runs: same kernels, same order of additions
-    const size_t partial_bytes = (p.partial_bytes + 255) / 256 * 256;
-    if (partial_bytes + p.operand_bytes > STATIC_WORKSPACE_BYTES) {
-        HLOG("hgemm_auto_static_workspace: the plan for M=%zu N=%zu K=%zu keeps %zu bytes of partial sums and %zu bytes "
-             "of padded operands, the static workspace holds %zu; nothing was launched (hgemm_auto has no such limit)",
-             M, N, K, p.partial_bytes, p.operand_bytes, STATIC_WORKSPACE_BYTES);
-        return 1;
+    const Plan *chosen = &cached_plan(M, N, K);  // the plan hgemm_auto runs: same kernels, same order of additions
+    if (!fits_static_workspace(*chosen)) {
+        if (!runs_unaided(M, N, K)) {
+            HLOG("hgemm_auto_static_workspace: the plan for M=%zu N=%zu K=%zu keeps %zu bytes of partial sums and %zu bytes "
+                 "of padded operands, the static workspace holds %zu; nothing was launched (hgemm_auto has no such limit)",
+                 M, N, K, chosen->partial_bytes, chosen->operand_bytes, STATIC_WORKSPACE_BYTES);
+            return 1;
+        }
+        chosen = &cached_plan(M, N, K, true);
     }
+    const Plan &p = *chosen;
+    const size_t partial_bytes = (p.partial_bytes + 255) / 256 * 256;
     Workspace ws;
     if (partial_bytes + p.operand_bytes > 0) {
         unsigned char *base = static_scratch();

@@ -96,3 +96,19 @@ def test_static_workspace_allocates_nothing_and_rejects_what_does_not_fit(oracle
     B = torch.zeros((N, K), dtype=torch.float16, device=gpu)
     rc, got = _call(hgemm_lib, "hgemm_auto_static_workspace", A, B, M, N, K, gpu)
     assert rc == 1 and np.all(got == POISON)
+
+
+# K % 8 != 0 with copies beyond the array (the gather kernel runs instead), and K slices that do not fit it on sizes that
+# end inside a tile and a chunk (the same tile unsliced)
+@pytest.mark.parametrize("M,N,K", [(5, 35434, 1547), (11, 36904, 1180), (16, 8192, 4097), (45328, 104, 16184)])
+def test_static_workspace_runs_what_needs_none_where_the_plan_does_not_fit(oracle, hgemm_lib, gpu, M, N, K):
+    import torch
+    need = hgemm_lib.auto_workspace_bytes(M, N, K)
+    assert need["partial"] + need["operands"] > hgemm_lib.static_workspace_bytes()
+    gen = torch.Generator(device=gpu).manual_seed(94)
+    A, B = (torch.randint(-1, 2, (rows, K), generator=gen, device=gpu, dtype=torch.int8).half() for rows in (M, N))
+    rc, got = _call(hgemm_lib, "hgemm_auto_static_workspace", A, B, M, N, K, gpu)
+    assert rc == 0
+    for m0 in sorted({0, max(0, M - 16)}):    # ternary operands: sums are whole numbers, rounded to fp16 once
+        rows = slice(m0, min(M, m0 + 16))
+        assert np.array_equal(got[rows], oracle.hgemm(_bits(A[rows].contiguous()), _bits(B))), (M, N, K, m0)
