@@ -782,9 +782,11 @@ Plan plan_for(size_t M, size_t N, size_t K, const PlanLimits &limits) {
         }
     }
     if (p.kernel != KERNEL_NONE) {
-        if (K % 64) {  // copied to rows of whole lines first?
+        if (K % 64) {  // copied to rows of whole lines first?  Not where the model has nothing to say about the copies' plan:
+            // M = 129 ... 192 and K = 1992 ... 2040 reach the one-row rule above only with the copies' K, and a copy of all of
+            // B before a product that is bound by reading B costs 1.4 ... 3x (160 x 28672 x 2040: 73.0 us, 38.3 without)
             Plan copied = plan_on_copies(M, N, K, limits);
-            if (copied.kernel != KERNEL_NONE && copied.est_us < p.est_us && !left_out(limits, copied)) return copied;
+            if (copied.est_us > 0.0 && copied.est_us < p.est_us && !left_out(limits, copied)) return copied;
         }
         return p;
     }
