@@ -8,3 +8,11 @@ def test_no_copies_below_the_one_row_rule(hgemm_lib, M, N):
     """K just short of 2048: the copies' padded K would be the first the 192x128 one-row rule covers."""
     for K in range(1992, 2048, 8):
         assert hgemm_lib.auto_workspace_bytes(M, N, K)["operands"] == 0, K
+
+
+@pytest.mark.parametrize("size", [4600, 5112, 6200])
+def test_tuner_times_direct_plans_beside_copies(hgemm_lib, size):
+    """K a multiple of 8 and not of 64: copied operands are one plan of several, wherever they come in the order."""
+    plans = hgemm_lib.tune_plans(size, size, size, 8)
+    on_copies = [p["kernel"].startswith("zero-padded") for p in plans]
+    assert len(plans) >= 4 and sum(on_copies) == 1, plans
