@@ -303,12 +303,16 @@ constexpr double OFF_LINE = 1.27;
 constexpr double COPY_US = 3.5, COPY_BYTES_PER_US = 5500e3;
 size_t padded_n(size_t N) { return (N + 7) / 8 * 8; }
 size_t padded_k(size_t K) { return (K + 63) / 64 * 64; }
-// What a plan with copied operands reserves, and hgemm_auto_workspace_bytes reports: A' (M x K'), B' (N' x K') and, when N
-// is no multiple of 8, as much again as a C' (M x N') would take.  The copies are M + N rows of K'; the rest is a bound that
-// callers size their reservations by.
-size_t padded_bytes(size_t M, size_t N, size_t K) {
+// What a plan with copied operands keeps in the workspace: M + N rows of whole chunks.
+size_t copy_bytes(size_t M, size_t N, size_t K) { return (M + N) * padded_k(K) * sizeof(half_t); }
+// What hgemm_auto_workspace_bytes reports for it and hgemm_auto_static_workspace holds against its array: where N is no
+// multiple of 8 also room for a C' (M x N'), up to the cap of the heap workspace.  C is written in place and nothing is
+// kept there; callers have sized reservations by the figure, so it stays, and decides no plan.
+size_t reported_copy_bytes(size_t M, size_t N, size_t K) {
     const size_t Np = padded_n(N), Kp = padded_k(K);
-    return ((M + Np) * Kp + (Np != N ? M * Np : 0)) * sizeof(half_t);
+    const size_t bytes = ((M + Np) * Kp + (Np != N ? M * Np : 0)) * sizeof(half_t);
+    const size_t kept = copy_bytes(M, N, K);
+    return bytes <= MAX_PADDED_BYTES ? bytes : kept > MAX_PADDED_BYTES ? kept : MAX_PADDED_BYTES;
 }
 
 double predict_us(const Candidate &c, size_t M, size_t N, size_t K, int splits, size_t cus) {
@@ -592,7 +596,7 @@ bool left_out(const PlanLimits &limits, int kernel, int splits, int tail_tiles =
 // One pass that copies A and B with rows of whole 64-wide chunks, then the plan for that K (same products, same result);
 // no plan where the copies do not fit.
 Plan plan_on_copies(size_t M, size_t N, size_t K, const PlanLimits &limits) {
-    if (K < 192 || padded_bytes(M, N, K) > limits.operand_bytes) return Plan();
+    if (K < 192 || copy_bytes(M, N, K) > limits.operand_bytes) return Plan();
     PlanLimits inner_limits;
     inner_limits.partial_bytes = limits.partial_bytes;
     inner_limits.operand_bytes = 0;
@@ -600,7 +604,7 @@ Plan plan_on_copies(size_t M, size_t N, size_t K, const PlanLimits &limits) {
     p.inner_kernel = p.kernel;
     p.kernel = KERNEL_PADDED;
     if (p.est_us > 0.0) p.est_us += COPY_US + 4.0 * (double)((M + N) * padded_k(K)) / COPY_BYTES_PER_US;
-    p.operand_bytes = padded_bytes(M, N, K);
+    p.operand_bytes = copy_bytes(M, N, K);
     return p;
 }
 
@@ -1207,8 +1211,8 @@ extern "C" void hgemm_release_workspace(void) {
     g_heap[dev] = HeapState();
 }
 
-static bool fits_static_workspace(const Plan &p) {
-    return (p.partial_bytes + 255) / 256 * 256 + p.operand_bytes <= STATIC_WORKSPACE_BYTES;
+static bool fits_static_workspace(const Plan &p, size_t M, size_t N, size_t K) {
+    return (p.partial_bytes + 255) / 256 * 256 + (p.operand_bytes ? reported_copy_bytes(M, N, K) : 0) <= STATIC_WORKSPACE_BYTES;
 }
 
 // What hgemm_auto_static_workspace does with a shape whose plan needs more than its array: true, the best plan without a
@@ -1216,10 +1220,10 @@ static bool fits_static_workspace(const Plan &p) {
 // is too many K slices of a large C).  Others run a kernel with guarded edges; where that is the gather kernel (K % 8 != 0),
 // up to twice the time of the copies it does without, at the rates that kernel was once chosen by (80 TFLOP/s against
 // passes at 3.5 TB/s and 4 TB/s for a B that is only streamed): decode shapes, 16 x 8192 x 4097, but not 4095^3, 1.7 ms of
-// gathering for 0.12 ms.  Copies of more than the heap workspace ever holds leave no other way.
+// gathering for 0.12 ms.  Where the reported figure reaches the cap of the heap workspace, the gather kernel is what has always run.
 static bool runs_unaided(size_t M, size_t N, size_t K) {
     if (N % 8 == 0 && K % 64 == 0) return false;
-    if (cached_plan(M, N, K, true).kernel != KERNEL_RAGGED || padded_bytes(M, N, K) > MAX_PADDED_BYTES) return true;
+    if (cached_plan(M, N, K, true).kernel != KERNEL_RAGGED || reported_copy_bytes(M, N, K) >= MAX_PADDED_BYTES) return true;
     const size_t Np = padded_n(N), Kp = padded_k(K);
     PlanLimits inner_limits;
     inner_limits.operand_bytes = 0;
@@ -1233,11 +1237,11 @@ extern "C" int hgemm_auto_static_workspace(const hgemm_half *A, const hgemm_half
                                            size_t K) {
     check_operands(A, B, C, M, N, K);
     const Plan *chosen = &cached_plan(M, N, K);  // the plan hgemm_auto runs: same kernels, same order of additions
-    if (!fits_static_workspace(*chosen)) {
+    if (!fits_static_workspace(*chosen, M, N, K)) {
         if (!runs_unaided(M, N, K)) {
             HLOG("hgemm_auto_static_workspace: the plan for M=%zu N=%zu K=%zu keeps %zu bytes of partial sums and %zu bytes "
                  "of padded operands, the static workspace holds %zu; nothing was launched (hgemm_auto has no such limit)",
-                 M, N, K, chosen->partial_bytes, chosen->operand_bytes, STATIC_WORKSPACE_BYTES);
+                 M, N, K, chosen->partial_bytes, chosen->operand_bytes ? reported_copy_bytes(M, N, K) : 0, STATIC_WORKSPACE_BYTES);
             return 1;
         }
         chosen = &cached_plan(M, N, K, true);
@@ -1267,7 +1271,7 @@ extern "C" size_t hgemm_static_workspace_bytes(void) { return STATIC_WORKSPACE_B
 
 extern "C" size_t hgemm_auto_workspace_bytes(size_t M, size_t N, size_t K, size_t *operand_bytes) {
     const Plan p = current_plan(M, N, K);
-    if (operand_bytes) *operand_bytes = p.operand_bytes;
+    if (operand_bytes) *operand_bytes = p.operand_bytes ? reported_copy_bytes(M, N, K) : 0;
     return p.partial_bytes;
 }
 extern "C" int hgemm_auto_supports(size_t M, size_t N, size_t K) { return M > 0 && N > 0 && K > 0; }

@@ -16,3 +16,11 @@ def test_tuner_times_direct_plans_beside_copies(hgemm_lib, size):
     plans = hgemm_lib.tune_plans(size, size, size, 8)
     on_copies = [p["kernel"].startswith("zero-padded") for p in plans]
     assert len(plans) >= 4 and sum(on_copies) == 1, plans
+
+
+@pytest.mark.parametrize("M,N,K", [(24001, 24001, 1001), (16385, 16385, 8191), (20001, 20001, 4001)])
+def test_copies_are_planned_by_what_is_copied(hgemm_lib, M, N, K):
+    """(M + N) rows of whole chunks within the workspace's 1 GiB, whatever a C of that size would take."""
+    assert 2 * (M + N) * ((K + 63) // 64 * 64) <= 1 << 30
+    assert hgemm_lib.auto_plan(M, N, K)["kernel"].startswith("zero-padded")
+    assert hgemm_lib.auto_workspace_bytes(M, N, K)["operands"] <= 1 << 30
