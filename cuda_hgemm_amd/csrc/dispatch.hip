@@ -18,6 +18,7 @@ namespace {
 
 constexpr size_t MAX_PARTIAL_BYTES = PlanLimits().partial_bytes;
 constexpr size_t MAX_PADDED_BYTES = PlanLimits().operand_bytes;
+constexpr size_t SMALL_PADDED_BYTES = (size_t)64 << 20;
 constexpr int MAX_DEVICES = 64;
 
 int current_device() {
@@ -30,7 +31,9 @@ int current_device() {
 // Heap workspaces of hgemm_auto / hgemm_skinny, one pair per device, kept for the life of
 // the process (the reference keeps its vendor handle the same way,
 // src/cublas_tensor_op.cu:18).  Each is allocated once, at its cap, the first time a plan
-// needs it (or by hgemm_reserve_workspace).  If the cap cannot be had, the size asked for is
+// needs it (or by hgemm_reserve_workspace).  Operand copies have two buffers: most calls that need one copy a few MB
+// (192 x 192 x 1001: 0.8 MB) and are no reason to hold 1 GiB, so copies of up to 64 MiB get a buffer of that size, unless the
+// large one is there.  If the cap cannot be had, the size asked for is
 // tried, and sizes hipMalloc has refused are remembered so that no later call asks again.
 // An entry point never frees or replaces a buffer: a plan that needs more than the buffer
 // holds (possible only after such a refusal) is not run, the caller plans again without a
@@ -43,7 +46,9 @@ int current_device() {
 // partial-sum kernel with the other's reduction, and no thread holds a workspace pointer
 // while another frees it.
 struct HeapState {
-    Workspace ws;
+    Workspace ws;  // partial sums, large operand copies
+    unsigned char *small_operands = nullptr;
+    size_t small_bytes = 0, small_refused = SIZE_MAX;
     size_t partial_refused = SIZE_MAX, operand_refused = SIZE_MAX;  // smallest size hipMalloc has refused
 };
 std::mutex g_heap_mutex;
@@ -82,10 +87,15 @@ bool heap_workspace(size_t partial_bytes, size_t operand_bytes, Workspace *out, 
     if (partial_bytes > w.partial_bytes)
         ok = grow(reinterpret_cast<void **>(&w.partial), &w.partial_bytes, partial_bytes, MAX_PARTIAL_BYTES,
                   &h.partial_refused, may_replace) && ok;
-    if (operand_bytes > w.operand_bytes)
+    const bool small = !may_replace && operand_bytes > w.operand_bytes && operand_bytes <= SMALL_PADDED_BYTES;
+    if (small)
+        ok = grow(reinterpret_cast<void **>(&h.small_operands), &h.small_bytes, operand_bytes, SMALL_PADDED_BYTES,
+                  &h.small_refused, false) && ok;
+    else if (operand_bytes > w.operand_bytes)
         ok = grow(reinterpret_cast<void **>(&w.operands), &w.operand_bytes, operand_bytes, MAX_PADDED_BYTES,
                   &h.operand_refused, may_replace) && ok;
     *out = w;
+    if (small) out->operands = h.small_operands, out->operand_bytes = h.small_bytes;
     return ok;
 }
 
@@ -1205,7 +1215,9 @@ extern "C" void hgemm_release_workspace(void) {
     const int dev = current_device();
     std::lock_guard<std::mutex> lock(g_heap_mutex);
     Workspace &w = g_heap[dev].ws;
-    if (w.partial || w.operands) HGEMM_CHECK_HIP_ERROR(hipDeviceSynchronize());  // launches may still use them
+    unsigned char *small = g_heap[dev].small_operands;
+    if (w.partial || w.operands || small) HGEMM_CHECK_HIP_ERROR(hipDeviceSynchronize());  // launches may still use them
+    if (small) HGEMM_CHECK_HIP_ERROR(hipFree(small));
     if (w.partial) HGEMM_CHECK_HIP_ERROR(hipFree(w.partial));
     if (w.operands) HGEMM_CHECK_HIP_ERROR(hipFree(w.operands));
     g_heap[dev] = HeapState();

@@ -169,11 +169,11 @@ int hgemm_small_m_rule(int index, size_t *bounds, int *flags);
 
 /* ---- workspace of hgemm_auto / hgemm_skinny.  Plans that cut K into slices keep fp32
  * partial sums in device memory, and shapes with K % 8 != 0 (large ones with K % 64 != 0 too)
- * run on zero-padded copies of A and B.  Both buffers belong to the library, one pair per device,
+ * run on zero-padded copies of A and B.  These buffers belong to the library, one set per device,
  * and live until hgemm_release_workspace or the end of the process (the reference keeps its
  * vendor handle the same way, src/cublas_tensor_op.cu:18).  Each is allocated ONCE, at its
- * cap (512 MiB of partial sums, 1 GiB of operand copies), by the first call that needs it:
- * that one call contains a hipMalloc; no later call frees or synchronises, and none
+ * cap (512 MiB of partial sums; 64 MiB of operand copies, a second buffer of 1 GiB for larger ones), by
+ * the first call that needs it: that one call contains a hipMalloc; no later call frees or synchronises, and none
  * allocates unless that first hipMalloc was refused (then the size the plan needs is tried
  * once; refused sizes are remembered and not asked for again).  Callers that cannot have
  * even that (a timed loop) reserve beforehand.  If the memory cannot be had, hgemm_auto

@@ -112,3 +112,26 @@ def test_static_workspace_runs_what_needs_none_where_the_plan_does_not_fit(oracl
     for m0 in sorted({0, max(0, M - 16)}):    # ternary operands: sums are whole numbers, rounded to fp16 once
         rows = slice(m0, min(M, m0 + 16))
         assert np.array_equal(got[rows], oracle.hgemm(_bits(A[rows].contiguous()), _bits(B))), (M, N, K, m0)
+
+
+def test_small_operand_copies_hold_a_small_buffer(oracle, hgemm_lib, gpu):
+    """K % 8 != 0: 0.5 ... 34 MB of copies take a workspace of 64 MiB, not the 1 GiB that large copies share, and a large one
+    that is there already serves them too."""
+    import torch
+    for M, N, K in [(1, 1000, 193), (192, 192, 1001), (64, 4096, 4097), (700, 1333, 515)]:
+        Ab, Bb = oracle.fill((M, K), 95, 1, oracle.TERNARY, 0, 1), oracle.fill((N, K), 95, 2, oracle.TERNARY, 0, 1)
+        A, B, C = _to_gpu(Ab, gpu), _to_gpu(Bb, gpu), torch.empty((M, N), dtype=torch.float16, device=gpu)
+        partial = hgemm_lib.auto_workspace_bytes(M, N, K)["partial"]
+        for reserved in (0, 1 << 20):
+            hgemm_lib.release_workspace()
+            print(f"[gpu] hgemm_auto M={M} N={N} K={K}", flush=True)
+            hgemm_lib.call("hgemm_auto", A, B, C, M, N, K)      # loads the kernels
+            hgemm_lib.release_workspace()
+            hgemm_lib.reserve_workspace(partial, reserved)
+            torch.cuda.synchronize()
+            free_before = torch.cuda.mem_get_info()[0]
+            C.zero_()
+            hgemm_lib.call("hgemm_auto", A, B, C, M, N, K)
+            assert np.array_equal(_bits(C), oracle.hgemm(Ab, Bb)), (M, N, K)
+            assert free_before - torch.cuda.mem_get_info()[0] <= (0 if reserved else 66 << 20), (M, N, K, reserved)
+    hgemm_lib.release_workspace()
