@@ -62,7 +62,7 @@ __global__ void __launch_bounds__(RING_MAX_WAVES * 64)
     const int n0 = blockIdx.x * 16;
     int k_begin = wave * k_per_wave, num_k = k_per_wave / 64;
     if constexpr (EDGE) {
-        slice_of_k((K + 63) / 64, waves, wave, k_begin, num_k);
+        slice_of_k(chunks_of(K, 64), waves, wave, k_begin, num_k);
         k_begin *= 64;
     }
     const int tail_dup = EDGE && wave == waves - 1 ? tail_pieces(K, 64) : 0;

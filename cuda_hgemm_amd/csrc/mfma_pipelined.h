@@ -366,7 +366,7 @@ struct PipeFrame {
         tile_m = __builtin_amdgcn_readfirstlane(tile_m);  // wave-uniform by construction: keep them in SGPRs
         tile_n = __builtin_amdgcn_readfirstlane(tile_n);
         int first_chunk;
-        const int chunks = EDGE == EDGE_ANY ? (K + BK - 1) / BK : K / BK;
+        const int chunks = EDGE == EDGE_ANY ? chunks_of(K, BK) : K / BK;
         slice_of_k(chunks, slices, slice, first_chunk, num_k);
         const int k_begin = first_chunk * BK;
         tail_dup = EDGE == EDGE_ANY && first_chunk + num_k == chunks ? tail_pieces(K, BK) : 0;

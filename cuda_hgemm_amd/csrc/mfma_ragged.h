@@ -37,7 +37,7 @@ __global__ void __launch_bounds__(RaggedConfig::THREADS)
     // one-dimensional grid, row-major over the tiles of C: no 65535 limit on either dimension
     const int tiles_n = (N + Cfg::BN - 1) / Cfg::BN;
     const int m0 = (int)(blockIdx.x / tiles_n) * Cfg::BM, n0 = (int)(blockIdx.x % tiles_n) * Cfg::BN;
-    const int num_k = (K + BK - 1) / BK;
+    const int num_k = chunks_of(K, BK);
 
     // eight consecutive k of one row, zero where the row or k is outside the matrix
     auto fetch = [&](const half_t *__restrict__ base, int row, int rows, int k) -> half8 {

@@ -48,7 +48,7 @@ __global__ void __launch_bounds__(Cfg::THREADS)
     const int tile_n = (int)blockIdx.x % tiles_n, tile_m = (int)blockIdx.x / tiles_n, split = blockIdx.y;
     const int m0 = tile_m * BM;
     int first_chunk, num_k;  // K's chunks are dealt to the slices as evenly as whole chunks allow
-    const int chunks = EDGE ? (K + BK - 1) / BK : K / BK;
+    const int chunks = EDGE ? chunks_of(K, BK) : K / BK;
     slice_of_k(chunks, splits, split, first_chunk, num_k);
     const int k_begin = first_chunk * BK;
     const int tail_dup = EDGE && first_chunk + num_k == chunks ? tail_pieces(K, BK) : 0;

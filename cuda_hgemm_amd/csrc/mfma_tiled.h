@@ -28,6 +28,7 @@
 #include <type_traits>
 
 #include "common.h"
+#include "k_chunks.h"
 #include "tile_order.h"
 
 namespace hgemm {
@@ -88,24 +89,11 @@ struct TileConfig {
     }
 };
 
-// K in slices of whole chunks, as even as that allows: the first `chunks % slices` slices walk one chunk more.
-// Slice `slice` starts at chunk `first` and walks `count`.
-__host__ __device__ __forceinline__ void slice_of_k(int chunks, int slices, int slice, int &first, int &count) {
-    const int base = chunks / slices, longer = chunks % slices;
-    first = slice * base + (slice < longer ? slice : longer);
-    count = base + (slice < longer ? 1 : 0);
-}
 // the length of the shortest of `splits` such slices of K (chunks of `bk`, the last one perhaps not full), in whole
 // chunks: what a kernel's minimum K applies to
 inline size_t shortest_slice(size_t K, int bk, int splits) { return div_ceil(K, (size_t)bk) / (size_t)splits * (size_t)bk; }
 
-// ---- K that ends inside a chunk (K % 8 == 0, so rows still start on 16-byte boundaries).  The last chunk is read from
-// K - 64 on instead of from its own beginning: every copy stays inside the matrix and as aligned as the others, and
-// only a wave-uniform base address changes.  The chunk then starts with `tail_dup` 16-byte pieces that the chunk
-// before it has already multiplied; both operands' registers of those pieces are cleared before the last chunk's MFMAs
-// (both, because a product of a cleared and an infinite element would be NaN).  Padding the operands instead cost two
-// launches and 4 (M + N) K bytes: 1000^3 16.4 -> 7.8 us.
-__device__ __forceinline__ int tail_pieces(int K, int bk) { return ((K + bk - 1) / bk * bk - K) >> 3; }
+// what `tail_pieces` leaves of an operand register
 __device__ __forceinline__ half8 keep_or_zero(half8 v, bool keep) {
     u32x4 bits = __builtin_bit_cast(u32x4, v);
 #pragma unroll
@@ -295,7 +283,7 @@ __global__ void __launch_bounds__(Cfg::THREADS)
     }
 
     int first_chunk, num_k;
-    const int chunks = EDGE ? (K + BK - 1) / BK : K / BK;
+    const int chunks = EDGE ? chunks_of(K, BK) : K / BK;
     slice_of_k(chunks, slices, slice, first_chunk, num_k);
     const int k_begin = first_chunk * BK;
     const int tail_dup = EDGE && first_chunk + num_k == chunks ? tail_pieces(K, BK) : 0;

@@ -94,3 +94,16 @@ def test_call_refuses_what_it_refused_before_on_every_call(hgemm_lib, gpu):
             hgemm_lib.call("hgemm_mfma_base", A, B, C, 48, 40, 64)
         with pytest.raises(KeyError, match="no such"):
             hgemm_lib.call("no such", A, B, C, 48, 40, 64)
+
+
+def test_the_longest_k(hgemm_lib, gpu):
+    """K within one chunk of 2^31: chunk counts round up without leaving 32 bits."""
+    import torch
+    K = (1 << 31) - 56
+    A, B = torch.zeros((1, K), dtype=torch.float16, device=gpu), torch.zeros((1, K), dtype=torch.float16, device=gpu)
+    at = torch.tensor([0, 7, 63, 64, K // 2, K - 65, K - 64, K - 57, K - 56, K - 9, K - 8, K - 1], device=gpu)
+    A[0, at], B[0, at] = 1.0, 3.0
+    C = torch.empty((1, 1), dtype=torch.float16, device=gpu)
+    print(f"[gpu] hgemm_auto M=1 N=1 K={K}", flush=True)
+    hgemm_lib.call("hgemm_auto", A, B, C, 1, 1, K)
+    assert C.item() == 3.0 * len(at)
