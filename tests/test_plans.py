@@ -24,3 +24,13 @@ def test_copies_are_planned_by_what_is_copied(hgemm_lib, M, N, K):
     assert 2 * (M + N) * ((K + 63) // 64 * 64) <= 1 << 30
     assert hgemm_lib.auto_plan(M, N, K)["kernel"].startswith("zero-padded")
     assert hgemm_lib.auto_workspace_bytes(M, N, K)["operands"] <= 1 << 30
+
+
+@pytest.mark.parametrize("M,K,sliced", [(58, 1664, True), (83, 1072, True), (121, 2304, True), (13, 512, False), (26, 544, False)])
+def test_slice_counts_below_one_tile_of_columns(hgemm_lib, M, K, sliced):
+    """The split-K family goes by whole tiles: N = 8 and 17 as N = 64, except below K = 896, where they stay unsliced."""
+    whole = hgemm_lib.auto_plan(M, 64, K)
+    for N in (8, 17):
+        plan = hgemm_lib.auto_plan(M, N, K)
+        if plan["kernel"] == whole["kernel"]:
+            assert plan["splits"] == (whole["splits"] if sliced else 1), (N, plan)
