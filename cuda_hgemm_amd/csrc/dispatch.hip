@@ -537,6 +537,39 @@ int small_m_edge_kernel(int kernel, size_t M, size_t N, size_t K) {
     }
 }
 
+// Whole chunks with aligned rows of C (N % 8 == 0, K % 64 == 0): the pipelined tiles further below run these with guarded
+// edges too, so a row's stand-in has to be the faster one.  Timed against them over M = 1 ... 128, N = 8 ... 65536, K = 64 ...
+// 32768 (5500 shapes; what they take, then the stand-in):
+// * Ring kernel: 1.0 ... 2.3x ahead, but behind where few workgroups walk a long K (N <= 1024 from K of about 16384 on, N <= 1536
+//   from 20480: 4 x 96 x 32704 11.6 us, 18.3), where eight waves a workgroup leave a CU no room for a second one and the
+//   second or third round fills less than a third of the chip (8 x 4200 x 19008 33.2 us, 43.1), and by 1 ... 12 % for M > 32
+//   with more workgroups than CUs up to K = 512.
+// * 32x64 and 64x64 split-K tiles: 1.0 ... 1.5x ahead, but 0.86 ... 1.0x beyond K = 16384 at N <= 64, where their 16 slices end
+//   (42 x 8 x 29568 10.8 us, 12.7), and the latter 0.69 ... 0.95x at M > 32 from N = 16384 on.
+// * 128x64 split-K tile: 1.0 ... 1.1x ahead up to K = 1664, and 0.95 ... 1.15x up to K = 8192 at N <= 4096 and for N = 1536 ... 3072;
+//   beyond, 0.73 ... 1.05x (75 x 5808 x 25920 57.8 us, 79.0) until its unsliced tiles fill three quarters of the chip (113 x
+//   12496 x 2368 25.8 us, 19.5); 0.6 ... 1.0x at N <= 2048 between K = 128 and 2560, where partial sums of more than 64 rows
+//   outweigh so short a K (117 x 8 x 1216 6.4 us, 10.5), except for N up to 256 from K = 12 M on (102 x 40 x 1664 7.0, 5.8).
+// * The 128-column split-K tiles: 0.53 ... 1.1x, geomean 0.8 (114 x 50336 x 128 6.2 us, 11.7).
+bool stand_in_pays(int kernel, size_t M, size_t N, size_t K, size_t cus) {
+    if (N % 8 || K % 64) return true;
+    switch (kernel) {
+        case KERNEL_DECODE_RING_EDGE: {
+            const size_t tiles = div_ceil(N, (size_t)16), last = tiles % cus;
+            if ((N <= 1024 && K > 16384) || (N <= 1536 && K > 20480) || (M > 32 && tiles > cus && K <= 512)) return false;
+            return decode_ring_edge_waves(M, N, K, cus) < 8 || tiles <= cus || tiles > 3 * cus || last == 0 || last * 3 >= cus;
+        }
+        case KERNEL_SPLIT_32x64: return N > 64 || K <= 16384;
+        case KERNEL_SPLIT_64x64: return N < 16384 && (N > 64 || K <= 16384);
+        case KERNEL_SPLIT_128x64:
+            if (N >= 16384 || (N <= 2048 && K > 128 && K < 2560 && (N > 256 || K < 896 || K < 12 * M))) return false;
+            return K <= 1664 || (N <= 4096 && K <= 8192) || (N >= 1536 && N <= 3072) || div_ceil(N, (size_t)64) * 4 > cus * 3;
+        case KERNEL_SPLIT_64x128:
+        case KERNEL_SPLIT_128x128: return false;
+        default: return true;
+    }
+}
+
 // An odd number of whole chunks, which no two waves share evenly: on rows of the ring kernel its guarded form instead of the
 // split-K family with its second launch.  M = 1 ... 8, N = 1024 ... 28672, K = 1088 ... 4032: 1.08 ... 1.74x (1 x 1984 x 1344
 // 5.9 -> 3.5 us, 8 x 28672 x 3008 32.6 -> 27.7); M = 9 ... 16 up to N = 8192: 1.06 ... 1.30x; from K = 6000 on mixed (0.93 ...
@@ -637,6 +670,10 @@ Plan plan_for(size_t M, size_t N, size_t K, const PlanLimits &limits) {
         p = Plan();
         p.kernel = edges || odd_chunks ? small_m_edge_kernel(r.kernel, M, N, K) : r.kernel;
         if (p.kernel == KERNEL_NONE) continue;
+        if (edges && !limits.every_small_m_kernel && !stand_in_pays(p.kernel, M, N, K, cus)) {
+            p = Plan();
+            break;
+        }
         switch (p.kernel) {
             case KERNEL_DECODE_RING: {
                 p.splits = decode_ring_waves(M, N, K, cus);

@@ -34,3 +34,26 @@ def test_slice_counts_below_one_tile_of_columns(hgemm_lib, M, K, sliced):
         plan = hgemm_lib.auto_plan(M, N, K)
         if plan["kernel"] == whole["kernel"]:
             assert plan["splits"] == (whole["splits"] if sliced else 1), (N, plan)
+
+
+# shape -> what runs it, on whole chunks with aligned rows of C that no row of the small-M table divides: the faster of a
+# pipelined tile and a table kernel's guarded form (microseconds of the two when they were compared)
+@pytest.mark.parametrize("shape,kernel", [
+    ((114, 50336, 128), "pipelined 128x128x64, 4 waves, 2"),   # 6.2, 11.7 on 128x128 split-K
+    ((40, 57864, 128), "pipelined 128x128x64, 4 waves, 2"),    # 6.1, 8.3 on 64x128 split-K
+    ((117, 8, 1216), "pipelined 64x64"),                       # 6.4, 10.5 on 128x64 split-K
+    ((75, 5808, 25920), "pipelined 128x128"),                  # 57.8, 79.0
+    ((42, 8, 29568), "pipelined 64x64"),                       # 10.8, 12.7 on 64x64 split-K
+    ((4, 96, 32704), "pipelined 64x64"),                       # 11.6, 18.3 on the ring kernel
+    ((8, 4200, 19008), "pipelined 64x64"),                     # 33.2, 43.1
+    ((50, 8072, 320), "pipelined 64x64"),                      # 4.6, 5.3
+    ((1, 3544, 25216), "streaming decode"),                    # 37.1 on the 64x64 tile, 29.0
+    ((6, 640, 640), "streaming decode"),
+    ((113, 12496, 2368), "split-K 128x64"),                    # 25.8, 19.5
+    ((102, 40, 1664), "split-K 128x64"),                       # 7.0, 5.8
+    ((28, 7968, 21952), "split-K 32x64"),                      # 65.1, 57.1
+    ((59, 3240, 24896), "split-K 64x64"),                      # 37.5, 33.4
+    ((84, 11736, 832), "split-K 128x64"),                      # 9.2, 8.4
+])
+def test_small_m_on_whole_chunks_of_ragged_columns(hgemm_lib, shape, kernel):
+    assert hgemm_lib.auto_plan(*shape)["kernel"].startswith(kernel)
