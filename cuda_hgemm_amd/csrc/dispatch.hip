@@ -533,6 +533,8 @@ int small_m_edge_kernel(int kernel, size_t M, size_t N, size_t K) {
         case KERNEL_MID128:
         case KERNEL_ROW64x128: return chunks >= 5 ? kernel : (int)KERNEL_NONE;
         case KERNEL_T192: return chunks >= 3 ? kernel : (int)KERNEL_NONE;
+        // below K = 320, where no pipelined row covers N >= 16384: 0.75 ... 1.0x of the time, geomean 0.84 (35 x 52088 x 88 7.5 -> 5.9 us)
+        case KERNEL_SPLIT_64x128: return N % 8 == 0 && K < 320 ? (int)KERNEL_SPLIT_64x64 : kernel;
         default: return kernel;  // the split-K family
     }
 }
@@ -550,9 +552,12 @@ int small_m_edge_kernel(int kernel, size_t M, size_t N, size_t K) {
 //   beyond, 0.73 ... 1.05x (75 x 5808 x 25920 57.8 us, 79.0) until its unsliced tiles fill three quarters of the chip (113 x
 //   12496 x 2368 25.8 us, 19.5); 0.6 ... 1.0x at N <= 2048 between K = 128 and 2560, where partial sums of more than 64 rows
 //   outweigh so short a K (117 x 8 x 1216 6.4 us, 10.5), except for N up to 256 from K = 12 M on (102 x 40 x 1664 7.0, 5.8).
-// * The 128-column split-K tiles: 0.53 ... 1.1x, geomean 0.8 (114 x 50336 x 128 6.2 us, 11.7).
+// * The 128-column split-K tiles: 0.53 ... 1.1x, geomean 0.8 (114 x 50336 x 128 6.2 us, 11.7).  The 128x128 one also where K ends
+//   inside a chunk, below K = 320 (N = 16384 ... 65536: 0.49 ... 0.97x of the 2-stage 128x128 tile, geomean 0.72; 65 x 34344 x 120
+//   6.9 us, 10.0); not where N % 8 != 0, which costs the pipelined tiles their aligned stores.
 bool stand_in_pays(int kernel, size_t M, size_t N, size_t K, size_t cus) {
-    if (N % 8 || K % 64) return true;
+    if (N % 8) return true;
+    if (K % 64) return K >= 320 || kernel != KERNEL_SPLIT_128x128;
     switch (kernel) {
         case KERNEL_DECODE_RING_EDGE: {
             const size_t tiles = div_ceil(N, (size_t)16), last = tiles % cus;

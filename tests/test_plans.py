@@ -57,3 +57,14 @@ def test_slice_counts_below_one_tile_of_columns(hgemm_lib, M, K, sliced):
 ])
 def test_small_m_on_whole_chunks_of_ragged_columns(hgemm_lib, shape, kernel):
     assert hgemm_lib.auto_plan(*shape)["kernel"].startswith(kernel)
+
+
+# K ends inside one of its first five chunks, N = 16384 ... 65536 with aligned rows of C (microseconds before and after)
+@pytest.mark.parametrize("shape,kernel", [
+    ((65, 34344, 120), "pipelined 128x128x64, 4 waves, 2"),    # 10.0, 6.9 (128x128 split-K before)
+    ((117, 40784, 104), "pipelined 128x128x64, 4 waves, 2"),
+    ((35, 52088, 88), "split-K 64x64"),                        # 7.5, 5.9 (64x128 split-K before)
+    ((69, 23286, 88), "split-K 128x128"),                      # rows of C not aligned
+])
+def test_small_m_on_short_k(hgemm_lib, shape, kernel):
+    assert hgemm_lib.auto_plan(*shape)["kernel"].startswith(kernel)
