@@ -68,3 +68,19 @@ def test_small_m_on_whole_chunks_of_ragged_columns(hgemm_lib, shape, kernel):
 ])
 def test_small_m_on_short_k(hgemm_lib, shape, kernel):
     assert hgemm_lib.auto_plan(*shape)["kernel"].startswith(kernel)
+
+
+# K of one chunk, or one and a part, on ragged sizes (microseconds on the tile that ran them before, now)
+@pytest.mark.parametrize("shape,kernel", [
+    ((2308, 40, 80), "split-K 64x64"),                         # 4.4, 3.8
+    ((163, 991, 128), "split-K 64x64"),                        # 4.8, 3.5
+    ((147, 20, 72), "pipelined 128x128"),                      # less than one 64-column tile, rows of C not aligned
+    ((428, 10574, 96), "pipelined 128x128"),                   # too many tiles
+    ((11111, 10444, 72), "guarded"),                           # 119, 98
+    ((8077, 37696, 72), "pipelined 128x128"),                  # whole lines of C
+    ((2315, 55336, 64), "guarded"),                            # 153, 99
+    ((2315, 55296, 64), "split-K 64x64"),                      # whole tiles of columns
+    ((300, 1000, 64), "split-K 64x64"),                        # small C
+])
+def test_ragged_sizes_on_one_or_two_chunks(hgemm_lib, shape, kernel):
+    assert hgemm_lib.auto_plan(*shape)["kernel"].startswith(kernel)
