@@ -307,9 +307,19 @@ double reduce_us(int slices, double elems) {
 constexpr double TAIL_US = 3.6, TAIL_SUB_US = 4.4;
 // K that is no multiple of 64: a 128-byte piece of a row straddles two cache lines, so the copies into LDS ask L2 for twice
 // the lines.  Chunk times grow by this factor (5112^3 269 us where 5120^3 takes 208; 1.18 ... 1.30 from 1000^3 to 8184^3), and from
-// about 4500^3 on it is cheaper to copy both operands first (5112^3 245 us, 8184^3 863 -> 802 us; 4000^2 x 4040 103 against 112).
+// about 4500^3 on it is cheaper to copy both operands first (5112^3 266 us directly, 196 on copies; 4000^2 x 4040 97, 110).
 constexpr double OFF_LINE = 1.27;
-// that copy: fixed, and per byte read and written (20 us for 4095^2 twice)
+// On tiles of 192x192 and unsliced ones of 256x128, K = 4200 ... 12000 (in slices from 6000), a direct product takes longer than
+// that in proportion.  75 shapes where the figures alone prefer it by less than this: 1.15x as long as on copies, 54 of them by more
+// than 5 %, 7 shorter (1391 x 4586 x 7592 146 us directly, 102 on copies; 2190 x 3878 x 11528 207, 158; 757 x 14816 x 11168 259,
+// 332).  Not on other tiles, where it is ahead as often as behind.
+double direct_weight(int kernel, int splits, size_t K) {
+    const bool longer = kernel == KERNEL_T192 || (kernel == KERNEL_R256x128 && splits == 1);
+    return longer && K >= (splits == 1 ? 4200u : 6000u) && K < 12000 ? 1.18 : 1.0;
+}
+// that copy: launch and gap, and per byte read and written.  Measured 5.0 us for 8 MB, 11.2 for 72, 23.7 for 134 (4095^2 twice) and
+// 87.2 for 536; the rate is lower than those say by the 1.14 by which the tiles' figures exceed measurement, so that the two
+// compare (27.9 for 134 MB)
 constexpr double COPY_US = 3.5, COPY_BYTES_PER_US = 5500e3;
 size_t padded_n(size_t N) { return (N + 7) / 8 * 8; }
 size_t padded_k(size_t K) { return (K + 63) / 64 * 64; }
@@ -865,7 +875,7 @@ Plan plan_for(size_t M, size_t N, size_t K, const PlanLimits &limits) {
             // M = 129 ... 192 and K = 1992 ... 2040 reach the one-row rule above only with the copies' K, and a copy of all of
             // B before a product that is bound by reading B costs 1.4 ... 3x (160 x 28672 x 2040: 73.0 us, 38.3 without)
             Plan copied = plan_on_copies(M, N, K, limits);
-            if (copied.est_us > 0.0 && copied.est_us < p.est_us && !left_out(limits, copied)) return copied;
+                        if (copied.est_us > 0.0 && copied.est_us < p.est_us * direct_weight(p.kernel, p.splits, K) && !left_out(limits, copied)) return copied;
         }
         return p;
     }

@@ -84,3 +84,17 @@ def test_small_m_on_short_k(hgemm_lib, shape, kernel):
 ])
 def test_ragged_sizes_on_one_or_two_chunks(hgemm_lib, shape, kernel):
     assert hgemm_lib.auto_plan(*shape)["kernel"].startswith(kernel)
+
+
+@pytest.mark.parametrize("shape,copied", [
+    ((1391, 4586, 7592), True),      # 146 us directly, 102
+    ((2190, 3878, 11528), True),     # 207, 158
+    ((5112, 5112, 5112), True),      # 266, 196
+    ((1198, 9512, 11240), False),    # 210, 286
+    ((4000, 4000, 4000), False),     # 81.5, 98.0
+    ((3296, 3584, 3488), False),     # 54.6, 64.8
+    ((1000, 1000, 1000), False),
+])
+def test_copies_of_aligned_rows_where_they_pay(hgemm_lib, shape, copied):
+    """K a multiple of 8 and not of 64 runs on guarded kernels or on copies with rows of whole cache lines."""
+    assert hgemm_lib.auto_plan(*shape)["kernel"].startswith("zero-padded") == copied
