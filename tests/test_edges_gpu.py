@@ -76,6 +76,41 @@ def test_sizes_inside_tiles_and_chunks(oracle, hgemm_lib, gpu, shape, kernel):
     assert M == 1 or bool(torch.isfinite(C[:row]).all())
 
 
+# The tiles between 128x128 and 256x256 on whole chunks with aligned rows of C: M and N whole tiles, or ending inside one, each a
+# form of its own, and on the interleaved or (K of 4096 on; three of the tiles have it) the chained kernel, with stores of its own
+FORMS = [
+    ((160, 16640, 320), "160x128x64", False), ((131, 17008, 320), "160x128x64", False),
+    ((320, 19840, 320), "160x160x64", False), ((139, 33016, 320), "160x160x64", False),
+    ((320, 24832, 256), "160x256x64", False), ((259, 22120, 256), "160x256x64", False),
+    ((640, 11776, 4096), "160x256x64", True), ((277, 24016, 4160), "160x256x64", True), ((600, 14336, 4096), "160x256x64", True),
+    ((384, 25600, 320), "192x256x64", False), ((486, 16608, 320), "192x256x64", False),
+    ((1344, 7424, 4160), "192x256x64", True), ((652, 13080, 4288), "192x256x64", True),
+    ((224, 33280, 320), "224x256x64", False), ((408, 22168, 320), "224x256x64", False),
+    ((448, 22272, 4096), "224x256x64", True), ((389, 22560, 4096), "224x256x64", True),
+]
+
+
+@pytest.mark.parametrize("shape,tile,chained", FORMS)
+def test_every_form_of_the_tiles_between(oracle, hgemm_lib, gpu, shape, tile, chained):
+    """Exact on ternary inputs inside a guard band, C starting as NaN: eight rows from every 61 (so every row of tiles, wave and
+    register group of one) against the checker, the rest written and finite."""
+    import torch
+    M, N, K = shape
+    plan = hgemm_lib.auto_plan(M, N, K)
+    assert plan["kernel"].startswith(tile) and plan["chained"] == chained and plan["splits"] == 1 and plan["tail_tiles"] == 0, plan
+    A, B = oracle.fill((M, K), 33, 1, oracle.TERNARY, 0, 1), oracle.fill((N, K), 33, 2, oracle.TERNARY, 0, 1)
+    buf = torch.full((GUARD + M * N + GUARD,), POISON, dtype=torch.int16, device=gpu)
+    C = buf[GUARD:GUARD + M * N].view(torch.float16).view(M, N)
+    print(f"[gpu] hgemm_auto M={M} N={N} K={K} {plan['kernel']} chained {chained}", flush=True)
+    hgemm_lib.call("hgemm_auto", _gpu_bits(A, gpu), _gpu_bits(B, gpu), C, M, N, K)
+    host = buf.cpu().numpy().view(np.uint16)
+    assert np.all(host[:GUARD] == POISON) and np.all(host[GUARD + M * N:] == POISON)
+    got = host[GUARD:GUARD + M * N].reshape(M, N)
+    assert not np.any((got & 0x7C00) == 0x7C00), "outputs left unwritten or non-finite"
+    rows = np.unique(np.concatenate([np.arange(m0, min(M, m0 + 8)) for m0 in range(0, M, 61)] + [np.arange(M - 8, M)]))
+    assert np.array_equal(got[rows], oracle.hgemm(np.ascontiguousarray(A[rows]), B))
+
+
 def test_call_refuses_what_it_refused_before_on_every_call(hgemm_lib, gpu):
     """Operands pass the binding's one-expression check or are told why not, also after calls that were in order."""
     import torch

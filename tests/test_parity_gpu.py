@@ -355,7 +355,8 @@ def test_auto_last_round_of_a_large_grid(oracle, hgemm_lib, gpu, shape, mode):
 
 
 @pytest.mark.parametrize("variant,shape", [
-    ("hgemm_auto", (520, 9480, 8192)),                    # 3 x 38 tiles of 256: clipped blocks, ragged M and N
+    ("hgemm_auto", (520, 9480, 8192)),                    # 4 x 60 tiles of 160: clipped blocks, ragged M and N
+    ("hgemm_mfma_chained_256x256", (520, 9480, 8192)),    # 3 x 38 tiles of 256, clipped likewise
     ("hgemm_auto", (4352, 9472, 8192)),                   # 17 x 37 tiles: whole rounds plus a last, separately launched one
     ("hgemm_mfma_chained_256x256", (2304, 9472, 8192)),   # 9 x 37 tiles in one launch
     ("hgemm_mfma_pipelined_256x256", (2304, 9472, 8192)),
