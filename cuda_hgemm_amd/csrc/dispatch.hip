@@ -285,7 +285,7 @@ constexpr Candidate CANDIDATES[] = {
 // load differs from one board to the next; only ratios matter to the choice).  One is taken in place of a plan of whole,
 // unsliced tiles where it is predicted BETWEEN_MARGIN ahead, about the error of the fits.  A plan that already fills its
 // last round, in K slices or on smaller tiles, stays: there these measured 0.90 ... 1.12x, not what was predicted.
-// 600 x 14336 x 4096 78.4 -> 61.8 us (160x256), 1.06 ... 1.16x on drawn shapes of 10 ... 35 us.
+// 600 x 14336 x 4096 83 -> 67 us (160x256; operands that change from call to call), 1.06 ... 1.16x on drawn shapes of 10 ... 35 us.
 constexpr Candidate BETWEEN_TILES[] = {
     {KERNEL_T160x128, 160, 128, 1, 4, 3.60, 0.341, 0.547}, {KERNEL_T160x160, 160, 160, 1, 4, 4.89, 0.336, 0.667},
     {KERNEL_T160x256, 160, 256, 1, 3, 4.83, 0.543, 1.018}, {KERNEL_T192x256, 192, 256, 1, 2, 5.57, 0.612, 1.181},
@@ -587,7 +587,8 @@ bool stand_in_pays(int kernel, size_t M, size_t N, size_t K, size_t cus) {
 
 // An odd number of whole chunks, which no two waves share evenly: on rows of the ring kernel its guarded form instead of the
 // split-K family with its second launch.  M = 1 ... 8, N = 1024 ... 28672, K = 1088 ... 4032: 1.08 ... 1.74x (1 x 1984 x 1344
-// 5.9 -> 3.5 us, 8 x 28672 x 3008 32.6 -> 27.7); M = 9 ... 16 up to N = 8192: 1.06 ... 1.30x; from K = 6000 on mixed (0.93 ...
+// 5.9 -> 3.5 us, 8 x 28672 x 3008 32.6 -> 27.7); M = 9 ... 16 up to N = 8192: 1.06 ... 1.30x; M = 17 ... 32, N = 1024 ... 4096, up to
+// K = 4032: 1.47 ... 2.15x, M = 33 ... 64 up to K = 1984: 0.99 ... 1.90x (62 x 1792 x 1472 7.2 -> 5.0); from K = 6000 on mixed (0.93 ...
 // 1.11x).  On rows of the streaming kernel, which such a K shuts out too, below 48 MB of B (17728 x 1088: 1.25 ... 1.35x;
 // 24000 x 1856: 0.96 ... 0.98x).  Below N = 1024 few workgroups share the chip and K slices across them stay.
 bool odd_chunks_on_ring(int kernel, size_t N, size_t K) {
@@ -710,7 +711,7 @@ Plan plan_for(size_t M, size_t N, size_t K, const PlanLimits &limits) {
                 // Chunks that do not come out even over the waves the rule asks for: dealt unevenly rather than to half as
                 // many waves, where those would walk more than 1024 of K each and a CU has one workgroup at most
                 // (N = 1216 ... 4096, K = 2176 ... 15744: 0.99 ... 1.68x, median 1.25x; 1 x 1984 x 9600 18.4 -> 11.5 us on
-                // eight waves for two).  A shorter walk is latency either way (0.98 ... 1.11x), and with more workgroups
+                // eight waves for two; N = 16 ... 1200, K up to 25500: 0.99 ... 2.30x, geomean 1.58).  A shorter walk is latency either way (0.98 ... 1.11x), and with more workgroups
                 // they hide the difference and the even form is ahead (N = 5184 ... 46592: 0.84 ... 1.07x).
                 const int uneven = decode_ring_edge_waves(M, N, K, cus);
                 if (uneven > p.splits && N / 16 <= cus && K > 1024 * (size_t)p.splits) p.kernel = KERNEL_DECODE_RING_EDGE, p.splits = uneven;

@@ -784,7 +784,8 @@ namespace hgemm {
 // not issue slots) and a K long enough to pay for its longer prologue.  Measured on an MI355X
 // against the interleaved kernel, tile by tile, over grids of 64 to 1024 tiles and K from 512
 // to 8192: 256x256 ahead (1-4 %) from K = 1536 on once most CUs have a tile, 256x128 and
-// 192x192 from K = 4096 on, 128x128 and 64x64 behind everywhere.
+// 192x192 from K = 4096 on, 128x128 and 64x64 behind everywhere.  160x256: level up to K = 3000, 1.03x on average from there
+// (1.0 ... 1.14); 192x256 and 224x256: level at every K from 1000 to 10000 (0.97 ... 1.03x, 140 shapes), so they share the rule.
 enum class PipeKernel { Auto, Interleaved, Chained };
 template <class Cfg>
 constexpr bool chained_available() {

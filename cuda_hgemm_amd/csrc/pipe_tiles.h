@@ -20,7 +20,8 @@ using Row192x128 = PipeConfig<192, 128, 64, 2, 2, 4, 16>;
 using Tile192 = PipeConfig<192, 192, 64, 2, 2, 3, 16>;
 using Rect256x128 = PipeConfig<256, 128, 64, 2, 2, 3, 16>;
 // Sizes between those, for products whose tiles of the sizes above leave part of the chip idle in their last round or run
-// past M: 600 x 14336 x 4096 is 168 tiles of 256x256 (78.4 us), 224 of 160x256 (61.8 us).  Wave tiles are any multiple
+// past M: 600 x 14336 x 4096 is 168 tiles of 256x256 (84 us on operands that stay cached, 83 on operands that change from call
+// to call), 224 of 160x256 (60, 67).  Wave tiles are any multiple
 // of the 16x16 MFMA tile.  The rings are as deep as 160 KB allow (192 and 224 rows: two B buffers, three A buffers).
 using Tile160x128 = PipeConfig<160, 128, 64, 2, 2, 4, 16>;
 using Tile160x160 = PipeConfig<160, 160, 64, 2, 2, 4, 16>;
