@@ -657,14 +657,14 @@ bool left_out(const PlanLimits &limits, int kernel, int splits, int tail_tiles =
 // * Fewer 128x128 tiles than half the CUs: the 64x64 split-K tile, 0.60 ... 0.89x of the time (2308 x 40 x 80 4.4 -> 3.8 us).  N of
 //   less than one such tile only with aligned rows of C.
 // * Bound by writing C, in lines that rows not a multiple of 32 bytes straddle: the guarded 128x128x32 kernel, whose 8-byte
-//   stores merge in L2.  One chunk from C of 3 M elements on 0.64 ... 1.13x (2315 x 55336 x 64 153 us, 99); up to K = 80 from
-//   16 rounds of 128x128 tiles on 0.77 ... 0.96x (11111 x 10444 x 72 119 us, 98).
+//   stores merge in L2.  One chunk from C of 3 M elements on 0.64 ... 1.13x (2315 x 55336 x 64 153 us, 99); up to K = 96 from
+//   16 rounds of 128x128 tiles on 0.77 ... 0.96x (11111 x 10444 x 72 119 us, 98; 7873 x 56748 x 88 471, 399).
 int short_k_kernel(size_t M, size_t N, size_t K, size_t cus) {
     const size_t tiles = div_ceil(M, (size_t)128) * div_ceil(N, (size_t)128);
     if (K > 128 || (N % 8 == 0 && K % 64 == 0 && K > 64)) return KERNEL_NONE;
     if (K == 64) return N % 64 && N % 4 == 0 && M * N >= ((size_t)3 << 20) ? KERNEL_RAGGED : KERNEL_NONE;
     if (M > 128 && tiles * 2 <= cus && (N % 8 == 0 || N >= 64)) return KERNEL_SPLIT_64x64;
-    return K <= 80 && N % 4 == 0 && N % 16 && tiles > 16 * cus ? KERNEL_RAGGED : KERNEL_NONE;
+    return K <= 96 && N % 4 == 0 && N % 16 && tiles > 16 * cus ? KERNEL_RAGGED : KERNEL_NONE;
 }
 
 // One pass that copies A and B with rows of whole 64-wide chunks, then the plan for that K (same products, same result);

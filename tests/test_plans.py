@@ -77,6 +77,7 @@ def test_small_m_on_short_k(hgemm_lib, shape, kernel):
     ((147, 20, 72), "pipelined 128x128"),                      # less than one 64-column tile, rows of C not aligned
     ((428, 10574, 96), "pipelined 128x128"),                   # too many tiles
     ((11111, 10444, 72), "guarded"),                           # 119, 98
+    ((7873, 56748, 88), "guarded"),                            # 471, 399
     ((8077, 37696, 72), "pipelined 128x128"),                  # whole lines of C
     ((2315, 55336, 64), "guarded"),                            # 153, 99
     ((2315, 55296, 64), "split-K 64x64"),                      # whole tiles of columns
