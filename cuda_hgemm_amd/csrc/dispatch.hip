@@ -317,8 +317,8 @@ double direct_weight(int kernel, int splits, size_t K) {
     const bool longer = kernel == KERNEL_T192 || (kernel == KERNEL_R256x128 && splits == 1);
     return longer && K >= (splits == 1 ? 4200u : 6000u) && K < 12000 ? 1.18 : 1.0;
 }
-// that copy: launch and gap, and per byte read and written.  Measured 5.0 us for 8 MB, 11.2 for 72, 23.7 for 134 (4095^2 twice) and
-// 87.2 for 536; the rate is lower than those say by the 1.14 by which the tiles' figures exceed measurement, so that the two
+// that copy: launch and gap, and per byte read and written.  Measured on operands that change 5.0 us for 8 MB, 11.2 for 72, 23.7 for 134
+// (4095^2 twice; 19.6 on operands that stay cached) and 87.2 for 536; the rate is lower than those say by the 1.14 by which the tiles' figures exceed measurement, so that the two
 // compare (27.9 for 134 MB)
 constexpr double COPY_US = 3.5, COPY_BYTES_PER_US = 5500e3;
 size_t padded_n(size_t N) { return (N + 7) / 8 * 8; }
