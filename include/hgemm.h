@@ -191,7 +191,8 @@ int hgemm_reserve_workspace(size_t partial_bytes, size_t operand_bytes);
 /* Waits for the device and frees its workspaces. */
 void hgemm_release_workspace(void);
 /* Bytes of partial sums (return value) and of operand copies (*operand_bytes, if not NULL)
- * that hgemm_auto's plan for the shape uses. */
+ * that hgemm_auto's plan for the shape uses (copies: with room for a padded C where N % 8 != 0, up to
+ * 1 GiB, an upper bound). */
 size_t hgemm_auto_workspace_bytes(size_t M, size_t N, size_t K, size_t *operand_bytes);
 
 /* hgemm_auto for callers that cannot allocate device memory (serving loops, harnesses that
