@@ -746,9 +746,10 @@ Plan plan_for(size_t M, size_t N, size_t K, const PlanLimits &limits) {
             default: {  // the split-K family: K slices across workgroups, then the ordered reduction
                 const size_t bn = (r.kernel == KERNEL_SPLIT_64x128 || r.kernel == KERNEL_SPLIT_128x128) ? 128 : 64;
                 // By whole tiles: an N of 8 takes as long as one of 64 (57 x 8 x 1552 unsliced 8.9 us, in 12 slices as at N = 64
-                // 5.5; 83 x 17 x 1072 9.5, 6.0).  Below K = 896 what N itself asks for, i.e. no slices at N < 64: the second
-                // launch costs more than they return (9 x 24 x 424 3.8 us, in three slices 6.0; level from 830 to 950).
-                const size_t columns = K >= 896 ? div_ceil(N, bn) * bn : N;
+                // 5.5; 83 x 17 x 1072 9.5, 6.0).  Below K = 896, and 1280 on the 32-row tile, what N itself asks for, which is
+                // no slices at N = 8: the second launch costs more than they return (9 x 24 x 424 3.8 us, in three slices 6.0;
+                // 16 x 3 x 1072 6.4, 7.4; 48 x 8 x 944 6.1, 5.9).
+                const size_t columns = K >= (p.kernel == KERNEL_SPLIT_32x64 ? 1280u : 896u) ? div_ceil(N, bn) * bn : N;
                 p.splits = choose_splits(div_ceil(N, bn), M, columns, cus, K, slice_bytes, limits.partial_bytes);
                 if (p.splits > 1) p.partial_bytes = (size_t)p.splits * slice_bytes;
             }

@@ -26,14 +26,15 @@ def test_copies_are_planned_by_what_is_copied(hgemm_lib, M, N, K):
     assert hgemm_lib.auto_workspace_bytes(M, N, K)["operands"] <= 1 << 30
 
 
-@pytest.mark.parametrize("M,K,sliced", [(58, 1664, True), (83, 1072, True), (121, 2304, True), (13, 512, False), (26, 544, False)])
-def test_slice_counts_below_one_tile_of_columns(hgemm_lib, M, K, sliced):
-    """The split-K family goes by whole tiles: N = 8 and 17 as N = 64, except below K = 896, where they stay unsliced."""
-    whole = hgemm_lib.auto_plan(M, 64, K)
-    for N in (8, 17):
-        plan = hgemm_lib.auto_plan(M, N, K)
-        if plan["kernel"] == whole["kernel"]:
-            assert plan["splits"] == (whole["splits"] if sliced else 1), (N, plan)
+@pytest.mark.parametrize("shape,sliced", [
+    ((58, 8, 1664), True), ((58, 17, 1664), True), ((83, 17, 1072), True), ((121, 17, 2304), True), ((20, 9, 1608), True),
+    ((13, 8, 512), False), ((13, 17, 512), False), ((26, 8, 544), False), ((13, 8, 904), False), ((16, 3, 1072), False)])
+def test_slice_counts_below_one_tile_of_columns(hgemm_lib, shape, sliced):
+    """The split-K family goes by whole tiles, N = 3 ... 17 as N = 64, but for a K of less than 896 (1280 up to M = 32)."""
+    M, N, K = shape
+    plan = hgemm_lib.auto_plan(M, N, K)
+    assert plan["kernel"].startswith("split-K")
+    assert plan["splits"] == (hgemm_lib.auto_plan(M, 64, (K + 63) // 64 * 64)["splits"] if sliced else 1), plan
 
 
 # shape -> what runs it, on whole chunks with aligned rows of C that no row of the small-M table divides: the faster of a
