@@ -6,6 +6,7 @@
 #include "pipe_tiles.h"
 #include "mfma_ragged.h"
 #include "mfma_skinny.h"
+#include "mfma_unaligned.h"
 #include "plan.h"
 
 #include <atomic>
@@ -250,6 +251,12 @@ void launch_small64_w4(const void *A, const void *B, void *C, size_t M, size_t N
     else
         launch_tiled_split<Small64W4Deep, EDGE>(A, B, ws.partial, M, N, K, splits, "hgemm_auto");
     launch_splitk_reduce(ws.partial, reinterpret_cast<half_t *>(C), M, N, splits);
+}
+
+template <class Cfg>
+void launch_unaligned_plan(const void *A, const void *B, void *C, size_t M, size_t N, size_t K, int splits, const Workspace &ws) {
+    HGEMM_CHECK(splits == 1 || (ws.partial != nullptr && ws.partial_bytes >= (size_t)splits * M * partial_ld(N) * sizeof(float)));
+    launch_unaligned<Cfg>(A, B, C, M, N, K, splits, ws.partial);
 }
 
 // ---- cost model for the tile-aligned shapes.  A candidate is a tile (its kernel), how
@@ -682,6 +689,44 @@ Plan plan_on_copies(size_t M, size_t N, size_t K, const PlanLimits &limits) {
     return p;
 }
 
+// K % 8 != 0 read where it lies (mfma_unaligned.h).  Times as in CANDIDATES, of a 128-wide chunk, fitted on 80 shapes (M = 2 ... 4863,
+// N = 5 ... 19948, K = 215 ... 14927, up to 16 slices; rms 6 ... 11 %) and on the same scale as those.  64x64 twice: one
+// workgroup to a CU, and two that share its load path.
+constexpr Candidate UNALIGNED_TILES[] = {
+    {KERNEL_UNALIGNED64, 64, 64, 1, 1, 3.60, 0.539, 0.709},
+    {KERNEL_UNALIGNED64, 64, 64, 2, 1, 3.44, 0.824, 1.361},
+    {KERNEL_UNALIGNED96, 96, 96, 1, 1, 4.81, 0.944, 1.007},
+    {KERNEL_UNALIGNED128x64, 128, 64, 1, 1, 3.95, 0.935, 0.962},
+    {KERNEL_UNALIGNED128, 128, 128, 1, 1, 5.09, 1.206, 1.516},
+};
+// The figures for copies understate them by about this up to some 35 us (1595^2 x 911 18.6 us on copies where they say 13.4, 905^2 x
+// 2305 20.8 and 14.3); beyond, both tables are off by as much either way (880 x 1672 x 7165 40.9 us on copies, 48.9 without).
+constexpr double COPIES_UNDERSTATED_US = 4.0, COPIES_UNDERSTATED_BELOW_US = 40.0;
+bool reads_unaligned_rows(int kernel) {
+    return kernel == KERNEL_UNALIGNED64 || kernel == KERNEL_UNALIGNED96 || kernel == KERNEL_UNALIGNED128x64 || kernel == KERNEL_UNALIGNED128;
+}
+Plan plan_on_unaligned_rows(size_t M, size_t N, size_t K, size_t cus, const PlanLimits &limits) {
+    Plan p;
+    if (!unaligned_runs(K)) return p;
+    const size_t slice_bytes = M * partial_ld(N) * sizeof(float), chunks = div_ceil(K, (size_t)128);
+    for (const Candidate &c : UNALIGNED_TILES) {
+        const size_t tiles = div_ceil(M, (size_t)c.bm) * div_ceil(N, (size_t)c.bn);
+        for (int s = 1; s <= 16 && (size_t)s <= chunks; ++s) {
+            const size_t wgs = tiles * (size_t)s, slots = cus * (size_t)c.per_cu;
+            if (s > 1 && (wgs > 2 * slots || (size_t)s * slice_bytes > limits.partial_bytes)) break;
+            if (wgs >= (size_t)1 << 31 || left_out(limits, c.kernel, s)) continue;
+            if (c.kernel == KERNEL_UNALIGNED64 && (c.per_cu == 1) != (wgs <= cus)) continue;
+            const double t = predict_us(c, M, N, div_ceil(K, (size_t)128) * 64, s, cus);  // (predict_us counts chunks of 64)
+            if (p.kernel != KERNEL_NONE && t >= p.est_us) continue;
+            p.kernel = c.kernel;
+            p.splits = s;
+            p.est_us = t;
+            p.partial_bytes = s > 1 ? (size_t)s * slice_bytes : 0;
+        }
+    }
+    return p;
+}
+
 // M <= 128: choices come from timing every candidate (tile x slices) on the specification's
 // decode shapes on an MI355X, operands rotated so small problems read HBM.  Larger,
 // tile-aligned shapes: the cheapest (tile, slices) pair under the cost model above.
@@ -876,22 +921,38 @@ Plan plan_for(size_t M, size_t N, size_t K, const PlanLimits &limits) {
         if (K % 64) {  // copied to rows of whole lines first?  Not where the model has nothing to say about the copies' plan:
             // M = 129 ... 192 and K = 1992 ... 2040 reach the one-row rule above only with the copies' K, and a copy of all of
             // B before a product that is bound by reading B costs 1.4 ... 3x (160 x 28672 x 2040: 73.0 us, 38.3 without)
-            Plan copied = plan_on_copies(M, N, K, limits);
-                        if (copied.est_us > 0.0 && copied.est_us < p.est_us * direct_weight(p.kernel, p.splits, K) && !left_out(limits, copied)) return copied;
+            const Plan copied = plan_on_copies(M, N, K, limits);
+            if (copied.est_us > 0.0 && copied.est_us < p.est_us * direct_weight(p.kernel, p.splits, K) && !left_out(limits, copied)) return copied;
         }
         return p;
     }
+    if (K % 8) {
+        // Rows of A and B not 16-byte aligned: read where they lie (K from 129 on) or copied first (from 192 on), whichever is
+        // predicted faster.  Against copies alone, 206 shapes drawn over the whole range: 0.96 ... 2.5x, geomean 1.35 (929^3 12.0 -> 8.2 us,
+        // 439^2 x 7179 21.0 -> 13.4, 16 x 8192 x 4097 39.8 -> 18.2, 147 x 22092 x 1853 46.3 -> 35.9); copies stay ahead for large products
+        // (2603^3 46 us, 62 without).  The small-M kernels have no estimate: there B is most of what would be copied, and only where
+        // one to eight rows meet a B of less than 2 MB are copies and the ring kernel ahead (2 x 110 x 1083 5.4 us, 6.1).  K below 129,
+        // and beyond 2^23 where the copies do not fit: the guarded kernel, which gathers such rows element by element (170 x
+        // 214 x 153 23.3 us, 4.6 here).
+        Plan copied = plan_on_copies(M, N, K, limits);
+        if (copied.kernel != KERNEL_NONE && left_out(limits, copied)) copied = Plan();
+        Plan direct = plan_on_unaligned_rows(M, N, K, cus, limits);
+        direct.copies_partial_bytes = copied.partial_bytes;
+        const bool short_b = M <= 8 && N * K < ((size_t)1 << 20);
+        const double understated = copied.est_us < COPIES_UNDERSTATED_BELOW_US ? COPIES_UNDERSTATED_US : 0.0;
+        const bool copy = copied.est_us > 0.0 ? copied.est_us + understated <= direct.est_us : short_b;
+        if (direct.kernel != KERNEL_NONE && !(copied.kernel != KERNEL_NONE && copy)) return direct;
+        if (copied.kernel != KERNEL_NONE) return copied;
+        if (limits.excluded_count == 0) p.kernel = KERNEL_RAGGED;
+        return p;
+    }
     if (limits.excluded_count > 0) return Plan();  // the tuner's question has no further answer
-    if (K % 8 == 0 && K >= 64) {  // K of one or two chunks; any M and N: guarded
+    if (K >= 64) {  // K of one or two chunks; any M and N: guarded
         p.kernel = KERNEL_SPLIT_64x64;
         p.splits = choose_splits(div_ceil(M, 64) * div_ceil(N, 64), M, N, cus, K, slice_bytes, limits.partial_bytes);
         if (p.splits > 1) p.partial_bytes = (size_t)p.splits * slice_bytes;
         return p;
     }
-    // Rows of A and B not 16-byte aligned: on copies from K = 192 on.  Below, and where the copies do not fit, the guarded
-    // kernel, which gathers such rows element by element (4 ... 5 us per 32 of K).
-    const Plan copied = plan_on_copies(M, N, K, limits);
-    if (copied.kernel != KERNEL_NONE) return copied;
     p.kernel = KERNEL_RAGGED;
     return p;
 }
@@ -974,6 +1035,10 @@ void run_plan(const Plan &p, const Workspace &ws, const void *A, const void *B, 
         case KERNEL_DECODE_RING: launch_decode_ring(A, B, C, M, N, K, p.splits); break;
         case KERNEL_DECODE_RING_EDGE: launch_decode_ring_edge(A, B, C, M, N, K, p.splits); break;
         case KERNEL_DECODE_RESIDENT: launch_decode_resident(A, B, C, M, N, K, compute_units()); break;
+        case KERNEL_UNALIGNED64: launch_unaligned_plan<Unaligned64>(A, B, C, M, N, K, p.splits, ws); break;
+        case KERNEL_UNALIGNED96: launch_unaligned_plan<Unaligned96>(A, B, C, M, N, K, p.splits, ws); break;
+        case KERNEL_UNALIGNED128x64: launch_unaligned_plan<Unaligned128x64>(A, B, C, M, N, K, p.splits, ws); break;
+        case KERNEL_UNALIGNED128: launch_unaligned_plan<Unaligned128>(A, B, C, M, N, K, p.splits, ws); break;
         case KERNEL_RAGGED: launch_ragged(A, B, C, M, N, K); break;
         case KERNEL_PADDED: run_padded(p, ws, A, B, C, M, N, K); break;
         case KERNEL_SIMT:
@@ -1300,19 +1365,27 @@ extern "C" void hgemm_release_workspace(void) {
     g_heap[dev] = HeapState();
 }
 
+// Operand bytes reported for a plan: rows read where they lie count as the copies that they once were, so that reservations and
+// what fits the static workspace stay what they were.
+static size_t reported_operand_bytes(const Plan &p, size_t M, size_t N, size_t K) {
+    const bool once_copied = reads_unaligned_rows(p.kernel) && K >= 192 && copy_bytes(M, N, K) <= MAX_PADDED_BYTES;
+    return p.operand_bytes || once_copied ? reported_copy_bytes(M, N, K) : 0;
+}
+static size_t padded_partial_bytes(size_t bytes) { return (bytes + 255) / 256 * 256; }
 static bool fits_static_workspace(const Plan &p, size_t M, size_t N, size_t K) {
-    return (p.partial_bytes + 255) / 256 * 256 + (p.operand_bytes ? reported_copy_bytes(M, N, K) : 0) <= STATIC_WORKSPACE_BYTES;
+    const size_t partial_bytes = reads_unaligned_rows(p.kernel) ? p.copies_partial_bytes : p.partial_bytes;
+    return padded_partial_bytes(partial_bytes) + reported_operand_bytes(p, M, N, K) <= STATIC_WORKSPACE_BYTES;
 }
 
 // What hgemm_auto_static_workspace does with a shape whose plan needs more than its array: true, the best plan without a
 // workspace; false, it says so and launches nothing.  Products in whole chunks with aligned rows of C are refused (their plan
-// is too many K slices of a large C).  Others run a kernel with guarded edges; where that is the gather kernel (K % 8 != 0),
-// up to twice the time of the copies it does without, at the rates that kernel was once chosen by (80 TFLOP/s against
-// passes at 3.5 TB/s and 4 TB/s for a B that is only streamed): decode shapes, 16 x 8192 x 4097, but not 4095^3, 1.7 ms of
-// gathering for 0.12 ms.  Where the reported figure reaches the cap of the heap workspace, the gather kernel is what has always run.
+// is too many K slices of a large C).  Others run a kernel with guarded edges.  Where rows of A and B are not aligned (K % 8 != 0),
+// which products are run was settled when only the gather kernel could: those it took up to twice the time of the copies for, at
+// the rates it was once chosen by (80 TFLOP/s against passes at 3.5 TB/s and 4 TB/s for a B that is only streamed): decode
+// shapes, 16 x 8192 x 4097, but not 4095^3.  Where the reported figure reaches the cap of the heap workspace, all are run.
 static bool runs_unaided(size_t M, size_t N, size_t K) {
     if (N % 8 == 0 && K % 64 == 0) return false;
-    if (cached_plan(M, N, K, true).kernel != KERNEL_RAGGED || reported_copy_bytes(M, N, K) >= MAX_PADDED_BYTES) return true;
+    if ((K % 8 == 0 && cached_plan(M, N, K, true).kernel != KERNEL_RAGGED) || reported_copy_bytes(M, N, K) >= MAX_PADDED_BYTES) return true;
     const size_t Np = padded_n(N), Kp = padded_k(K);
     PlanLimits inner_limits;
     inner_limits.operand_bytes = 0;
@@ -1330,13 +1403,15 @@ extern "C" int hgemm_auto_static_workspace(const hgemm_half *A, const hgemm_half
         if (!runs_unaided(M, N, K)) {
             HLOG("hgemm_auto_static_workspace: the plan for M=%zu N=%zu K=%zu keeps %zu bytes of partial sums and %zu bytes "
                  "of padded operands, the static workspace holds %zu; nothing was launched (hgemm_auto has no such limit)",
-                 M, N, K, chosen->partial_bytes, chosen->operand_bytes ? reported_copy_bytes(M, N, K) : 0, STATIC_WORKSPACE_BYTES);
+                 M, N, K, chosen->partial_bytes, reported_operand_bytes(*chosen, M, N, K), STATIC_WORKSPACE_BYTES);
             return 1;
         }
         chosen = &cached_plan(M, N, K, true);
+    } else if (padded_partial_bytes(chosen->partial_bytes) + chosen->operand_bytes > STATIC_WORKSPACE_BYTES) {
+        chosen = &cached_plan(M, N, K, true);  // (rows read where they lie, in more slices than their copies took)
     }
     const Plan &p = *chosen;
-    const size_t partial_bytes = (p.partial_bytes + 255) / 256 * 256;
+    const size_t partial_bytes = padded_partial_bytes(p.partial_bytes);
     Workspace ws;
     if (partial_bytes + p.operand_bytes > 0) {
         unsigned char *base = static_scratch();
@@ -1360,7 +1435,7 @@ extern "C" size_t hgemm_static_workspace_bytes(void) { return STATIC_WORKSPACE_B
 
 extern "C" size_t hgemm_auto_workspace_bytes(size_t M, size_t N, size_t K, size_t *operand_bytes) {
     const Plan p = current_plan(M, N, K);
-    if (operand_bytes) *operand_bytes = p.operand_bytes ? reported_copy_bytes(M, N, K) : 0;
+    if (operand_bytes) *operand_bytes = reported_operand_bytes(p, M, N, K);
     return p.partial_bytes;
 }
 extern "C" int hgemm_auto_supports(size_t M, size_t N, size_t K) { return M > 0 && N > 0 && K > 0; }
@@ -1440,6 +1515,10 @@ extern "C" const char *hgemm_kernel_name(int kernel) {
         case KERNEL_DECODE_RESIDENT: return "decode with A in registers, persistent workgroups over 16-column tiles, one wave per K slice";
         case KERNEL_RAGGED: return "guarded 128x128x32, 4 waves, any shape";
         case KERNEL_PADDED: return "zero-padded operand copies + kernel of the padded shape";
+        case KERNEL_UNALIGNED64: return "zero-padded chunks of rows read where they lie, 64x64x128, 4 waves";
+        case KERNEL_UNALIGNED96: return "zero-padded chunks of rows read where they lie, 96x96x128, 4 waves";
+        case KERNEL_UNALIGNED128x64: return "zero-padded chunks of rows read where they lie, 128x64x128, 8 waves";
+        case KERNEL_UNALIGNED128: return "zero-padded chunks of rows read where they lie, 128x128x128, 8 waves";
         case KERNEL_SIMT: return "scalar fallback";
         default: return "none";
     }

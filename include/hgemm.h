@@ -206,8 +206,8 @@ size_t hgemm_auto_workspace_bytes(size_t M, size_t N, size_t K, size_t *operand_
  * calls no hipMalloc, hipFree or other allocating routine.  Where the plan needs more than the
  * array holds (hgemm_auto_workspace_bytes tells beforehand) and M, N or K ends inside a tile or chunk
  * (N % 8 != 0 or K % 64 != 0), it runs the best plan that needs no workspace, whose sums may differ from
- * hgemm_auto's in the last bit: the tile without K slices, or for K % 8 != 0 the gather kernel
- * unless that takes more than about twice as long as the copies it does without.  Otherwise it
+ * hgemm_auto's in the last bit: the tile without K slices, or for K % 8 != 0 a kernel that
+ * reads unaligned rows where they lie, except for large products (4095^3).  Otherwise it
  * returns 1 with a message on stderr and nothing launched; else 0.  Other contract violations end
  * the process as everywhere.  All calls on one GPU share that GPU's array, which keeps the last call's
  * contents (nothing in it has to start at zero: every kernel reads only what an earlier
