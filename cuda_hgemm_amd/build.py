@@ -26,7 +26,11 @@ HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = "gfx950"
 # -packed-fp32-ops is switched off on purpose: the packed FP32 forms the compiler would
 # pick by itself are not trusted on this hardware pool.
-DEVICE_FLAGS = ["--offload-arch=" + ARCH, "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
+# Kernel arguments are preloaded: the dispatcher writes the first 14 to 16 dwords of them into scalar registers before a wave
+# starts, where it would otherwise begin with a load and its latency.  0.25 us of every launch that is short enough to show
+# it: 256^3 3.07 -> 2.80 us, 512^3 4.01 -> 3.72, 1 x 4096 x 4096 7.08 -> 6.86; level from about 15 us on.
+DEVICE_FLAGS = ["--offload-arch=" + ARCH, "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+                "-Xarch_device", "-mllvm=-amdgpu-kernarg-preload-count=16"]
 CXXFLAGS = ["-O3", "-std=c++17", "-fPIC", "-Wall", "-Wextra", "-Wno-unused-parameter", "-I" + INCLUDE]
 
 LIB_SOURCES = ["basic_kernels.hip", "ladder_sync.hip", "ladder_async.hip", "ladder_stages.hip", "tiles_256.hip",
