@@ -9,6 +9,8 @@ which is also torch's default stream.  Operands are torch CUDA tensors or
 from __future__ import annotations
 
 import ctypes as C
+import importlib.machinery
+import importlib.util
 import os
 import sys
 from typing import List, Optional
@@ -22,6 +24,10 @@ def lib_path() -> str:
 
 def vendor_lib_path() -> str:
     return os.path.join(_HERE, "lib", "libhgemm_hipblaslt.so")
+
+
+def call_module_path() -> str:
+    return os.path.join(_HERE, "lib", "_call.so")
 
 
 def driver_path() -> str:
@@ -67,6 +73,21 @@ def _share_hip_runtime_with_torch() -> None:
         import torch  # noqa: F401
     except ImportError:
         pass  # a caller without torch brings its own device pointers and the system runtime
+
+
+_call_module = None
+
+
+def _native_calls():
+    """The module that launches on torch tensors without ctypes (``csrc/python_call.cpp``); None in a process without torch,
+    and where torch was not installed when the library was built."""
+    global _call_module
+    if _call_module is None and "torch" in sys.modules and os.path.exists(call_module_path()):
+        loader = importlib.machinery.ExtensionFileLoader("_call", call_module_path())
+        module = importlib.util.module_from_spec(importlib.util.spec_from_loader("_call", loader))
+        loader.exec_module(module)
+        _call_module = module
+    return _call_module
 
 
 # torch.Tensor and torch.float16 from the first tensor on; a process without torch keeps the empty tuple, which nothing
@@ -153,6 +174,12 @@ class HgemmLibrary:
         d.hgemm_variant_run.argtypes, d.hgemm_variant_run.restype = [C.c_int] + _HGEMM_ARGS, C.c_int
         self._run = d.hgemm_variant_run
         self._indices = {}  # variant names seen by call() -> their indices
+        # operands that are plain torch tensors: checked and launched in one native call
+        self._run_address = C.cast(d.hgemm_variant_run, _PTR).value
+        native = _native_calls() if torch_runtime else None
+        self._native_product = native.product if native else None
+        if native:
+            self.call = native.Caller(self._run_address, self._indices, self.call)
         d.hgemm_profile_ms.argtypes = [HGEMM_FN, _PTR, _PTR, _PTR, _SZ, _SZ, _SZ, _SZ, _SZ]
         d.hgemm_profile_ms.restype = C.c_double
         d.hgemm_profile_rotating_ms.argtypes = [HGEMM_FN, C.POINTER(_PTR), C.POINTER(_PTR), C.POINTER(_PTR), _SZ, _SZ,
@@ -381,10 +408,17 @@ def vendor_library(torch_runtime: bool = True) -> VendorLibrary:
 
 def hgemm(A, B, variant: str = "hgemm_auto", out=None):
     """``C = A @ B.T`` for fp16 GPU tensors ``A (M, K)`` and ``B (N, K)`` through variant ``variant``."""
+    lib = _library or library()
+    if out is None and lib._native_product is not None:
+        index = lib._indices.get(variant)
+        if index is not None:
+            product = lib._native_product(lib._run_address, index, A, B)
+            if product is not None:
+                return product
     import torch
     M, K = A.shape
     N = B.shape[0]
     if out is None:
         out = torch.empty((M, N), dtype=torch.float16, device=A.device)
-    (_library or library()).call(variant, A, B, out, M, N, K)
+    lib.call(variant, A, B, out, M, N, K)
     return out

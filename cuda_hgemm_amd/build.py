@@ -2,6 +2,7 @@
 
     cuda_hgemm_amd/lib/libhgemm.so            the kernels + C ABI (include/hgemm.h)
     cuda_hgemm_amd/lib/libhgemm_hipblaslt.so  vendor comparator (include/hgemm_hipblaslt.h)
+    cuda_hgemm_amd/lib/_call.so               the Python calls' launcher for torch tensors (where torch is installed)
     cuda_hgemm_amd/bin/hgemm                  C++ benchmark / check driver
 
 Run as ``python -m cuda_hgemm_amd.build`` (add ``--force`` to rebuild everything).
@@ -10,10 +11,12 @@ hipcc cross-compiles without a GPU, so this works on a CPU-only machine.
 from __future__ import annotations
 
 import concurrent.futures as cf
+import importlib.util
 import os
 import re
 import subprocess
 import sys
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
@@ -37,6 +40,7 @@ LIB_SOURCES = ["basic_kernels.hip", "ladder_sync.hip", "ladder_async.hip", "ladd
                "tiles_224.hip", "tiles_192.hip", "tiles_160.hip", "tiles_128.hip", "tiles_64.hip", "tiles_unaligned.hip", "dispatch.hip", "api.hip"]
 VENDOR_SOURCES = ["vendor_hipblaslt.cpp"]
 DRIVER_SOURCES = ["driver/main.cpp"]
+PYTHON_CALL_SOURCE = "python_call.cpp"
 
 
 def _headers():
@@ -148,12 +152,28 @@ def _compile(src, force):
     return obj
 
 
+def _build_python_call(force):
+    """The module behind HgemmLibrary.call and hgemm() for torch tensors: host code only, against the installed torch."""
+    torch = importlib.util.find_spec("torch")
+    if torch is None or not torch.submodule_search_locations:
+        return None  # a machine without torch: nobody there has a torch tensor either
+    root = list(torch.submodule_search_locations)[0]
+    target, source = os.path.join(LIB, "_call.so"), os.path.join(CSRC, PYTHON_CALL_SOURCE)
+    if force or _stale(target, [source, os.path.join(root, "version.py")]):
+        _run(["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D_GLIBCXX_USE_CXX11_ABI=1", "-I" + os.path.join(root, "include"),
+              "-I" + os.path.join(root, "include", "torch", "csrc", "api", "include"), "-I" + sysconfig.get_path("include"), source,
+              "-o", target, "-L" + os.path.join(root, "lib"), "-ltorch_python", "-ltorch_cpu", "-lc10"])
+    return target
+
+
 def build(force: bool = False, verbose: bool = False) -> dict:
     for d in (OBJ, LIB, BIN):
         os.makedirs(d, exist_ok=True)
     sources = LIB_SOURCES + VENDOR_SOURCES + DRIVER_SOURCES
     with cf.ThreadPoolExecutor(max_workers=min(8, len(sources))) as pool:
+        python_call = pool.submit(_build_python_call, force)
         objs = dict(zip(sources, pool.map(lambda s: _compile(s, force), sources)))
+        python_call.result()
     libhgemm = os.path.join(LIB, "libhgemm.so")
     vendor = os.path.join(LIB, "libhgemm_hipblaslt.so")
     driver = os.path.join(BIN, "hgemm")
