@@ -145,8 +145,8 @@ void launch_splitk_form(const void *A, const void *B, void *C, size_t M, size_t 
     HGEMM_CHECK(EDGE ? K % 8 == 0 && K >= 64 : N % Cfg::BN == 0 && K % (size_t)Cfg::BK == 0);
     HGEMM_CHECK(splits >= 1 && div_ceil(K, (size_t)Cfg::BK) >= (size_t)splits);
     const size_t tiles_n = div_ceil(N, (size_t)Cfg::BN), tiles = tiles_n * div_ceil(M, (size_t)Cfg::BM);  // < 2^31
-    const dim3 grid((unsigned)tiles, (unsigned)splits);
-    HGEMM_CHECK(splits <= 65535);
+    HGEMM_CHECK(tiles * (size_t)splits < ((size_t)1 << 31));
+    const dim3 grid((unsigned)(tiles * (size_t)splits));
     float *partial = nullptr;
     if (splits > 1) {
         HGEMM_CHECK(ws.partial != nullptr && ws.partial_bytes >= (size_t)splits * M * partial_ld(N) * sizeof(float));
@@ -170,12 +170,27 @@ void launch_splitk(const void *A, const void *B, void *C, size_t M, size_t N, si
         launch_splitk_form<Cfg, true>(A, B, C, M, N, K, splits, ws);
 }
 
-//                             BM   BN  WM WN stages
-using Split32x64 = SkinnyConfig<32, 64, 1, 2, 4>;
-using Split64x64 = SkinnyConfig<64, 64, 2, 2, 4>;
-using Split64x128 = SkinnyConfig<64, 128, 2, 2, 4>;
-using Split128x64 = SkinnyConfig<128, 64, 2, 2, 4>;
-using Split128x128 = SkinnyConfig<128, 128, 2, 2, 4>;
+//                             BM   BN  WM WN stages look-ahead
+// Six and five stages leave a CU room for two workgroups (72 and 80 KB).
+using Split32x64 = SkinnyConfig<32, 64, 1, 2, 6>;
+using Split64x64 = SkinnyConfig<64, 64, 2, 2, 5>;
+// ... and for slices of few chunks; 32x64 also for more than two workgroups to a CU, of which three share one at a time
+// (18 x 59328 x 2624 52.5 us, 55.7 on six stages; 16 x 9689 x 14912 in five slices 47.0, 54.4)
+using Split32x64Short = SkinnyConfig<32, 64, 1, 2, 4, false>;
+using Split64x64Short = SkinnyConfig<64, 64, 2, 2, 4, false>;
+using Split64x128 = SkinnyConfig<64, 128, 2, 2, 4, false>;
+using Split128x64 = SkinnyConfig<128, 64, 2, 2, 4, false>;
+using Split128x128 = SkinnyConfig<128, 128, 2, 2, 4, false>;
+
+constexpr size_t SPLIT_SHORT_MAX_CHUNKS = 8;
+template <class Cfg, class Short>
+void launch_splitk_by_length(const void *A, const void *B, void *C, size_t M, size_t N, size_t K, int splits, const Workspace &ws) {
+    const size_t wgs = div_ceil(M, (size_t)Cfg::BM) * div_ceil(N, (size_t)Cfg::BN) * (size_t)splits;
+    if (div_ceil(div_ceil(K, (size_t)64), (size_t)splits) <= SPLIT_SHORT_MAX_CHUNKS || (Cfg::BM == 32 && wgs > 2 * (size_t)compute_units()))
+        launch_splitk<Short>(A, B, C, M, N, K, splits, ws);
+    else
+        launch_splitk<Cfg>(A, B, C, M, N, K, splits, ws);
+}
 
 // 64x64x64 on four waves (one 32x32 MFMA tile each) with the ladder's kernel: a small tile whose chunk takes a quarter
 // of the one-wave tile's matrix-pipe time; for grids that give a CU at most one tile.  Three forms by the number of
@@ -382,20 +397,26 @@ double predict_subtile_us(const Candidate &big, const Candidate &small, size_t M
     return t + TAIL_SUB_US;
 }
 
-// Number of K slices (1 ... 16) for `tiles` output tiles of a split-K kernel, by a model of its time fitted to 91
-// shapes (M = 7 ... 128, N = 1408 ... 65536, K = 384 ... 15104, all five tiles) timed at every slice count on an MI355X,
-// operands rotated so that B streams from HBM:
-//     t(s) = t_B (1 + [s > 1] 8 s M / K) / balance(s) + [s > 1] 1 us,    t_B = 2 N K bytes at 5 TB/s,
+// Number of K slices (1 ... 16) for `tiles` output tiles of a kernel for small M, by a model of its time:
+//     t(s) = t_B / balance(s) + [s > 1] (t_B weight s M / K + overhead),    t_B = 2 N K bytes at 5 TB/s,
 // balance(s) = w / (ceil(w / CUs) CUs) for w = tiles x s workgroups: the busiest CU runs ceil(w / CUs) of them, whether
 // side by side or one after the other, so 144 tiles run better in three slices (432 workgroups, two on most CUs) than
-// in two (288: two on a few CUs, one on the rest) -- M = 48, N = 9216, K = 8192: 43.8 / 45.0 / 35.8 / 41.9 us in 1 ... 4
-// slices.  The middle factor is the traffic of the fp32 partial sums (8 M bytes per slice and column of C, out and
-// back) against B's (2 K bytes per column), counted twice.  The model's choice is 1.2 % behind the best count on
-// average (16 % at worst); the rule it replaces (the smallest power of two that divides K's chunks and gives three
-// quarters of the CUs a workgroup) was 22 % behind on average.  A slice is a whole number of 64-wide chunks, at least
+// in two (288: two on a few CUs, one on the rest).  The second term is the traffic of the fp32 partial sums (8 M bytes per
+// slice and column of C, out and back) against B's (2 K bytes per column), and the launch that adds them.
+//   `weight`, `overhead` (us): 16 and 4 on the tiles up to 64x64, fitted to 140 shapes (M = 9 ... 128, N = 1024 ...
+// 64448, K = 1024 ... 16256, operands rotated) timed at ten counts: 1 ... 4 % behind the best count on average.  Partial sums
+// scaled by the balance too, 8 and 1 us, which this replaced there, chose too many slices since the tiles' loop is faster
+// (6 ... 10 % behind: 12 x 8448 x 1280 in three slices 1.42x the time of one).  The wider and the pipelined tiles keep the older
+// form (`scaled`), fitted to 91 shapes.
+// A slice is a whole number of 64-wide chunks, at least
 // two (`min_chunks`: the pipelined tiles need as many as their ring has stages); slices differ by at most one chunk.
 // `slice_bytes`: fp32 partial sums of one slice; the slices together stay within `limit`.
-int choose_splits(size_t tiles, size_t M, size_t N, size_t cus, size_t K, size_t slice_bytes, size_t limit,
+struct SliceModel {
+    double weight, overhead;
+    bool scaled;  // partial sums scaled by the balance
+};
+constexpr SliceModel SLICES{16.0, 4.0, false}, SLICES_WIDE_TILE{8.0, 1.0, true};
+int choose_splits(const SliceModel &model, size_t tiles, size_t M, size_t N, size_t cus, size_t K, size_t slice_bytes, size_t limit,
                   size_t min_chunks = 2) {
     int best = 1;
     double best_us = 0.0;
@@ -404,8 +425,8 @@ int choose_splits(size_t tiles, size_t M, size_t N, size_t cus, size_t K, size_t
         if (s > 1 && (K % 8 != 0 || div_ceil(K, (size_t)64) / (size_t)s < min_chunks || (size_t)s * slice_bytes > limit)) break;
         const size_t wgs = tiles * (size_t)s;
         const double balance = (double)wgs / (double)(div_ceil(wgs, cus) * cus);
-        const double partials = s > 1 ? 8.0 * s * (double)M / (double)K : 0.0;
-        const double us = stream_us * (1.0 + partials) / balance + (s > 1 ? 1.0 : 0.0);
+        const double partials = s > 1 ? stream_us * model.weight * s * (double)M / (double)K : 0.0;
+        const double us = stream_us / balance + (model.scaled ? partials / balance : partials) + (s > 1 ? model.overhead : 0.0);
         if (s == 1 || us < best_us - 1e-9) {
             best_us = us;
             best = s;
@@ -443,8 +464,7 @@ constexpr SmallMRule SMALL_M_RULES[] = {
     // 57344, M = 1: 0.97 ... 1.18x (N = 28672, K = 4096: 39.2 -> 35.9 us, 82 % of 8 TB/s; N = 57344: 87 %), M = 8:
     // 0.95 ... 1.31x from K = 2048 (ties at K = 1024).
     {1, 8, 1, 8192, 256, 2047, 0, ANY, 0, KERNEL_DECODE_RING},
-    {1, 8, 1, ANY, 2048, 8191, 0, LARGE_B - 1, 0, KERNEL_DECODE_RING},
-    {1, 8, 1, ANY, 8192, ANY, 0, LARGE_B - 1, 0, KERNEL_DECODE_RING},
+    {1, 8, 1, ANY, 2048, ANY, 0, LARGE_B - 1, 0, KERNEL_DECODE_RING},
     {1, 8, 1, ANY, 8192, ANY, LARGE_B, ANY, RULE_K_NOT_16384S, KERNEL_DECODE_RING},
     {1, 5, 1, ANY, 1024, 8191, LARGE_B, ANY, 0, KERNEL_DECODE_RING},
     {6, 8, 1, ANY, 2048, 8191, LARGE_B, ANY, 0, KERNEL_DECODE_RING},
@@ -462,10 +482,8 @@ constexpr SmallMRule SMALL_M_RULES[] = {
     // 151936 (the 64x128 tile's second and later rounds cost it more), so from N = 32768; K <= 3072 mixed (0.68 ... 1.2x),
     // so not taken.
     {9, 16, 18432, ANY, 5120, 5120, (size_t)24 << 20, ANY, 0, KERNEL_DECODE_RESIDENT},
-    {9, 16, 14336, ANY, 10240, 10240, (size_t)24 << 20, ANY, 0, KERNEL_DECODE_RESIDENT},
-    {9, 16, 14336, ANY, 12288, 12288, (size_t)24 << 20, ANY, 0, KERNEL_DECODE_RESIDENT},
-    {9, 16, 14336, ANY, 6144, 6144, (size_t)24 << 20, ANY, 0, KERNEL_DECODE_RESIDENT},
-    {9, 16, 14336, ANY, 8192, 8192, (size_t)24 << 20, ANY, 0, KERNEL_DECODE_RESIDENT},
+    // (of these K the kernel takes 6144, 8192, 10240 and 12288)
+    {9, 16, 14336, ANY, 6144, 12288, (size_t)24 << 20, ANY, 0, KERNEL_DECODE_RESIDENT},
     {13, 16, 18432, ANY, 4096, 4096, (size_t)24 << 20, ANY, 0, KERNEL_DECODE_RESIDENT},
     {17, 24, 18432, ANY, 4096, 4096, (size_t)24 << 20, ANY, 0, KERNEL_DECODE_RESIDENT},
     {25, 32, 32768, ANY, 4096, 4096, (size_t)24 << 20, ANY, 0, KERNEL_DECODE_RESIDENT},
@@ -474,7 +492,8 @@ constexpr SmallMRule SMALL_M_RULES[] = {
     // K = 2048, 4096 and 8192, where every wave walks 1024 of K (M = 12: 1.05 ... 1.29x, M = 16: 0.97 ... 1.23x over
     // N = 10240 ... 57344); at K = 1024, 3072, 6144 and 12288 the split-K kernel stays ahead (0.84 ... 1.06x).
     {9, 16, 1, 8192, 256, 4096, 0, ANY, RULE_K_BELOW_4N, KERNEL_DECODE_RING},
-    {9, 16, 1, 4096, 4097, 8192, 0, ANY, RULE_K_BELOW_4N, KERNEL_DECODE_RING},
+    // (for K of 4 N and more too: 9 x 1344 x 7936 1.18x, 16 x 1603 x 6848 1.16x)
+    {9, 16, 1024, 4096, 4097, 8192, 0, ANY, 0, KERNEL_DECODE_RING},
     {9, 16, 8193, ANY, 2048, 2048, (size_t)24 << 20, ANY, 0, KERNEL_DECODE_RING},
     {9, 16, 8193, ANY, 4096, 4096, (size_t)24 << 20, ANY, 0, KERNEL_DECODE_RING},
     {9, 16, 8193, ANY, 8192, 8192, (size_t)24 << 20, ANY, 0, KERNEL_DECODE_RING},
@@ -485,6 +504,11 @@ constexpr SmallMRule SMALL_M_RULES[] = {
     {17, 64, 1, 8192, 256, 1023, 0, ANY, RULE_K_BELOW_4N, KERNEL_DECODE_RING},
     {17, 64, 1, 4096, 1024, 2048, 0, ANY, RULE_K_BELOW_4N, KERNEL_DECODE_RING},
     {17, 24, 3072, 4096, 2049, 4096, 0, ANY, RULE_K_BELOW_4N, KERNEL_DECODE_RING},
+    // Up to M = 32 also where K is longer or N larger than that, against the split-K family at its best count on look-ahead
+    // loops: N = 1600 ... 4000, K = 2176 ... 7000 1.12 ... 1.36x (24 x 3712 x 4800 1.27x, 32 x 3369 x 5376 1.26x; level at N = 4096,
+    // 0.95x beyond: 18 x 4608 x 6656), N = 4300 ... 8000, K = 1024 ... 1728 1.08 ... 1.34x.
+    {17, 32, 1536, 4095, 2049, 7168, 0, ANY, 0, KERNEL_DECODE_RING},
+    {17, 32, 4097, 8192, 1024, 1792, 0, ANY, 0, KERNEL_DECODE_RING},
     // --- M = 65 ... 128 (eight row tiles): the ring kernel for K <= 512 up to N = 8192, K <= 1024 up to N = 4096
     // (median 1.45x).
     {65, 128, 1, 8192, 256, 512, 0, ANY, RULE_K_BELOW_4N, KERNEL_DECODE_RING},
@@ -517,7 +541,10 @@ constexpr SmallMRule SMALL_M_RULES[] = {
     // N = 10240, K = 16384: 106.9 -> 79.8 us); at K = 4096 mixed (0.92 ... 1.13x), at K = 2048 behind (0.80 ... 1.07x).
     // M = 65 ... 128 already from K = 6144: 1.01 ... 1.30x over N = 6144 ... 14336 at K = 6144 and 7168 (median 1.12x).
     {65, 128, 6144, ANY, 6144, ANY, 0, ANY, 0, KERNEL_MID128},
-    {33, 64, 6144, ANY, 8192, ANY, 0, ANY, 0, KERNEL_ROW64x128},
+    // From K = 7168 also against N = 3584 ... 6143 (M > 64; 66 x 4800 x 12928 1.34x, 73 x 4288 x 15680 1.30x, 124 x 5568 x 8000 1.25x) and
+    // 4096 ... 6143 (M = 33 ... 64; 53 x 6039 x 7488 1.09x, 61 x 4224 x 16064 1.09x).
+    {65, 128, 3584, 6143, 7168, ANY, 0, ANY, 0, KERNEL_MID128},
+    {33, 64, 4096, ANY, 7168, ANY, 0, ANY, 0, KERNEL_ROW64x128},
     // --- everything else with N % 64 == 0 and K % 64 == 0: the split-K family, the tile by M; 128-wide tiles where
     // N gives enough of them and is a multiple of 128 (they stream B better).
     {1, 32, 1, ANY, 1, ANY, 0, ANY, 0, KERNEL_SPLIT_32x64},
@@ -595,11 +622,11 @@ bool stand_in_pays(int kernel, size_t M, size_t N, size_t K, size_t cus) {
 // An odd number of whole chunks, which no two waves share evenly: on rows of the ring kernel its guarded form instead of the
 // split-K family with its second launch.  M = 1 ... 8, N = 1024 ... 28672, K = 1088 ... 4032: 1.08 ... 1.74x (1 x 1984 x 1344
 // 5.9 -> 3.5 us, 8 x 28672 x 3008 32.6 -> 27.7); M = 9 ... 16 up to N = 8192: 1.06 ... 1.30x; M = 17 ... 32, N = 1024 ... 4096, up to
-// K = 4032: 1.47 ... 2.15x, M = 33 ... 64 up to K = 1984: 0.99 ... 1.90x (62 x 1792 x 1472 7.2 -> 5.0); from K = 6000 on mixed (0.93 ...
-// 1.11x).  On rows of the streaming kernel, which such a K shuts out too, below 48 MB of B (17728 x 1088: 1.25 ... 1.35x;
+// K = 4032: 1.47 ... 2.15x, M = 33 ... 64 up to K = 1984: 0.99 ... 1.90x (62 x 1792 x 1472 7.2 -> 5.0); K = 4224 ... 8192 up to N = 4096 1.02 ... 1.27x
+// (21 x 3328 x 6976 1.26x; beyond, eight waves leave a CU one workgroup and the second round costs more: 1 x 4800 x 6976 13.9 us, 17.0).  On rows of the streaming kernel, which such a K shuts out too, below 48 MB of B (17728 x 1088: 1.25 ... 1.35x;
 // 24000 x 1856: 0.96 ... 0.98x).  Below N = 1024 few workgroups share the chip and K slices across them stay.
 bool odd_chunks_on_ring(int kernel, size_t N, size_t K) {
-    if (N % 16 != 0 || N < 1024 || K % 128 != 64 || K < 1024 || K > 4096) return false;
+    if (N % 16 != 0 || N < 1024 || K % 128 != 64 || K < 1024 || (K > 4096 && (K < 4224 || K > 8192 || N > 4096))) return false;
     return kernel == KERNEL_DECODE_RING || (kernel == KERNEL_DECODE_BN16 && N * K < ((size_t)24 << 20));
 }
 
@@ -783,7 +810,7 @@ Plan plan_for(size_t M, size_t N, size_t K, const PlanLimits &limits) {
                 const size_t tiles = div_ceil(N, (size_t)128);
                 // (from K = 6144: below, slices were measured level or behind -- M = 96, N = 18432, K = 4096: 40.8 us
                 // unsliced, 43.6 in three; at K = 6144 and 7168 against N = 18432 1.00 ... 1.04x)
-                p.splits = tiles <= cus && K >= 6144 ? choose_splits(tiles, M, N, cus, K, slice_bytes, limits.partial_bytes, 5) : 1;
+                p.splits = tiles <= cus && K >= 6144 ? choose_splits(SLICES_WIDE_TILE, tiles, M, N, cus, K, slice_bytes, limits.partial_bytes, 5) : 1;
                 if (p.splits > 1) p.partial_bytes = (size_t)p.splits * slice_bytes;
                 if (tiles > cus) one_row_tail(p, r.kernel == KERNEL_MID128 ? 128 : 64, 5, N, K, cus, limits.partial_bytes);
                 break;
@@ -795,7 +822,14 @@ Plan plan_for(size_t M, size_t N, size_t K, const PlanLimits &limits) {
                 // no slices at N = 8: the second launch costs more than they return (9 x 24 x 424 3.8 us, in three slices 6.0;
                 // 16 x 3 x 1072 6.4, 7.4; 48 x 8 x 944 6.1, 5.9).
                 const size_t columns = K >= (p.kernel == KERNEL_SPLIT_32x64 ? 1280u : 896u) ? div_ceil(N, bn) * bn : N;
-                p.splits = choose_splits(div_ceil(N, bn), M, columns, cus, K, slice_bytes, limits.partial_bytes);
+                size_t tiles = div_ceil(N, bn);
+                // M = 65 ... 128 against a B of less than 32 MB: as two rows of 64x64 tiles, whose rings leave a CU room for two
+                // workgroups, and half as many slices.  Against the 128x64 tile at its best count: 75 x 1024 x 1664 7.7 -> 6.4 us, 113 x
+                // 2560 x 1792 11.2 -> 8.0, 82 x 2112 x 12096 20.8 -> 17.5; level from there on (99 x 3776 x 4480 13.0, 12.6; 124 x 5568 x 8000
+                // 36.7, 36.0).
+                if (p.kernel == KERNEL_SPLIT_128x64 && N * K < ((size_t)1 << 24)) p.kernel = KERNEL_SPLIT_2x64x64, tiles *= div_ceil(M, (size_t)64);
+                const bool wide = p.kernel != KERNEL_SPLIT_32x64 && p.kernel != KERNEL_SPLIT_64x64;
+                p.splits = choose_splits(wide ? SLICES_WIDE_TILE : SLICES, tiles, M, columns, cus, K, slice_bytes, limits.partial_bytes);
                 if (p.splits > 1) p.partial_bytes = (size_t)p.splits * slice_bytes;
             }
         }
@@ -949,7 +983,7 @@ Plan plan_for(size_t M, size_t N, size_t K, const PlanLimits &limits) {
     if (limits.excluded_count > 0) return Plan();  // the tuner's question has no further answer
     if (K >= 64) {  // K of one or two chunks; any M and N: guarded
         p.kernel = KERNEL_SPLIT_64x64;
-        p.splits = choose_splits(div_ceil(M, 64) * div_ceil(N, 64), M, N, cus, K, slice_bytes, limits.partial_bytes);
+        p.splits = choose_splits(SLICES_WIDE_TILE, div_ceil(M, 64) * div_ceil(N, 64), M, N, cus, K, slice_bytes, limits.partial_bytes);
         if (p.splits > 1) p.partial_bytes = (size_t)p.splits * slice_bytes;
         return p;
     }
@@ -1025,8 +1059,9 @@ void run_plan(const Plan &p, const Workspace &ws, const void *A, const void *B, 
         case KERNEL_SMALL64: launch_pipelined_plan<Small64>(A, B, C, M, N, K, p, ws); break;
         case KERNEL_SMALL64_W4: launch_small64_w4<false>(A, B, C, M, N, K, p.splits, ws); break;
         case KERNEL_SMALL64_W4_EDGE: launch_small64_w4<true>(A, B, C, M, N, K, p.splits, ws); break;
-        case KERNEL_SPLIT_32x64: launch_splitk<Split32x64>(A, B, C, M, N, K, p.splits, ws); break;
-        case KERNEL_SPLIT_64x64: launch_splitk<Split64x64>(A, B, C, M, N, K, p.splits, ws); break;
+        case KERNEL_SPLIT_32x64: launch_splitk_by_length<Split32x64, Split32x64Short>(A, B, C, M, N, K, p.splits, ws); break;
+        case KERNEL_SPLIT_2x64x64:
+        case KERNEL_SPLIT_64x64: launch_splitk_by_length<Split64x64, Split64x64Short>(A, B, C, M, N, K, p.splits, ws); break;
         case KERNEL_SPLIT_64x128: launch_splitk<Split64x128>(A, B, C, M, N, K, p.splits, ws); break;
         case KERNEL_SPLIT_128x64: launch_splitk<Split128x64>(A, B, C, M, N, K, p.splits, ws); break;
         case KERNEL_SPLIT_128x128: launch_splitk<Split128x128>(A, B, C, M, N, K, p.splits, ws); break;
@@ -1503,10 +1538,11 @@ extern "C" const char *hgemm_kernel_name(int kernel) {
         case KERNEL_T160x256: return "160x256x64 pipelined, 4 waves, 3-stage ring";
         case KERNEL_T192x256: return "192x256x64 pipelined, 4 waves, LDS ring 3 (A) + 2 (B)";
         case KERNEL_T224x256: return "224x256x64 pipelined, 4 waves, LDS ring 3 (A) + 2 (B)";
-        case KERNEL_SPLIT_32x64: return "split-K 32x64x64, 2 waves, 4-stage ring";
-        case KERNEL_SPLIT_64x64: return "split-K 64x64x64, 4 waves, 4-stage ring";
+        case KERNEL_SPLIT_32x64: return "split-K 32x64x64, 2 waves, look-ahead 6-stage or 4-stage ring";
+        case KERNEL_SPLIT_64x64: return "split-K 64x64x64, 4 waves, look-ahead 5-stage or 4-stage ring";
         case KERNEL_SPLIT_64x128: return "split-K 64x128x64, 4 waves, 4-stage ring";
         case KERNEL_SPLIT_128x64: return "split-K 128x64x64, 4 waves, 4-stage ring";
+        case KERNEL_SPLIT_2x64x64: return "split-K 128x64x64, as two 64x64x64 tiles, 4 waves each, 5-stage ring";
         case KERNEL_SPLIT_128x128: return "split-K 128x128x64, 4 waves, 4-stage ring";
         case KERNEL_DECODE_BN16: return "streaming decode, 16 columns per workgroup, one wave per K slice";
         case KERNEL_DECODE_BN32: return "streaming decode, 32 columns per workgroup, one wave per K slice";

@@ -19,8 +19,9 @@
 
 namespace hgemm {
 
-template <int BM_, int BN_, int WAVES_M_, int WAVES_N_, int STAGES_>
-struct SkinnyConfig : TileConfig<BM_, BN_, 64, WAVES_M_, WAVES_N_, STAGES_, LOAD_DMA, LDS_SWIZZLE, true> {};
+// LOOKAHEAD: see the loop
+template <int BM_, int BN_, int WAVES_M_, int WAVES_N_, int STAGES_, bool LOOKAHEAD_ = true>
+struct SkinnyConfig : TileConfig<BM_, BN_, 64, WAVES_M_, WAVES_N_, STAGES_, LOAD_DMA, LDS_SWIZZLE, true, LOOKAHEAD_> {};
 
 // STREAM_B: B is copied with the non-temporal hint.  Every byte of B is read once; when B is larger than the
 // Infinity Cache keeps (N = 28672, K = 4096: 235 MB) the hint is worth 11-12 % (M = 16 ... 64: 64.5 -> 72.6 %, 63.6 ->
@@ -44,8 +45,17 @@ __global__ void __launch_bounds__(Cfg::THREADS)
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave / Cfg::WAVES_N, wn = wave % Cfg::WAVES_N;
 
-    // grid: x = tiles of C, row-major (no 65535 limit on the number of row or column tiles), y = K slice
-    const int tile_n = (int)blockIdx.x % tiles_n, tile_m = (int)blockIdx.x / tiles_n, split = blockIdx.y;
+    // One-dimensional grid, slice-major.  Up to two workgroups of a look-ahead tile to a CU are dealt so that those an XCD runs
+    // together are neighbours in a slice (32x64, M = 9 ... 16: 1.01 ... 1.05x).  More of them go round the XCDs, and so do the wider
+    // tiles (0.94 ... 1.0x the other way).
+    const int tiles_m = (M + BM - 1) / BM, tiles = tiles_m * tiles_n;
+    int split, slot;
+    if (Cfg::LOOKAHEAD && gridDim.x <= 512)
+        slice_and_slot_of_workgroup((int)blockIdx.x, tiles, splits, split, slot);
+    else
+        split = (int)blockIdx.x / tiles, slot = (int)blockIdx.x - split * tiles;
+    split = __builtin_amdgcn_readfirstlane(split);
+    const int tile_n = __builtin_amdgcn_readfirstlane(slot / tiles_m), tile_m = __builtin_amdgcn_readfirstlane(slot % tiles_m);
     const int m0 = tile_m * BM;
     int first_chunk, num_k;  // K's chunks are dealt to the slices as evenly as whole chunks allow
     const int chunks = EDGE ? chunks_of(K, BK) : K / BK;
@@ -101,51 +111,106 @@ __global__ void __launch_bounds__(Cfg::THREADS)
 #pragma unroll
             for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
 
-    // drop: 16-byte pieces at the start of the chunk that must not count (EDGE, last chunk)
-    auto compute_stage = [&](int stage, int drop) {
+    // All operands of a chunk.  drop: 16-byte pieces at its start that must not count (EDGE, last chunk)
+    constexpr int SETS = Cfg::LOOKAHEAD ? 2 : 1;
+    half8 af[SETS][KSTEPS][TM], bf[SETS][KSTEPS][TN];
+    auto load_chunk = [&](int stage, int drop, half8 (&a)[KSTEPS][TM], half8 (&b)[KSTEPS][TN]) {
         const unsigned char *s = lds + stage * Cfg::STAGE_BYTES;
 #pragma unroll
         for (int kk = 0; kk < KSTEPS; ++kk) {
             const uint32_t chunk = (uint32_t)((kk * 2) ^ frag_x) << 4;
-            half8 af[TM], bf[TN];
 #pragma unroll
             for (int i = 0; i < TM; ++i)
-                af[i] = *reinterpret_cast<const half8 *>(s + a_frag_off + i * 32 * ROW_BYTES + chunk);
+                a[kk][i] = *reinterpret_cast<const half8 *>(s + a_frag_off + i * 32 * ROW_BYTES + chunk);
 #pragma unroll
             for (int j = 0; j < TN; ++j)
-                bf[j] = *reinterpret_cast<const half8 *>(s + b_frag_off + j * 32 * ROW_BYTES + chunk);
+                b[kk][j] = *reinterpret_cast<const half8 *>(s + b_frag_off + j * 32 * ROW_BYTES + chunk);
             if constexpr (EDGE) {
                 if (drop > 0) {
                     const bool keep = kk * 2 + (lane >> 5) >= drop;
 #pragma unroll
-                    for (int i = 0; i < TM; ++i) af[i] = keep_or_zero(af[i], keep);
+                    for (int i = 0; i < TM; ++i) a[kk][i] = keep_or_zero(a[kk][i], keep);
 #pragma unroll
-                    for (int j = 0; j < TN; ++j) bf[j] = keep_or_zero(bf[j], keep);
+                    for (int j = 0; j < TN; ++j) b[kk][j] = keep_or_zero(b[kk][j], keep);
                 }
             }
+        }
+    };
+
+    auto multiply = [&](half8 (&a)[KSTEPS][TM], half8 (&b)[KSTEPS][TN]) {
+#pragma unroll
+        for (int kk = 0; kk < KSTEPS; ++kk)
 #pragma unroll
             for (int i = 0; i < TM; ++i)
 #pragma unroll
                 for (int j = 0; j < TN; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(bf[j], af[i], acc[i][j], 0, 0, 0);
-        }
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(b[kk][j], a[kk][i], acc[i][j], 0, 0, 0);
     };
 
-    // ---- ring of STAGES buffers, STAGES-1 chunks in flight
+    // ---- ring of STAGES buffers, STAGES-1 chunks in flight, barrier one chunk ahead (as the look-ahead loop of mfma_tiled.h,
+    // for any number of chunks): at the top of iteration kt every operand of chunk kt is on its way into registers; the wait
+    // and the barrier confirm chunk kt+1 and retire every wave's reads of chunk kt-1, whose buffer the new copy refills; then
+    // the wave issues all operand reads of chunk kt+1, the copy, and only then the MFMAs of chunk kt.  Against a loop that reads a
+    // chunk's operands behind its own barrier, at the best slice counts of both: 32x64 1.02 ... 1.05x, 64x64 1.05x (14 ... 18 shapes a
+    // class of M; 64 x 4096 x 4096 11.2 -> 10.1 us, unsliced 19.9 -> 14.6).  That loop (!LOOKAHEAD) stays for a few
+    // chunks, where it is 0.2 ... 0.3 us ahead (38 x 40 x 136 3.0 us, 3.4), and on the wider tiles, whose waves have more
+    // than one MFMA to a k-step (128x64 0.87 ... 1.0x, 64x128 0.89 ... 1.0x, 128x128 1.01x by ring depth).
 #pragma unroll
     for (int s = 0; s < STAGES - 1; ++s)
         if (s < num_k) dma_fetch(s, s);
-    int cur = 0, fill = STAGES - 1;
-    for (int kt = 0; kt < num_k; ++kt) {
-        if (num_k - 1 - kt >= STAGES - 2)
+    int cur = 0, fill = STAGES - 1, kt = 0;
+    if constexpr (!Cfg::LOOKAHEAD) {
+        for (; kt < num_k; ++kt) {
+            if (num_k - 1 - kt >= STAGES - 2)
+                wait_vmcnt<(STAGES - 2) * L>();
+            else
+                wait_vmcnt<0>();
+            __syncthreads();
+            if (kt + STAGES - 1 < num_k) dma_fetch(kt + STAGES - 1, fill);
+            load_chunk(cur, kt == num_k - 1 ? tail_dup : 0, af[0], bf[0]);
+            multiply(af[0], bf[0]);
+            cur = (cur + 1 == STAGES) ? 0 : cur + 1;
+            fill = (fill + 1 == STAGES) ? 0 : fill + 1;
+        }
+    } else {
+        if (num_k >= STAGES - 1)
             wait_vmcnt<(STAGES - 2) * L>();
         else
             wait_vmcnt<0>();
         __syncthreads();
-        if (kt + STAGES - 1 < num_k) dma_fetch(kt + STAGES - 1, fill);
-        compute_stage(cur, kt == num_k - 1 ? tail_dup : 0);
-        cur = (cur + 1 == STAGES) ? 0 : cur + 1;
-        fill = (fill + 1 == STAGES) ? 0 : fill + 1;
+        load_chunk(0, num_k == 1 ? tail_dup : 0, af[0], bf[0]);
+        // STEADY: the copy of chunk kt+STAGES-1 exists (so does chunk kt+1, and the wait count is the full one)
+        auto iteration = [&](auto steady, int kt, half8 (&ca)[KSTEPS][TM], half8 (&cb)[KSTEPS][TN], half8 (&na)[KSTEPS][TM],
+                             half8 (&nb)[KSTEPS][TN]) __attribute__((always_inline)) {
+            constexpr bool STEADY = decltype(steady)::value;
+            const int nxt = (cur + 1 == STAGES) ? 0 : cur + 1;
+            if (STEADY || kt + 1 < num_k) {
+                // copies issued so far: chunks up to min(kt+STAGES-2, num_k-1); all but those beyond kt+1 must land
+                if (STEADY || num_k - 1 - (kt + 1) >= STAGES - 3)
+                    wait_vmcnt<(STAGES - 3) * L>();
+                else
+                    wait_vmcnt<0>();
+                // a bare barrier: the fence of __syncthreads() would wait for this wave's own operand reads of chunk kt, which
+                // nothing behind the barrier overwrites
+                __builtin_amdgcn_sched_barrier(0);  // the MFMAs of chunk kt-1 (and their waits) stay in front
+                asm volatile("s_barrier" ::: "memory");
+                load_chunk(nxt, !STEADY && kt + 1 == num_k - 1 ? tail_dup : 0, na, nb);
+            }
+            if (STEADY || kt + STAGES - 1 < num_k) dma_fetch(kt + STAGES - 1, fill);
+            __builtin_amdgcn_sched_barrier(0);
+            multiply(ca, cb);
+            cur = nxt;
+            fill = (fill + 1 == STAGES) ? 0 : fill + 1;
+        };
+        const int steady_end = num_k - (STAGES - 1);
+        for (; kt + 2 <= steady_end; kt += 2) {
+            iteration(std::true_type{}, kt, af[0], bf[0], af[1], bf[1]);
+            iteration(std::true_type{}, kt + 1, af[1], bf[1], af[0], bf[0]);
+        }
+        for (; kt < num_k; kt += 2) {
+            iteration(std::false_type{}, kt, af[0], bf[0], af[1], bf[1]);
+            if (kt + 1 < num_k) iteration(std::false_type{}, kt + 1, af[1], bf[1], af[0], bf[0]);
+        }
     }
 
     // ---- epilogue.  Lane l holds row l%32 of each 32x32 tile and four consecutive n per

@@ -39,6 +39,7 @@ enum KernelId {
     KERNEL_UNALIGNED96,
     KERNEL_UNALIGNED128x64,
     KERNEL_UNALIGNED128,
+    KERNEL_SPLIT_2x64x64,  // KERNEL_SPLIT_128x64's block as two rows of KERNEL_SPLIT_64x64's tiles
 };
 
 struct Plan {
