@@ -331,6 +331,11 @@ constexpr double TAIL_US = 3.6, TAIL_SUB_US = 4.4;
 // the lines.  Chunk times grow by this factor (5112^3 269 us where 5120^3 takes 208; 1.18 ... 1.30 from 1000^3 to 8184^3), and from
 // about 4500^3 on it is cheaper to copy both operands first (5112^3 266 us directly, 196 on copies; 4000^2 x 4040 97, 110).
 constexpr double OFF_LINE = 1.27;
+// By how much the tiles for unaligned rows may be predicted behind such a product on the four-wave 64x64 tile, or on another, and
+// still be ahead: both sides' figures leave out some of what the lines cost.  Their time over that of the plan without them, where
+// they are taken: 0.78 ... 0.95 (1400^3 15.7 -> 12.5 us, 1528^2 x 2632 27.5 -> 21.4, 1224^2 x 2056 19.3 -> 16.4; 1000^3, left
+// alone, 7.8 us and 7.8).  In K slices it was 0.85 ... 1.15 without a pattern (584^2 x 3000 12.9 us, 14.9 on them): not taken.
+constexpr double OFF_LINE_SMALL = 1.25, OFF_LINE_OTHERS = 1.12;
 // On tiles of 192x192 and unsliced ones of 256x128, K = 4200 ... 12000 (in slices from 6000), a direct product takes longer than
 // that in proportion.  75 shapes where the figures alone prefer it by less than this: 1.15x as long as on copies, 54 of them by more
 // than 5 %, 7 shorter (1391 x 4586 x 7592 146 us directly, 102 on copies; 2190 x 3878 x 11528 207, 158; 757 x 14816 x 11168 259,
@@ -854,7 +859,9 @@ Plan plan_for(size_t M, size_t N, size_t K, const PlanLimits &limits) {
     }
     // Pipelined tiles: M and N may end inside a tile and K inside a chunk (guarded edges; the model charges whole
     // tiles and chunks), as long as rows of A and B stay 16-byte aligned.
-    // M and N that 64 does not divide while K does and rows of C are aligned: fitted on the one-wave tile, left to it
+    // M and N that 64 does not divide while K does and rows of C are aligned: the one-wave tile keeps M <= 128, a short K in slices
+    // (227 x 128 x 1216) and a long K without (555 x 2688 x 4224 21.0 us, 25.9 on the four-wave tile).  Else the four-wave tile is
+    // ahead: 1000^2 x 1024 9.9 -> 6.7 us, 504^2 x 512 5.0 -> 4.2, 416^2 x 8192 14.6 -> 11.9
     const bool one_wave = (M % 64 || N % 64) && N % 8 == 0 && K % 64 == 0;
     if (K % 8 == 0 && K >= 64 && limits.excluded_count == 0) {
         p.kernel = short_k_kernel(M, N, K, cus);
@@ -866,8 +873,8 @@ Plan plan_for(size_t M, size_t N, size_t K, const PlanLimits &limits) {
         if (K % 64) c.lo *= OFF_LINE, c.hi *= OFF_LINE;
         const bool w4 = c.kernel == KERNEL_SMALL64_W4;
         const int kernel = w4 && (M % 64 || N % 64 || K % 64) ? (int)KERNEL_SMALL64_W4_EDGE : c.kernel;
-        if (w4 && one_wave) continue;
         for (int s = 1; s <= 32; ++s) {  // K slices: whole chunks, as even as that allows
+            if (w4 && one_wave && (M <= 128 || (s > 1 ? K < 2048 : K > 2048))) continue;
             if (w4) {
                 const size_t wgs = div_ceil(M, (size_t)c.bm) * div_ceil(N, (size_t)c.bn) * (size_t)s;
                 if (wgs > cus * (size_t)c.per_cu) break;
@@ -957,6 +964,13 @@ Plan plan_for(size_t M, size_t N, size_t K, const PlanLimits &limits) {
             // B before a product that is bound by reading B costs 1.4 ... 3x (160 x 28672 x 2040: 73.0 us, 38.3 without)
             const Plan copied = plan_on_copies(M, N, K, limits);
             if (copied.est_us > 0.0 && copied.est_us < p.est_us * direct_weight(p.kernel, p.splits, K) && !left_out(limits, copied)) return copied;
+            // ... or on the tiles for unaligned rows, whose 128-wide chunks straddle half as many lines
+            if (limits.excluded_count == 0 && M >= 256 && N >= 256) {
+                Plan direct = plan_on_unaligned_rows(M, N, K, cus, limits);
+                direct.copies_partial_bytes = p.partial_bytes;
+                const double weight = p.kernel == KERNEL_SMALL64_W4_EDGE ? OFF_LINE_SMALL : OFF_LINE_OTHERS;
+                if (direct.kernel != KERNEL_NONE && direct.splits == 1 && direct.est_us < p.est_us * weight) return direct;
+            }
         }
         return p;
     }
@@ -1403,7 +1417,7 @@ extern "C" void hgemm_release_workspace(void) {
 // Operand bytes reported for a plan: rows read where they lie count as the copies that they once were, so that reservations and
 // what fits the static workspace stay what they were.
 static size_t reported_operand_bytes(const Plan &p, size_t M, size_t N, size_t K) {
-    const bool once_copied = reads_unaligned_rows(p.kernel) && K >= 192 && copy_bytes(M, N, K) <= MAX_PADDED_BYTES;
+    const bool once_copied = K % 8 && reads_unaligned_rows(p.kernel) && K >= 192 && copy_bytes(M, N, K) <= MAX_PADDED_BYTES;
     return p.operand_bytes || once_copied ? reported_copy_bytes(M, N, K) : 0;
 }
 static size_t padded_partial_bytes(size_t bytes) { return (bytes + 255) / 256 * 256; }

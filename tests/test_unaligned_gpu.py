@@ -19,6 +19,17 @@ CASES = [
     ((779, 779, 11221), "128x128x128", True), ((1009, 1009, 7364), "128x128x128", True),
 ]
 
+# 64 does not divide K though 8 does: the same tiles, unsliced, for products that they are ahead on; 64 divides K but not M or N:
+# the four-wave tile of 64x64 on whole chunks, unsliced up to K = 2048 and in slices from there on
+ALIGNED_CASES = [
+    ((1264, 1264, 1264), "where they lie, 128x64x128", False), ((1403, 1318, 1416), "where they lie, 128x64x128", False),
+    ((1193, 1591, 1848), "where they lie, 128x64x128", False), ((377, 5817, 1240), "where they lie, 96x96x128", False),
+    ((1416, 1416, 3096), "where they lie, 96x96x128", False), ((462, 4128, 3912), "where they lie, 96x96x128", False),
+    ((129, 1000, 640), "edge-guarded 64x64x64", False), ((1000, 1000, 1024), "edge-guarded 64x64x64", False),
+    ((1000, 1000, 2048), "edge-guarded 64x64x64", False), ((376, 376, 2048), "edge-guarded 64x64x64", True),
+    ((177, 1088, 2432), "edge-guarded 64x64x64", True), ((264, 264, 6784), "edge-guarded 64x64x64", True),
+]
+
 
 def _gpu_bits(bits, gpu):
     import torch
@@ -29,10 +40,20 @@ def _gpu_bits(bits, gpu):
 def test_unaligned_rows(oracle, hgemm_lib, gpu, shape, tile, sliced):
     """Exact on ternary inputs (sums are integers below 2048) inside a guard band; then with an infinity in one row of A, at a
     k that the last chunk and the one before it both read: that row is infinite with B's sign, no other changes."""
+    _exact_and_infinite(oracle, hgemm_lib, gpu, shape, f"where they lie, {tile}", sliced)
+
+
+@pytest.mark.parametrize("shape,kernel,sliced", ALIGNED_CASES)
+def test_aligned_rows_off_the_lines(oracle, hgemm_lib, gpu, shape, kernel, sliced):
+    """The same for products whose rows are 16-byte aligned and whose K, M or N no tile divides."""
+    _exact_and_infinite(oracle, hgemm_lib, gpu, shape, kernel, sliced)
+
+
+def _exact_and_infinite(oracle, hgemm_lib, gpu, shape, kernel, sliced):
     import torch
     M, N, K = shape
     plan = hgemm_lib.auto_plan(M, N, K)
-    assert f"where they lie, {tile}" in plan["kernel"] and (plan["splits"] > 1) == sliced, plan
+    assert kernel in plan["kernel"] and (plan["splits"] > 1) == sliced, plan
     A, B = oracle.fill((M, K), 41, 1, oracle.TERNARY, 0, 1), oracle.fill((N, K), 41, 2, oracle.TERNARY, 0, 1)
     expect = oracle.hgemm(A, B)
     assert np.abs(expect.view(np.float16).astype(np.float32)).max() < 2048
