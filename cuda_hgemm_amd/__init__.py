@@ -2,7 +2,8 @@
 
 The product is the native library ``lib/libhgemm.so`` (hand-written HIP kernels behind
 ``include/hgemm.h``) and the C++ driver ``bin/hgemm``.  This package only loads the
-library through ctypes so that tests and the benchmark can call the same entry points a
+library through ctypes -- and, for torch tensors, through ``lib/_call.so``, which checks them and
+launches in one native call -- so that tests and the benchmark can call the same entry points a
 C++ caller links against.  PyTorch is used for device memory and nothing else.
 
 There is no fallback: if the library has not been built, importing a symbol raises.

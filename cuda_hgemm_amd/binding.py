@@ -1,4 +1,4 @@
-"""ctypes binding of ``include/hgemm.h`` / ``include/hgemm_hipblaslt.h``.
+"""Binding of ``include/hgemm.h`` / ``include/hgemm_hipblaslt.h``: ctypes, and ``csrc/python_call.cpp`` for torch tensors.
 
 Operand layouts are the reference's (``src/common/tester.h:117-120``): ``A`` is ``(M, K)``
 row-major, ``B`` is handed over as its ``(N, K)`` storage (column-major ``K x N``), ``C`` is
