@@ -116,8 +116,9 @@ HGEMM_FUNC(hgemm_skinny);
 
 /* Dispatcher: picks tile, kernel and number of K slices for the shape from a cost model
  * fitted to measurements; accepts every shape.  M and N may end anywhere inside a tile and K,
- * a multiple of 8, anywhere inside a chunk (edges are guarded); other K from 192 on run on
- * copies of A and B whose rows are aligned, shorter ones on a fully guarded MFMA kernel.  This is the entry point the benchmark measures. */
+ * a multiple of 8, anywhere inside a chunk (edges are guarded); other K from 129 on are read
+ * where they lie or, from 192 on, copied to aligned rows first, whichever is predicted faster; shorter ones run on a fully guarded
+ * MFMA kernel.  This is the entry point the benchmark measures. */
 HGEMM_FUNC(hgemm_auto);
 
 /* Kernel hgemm_auto would pick for a shape (an id for hgemm_kernel_name) and, through
