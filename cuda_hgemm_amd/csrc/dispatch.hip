@@ -861,7 +861,8 @@ Plan plan_for(size_t M, size_t N, size_t K, const PlanLimits &limits) {
     // tiles and chunks), as long as rows of A and B stay 16-byte aligned.
     // M and N that 64 does not divide while K does and rows of C are aligned: the one-wave tile keeps M <= 128, a short K in slices
     // (227 x 128 x 1216) and a long K without (555 x 2688 x 4224 21.0 us, 25.9 on the four-wave tile).  Else the four-wave tile is
-    // ahead: 1000^2 x 1024 9.9 -> 6.7 us, 504^2 x 512 5.0 -> 4.2, 416^2 x 8192 14.6 -> 11.9
+    // ahead: 1000^2 x 1024 9.9 -> 6.7 us, 504^2 x 512 5.0 -> 4.2, 416^2 x 8192 14.6 -> 11.9.  Not in slices of more than 44 chunks,
+    // where 128x128 in slices is (456^2 x 11200, 44 chunks, 14.9 us and 15.3; 480^2 x 14720, 58 chunks, 17.1 and 15.3)
     const bool one_wave = (M % 64 || N % 64) && N % 8 == 0 && K % 64 == 0;
     if (K % 8 == 0 && K >= 64 && limits.excluded_count == 0) {
         p.kernel = short_k_kernel(M, N, K, cus);
@@ -874,7 +875,7 @@ Plan plan_for(size_t M, size_t N, size_t K, const PlanLimits &limits) {
         const bool w4 = c.kernel == KERNEL_SMALL64_W4;
         const int kernel = w4 && (M % 64 || N % 64 || K % 64) ? (int)KERNEL_SMALL64_W4_EDGE : c.kernel;
         for (int s = 1; s <= 32; ++s) {  // K slices: whole chunks, as even as that allows
-            if (w4 && one_wave && (M <= 128 || (s > 1 ? K < 2048 : K > 2048))) continue;
+            if (w4 && one_wave && (M <= 128 || (s > 1 ? K < 2048 || K > 64 * 44 * (size_t)s : K > 2048))) continue;
             if (w4) {
                 const size_t wgs = div_ceil(M, (size_t)c.bm) * div_ceil(N, (size_t)c.bn) * (size_t)s;
                 if (wgs > cus * (size_t)c.per_cu) break;
