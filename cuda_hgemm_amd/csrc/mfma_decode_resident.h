@@ -64,6 +64,11 @@ __global__ void __launch_bounds__(512)
 
     int tile = blockIdx.x;  // the launcher starts no workgroup without a tile
     const half_t *rows = B + (size_t)tile * 16 * K;
+    // 128 clocks of pause: since arguments are preloaded a wave gets here without waiting for them, and M = 15 and 16 at K = 4096 lost
+    // 0.4 ... 0.8 % by it (16 x 28672 x 4096 38.3 -> 38.5 us, 16 x 24576 x 4096 33.9 -> 34.2).  With the pause they are 0.7 ... 1.0 % ahead of
+    // the waiting form (37.9, 33.6), twelve shapes of M = 10 ... 30 and K = 4096 ... 12288 0.1 ... 1.0 %; 64 clocks give half of that, and a
+    // barrier instead, i.e. all waves of a workgroup at once, costs 1 ... 2 %.
+    __builtin_amdgcn_s_sleep(2);
 #pragma unroll
     for (int s = 0; s < STAGES - 1; ++s) fetch(rows, s, s);
 
