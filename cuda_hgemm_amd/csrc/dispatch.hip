@@ -624,6 +624,15 @@ bool stand_in_pays(int kernel, size_t M, size_t N, size_t K, size_t cus) {
     }
 }
 
+// Sizes in a row's box at which its stand-in is behind what a later row covers them with: the row is passed over.
+// * The persistent kernel's K come as a range in the table and it takes four of them.  At any other K the ring kernel's guarded form in its
+//   place takes 1.04 ... 1.47 times as long as the 32x64 split-K tile (30 shapes of M = 9 ... 16, N = 14336 ... 40000, K = 6144 ... 12288, geomean
+//   1.13: 16 x 15040 x 10648 66.8 us, 98.4; 10 x 14800 x 7232 37.6, 41.3).
+bool stand_in_covers(const SmallMRule &r, size_t M, size_t K) {
+    int chunks = 0;
+    return r.kernel != KERNEL_DECODE_RESIDENT || decode_resident_waves(M, K, &chunks) > 0;
+}
+
 // An odd number of whole chunks, which no two waves share evenly: on rows of the ring kernel its guarded form instead of the
 // split-K family with its second launch.  M = 1 ... 8, N = 1024 ... 28672, K = 1088 ... 4032: 1.08 ... 1.74x (1 x 1984 x 1344
 // 5.9 -> 3.5 us, 8 x 28672 x 3008 32.6 -> 27.7); M = 9 ... 16 up to N = 8192: 1.06 ... 1.30x; M = 17 ... 32, N = 1024 ... 4096, up to
@@ -778,6 +787,10 @@ Plan plan_for(size_t M, size_t N, size_t K, const PlanLimits &limits) {
         p = Plan();
         p.kernel = edges || odd_chunks ? small_m_edge_kernel(r.kernel, M, N, K) : r.kernel;
         if (p.kernel == KERNEL_NONE) continue;
+        if (edges && !limits.every_small_m_kernel && !stand_in_covers(r, M, K)) {
+            p = Plan();
+            continue;
+        }
         if (edges && !limits.every_small_m_kernel && !stand_in_pays(p.kernel, M, N, K, cus)) {
             p = Plan();
             break;

@@ -100,3 +100,16 @@ def test_ragged_sizes_on_one_or_two_chunks(hgemm_lib, shape, kernel):
 def test_copies_of_aligned_rows_where_they_pay(hgemm_lib, shape, copied):
     """K a multiple of 8 and not of 64 runs on guarded kernels or on copies with rows of whole cache lines."""
     assert hgemm_lib.auto_plan(*shape)["kernel"].startswith("zero-padded") == copied
+
+
+# M = 9 ... 16 against N from 14336 on (microseconds on the ring kernel's guarded form, on the split-K tile)
+@pytest.mark.parametrize("shape,kernel", [
+    ((16, 15040, 10648), "split-K 32x64"),                     # 98.4, 66.8
+    ((10, 14800, 7232), "split-K 32x64"),                      # 41.3, 37.6
+    ((16, 15257, 8320), "split-K 32x64"),                      # 51.3, 39.8
+    ((12, 28672, 6152), "split-K 32x64"),
+    ((12, 20001, 8192), "streaming decode"),                   # a K of the persistent kernel's: its row's stand-in
+    ((12, 20000, 8192), "decode with A in registers"),
+])
+def test_rows_of_the_persistent_kernel_hold_at_its_k_only(hgemm_lib, shape, kernel):
+    assert hgemm_lib.auto_plan(*shape)["kernel"].startswith(kernel)
