@@ -636,11 +636,12 @@ bool stand_in_covers(const SmallMRule &r, size_t M, size_t K) {
 // An odd number of whole chunks, which no two waves share evenly: on rows of the ring kernel its guarded form instead of the
 // split-K family with its second launch.  M = 1 ... 8, N = 1024 ... 28672, K = 1088 ... 4032: 1.08 ... 1.74x (1 x 1984 x 1344
 // 5.9 -> 3.5 us, 8 x 28672 x 3008 32.6 -> 27.7); M = 9 ... 16 up to N = 8192: 1.06 ... 1.30x; M = 17 ... 32, N = 1024 ... 4096, up to
-// K = 4032: 1.47 ... 2.15x, M = 33 ... 64 up to K = 1984: 0.99 ... 1.90x (62 x 1792 x 1472 7.2 -> 5.0); K = 4224 ... 8192 up to N = 4096 1.02 ... 1.27x
-// (21 x 3328 x 6976 1.26x; beyond, eight waves leave a CU one workgroup and the second round costs more: 1 x 4800 x 6976 13.9 us, 17.0).  On rows of the streaming kernel, which such a K shuts out too, below 48 MB of B (17728 x 1088: 1.25 ... 1.35x;
-// 24000 x 1856: 0.96 ... 0.98x).  Below N = 1024 few workgroups share the chip and K slices across them stay.
+// K = 4032: 1.47 ... 2.15x, M = 33 ... 64 up to K = 1984: 0.99 ... 1.90x (62 x 1792 x 1472 7.2 -> 5.0).  Up to N = 4096 also at K = 4160 ...
+// 8192: 1.02 ... 1.27x (21 x 3328 x 6976), M = 1 ... 32 at K = 4160 1.00 ... 1.58x; beyond, eight waves leave a CU one workgroup and the second
+// round costs more (1 x 4800 x 6976 13.9 us, 17.0).  On rows of the streaming kernel, which such a K shuts out too, below 48 MB of B
+// (17728 x 1088: 1.25 ... 1.35x; 24000 x 1856: 0.96 ... 0.98x).  Below N = 1024 few workgroups share the chip and K slices across them stay.
 bool odd_chunks_on_ring(int kernel, size_t N, size_t K) {
-    if (N % 16 != 0 || N < 1024 || K % 128 != 64 || K < 1024 || (K > 4096 && (K < 4224 || K > 8192 || N > 4096))) return false;
+    if (N % 16 != 0 || N < 1024 || K % 128 != 64 || K < 1024 || K > (N <= 4096 ? 8192u : 4096u)) return false;
     return kernel == KERNEL_DECODE_RING || (kernel == KERNEL_DECODE_BN16 && N * K < ((size_t)24 << 20));
 }
 

@@ -142,7 +142,9 @@ def test_small_m_rule_table(hgemm_lib):
             chunk_options = (8,) if M > 16 else (8, 12, 16, 20, 24)
             return M <= 32 and N % 16 == 0 and K % 64 == 0 and any(K // 64 == w * c for w in (2, 4, 8) for c in chunk_options)
         if "LDS ring per K slice" in kernel:
-            return N % 16 == 0 and K % 128 == 0
+            # ... or, on its guarded form, an odd number of whole chunks
+            odd = K % 128 == 64 and N >= 1024 and 1024 <= K <= (8192 if N <= 4096 else 4096)
+            return N % 16 == 0 and (K % 128 == 0 or odd)
         if kernel.startswith("streaming decode"):
             return M <= 32 and N % 32 == 0 and K % 256 == 0
         if kernel.startswith(("pipelined 128x128", "pipelined 64x128")):

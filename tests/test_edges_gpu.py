@@ -39,6 +39,8 @@ CASES = [
     ((3, 1984, 1344), "streaming decode, 16 columns per workgroup, per-wave"),             # an odd number of whole chunks
     ((16, 1024, 4032), "streaming decode, 16 columns per workgroup, per-wave"),
     ((8, 17728, 1088), "streaming decode, 16 columns per workgroup, per-wave"),
+    ((5, 2048, 4160), "streaming decode, 16 columns per workgroup, per-wave"),
+    ((30, 1536, 6976), "streaming decode, 16 columns per workgroup, per-wave"),
     ((511, 511, 511), "zero-padded"), ((296, 299, 2113), "zero-padded"), ((3, 1001, 4099), "zero-padded"),
     ((1027, 520, 193), "zero-padded"), ((2591, 11875, 1833), "zero-padded"),
 ]
