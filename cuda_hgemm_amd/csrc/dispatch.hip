@@ -509,10 +509,12 @@ constexpr SmallMRule SMALL_M_RULES[] = {
     {17, 64, 1, 8192, 256, 1023, 0, ANY, RULE_K_BELOW_4N, KERNEL_DECODE_RING},
     {17, 64, 1, 4096, 1024, 2048, 0, ANY, RULE_K_BELOW_4N, KERNEL_DECODE_RING},
     {17, 24, 3072, 4096, 2049, 4096, 0, ANY, RULE_K_BELOW_4N, KERNEL_DECODE_RING},
-    // Up to M = 32 also where K is longer or N larger than that, against the split-K family at its best count on look-ahead
-    // loops: N = 1600 ... 4000, K = 2176 ... 7000 1.12 ... 1.36x (24 x 3712 x 4800 1.27x, 32 x 3369 x 5376 1.26x; level at N = 4096,
-    // 0.95x beyond: 18 x 4608 x 6656), N = 4300 ... 8000, K = 1024 ... 1728 1.08 ... 1.34x.
-    {17, 32, 1536, 4095, 2049, 7168, 0, ANY, 0, KERNEL_DECODE_RING},
+    // Up to M = 32 also where K is longer or N larger than that, against the split-K family at its best count: N = 1536 ... 4095,
+    // K = 2049 ... 5631 1.02 ... 1.64x (24 x 3712 x 4800 1.27x, 32 x 3369 x 5376 1.26x; level at N = 4096, 0.95x beyond: 18 x 4608 x 6656);
+    // from there on what eight waves' walk costs more than slices do grows with M and N: up to K = 7168 1.03 ... 1.29x below N = 2304, and
+    // 0.88 ... 1.06x from there on (32 x 2944 x 6912 11.5 us, 14.0).  N = 4300 ... 8000, K = 1024 ... 1792 1.08 ... 1.34x.
+    {17, 32, 1536, 2303, 2049, 7168, 0, ANY, 0, KERNEL_DECODE_RING},
+    {17, 32, 2304, 4095, 2049, 6143, 0, ANY, 0, KERNEL_DECODE_RING},
     {17, 32, 4097, 8192, 1024, 1792, 0, ANY, 0, KERNEL_DECODE_RING},
     // --- M = 65 ... 128 (eight row tiles): the ring kernel for K <= 512 up to N = 8192, K <= 1024 up to N = 4096
     // (median 1.45x).
@@ -628,9 +630,15 @@ bool stand_in_pays(int kernel, size_t M, size_t N, size_t K, size_t cus) {
 // * The persistent kernel's K come as a range in the table and it takes four of them.  At any other K the ring kernel's guarded form in its
 //   place takes 1.04 ... 1.47 times as long as the 32x64 split-K tile (30 shapes of M = 9 ... 16, N = 14336 ... 40000, K = 6144 ... 12288, geomean
 //   1.13: 16 x 15040 x 10648 66.8 us, 98.4; 10 x 14800 x 7232 37.6, 41.3).
-bool stand_in_covers(const SmallMRule &r, size_t M, size_t K) {
+// * The ring kernel's rows for M = 17 ... 32 where K ends inside a chunk, whose rows straddle lines: up to N = 4096 to K = 4608 (1.02 ... 1.37x;
+//   beyond 0.67 ... 1.13x, geomean 0.86: 20 x 2624 x 7000 11.4 us, 16.6), beyond that N below K = 1024 (from there on level, 0.90 ... 1.10x).
+//   M = 9 ... 16 there with K of 4 N and more: to K = 6144 (1.00 ... 1.26x; beyond 0.91 ... 1.03x).
+bool stand_in_covers(const SmallMRule &r, size_t M, size_t N, size_t K) {
     int chunks = 0;
-    return r.kernel != KERNEL_DECODE_RESIDENT || decode_resident_waves(M, K, &chunks) > 0;
+    if (r.kernel == KERNEL_DECODE_RESIDENT) return decode_resident_waves(M, K, &chunks) > 0;
+    if (r.kernel != KERNEL_DECODE_RING || K % 64 == 0 || M <= 8 || M > 32) return true;
+    if (M <= 16) return K <= 6144 || K < 4 * N;
+    return N <= 4096 ? K <= 4608 : K < 1024;
 }
 
 // An odd number of whole chunks, which no two waves share evenly: on rows of the ring kernel its guarded form instead of the
@@ -788,7 +796,7 @@ Plan plan_for(size_t M, size_t N, size_t K, const PlanLimits &limits) {
         p = Plan();
         p.kernel = edges || odd_chunks ? small_m_edge_kernel(r.kernel, M, N, K) : r.kernel;
         if (p.kernel == KERNEL_NONE) continue;
-        if (edges && !limits.every_small_m_kernel && !stand_in_covers(r, M, K)) {
+        if (edges && !limits.every_small_m_kernel && !stand_in_covers(r, M, N, K)) {
             p = Plan();
             continue;
         }

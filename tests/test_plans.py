@@ -113,3 +113,20 @@ def test_copies_of_aligned_rows_where_they_pay(hgemm_lib, shape, copied):
 ])
 def test_rows_of_the_persistent_kernel_hold_at_its_k_only(hgemm_lib, shape, kernel):
     assert hgemm_lib.auto_plan(*shape)["kernel"].startswith(kernel)
+
+
+# M = 9 ... 32 against N up to 8192 (microseconds on the split-K tile, on the ring kernel)
+@pytest.mark.parametrize("shape,kernel", [
+    ((32, 2944, 6912), "split-K 32x64"),                       # 11.5, 14.0
+    ((30, 1536, 6976), "streaming decode"),                    # the longer K below N = 2304
+    ((24, 2560, 6080), "streaming decode"),
+    ((20, 2624, 7000), "split-K 32x64"),                       # 11.4, 16.6: K ends inside a chunk
+    ((29, 2511, 7024), "split-K 32x64"),                       # 11.7, 17.6
+    ((24, 2560, 4600), "streaming decode"),
+    ((24, 4400, 1672), "split-K 32x64"),
+    ((24, 6400, 1664), "streaming decode"),
+    ((14, 1504, 7080), "split-K 32x64"),                       # 8.8, 9.9
+    ((14, 2048, 7080), "streaming decode"),
+])
+def test_ring_kernel_for_few_rows_and_a_long_k(hgemm_lib, shape, kernel):
+    assert hgemm_lib.auto_plan(*shape)["kernel"].startswith(kernel)
