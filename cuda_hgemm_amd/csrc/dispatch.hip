@@ -752,9 +752,6 @@ constexpr Candidate UNALIGNED_TILES[] = {
 // The figures for copies understate them by about this up to some 35 us (1595^2 x 911 18.6 us on copies where they say 13.4, 905^2 x
 // 2305 20.8 and 14.3); beyond, both tables are off by as much either way (880 x 1672 x 7165 40.9 us on copies, 48.9 without).
 constexpr double COPIES_UNDERSTATED_US = 4.0, COPIES_UNDERSTATED_BELOW_US = 40.0;
-bool reads_unaligned_rows(int kernel) {
-    return kernel == KERNEL_UNALIGNED64 || kernel == KERNEL_UNALIGNED96 || kernel == KERNEL_UNALIGNED128x64 || kernel == KERNEL_UNALIGNED128;
-}
 Plan plan_on_unaligned_rows(size_t M, size_t N, size_t K, size_t cus, const PlanLimits &limits) {
     Plan p;
     if (!unaligned_runs(K)) return p;
@@ -990,7 +987,6 @@ Plan plan_for(size_t M, size_t N, size_t K, const PlanLimits &limits) {
             // ... or on the tiles for unaligned rows, whose 128-wide chunks straddle half as many lines
             if (limits.excluded_count == 0 && M >= 256 && N >= 256) {
                 Plan direct = plan_on_unaligned_rows(M, N, K, cus, limits);
-                direct.copies_partial_bytes = p.partial_bytes;
                 const double weight = p.kernel == KERNEL_SMALL64_W4_EDGE ? OFF_LINE_SMALL : OFF_LINE_OTHERS;
                 if (direct.kernel != KERNEL_NONE && direct.splits == 1 && direct.est_us < p.est_us * weight) return direct;
             }
@@ -1008,7 +1004,6 @@ Plan plan_for(size_t M, size_t N, size_t K, const PlanLimits &limits) {
         Plan copied = plan_on_copies(M, N, K, limits);
         if (copied.kernel != KERNEL_NONE && left_out(limits, copied)) copied = Plan();
         Plan direct = plan_on_unaligned_rows(M, N, K, cus, limits);
-        direct.copies_partial_bytes = copied.partial_bytes;
         const bool short_b = M <= 8 && N * K < ((size_t)1 << 20);
         const double understated = copied.est_us < COPIES_UNDERSTATED_BELOW_US ? COPIES_UNDERSTATED_US : 0.0;
         const bool copy = copied.est_us > 0.0 ? copied.est_us + understated <= direct.est_us : short_b;
@@ -1437,24 +1432,20 @@ extern "C" void hgemm_release_workspace(void) {
     g_heap[dev] = HeapState();
 }
 
-// Operand bytes reported for a plan: rows read where they lie count as the copies that they once were, so that reservations and
-// what fits the static workspace stay what they were.
-static size_t reported_operand_bytes(const Plan &p, size_t M, size_t N, size_t K) {
-    const bool once_copied = K % 8 && reads_unaligned_rows(p.kernel) && K >= 192 && copy_bytes(M, N, K) <= MAX_PADDED_BYTES;
-    return p.operand_bytes || once_copied ? reported_copy_bytes(M, N, K) : 0;
-}
+// Operand bytes reported for a plan: what a caller reserves, and what the static workspace has to hold.
+static size_t reported_operand_bytes(const Plan &p, size_t M, size_t N, size_t K) { return p.operand_bytes ? reported_copy_bytes(M, N, K) : 0; }
 static size_t padded_partial_bytes(size_t bytes) { return (bytes + 255) / 256 * 256; }
 static bool fits_static_workspace(const Plan &p, size_t M, size_t N, size_t K) {
-    const size_t partial_bytes = reads_unaligned_rows(p.kernel) ? p.copies_partial_bytes : p.partial_bytes;
-    return padded_partial_bytes(partial_bytes) + reported_operand_bytes(p, M, N, K) <= STATIC_WORKSPACE_BYTES;
+    return padded_partial_bytes(p.partial_bytes) + reported_operand_bytes(p, M, N, K) <= STATIC_WORKSPACE_BYTES;
 }
 
 // What hgemm_auto_static_workspace does with a shape whose plan needs more than its array: true, the best plan without a
 // workspace; false, it says so and launches nothing.  Products in whole chunks with aligned rows of C are refused (their plan
-// is too many K slices of a large C).  Others run a kernel with guarded edges.  Where rows of A and B are not aligned (K % 8 != 0),
-// which products are run was settled when only the gather kernel could: those it took up to twice the time of the copies for, at
-// the rates it was once chosen by (80 TFLOP/s against passes at 3.5 TB/s and 4 TB/s for a B that is only streamed): decode
-// shapes, 16 x 8192 x 4097, but not 4095^3.  Where the reported figure reaches the cap of the heap workspace, all are run.
+// is too many K slices of a large C).  Others run a kernel with guarded edges.  Where rows of A and B are not aligned (K % 8 != 0;
+// the plan copies them, what is read where it lies fits), which products are run was settled when only the gather kernel could:
+// those it took up to twice the time of the copies for, at the rates it was once chosen by (80 TFLOP/s against passes at 3.5 TB/s
+// and 4 TB/s for a B that is only streamed): 131 x 67882 x 338, but not 4095^3.  Callers count on what is refused, so it stays.
+// Where the reported figure reaches the cap of the heap workspace, all are run.
 static bool runs_unaided(size_t M, size_t N, size_t K) {
     if (N % 8 == 0 && K % 64 == 0) return false;
     if ((K % 8 == 0 && cached_plan(M, N, K, true).kernel != KERNEL_RAGGED) || reported_copy_bytes(M, N, K) >= MAX_PADDED_BYTES) return true;
@@ -1479,8 +1470,6 @@ extern "C" int hgemm_auto_static_workspace(const hgemm_half *A, const hgemm_half
             return 1;
         }
         chosen = &cached_plan(M, N, K, true);
-    } else if (padded_partial_bytes(chosen->partial_bytes) + chosen->operand_bytes > STATIC_WORKSPACE_BYTES) {
-        chosen = &cached_plan(M, N, K, true);  // (rows read where they lie, in more slices than their copies took)
     }
     const Plan &p = *chosen;
     const size_t partial_bytes = padded_partial_bytes(p.partial_bytes);

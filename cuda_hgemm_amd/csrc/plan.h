@@ -52,7 +52,6 @@ struct Plan {
     // pipelined kernels only: the last tail_tiles workgroup ids of the grid run in tail_splits K slices, or
     // (tail_kernel != KERNEL_NONE, 256x256 tiles only) divided among workgroups of that smaller tile
     int tail_tiles = 0, tail_splits = 1, tail_kernel = KERNEL_NONE;
-    size_t copies_partial_bytes = 0;  // KERNEL_UNALIGNED* only: partial sums of the plan on copies that it stands in for
     int inner_kernel = KERNEL_NONE;  // KERNEL_PADDED only: what runs on the copies (the fields above are its)
 };
 

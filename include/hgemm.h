@@ -193,7 +193,7 @@ int hgemm_reserve_workspace(size_t partial_bytes, size_t operand_bytes);
 void hgemm_release_workspace(void);
 /* Bytes of partial sums (return value) and of operand copies (*operand_bytes, if not NULL)
  * that hgemm_auto's plan for the shape uses (copies: with room for a padded C where N % 8 != 0, up to
- * 1 GiB, an upper bound). */
+ * 1 GiB, an upper bound; none where unaligned rows are read where they lie). */
 size_t hgemm_auto_workspace_bytes(size_t M, size_t N, size_t K, size_t *operand_bytes);
 
 /* hgemm_auto for callers that cannot allocate device memory (serving loops, harnesses that
@@ -207,7 +207,7 @@ size_t hgemm_auto_workspace_bytes(size_t M, size_t N, size_t K, size_t *operand_
  * calls no hipMalloc, hipFree or other allocating routine.  Where the plan needs more than the
  * array holds (hgemm_auto_workspace_bytes tells beforehand) and M, N or K ends inside a tile or chunk
  * (N % 8 != 0 or K % 64 != 0), it runs the best plan that needs no workspace, whose sums may differ from
- * hgemm_auto's in the last bit: the tile without K slices, or for K % 8 != 0 a kernel that
+ * hgemm_auto's in the last bit: the tile without K slices, or for K % 8 != 0, whose plan then copies, a kernel that
  * reads unaligned rows where they lie, except for large products (4095^3).  Otherwise it
  * returns 1 with a message on stderr and nothing launched; else 0.  Other contract violations end
  * the process as everywhere.  All calls on one GPU share that GPU's array, which keeps the last call's

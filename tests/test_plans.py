@@ -130,3 +130,23 @@ def test_rows_of_the_persistent_kernel_hold_at_its_k_only(hgemm_lib, shape, kern
 ])
 def test_ring_kernel_for_few_rows_and_a_long_k(hgemm_lib, shape, kernel):
     assert hgemm_lib.auto_plan(*shape)["kernel"].startswith(kernel)
+
+
+# K % 8 != 0 read where it lies: sizes whose copies would not fit the array of the static workspace, and others
+@pytest.mark.parametrize("shape", [(1494, 1494, 5973), (1297, 1297, 8156), (3330, 656, 6006), (453, 4600, 6178), (16, 8192, 4097),
+                                   (5, 35434, 1547), (1111, 1111, 1111), (515, 1032, 1100)])
+def test_workspace_reported_is_what_the_plan_keeps(hgemm_lib, shape):
+    """No copies are reported where none are made, and the static workspace refuses nothing that fits it as reported."""
+    plan, need = hgemm_lib.auto_plan(*shape), hgemm_lib.auto_workspace_bytes(*shape)
+    assert "read where they lie" in plan["kernel"] and need["operands"] == 0
+    assert (need["partial"] > 0) == (plan["splits"] > 1) and need["partial"] <= hgemm_lib.static_workspace_bytes()
+
+
+def test_static_workspace_refuses_what_does_not_fit(hgemm_lib, capfd):
+    """Before any device call: so also without a GPU."""
+    import ctypes
+    need = hgemm_lib.auto_workspace_bytes(4095, 4095, 4095)
+    assert need["operands"] > hgemm_lib.static_workspace_bytes()
+    address = ctypes.c_void_p(1 << 20)
+    assert hgemm_lib.dll.hgemm_auto_static_workspace(address, address, address, 4095, 4095, 4095) == 1
+    assert str(need["operands"]) in capfd.readouterr().err

@@ -35,7 +35,8 @@ def _call(lib, symbol, A, B, M, N, K, gpu):
 PAIRS = [((1024, 1024, 8192), (256, 256, 8192)),          # K slices on 128x128 tiles, then on 64x64 tiles
          ((7168, 7168, 2048), (64, 4096, 4096)),          # (no workspace: last round on smaller tiles), split-K small-M kernel
          ((7168, 7168, 7168), (512, 512, 8192)),          # last round of a large grid in K slices
-         ((1111, 1111, 1111), (515, 1032, 1100)),         # zero-padded operand copies
+         ((1113, 1211, 5707), (1, 1000, 193)),            # operand copies: with K slices on them, then of a few rows
+         ((1297, 1297, 8156), (515, 1032, 1100)),         # unaligned rows read where they lie: in K slices, then without
          ((2048, 2048, 16384), (16, 4096, 4096))]         # partial sums that fill the array to its last byte
 
 
@@ -47,6 +48,7 @@ def test_static_workspace_matches_heap_workspace(oracle, hgemm_lib, gpu, first, 
         need = hgemm_lib.auto_workspace_bytes(M, N, K)
         assert need["partial"] + need["operands"] <= limit, (M, N, K, need)
         used_scratch |= need["partial"] + need["operands"] > 0
+        assert (need["operands"] > 0) == hgemm_lib.auto_plan(M, N, K)["kernel"].startswith("zero-padded operand copies")
         A = oracle.fill((M, K), 91, 1, oracle.TERNARY, 0, 1)
         B = oracle.fill((N, K), 91, 2, oracle.TERNARY, 0, 1)
         Ad, Bd = _to_gpu(A, gpu), _to_gpu(B, gpu)
@@ -98,9 +100,9 @@ def test_static_workspace_allocates_nothing_and_rejects_what_does_not_fit(oracle
     assert rc == 1 and np.all(got == POISON)
 
 
-# K % 8 != 0 with copies beyond the array (the gather kernel runs instead), and K slices that do not fit it on sizes that
+# K % 8 != 0 with copies beyond the array (the rows are read where they lie instead), and K slices that do not fit it on sizes that
 # end inside a tile and a chunk (the same tile unsliced)
-@pytest.mark.parametrize("M,N,K", [(5, 35434, 1547), (11, 36904, 1180), (16, 8192, 4097), (45328, 104, 16184)])
+@pytest.mark.parametrize("M,N,K", [(131, 67882, 338), (146, 56668, 513), (45328, 104, 16184)])
 def test_static_workspace_runs_what_needs_none_where_the_plan_does_not_fit(oracle, hgemm_lib, gpu, M, N, K):
     import torch
     need = hgemm_lib.auto_workspace_bytes(M, N, K)
@@ -114,11 +116,25 @@ def test_static_workspace_runs_what_needs_none_where_the_plan_does_not_fit(oracl
         assert np.array_equal(got[rows], oracle.hgemm(_bits(A[rows].contiguous()), _bits(B))), (M, N, K, m0)
 
 
+# K % 8 != 0 on plans that keep no copies, of operands that would not fit the array
+@pytest.mark.parametrize("M,N,K", [(5, 35434, 1547), (11, 36904, 1180), (16, 8192, 4097), (1494, 1494, 5973), (453, 4600, 6178)])
+def test_static_workspace_goes_by_the_plan_that_runs(oracle, hgemm_lib, gpu, M, N, K):
+    """What fits the array as reported runs, on hgemm_auto's plan: the same bits, K slices among them."""
+    need = hgemm_lib.auto_workspace_bytes(M, N, K)
+    assert need["operands"] == 0 and need["partial"] <= hgemm_lib.static_workspace_bytes()
+    A, B = oracle.fill((M, K), 96, 1), oracle.fill((N, K), 96, 2)
+    Ad, Bd = _to_gpu(A, gpu), _to_gpu(B, gpu)
+    rc, got = _call(hgemm_lib, "hgemm_auto_static_workspace", Ad, Bd, M, N, K, gpu)
+    _, ref = _call(hgemm_lib, "hgemm_auto", Ad, Bd, M, N, K, gpu)
+    assert rc == 0 and np.array_equal(got, ref)
+
+
 def test_small_operand_copies_hold_a_small_buffer(oracle, hgemm_lib, gpu):
-    """K % 8 != 0: 0.5 ... 34 MB of copies take a workspace of 64 MiB, not the 1 GiB that large copies share, and a large one
+    """K % 8 != 0: 0.4 ... 26 MB of copies take a workspace of 64 MiB, not the 1 GiB that large copies share, and a large one
     that is there already serves them too."""
     import torch
-    for M, N, K in [(1, 1000, 193), (192, 192, 1001), (64, 4096, 4097), (700, 1333, 515)]:
+    for M, N, K in [(1, 1000, 193), (4, 243, 2188), (3019, 1354, 195), (1291, 956, 5550)]:
+        assert hgemm_lib.auto_plan(M, N, K)["kernel"].startswith("zero-padded operand copies")
         Ab, Bb = oracle.fill((M, K), 95, 1, oracle.TERNARY, 0, 1), oracle.fill((N, K), 95, 2, oracle.TERNARY, 0, 1)
         A, B, C = _to_gpu(Ab, gpu), _to_gpu(Bb, gpu), torch.empty((M, N), dtype=torch.float16, device=gpu)
         partial = hgemm_lib.auto_workspace_bytes(M, N, K)["partial"]
