@@ -74,14 +74,13 @@ def _exact_and_infinite(oracle, hgemm_lib, gpu, shape, kernel, sliced):
 
 
 def test_static_workspace_takes_what_it_took(hgemm_lib, gpu):
-    """What fits the array and what is refused goes by the copies these rows once needed; what runs without a workspace is the
-    unsliced kernel."""
+    """Rows read where they lie keep partial sums at most, which fit the array; copies beyond it are refused."""
     import torch
     limit = hgemm_lib.static_workspace_bytes()
     for (M, N, K), taken in [((1111, 1111, 5565), True), ((16, 8192, 4097), True), ((4095, 4095, 4095), False)]:
         need = hgemm_lib.auto_workspace_bytes(M, N, K)
-        assert need["operands"] >= 2 * (M + N) * K
-        assert (need["operands"] > limit) == ((M, N, K) != (1111, 1111, 5565))
+        assert need["operands"] == 0 if taken else need["operands"] >= 2 * (M + N) * K
+        assert (need["partial"] + need["operands"] <= limit) == taken
         gen = torch.Generator(device=gpu).manual_seed(7)
         A, B = (torch.randint(-1, 2, (rows, K), generator=gen, device=gpu, dtype=torch.int8).half() for rows in (M, N))
         C, D = torch.full((M, N), float("nan"), dtype=torch.float16, device=gpu), torch.empty((M, N), dtype=torch.float16, device=gpu)
