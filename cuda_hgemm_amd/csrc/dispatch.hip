@@ -1568,7 +1568,7 @@ extern "C" const char *hgemm_kernel_name(int kernel) {
         case KERNEL_SPLIT_64x64: return "split-K 64x64x64, 4 waves, look-ahead 5-stage or 4-stage ring";
         case KERNEL_SPLIT_64x128: return "split-K 64x128x64, 4 waves, 4-stage ring";
         case KERNEL_SPLIT_128x64: return "split-K 128x64x64, 4 waves, 4-stage ring";
-        case KERNEL_SPLIT_2x64x64: return "split-K 128x64x64, as two 64x64x64 tiles, 4 waves each, 5-stage ring";
+        case KERNEL_SPLIT_2x64x64: return "split-K 2x64x64x64, 4 waves a tile, look-ahead 5-stage or 4-stage ring";
         case KERNEL_SPLIT_128x128: return "split-K 128x128x64, 4 waves, 4-stage ring";
         case KERNEL_DECODE_BN16: return "streaming decode, 16 columns per workgroup, one wave per K slice";
         case KERNEL_DECODE_BN32: return "streaming decode, 32 columns per workgroup, one wave per K slice";
@@ -1577,10 +1577,10 @@ extern "C" const char *hgemm_kernel_name(int kernel) {
         case KERNEL_DECODE_RESIDENT: return "decode with A in registers, persistent workgroups over 16-column tiles, one wave per K slice";
         case KERNEL_RAGGED: return "guarded 128x128x32, 4 waves, any shape";
         case KERNEL_PADDED: return "zero-padded operand copies + kernel of the padded shape";
-        case KERNEL_UNALIGNED64: return "zero-padded chunks of rows read where they lie, 64x64x128, 4 waves";
-        case KERNEL_UNALIGNED96: return "zero-padded chunks of rows read where they lie, 96x96x128, 4 waves";
-        case KERNEL_UNALIGNED128x64: return "zero-padded chunks of rows read where they lie, 128x64x128, 8 waves";
-        case KERNEL_UNALIGNED128: return "zero-padded chunks of rows read where they lie, 128x128x128, 8 waves";
+        case KERNEL_UNALIGNED64: return "rows read where they lie, 64x64x128, 4 waves";
+        case KERNEL_UNALIGNED96: return "rows read where they lie, 96x96x128, 4 waves";
+        case KERNEL_UNALIGNED128x64: return "rows read where they lie, 128x64x128, 8 waves";
+        case KERNEL_UNALIGNED128: return "rows read where they lie, 128x128x128, 8 waves";
         case KERNEL_SIMT: return "scalar fallback";
         default: return "none";
     }

@@ -30,8 +30,10 @@ CASES = [
     ((492, 2108, 136), "pipelined 64x64"), ((2574, 1, 3112), "pipelined 64x64"),
     ((7, 20, 72), "split-K 32x64"), ((11, 5, 2792), "split-K 32x64"), ((39, 2, 176), "split-K 64x64"),
     ((34, 2, 7416), "split-K 64x64"), ((38, 18838, 96), "split-K 64x128"), ((38, 17733, 2136), "split-K 64x128"),
-    ((67, 1, 216), "split-K 128x64"), ((76, 2, 6272), "split-K 128x64"), ((69, 23286, 88), "split-K 128x128"),
+    ((67, 1, 216), "split-K 2x64x64x64"), ((76, 2, 6272), "split-K 2x64x64x64"), ((69, 23286, 88), "split-K 128x128"),
     ((74, 17395, 3824), "split-K 128x128"),
+    ((66, 10404, 1664), "split-K 128x64"), ((66, 9061, 1968), "split-K 128x64"), ((65, 674, 25472), "split-K 128x64"),
+    ((65, 899, 18768), "split-K 128x64"), ((65, 1900, 9048), "split-K 128x64"),
     ((1, 9, 312), "streaming decode"), ((4, 1475, 14528), "streaming decode"), ((18, 220, 288), "streaming decode"),
     ((56, 81, 312), "streaming decode"), ((67, 4295, 272), "streaming decode"), ((67, 146, 280), "streaming decode"),
     ((1, 1984, 9600), "streaming decode, 16 columns per workgroup, per-wave"),             # N and K even, the waves' shares not
@@ -41,8 +43,28 @@ CASES = [
     ((8, 17728, 1088), "streaming decode, 16 columns per workgroup, per-wave"),
     ((5, 2048, 4160), "streaming decode, 16 columns per workgroup, per-wave"),
     ((30, 1536, 6976), "streaming decode, 16 columns per workgroup, per-wave"),
-    ((511, 511, 511), "zero-padded"), ((296, 299, 2113), "zero-padded"), ((3, 1001, 4099), "zero-padded"),
-    ((1027, 520, 193), "zero-padded"), ((2591, 11875, 1833), "zero-padded"),
+    ((511, 511, 511), "rows read where they lie"), ((296, 299, 2113), "rows read where they lie"),
+    ((3, 1001, 4099), "rows read where they lie"), ((1027, 520, 193), "rows read where they lie"),
+    # operand copies: of a few rows, of short rows, with K slices on them, large ones
+    ((1, 1000, 193), "zero-padded operand copies"), ((5, 49, 2585), "zero-padded operand copies"),
+    ((3019, 1354, 195), "zero-padded operand copies"), ((1113, 1211, 5707), "zero-padded operand copies"),
+    ((2591, 11875, 1833), "zero-padded operand copies"),
+]
+
+# Split-K tiles on their look-ahead loop (more than eight chunks to a slice), which ends in a remainder of its steady part that goes by
+# the number of chunks: nine to fifteen of them, even and odd, with K ending inside the last one and not, in K slices that differ by
+# one chunk, and M one row into the second of two rows of tiles
+LOOKAHEAD = [
+    ((9, 1, 520), "split-K 32x64", 1), ((10, 1, 640), "split-K 32x64", 1), ((17, 45, 696), "split-K 32x64", 1),
+    ((32, 63, 744), "split-K 32x64", 1), ((22, 33, 824), "split-K 32x64", 1), ((31, 46, 888), "split-K 32x64", 1),
+    ((30, 46, 920), "split-K 32x64", 1), ((9, 1, 8248), "split-K 32x64", 16), ((21, 250, 9024), "split-K 32x64", 16),
+    ((13, 184, 18672), "split-K 32x64", 16), ((23, 98, 19800), "split-K 32x64", 16),
+    ((34, 1, 520), "split-K 64x64", 1), ((57, 144, 640), "split-K 64x64", 1), ((35, 87, 696), "split-K 64x64", 1),
+    ((48, 85, 760), "split-K 64x64", 1), ((33, 1, 8256), "split-K 64x64", 16), ((57, 181, 11976), "split-K 64x64", 16),
+    ((34, 134, 25600), "split-K 64x64", 16), ((52, 88, 27000), "split-K 64x64", 16),
+    ((65, 1, 536), "split-K 2x64x64x64", 1), ((122, 75, 600), "split-K 2x64x64x64", 1), ((95, 86, 672), "split-K 2x64x64x64", 1),
+    ((84, 81, 832), "split-K 2x64x64x64", 1), ((65, 1, 8560), "split-K 2x64x64x64", 16), ((113, 39, 22016), "split-K 2x64x64x64", 16),
+    ((119, 52, 16016), "split-K 2x64x64x64", 16), ((123, 34, 23696), "split-K 2x64x64x64", 16),
 ]
 
 
@@ -55,6 +77,19 @@ def _gpu_bits(bits, gpu):
 def test_sizes_inside_tiles_and_chunks(oracle, hgemm_lib, gpu, shape, kernel):
     """Exact on ternary inputs (sums are integers below 2048) inside a guard band; then with an infinity in one row of A, at
     the k that the last chunk and the one before it both read: that row is infinite with B's sign, no other changes."""
+    _exact_and_infinite(oracle, hgemm_lib, gpu, shape, kernel)
+
+
+@pytest.mark.parametrize("shape,kernel,slices", LOOKAHEAD)
+def test_look_ahead_split_k_at_its_edges(oracle, hgemm_lib, gpu, shape, kernel, slices):
+    M, N, K = shape
+    plan = hgemm_lib.auto_plan(M, N, K)
+    assert plan["splits"] == slices and -(-K // 64) > 8 * slices, plan
+    assert M > 32 or -(-N // 64) * slices <= 512      # (the 32-row tile has the other loop beyond two workgroups to a CU)
+    _exact_and_infinite(oracle, hgemm_lib, gpu, shape, kernel)
+
+
+def _exact_and_infinite(oracle, hgemm_lib, gpu, shape, kernel):
     import torch
     M, N, K = shape
     plan = hgemm_lib.auto_plan(M, N, K)

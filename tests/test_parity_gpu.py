@@ -291,12 +291,12 @@ def test_auto_every_tile_with_and_without_k_slices(oracle, hgemm_lib, gpu, shape
     ((1024, 8240, 3264), "pipelined 256x128x64", "tail"), ((1024, 8840, 4288), "pipelined 256x128x64", "tail chained"),
     ((640, 28672, 8192), "pipelined 256x256x64", "tail chained"),
     ((1, 192, 1344), "split-K 32x64x64", "main"), ((63, 64, 1216), "split-K 64x64x64", "main"),
-    ((37, 17152, 2176), "split-K 64x128x64", "main"), ((80, 64, 1088), "split-K 128x64x64", "main"),
+    ((37, 17152, 2176), "split-K 64x128x64", "main"), ((80, 64, 1088), "split-K 2x64x64x64", "main"),
     ((102, 16384, 1856), "split-K 128x128x64", "main"), ((110, 3072, 10112), "split-K 128x64x64", "main")])
 def test_k_slices_that_differ_by_a_chunk(oracle, hgemm_lib, gpu, shape, kernel, where):
     """K is cut into slices of whole 64-wide chunks, as even as that allows: where the slice count does not divide the
     chunk count the first slices walk one chunk more.  Every kernel that takes K slices (each pipelined tile,
-    interleaved and chained, the four-wave 64x64 tile, the last round of a large grid, the five split-K tiles), on a
+    interleaved and chained, the four-wave 64x64 tile, the last round of a large grid, the split-K tiles), on a
     shape whose plan has such slices."""
     M, N, K = shape
     plan = hgemm_lib.auto_plan(M, N, K)

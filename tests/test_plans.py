@@ -51,10 +51,10 @@ def test_slice_counts_below_one_tile_of_columns(hgemm_lib, shape, sliced):
     ((1, 3544, 25216), "streaming decode"),                    # 37.1 on the 64x64 tile, 29.0
     ((6, 640, 640), "streaming decode"),
     ((113, 12496, 2368), "split-K 128x64"),                    # 25.8, 19.5
-    ((102, 40, 1664), "split-K 128x64"),                       # 7.0, 5.8
+    ((102, 40, 1664), "split-K 2x64x64x64"),                   # 7.0, 5.8 on 128x64 split-K
     ((28, 7968, 21952), "split-K 32x64"),                      # 65.1, 57.1
     ((59, 3240, 24896), "split-K 64x64"),                      # 37.5, 33.4
-    ((84, 11736, 832), "split-K 128x64"),                      # 9.2, 8.4
+    ((84, 11736, 832), "split-K 2x64x64x64"),                  # 9.2, 8.4 on 128x64 split-K
 ])
 def test_small_m_on_whole_chunks_of_ragged_columns(hgemm_lib, shape, kernel):
     assert hgemm_lib.auto_plan(*shape)["kernel"].startswith(kernel)
