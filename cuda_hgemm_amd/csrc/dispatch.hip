@@ -1227,8 +1227,7 @@ int plans_to_time(size_t M, size_t N, size_t K, int max_plans, Plan *plans) {
         const Plan p = plan_for(M, N, K, limits);
         if (p.kernel == KERNEL_NONE) break;
         plans[count++] = p;
-        // nothing to choose from: the gather kernel, and copies of rows that nothing else reads (K % 8 != 0)
-        if ((p.kernel == KERNEL_PADDED && K % 8) || p.kernel == KERNEL_RAGGED || p.kernel == KERNEL_SIMT) break;
+        if (p.kernel == KERNEL_RAGGED || p.kernel == KERNEL_SIMT) break;  // nothing to choose from
     }
     return count;
 }

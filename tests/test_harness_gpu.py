@@ -140,7 +140,7 @@ def test_device_buffers_without_torch(oracle, hgemm_lib, gpu):
 
 
 @pytest.mark.parametrize("shape", [(384, 6144, 5120), (64, 4096, 4096), (16, 28672, 4096), (1000, 4000, 4096),
-                                   (100, 100, 100), (1000, 1000, 1000)])   # the last: direct plans and one on copies
+                                   (100, 100, 100), (1000, 1000, 1000), (1291, 956, 5550), (3, 100, 1001)])   # the last three: direct plans and one on copies
 def test_tuning_on_the_callers_operands(oracle, hgemm_lib, gpu, shape):
     """hgemm_auto_tune times the model's best plans for a shape and keeps the fastest: the kept plan is one of those
     hgemm_auto_tune_plans lists, the plan queries report it, C holds its product (within the tolerance of the

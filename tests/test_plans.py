@@ -18,6 +18,15 @@ def test_tuner_times_direct_plans_beside_copies(hgemm_lib, size):
     assert len(plans) >= 4 and sum(on_copies) == 1, plans
 
 
+@pytest.mark.parametrize("shape", [(2603, 2603, 2603), (4095, 4095, 4095), (600, 14336, 4095), (3, 100, 1001), (1111, 1111, 5565)])
+def test_tuner_times_rows_read_where_they_lie_beside_copies(hgemm_lib, shape):
+    """K % 8 != 0: copies are one plan of several, wherever they come in the order."""
+    plans = hgemm_lib.tune_plans(*shape, 12)
+    assert len({(p["kernel"], p["splits"]) for p in plans}) == len(plans) >= 5, plans
+    assert sum(p["kernel"].startswith("zero-padded operand copies") for p in plans) == 1, plans
+    assert all(p["kernel"].startswith(("zero-padded operand copies", "rows read where they lie")) for p in plans), plans
+
+
 @pytest.mark.parametrize("M,N,K", [(24001, 24001, 1001), (16385, 16385, 8191), (20001, 20001, 4001)])
 def test_copies_are_planned_by_what_is_copied(hgemm_lib, M, N, K):
     """(M + N) rows of whole chunks within the workspace's 1 GiB, whatever a C of that size would take."""
