@@ -12,7 +12,9 @@ import ctypes as C
 import importlib.machinery
 import importlib.util
 import os
+import re
 import sys
+import warnings
 from typing import List, Optional
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
@@ -79,13 +81,22 @@ _call_module = None
 
 
 def _native_calls():
-    """The module that launches on torch tensors without ctypes (``csrc/python_call.cpp``); None in a process without torch,
-    and where torch was not installed when the library was built."""
+    """The module that launches on torch tensors without ctypes (``csrc/python_call.cpp``).  None, and every call goes through
+    ctypes to the same kernels, in a process without torch, where torch was not installed when the library was built, and
+    (with a warning) where the module does not load into the torch of this process or was built against another one."""
     global _call_module
     if _call_module is None and "torch" in sys.modules and os.path.exists(call_module_path()):
         loader = importlib.machinery.ExtensionFileLoader("_call", call_module_path())
-        module = importlib.util.module_from_spec(importlib.util.spec_from_loader("_call", loader))
-        loader.exec_module(module)
+        try:
+            module = importlib.util.module_from_spec(importlib.util.spec_from_loader("_call", loader))
+            loader.exec_module(module)
+            torch_version = str(sys.modules["torch"].__version__)
+            if not re.match(re.escape(module.torch_version) + r"(?!\d)", torch_version):  # (2.10.0 also for 2.10.0+rocm7.0, 2.10.0a0)
+                raise ImportError(f"built against torch {module.torch_version}, this is {torch_version}")
+        except ImportError as e:
+            warnings.warn(f"{call_module_path()} is not used, calls on torch tensors take 1 ... 3 us longer: {e}; "
+                          "rebuild with `python -m cuda_hgemm_amd.build`", RuntimeWarning)
+            return None
         _call_module = module
     return _call_module
 
@@ -174,9 +185,9 @@ class HgemmLibrary:
         d.hgemm_variant_run.argtypes, d.hgemm_variant_run.restype = [C.c_int] + _HGEMM_ARGS, C.c_int
         self._run = d.hgemm_variant_run
         self._indices = {}  # variant names seen by call() -> their indices
-        # operands that are plain torch tensors: checked and launched in one native call
+        # operands that are plain torch tensors: checked and launched in one native call (a subclass's own call() stays in front)
         self._run_address = C.cast(d.hgemm_variant_run, _PTR).value
-        native = _native_calls() if torch_runtime else None
+        native = _native_calls() if torch_runtime and type(self).call is HgemmLibrary.call else None
         self._native_product = native.product if native else None
         if native:
             self.call = native.Caller(self._run_address, self._indices, self.call)

@@ -152,15 +152,25 @@ def _compile(src, force):
     return obj
 
 
+def _torch_string_abi(root):
+    """Which std::string the installed torch was built with (1: C++11's), from its CMake configuration; importing it takes seconds."""
+    config = os.path.join(root, "share", "cmake", "Torch", "TorchConfig.cmake")
+    found = re.search(r"_GLIBCXX_USE_CXX11_ABI=([01])", open(config).read()) if os.path.exists(config) else None
+    return found.group(1) if found else "1"
+
+
 def _build_python_call(force):
     """The module behind HgemmLibrary.call and hgemm() for torch tensors: host code only, against the installed torch."""
     torch = importlib.util.find_spec("torch")
     if torch is None or not torch.submodule_search_locations:
         return None  # a machine without torch: nobody there has a torch tensor either
+    if not os.path.exists(os.path.join(sysconfig.get_path("include"), "Python.h")):
+        print("Python's headers are not installed: calls on torch tensors will go through ctypes")
+        return None
     root = list(torch.submodule_search_locations)[0]
     target, source = os.path.join(LIB, "_call.so"), os.path.join(CSRC, PYTHON_CALL_SOURCE)
     if force or _stale(target, [source, os.path.join(root, "version.py")]):
-        _run(["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D_GLIBCXX_USE_CXX11_ABI=1", "-I" + os.path.join(root, "include"),
+        _run(["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D_GLIBCXX_USE_CXX11_ABI=" + _torch_string_abi(root), "-I" + os.path.join(root, "include"),
               "-I" + os.path.join(root, "include", "torch", "csrc", "api", "include"), "-I" + sysconfig.get_path("include"), source,
               "-o", target, "-L" + os.path.join(root, "lib"), "-ltorch_python", "-ltorch_cpu", "-lc10"])
     return target

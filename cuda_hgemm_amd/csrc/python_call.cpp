@@ -11,6 +11,7 @@
 #include <ATen/ATen.h>
 #include <ATen/PythonTorchFunctionTLS.h>
 #include <torch/csrc/autograd/python_variable.h>
+#include <torch/version.h>
 
 #include <stddef.h>
 
@@ -176,6 +177,8 @@ PyMODINIT_FUNC PyInit__call(void) {
     if (PyType_Ready(&g_caller_type) < 0) return nullptr;
     PyObject *module = PyModule_Create(&kModule);
     Py_INCREF(&g_caller_type);
-    if (module && PyModule_AddObject(module, "Caller", reinterpret_cast<PyObject *>(&g_caller_type)) < 0) Py_CLEAR(module);
+    if (module && (PyModule_AddObject(module, "Caller", reinterpret_cast<PyObject *>(&g_caller_type)) < 0 ||
+                   PyModule_AddStringConstant(module, "torch_version", TORCH_VERSION) < 0))
+        Py_CLEAR(module);
     return module;
 }

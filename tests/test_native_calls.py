@@ -40,6 +40,42 @@ def test_launcher_is_loaded_and_leaves_other_operands_alone(hgemm_lib):
     assert gone() is None
 
 
+def test_a_module_that_does_not_fit_is_left_out(hgemm_lib, monkeypatch, tmp_path):
+    """A launcher that does not load, or was built against another torch: a warning, and calls go through ctypes."""
+    import torch
+    from cuda_hgemm_amd import binding
+    A, B, C = torch.ones(4, 8).half(), torch.ones(5, 8).half(), torch.empty(4, 5).half()
+
+    def library_without_it():
+        monkeypatch.setattr(binding, "_call_module", None)
+        with pytest.warns(RuntimeWarning, match="is not used"):
+            lib = binding.HgemmLibrary(hgemm_lib.path)
+        assert lib._native_product is None and "call" not in vars(lib)
+        with pytest.raises(ValueError, match="GPU"):
+            lib.call("hgemm_auto", A, B, C, 4, 5, 8)
+
+    with monkeypatch.context() as m:
+        broken = tmp_path / "_call.so"
+        broken.write_bytes(b"not a shared object")
+        m.setattr(binding, "call_module_path", lambda: str(broken))
+        library_without_it()
+    if binding._native_calls() is not None:
+        with monkeypatch.context() as m:
+            m.setattr(torch, "__version__", "1.13.1")
+            library_without_it()
+
+
+def test_a_subclass_keeps_its_own_call(hgemm_lib):
+    from cuda_hgemm_amd import binding
+
+    class Counted(binding.HgemmLibrary):
+        def call(self, *args):
+            return "counted", args
+
+    lib = Counted(hgemm_lib.path)
+    assert lib.call("hgemm_auto", 1) == ("counted", ("hgemm_auto", 1)) and lib._native_product is None
+
+
 @pytest.mark.gpu
 def test_products_and_refusals(hgemm_lib, gpu):
     import torch
