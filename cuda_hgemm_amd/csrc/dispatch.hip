@@ -749,9 +749,16 @@ constexpr Candidate UNALIGNED_TILES[] = {
     {KERNEL_UNALIGNED128x64, 128, 64, 1, 1, 3.95, 0.935, 0.962},
     {KERNEL_UNALIGNED128, 128, 128, 1, 1, 5.09, 1.206, 1.516},
 };
-// The figures for copies understate them by about this up to some 35 us (1595^2 x 911 18.6 us on copies where they say 13.4, 905^2 x
-// 2305 20.8 and 14.3); beyond, both tables are off by as much either way (880 x 1672 x 7165 40.9 us on copies, 48.9 without).
-constexpr double COPIES_UNDERSTATED_US = 4.0, COPIES_UNDERSTATED_BELOW_US = 40.0;
+// What a plan on copies is taken to last beside those figures.  Its own estimate says too little for short products (15 ... 20 us of it
+// 1.17x: two launches back to back) and too much for long ones (60 us and more 0.90x), where the tiles above are at 0.93x throughout.
+// Of 2038 shapes timed both ways (M = 1 ... 5000, N = 16 ... 60000, K = 192 ... 16000) 18 run more than 5 % slower than on copies and the choice
+// is 0.27 % behind the better of the two on average; with 4 us more below an estimate of 40 us, and none beyond, 45 and 0.42 %
+// (636 x 3819 x 2821 31.8 us on copies, 39.4).  Copies that do not stay in the 256 MB Infinity Cache with what they are made of last
+// what they are estimated at (474 x 14498 x 9292 235 us, 193 without).
+double copies_us(const Plan &copied) {
+    const double more = 9.5 - 0.28 * copied.est_us, least = 2 * copied.operand_bytes > (size_t)256000000 ? 0.0 : -5.0;
+    return copied.est_us + (more > 4.0 ? 4.0 : more < least ? least : more);
+}
 Plan plan_on_unaligned_rows(size_t M, size_t N, size_t K, size_t cus, const PlanLimits &limits) {
     Plan p;
     if (!unaligned_runs(K)) return p;
@@ -1005,8 +1012,7 @@ Plan plan_for(size_t M, size_t N, size_t K, const PlanLimits &limits) {
         if (copied.kernel != KERNEL_NONE && left_out(limits, copied)) copied = Plan();
         Plan direct = plan_on_unaligned_rows(M, N, K, cus, limits);
         const bool short_b = M <= 8 && N * K < ((size_t)1 << 20);
-        const double understated = copied.est_us < COPIES_UNDERSTATED_BELOW_US ? COPIES_UNDERSTATED_US : 0.0;
-        const bool copy = copied.est_us > 0.0 ? copied.est_us + understated <= direct.est_us : short_b;
+        const bool copy = copied.est_us > 0.0 ? copies_us(copied) <= direct.est_us : short_b;
         if (direct.kernel != KERNEL_NONE && !(copied.kernel != KERNEL_NONE && copy)) return direct;
         if (copied.kernel != KERNEL_NONE) return copied;
         if (limits.excluded_count == 0) p.kernel = KERNEL_RAGGED;

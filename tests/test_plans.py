@@ -142,7 +142,7 @@ def test_ring_kernel_for_few_rows_and_a_long_k(hgemm_lib, shape, kernel):
 
 
 # K % 8 != 0 read where it lies: sizes whose copies would not fit the array of the static workspace, and others
-@pytest.mark.parametrize("shape", [(1494, 1494, 5973), (1297, 1297, 8156), (3330, 656, 6006), (453, 4600, 6178), (16, 8192, 4097),
+@pytest.mark.parametrize("shape", [(520, 520, 14561), (1000, 1000, 8001), (3330, 656, 6006), (453, 4600, 6178), (16, 8192, 4097),
                                    (5, 35434, 1547), (1111, 1111, 1111), (515, 1032, 1100)])
 def test_workspace_reported_is_what_the_plan_keeps(hgemm_lib, shape):
     """No copies are reported where none are made, and the static workspace refuses nothing that fits it as reported."""
@@ -159,3 +159,19 @@ def test_static_workspace_refuses_what_does_not_fit(hgemm_lib, capfd):
     address = ctypes.c_void_p(1 << 20)
     assert hgemm_lib.dll.hgemm_auto_static_workspace(address, address, address, 4095, 4095, 4095) == 1
     assert str(need["operands"]) in capfd.readouterr().err
+
+
+# K % 8 != 0, M > 8 (microseconds on copies, read where they lie)
+@pytest.mark.parametrize("shape,copied", [
+    ((636, 3819, 2821), True),       # 31.8, 39.4
+    ((2794, 693, 9069), True),       # 64.8, 87.1
+    ((264, 10926, 1455), True),      # 27.2, 34.2
+    ((1395, 1439, 8649), True),      # 62.0, 79.8
+    ((2603, 2603, 2603), True),      # 46, 62
+    ((929, 929, 929), False),        # 12.0, 8.2
+    ((2400, 414, 1458), False),      # 17.5, 12.4
+    ((339, 18066, 8334), False),     # 230, 172: copies beyond the Infinity Cache
+])
+def test_copies_of_unaligned_rows_where_they_pay(hgemm_lib, shape, copied):
+    kernel = hgemm_lib.auto_plan(*shape)["kernel"]
+    assert kernel.startswith("zero-padded operand copies" if copied else "rows read where they lie"), kernel
