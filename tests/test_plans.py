@@ -63,7 +63,7 @@ def test_slice_counts_below_one_tile_of_columns(hgemm_lib, shape, sliced):
     ((102, 40, 1664), "split-K 2x64x64x64"),                   # 7.0, 5.8 on 128x64 split-K
     ((28, 7968, 21952), "split-K 32x64"),                      # 65.1, 57.1
     ((59, 3240, 24896), "split-K 64x64"),                      # 37.5, 33.4
-    ((84, 11736, 832), "split-K 2x64x64x64"),                  # 9.2, 8.4 on 128x64 split-K
+    ((84, 11736, 832), "split-K 128x64"),                      # 9.2, 8.4
 ])
 def test_small_m_on_whole_chunks_of_ragged_columns(hgemm_lib, shape, kernel):
     assert hgemm_lib.auto_plan(*shape)["kernel"].startswith(kernel)
@@ -175,3 +175,23 @@ def test_static_workspace_refuses_what_does_not_fit(hgemm_lib, capfd):
 def test_copies_of_unaligned_rows_where_they_pay(hgemm_lib, shape, copied):
     kernel = hgemm_lib.auto_plan(*shape)["kernel"]
     assert kernel.startswith("zero-padded operand copies" if copied else "rows read where they lie"), kernel
+
+
+# M = 65 ... 128 against a B of less than 32 MB (microseconds on the 128x64 tile, as two rows of 64x64 tiles)
+@pytest.mark.parametrize("shape,two_rows", [
+    ((75, 1024, 1664), True),        # 7.7, 6.4
+    ((113, 2560, 1792), True),       # 11.2, 8.0
+    ((80, 8192, 576), True),
+    ((80, 8256, 576), False),        # more than one 64x64 tile to a CU
+    ((121, 10470, 152), True),       # 5.5, 4.8: level, or this, below K = 192
+    ((112, 37824, 128), True),       # 11.7, 8.9: more than one 128x64 tile too
+    ((80, 22592, 256), True),        # 8.5, 7.7
+    ((76, 10048, 480), False),       # 6.3, 8.1
+    ((125, 8832, 904), False),       # 13.3, 16.1
+    ((124, 4160, 3328), False),      # 15.0, 17.9
+    ((65, 4529, 3328), False),       # 13.9, 16.5
+    ((100, 1984, 8192), True),
+    ((65, 6493, 2416), True),        # 16.6, 15.3
+])
+def test_two_rows_of_split_k_tiles_where_they_pay(hgemm_lib, shape, two_rows):
+    assert hgemm_lib.auto_plan(*shape)["kernel"].startswith("split-K 2x64x64x64" if two_rows else "split-K 128x64")
