@@ -48,18 +48,22 @@ __global__ void __launch_bounds__(Cfg::THREADS)
     // One-dimensional grid, slice-major.  Up to two workgroups of a look-ahead tile to a CU are dealt so that those an XCD runs
     // together are neighbours in a slice (32x64, M = 9 ... 16: 1.01 ... 1.05x).  More of them go round the XCDs, and so do the wider
     // tiles (0.94 ... 1.0x the other way).
+    // K of one chunk against a large C lives by what a workgroup does beside its loads and stores: no division for what is not sliced or
+    // has at most two rows of tiles (each is 100 clocks and more of one chain), and operands of a k-step at a time in the loop below:
+    // 7505 x 8832 x 64 69.2 -> 58.5 us, 8768 x 11971 x 64 136 -> 110, 1664 x 12032 x 64 23.8 -> 20.5 (divisions alone 67.2, 116, 22.9).
     const int tiles_m = (M + BM - 1) / BM, tiles = tiles_m * tiles_n;
-    int split, slot;
+    int split = 0, slot = (int)blockIdx.x, tile_m, tile_n;
     if (Cfg::LOOKAHEAD && gridDim.x <= 512)
         slice_and_slot_of_workgroup((int)blockIdx.x, tiles, splits, split, slot);
-    else
+    else if (splits > 1)
         split = (int)blockIdx.x / tiles, slot = (int)blockIdx.x - split * tiles;
+    few_rows_tile(slot, tiles_m, tiles_n, tile_m, tile_n);
     split = __builtin_amdgcn_readfirstlane(split);
-    const int tile_n = __builtin_amdgcn_readfirstlane(slot / tiles_m), tile_m = __builtin_amdgcn_readfirstlane(slot % tiles_m);
+    tile_m = __builtin_amdgcn_readfirstlane(tile_m), tile_n = __builtin_amdgcn_readfirstlane(tile_n);
     const int m0 = tile_m * BM;
-    int first_chunk, num_k;  // K's chunks are dealt to the slices as evenly as whole chunks allow
     const int chunks = EDGE ? chunks_of(K, BK) : K / BK;
-    slice_of_k(chunks, splits, split, first_chunk, num_k);
+    int first_chunk = 0, num_k = chunks;  // K's chunks are dealt to the slices as evenly as whole chunks allow
+    if (splits > 1) slice_of_k(chunks, splits, split, first_chunk, num_k);
     const int k_begin = first_chunk * BK;
     const int tail_dup = EDGE && first_chunk + num_k == chunks ? tail_pieces(K, BK) : 0;
     const int last_koff = (num_k - 1) * BK - tail_dup * 8;  // where the last chunk is read from, relative to k_begin
@@ -111,40 +115,32 @@ __global__ void __launch_bounds__(Cfg::THREADS)
 #pragma unroll
             for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
 
-    // All operands of a chunk.  drop: 16-byte pieces at its start that must not count (EDGE, last chunk)
-    constexpr int SETS = Cfg::LOOKAHEAD ? 2 : 1;
-    half8 af[SETS][KSTEPS][TM], bf[SETS][KSTEPS][TN];
-    auto load_chunk = [&](int stage, int drop, half8 (&a)[KSTEPS][TM], half8 (&b)[KSTEPS][TN]) {
+    // Operands of k-step kk of a chunk.  drop: 16-byte pieces at the chunk's start that must not count (EDGE, last chunk)
+    auto load_step = [&](int stage, int drop, int kk, half8 (&a)[TM], half8 (&b)[TN]) __attribute__((always_inline)) {
         const unsigned char *s = lds + stage * Cfg::STAGE_BYTES;
+        const uint32_t chunk = (uint32_t)((kk * 2) ^ frag_x) << 4;
 #pragma unroll
-        for (int kk = 0; kk < KSTEPS; ++kk) {
-            const uint32_t chunk = (uint32_t)((kk * 2) ^ frag_x) << 4;
+        for (int i = 0; i < TM; ++i)
+            a[i] = *reinterpret_cast<const half8 *>(s + a_frag_off + i * 32 * ROW_BYTES + chunk);
 #pragma unroll
-            for (int i = 0; i < TM; ++i)
-                a[kk][i] = *reinterpret_cast<const half8 *>(s + a_frag_off + i * 32 * ROW_BYTES + chunk);
+        for (int j = 0; j < TN; ++j)
+            b[j] = *reinterpret_cast<const half8 *>(s + b_frag_off + j * 32 * ROW_BYTES + chunk);
+        if constexpr (EDGE) {
+            if (drop > 0) {
+                const bool keep = kk * 2 + (lane >> 5) >= drop;
 #pragma unroll
-            for (int j = 0; j < TN; ++j)
-                b[kk][j] = *reinterpret_cast<const half8 *>(s + b_frag_off + j * 32 * ROW_BYTES + chunk);
-            if constexpr (EDGE) {
-                if (drop > 0) {
-                    const bool keep = kk * 2 + (lane >> 5) >= drop;
+                for (int i = 0; i < TM; ++i) a[i] = keep_or_zero(a[i], keep);
 #pragma unroll
-                    for (int i = 0; i < TM; ++i) a[kk][i] = keep_or_zero(a[kk][i], keep);
-#pragma unroll
-                    for (int j = 0; j < TN; ++j) b[kk][j] = keep_or_zero(b[kk][j], keep);
-                }
+                for (int j = 0; j < TN; ++j) b[j] = keep_or_zero(b[j], keep);
             }
         }
     };
-
-    auto multiply = [&](half8 (&a)[KSTEPS][TM], half8 (&b)[KSTEPS][TN]) {
+    auto multiply_step = [&](half8 (&a)[TM], half8 (&b)[TN]) __attribute__((always_inline)) {
 #pragma unroll
-        for (int kk = 0; kk < KSTEPS; ++kk)
+        for (int i = 0; i < TM; ++i)
 #pragma unroll
-            for (int i = 0; i < TM; ++i)
-#pragma unroll
-                for (int j = 0; j < TN; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(b[kk][j], a[kk][i], acc[i][j], 0, 0, 0);
+            for (int j = 0; j < TN; ++j)
+                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(b[j], a[i], acc[i][j], 0, 0, 0);
     };
 
     // ---- ring of STAGES buffers, STAGES-1 chunks in flight, barrier one chunk ahead (as the look-ahead loop of mfma_tiled.h,
@@ -167,8 +163,13 @@ __global__ void __launch_bounds__(Cfg::THREADS)
                 wait_vmcnt<0>();
             __syncthreads();
             if (kt + STAGES - 1 < num_k) dma_fetch(kt + STAGES - 1, fill);
-            load_chunk(cur, kt == num_k - 1 ? tail_dup : 0, af[0], bf[0]);
-            multiply(af[0], bf[0]);
+            const int drop = kt == num_k - 1 ? tail_dup : 0;
+#pragma unroll
+            for (int kk = 0; kk < KSTEPS; ++kk) {
+                half8 a[TM], b[TN];
+                load_step(cur, drop, kk, a, b);
+                multiply_step(a, b);
+            }
             cur = (cur + 1 == STAGES) ? 0 : cur + 1;
             fill = (fill + 1 == STAGES) ? 0 : fill + 1;
         }
@@ -178,6 +179,11 @@ __global__ void __launch_bounds__(Cfg::THREADS)
         else
             wait_vmcnt<0>();
         __syncthreads();
+        half8 af[2][KSTEPS][TM], bf[2][KSTEPS][TN];
+        auto load_chunk = [&](int stage, int drop, half8 (&a)[KSTEPS][TM], half8 (&b)[KSTEPS][TN]) __attribute__((always_inline)) {
+#pragma unroll
+            for (int kk = 0; kk < KSTEPS; ++kk) load_step(stage, drop, kk, a[kk], b[kk]);
+        };
         load_chunk(0, num_k == 1 ? tail_dup : 0, af[0], bf[0]);
         // STEADY: the copy of chunk kt+STAGES-1 exists (so does chunk kt+1, and the wait count is the full one)
         auto iteration = [&](auto steady, int kt, half8 (&ca)[KSTEPS][TM], half8 (&cb)[KSTEPS][TN], half8 (&na)[KSTEPS][TM],
@@ -198,7 +204,8 @@ __global__ void __launch_bounds__(Cfg::THREADS)
             }
             if (STEADY || kt + STAGES - 1 < num_k) dma_fetch(kt + STAGES - 1, fill);
             __builtin_amdgcn_sched_barrier(0);
-            multiply(ca, cb);
+#pragma unroll
+            for (int kk = 0; kk < KSTEPS; ++kk) multiply_step(ca[kk], cb[kk]);
             cur = nxt;
             fill = (fill + 1 == STAGES) ? 0 : fill + 1;
         };

@@ -119,4 +119,16 @@ HGEMM_HOST_DEVICE void slice_and_slot_of_workgroup(int b, int count, int slices,
     slot = p - slice * count;
 }
 
+// Position -> tile of the kernels for few rows of C.  One or two rows of tiles: column by column, so that both rows read a
+// panel of B together.  More of them (any M, K of one or two chunks): row by row, which writes rows of C at a time.
+HGEMM_HOST_DEVICE void few_rows_tile(int slot, int tiles_m, int tiles_n, int &tile_m, int &tile_n) {
+    if (tiles_m <= 2) {
+        tile_m = slot & (tiles_m - 1);
+        tile_n = slot >> (tiles_m - 1);
+    } else {
+        tile_m = slot / tiles_n;
+        tile_n = slot - tile_m * tiles_n;
+    }
+}
+
 }  // namespace hgemm

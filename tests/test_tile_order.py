@@ -135,3 +135,39 @@ def test_orders_keep_their_locality(order_report):
 def test_blocked_order_threshold(order_report):
     # B = N x K halves: 128 MiB stays in strips, 162 MiB and 224 MiB go to blocks
     assert "blocked 0 1 1" in order_report
+
+
+FEW_ROWS = textwrap.dedent(
+    r"""
+    #include "%s"
+    #include <cstdio>
+    #include <vector>
+    using namespace hgemm;
+    int main() {
+        for (int tm = 1; tm <= 40; ++tm)
+            for (int tn = 1; tn <= 40; ++tn) {
+                std::vector<int> seen(tm * tn, 0);
+                int last = -1;
+                for (int slot = 0; slot < tm * tn; ++slot) {
+                    int m = -1, n = -1;
+                    few_rows_tile(slot, tm, tn, m, n);
+                    if (m < 0 || m >= tm || n < 0 || n >= tn || seen[m * tn + n]++) return printf("tile: grid %%d x %%d slot %%d\n", tm, tn, slot), 1;
+                    // one or two rows of tiles: column by column; more: row by row
+                    const int rank = tm <= 2 ? n * tm + m : m * tn + n;
+                    if (rank != last + 1) return printf("order: grid %%d x %%d slot %%d\n", tm, tn, slot), 1;
+                    last = rank;
+                }
+            }
+        return 0;
+    }
+    """
+)
+
+
+def test_few_rows_order(tmp_path):
+    """The split-K kernels' order: two rows of tiles read a panel of B together, more of them write rows of C at a time."""
+    src, exe = tmp_path / "few_rows.cpp", tmp_path / "few_rows"
+    src.write_text(FEW_ROWS % HEADER)
+    subprocess.run(["g++", "-O2", "-std=c++17", "-Wall", "-Werror", "-o", str(exe), str(src)], check=True)
+    done = subprocess.run([str(exe)], capture_output=True, text=True, timeout=60)
+    assert done.returncode == 0, done.stdout
