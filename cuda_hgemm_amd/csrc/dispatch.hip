@@ -857,12 +857,14 @@ Plan plan_for(size_t M, size_t N, size_t K, const PlanLimits &limits) {
                 // M = 65 ... 128 against a B of less than 32 MB: as two rows of 64x64 tiles, whose rings leave a CU room for two
                 // workgroups, and half as many slices.  Against the 128x64 tile: up to one of them to a CU, and less than 20 MB of B where K is 2500
                 // and more and N 2048, 355 shapes 0.85 ... 1.70x, geomean 1.19 (75 x 1024 x 1664 7.7 -> 6.4 us, 113 x 2560 x 1792 11.2 -> 8.0); more
-                // B than that 0.84 ... 1.0x (124 x 4160 x 3328 15.0 us, 17.9).  Two to a CU where the 128x64 tile has one, level below K = 192 and
-                // 0.78 ... 1.0x from there on (76 x 10048 x 480 6.3, 8.1); ahead again where that tile needs a second round (N > 16384: 1.04 ...
-                // 1.32x, 112 x 37824 x 128 11.7 -> 8.9).
+                // B than that 0.77 ... 1.07x where B comes from HBM, geomean 0.90 (124 x 4160 x 3328 15.2 us, 18.3; from the Infinity Cache the two
+                // rows are 4 % ahead), except N of more than a third of the CUs' 128x64 tiles, which leave room for two slices only (90 x
+                // 6272 x 2560 15.9 us from HBM and 13.1 from the cache, as two rows 15.2 and 11.0).  Two to a CU where the 128x64 tile has one:
+                // ahead below K = 192 and from M = 96 on (1.0 ... 1.16x; below 0.87 ... 1.0x), 0.78 ... 1.0x for longer K (76 x 10048 x 480 6.3, 8.1);
+                // ahead again where that tile needs a second round (N > 16384: 1.04 ... 1.32x, 112 x 37824 x 128 11.7 -> 8.9).
                 const size_t two_rows = tiles * div_ceil(M, (size_t)64);
                 if (p.kernel == KERNEL_SPLIT_128x64 && N * K < ((size_t)1 << 24) &&
-                    (two_rows <= cus ? K < 2500 || N < 2048 || N * K < (size_t)10000000 : K < 192 || tiles > cus))
+                    (two_rows <= cus ? K < 2500 || N < 2048 || N * K < (size_t)10000000 || 3 * tiles > cus : (K < 192 && M >= 96) || tiles > cus))
                     p.kernel = KERNEL_SPLIT_2x64x64, tiles = two_rows;
                 const bool wide = p.kernel != KERNEL_SPLIT_32x64 && p.kernel != KERNEL_SPLIT_64x64;
                 p.splits = choose_splits(wide ? SLICES_WIDE_TILE : SLICES, tiles, M, columns, cus, K, slice_bytes, limits.partial_bytes);

@@ -168,11 +168,11 @@ def test_small_m_rule_table(hgemm_lib):
                 return r["kernel"]
         return None
 
-    def family(name, N=0, K=0):
+    def family(name, M=0, N=0, K=0):
         # a row's 128x64 tile as two rows of 64x64 tiles, against less than 32 MB of B: up to 256 of them, but for a larger B under a
-        # longer K, and beyond that where K is short or the 128x64 tile itself needs a second round
+        # longer K where three slices of the 128x64 tile fit, and beyond that where K is short or the 128x64 tile itself needs a second round
         if name.startswith("split-K 128x64x64") and N and N * K < 1 << 24:
-            if (K < 2500 or N < 2048 or N * K < 10**7) if N <= 8192 else (K < 192 or N > 16384):
+            if (K < 2500 or N < 2048 or N * K < 10**7 or N > 5440) if N <= 8192 else (K < 192 and M >= 96 or N > 16384):
                 return "split-K 2x64x64x64"
         return name.split(",")[0].replace("32 columns", "16 columns")   # the streaming kernel's two widths
 
@@ -184,7 +184,7 @@ def test_small_m_rule_table(hgemm_lib):
                 if expect is None:
                     continue
                 got = hgemm_lib.auto_plan(M, N, K)["kernel"]
-                assert family(got) == family(expect, N, K), (M, N, K, got, expect)
+                assert family(got) == family(expect, M, N, K), (M, N, K, got, expect)
                 checked += 1
     assert checked > 2000, checked
     # the headline decode shapes, by row

@@ -183,7 +183,9 @@ def test_copies_of_unaligned_rows_where_they_pay(hgemm_lib, shape, copied):
     ((113, 2560, 1792), True),       # 11.2, 8.0
     ((80, 8192, 576), True),
     ((80, 8256, 576), False),        # more than one 64x64 tile to a CU
-    ((121, 10470, 152), True),       # 5.5, 4.8: level, or this, below K = 192
+    ((121, 10470, 152), True),       # 5.5, 4.8: below K = 192 from M = 96 on
+    ((77, 13632, 128), False),       # 3.9, 4.3
+    ((67, 14126, 64), False),        # 3.5, 3.9
     ((112, 37824, 128), True),       # 11.7, 8.9: more than one 128x64 tile too
     ((80, 22592, 256), True),        # 8.5, 7.7
     ((76, 10048, 480), False),       # 6.3, 8.1
@@ -192,6 +194,9 @@ def test_copies_of_unaligned_rows_where_they_pay(hgemm_lib, shape, copied):
     ((65, 4529, 3328), False),       # 13.9, 16.5
     ((100, 1984, 8192), True),
     ((65, 6493, 2416), True),        # 16.6, 15.3
+    ((90, 6272, 2560), True),        # 15.9, 15.2; 13.1, 11.0 with B in the Infinity Cache
+    ((100, 5696, 2752), True),       # 16.0, 15.5; 14.0, 11.2
+    ((83, 5056, 2624), False),       # 13.1, 14.1
 ])
 def test_two_rows_of_split_k_tiles_where_they_pay(hgemm_lib, shape, two_rows):
     assert hgemm_lib.auto_plan(*shape)["kernel"].startswith("split-K 2x64x64x64" if two_rows else "split-K 128x64")
