@@ -511,10 +511,13 @@ constexpr SmallMRule SMALL_M_RULES[] = {
     {17, 24, 3072, 4096, 2049, 4096, 0, ANY, RULE_K_BELOW_4N, KERNEL_DECODE_RING},
     // Up to M = 32 also where K is longer or N larger than that, against the split-K family at its best count: N = 1536 ... 4095,
     // K = 2049 ... 5631 1.02 ... 1.64x (24 x 3712 x 4800 1.27x, 32 x 3369 x 5376 1.26x; level at N = 4096, 0.95x beyond: 18 x 4608 x 6656);
-    // from there on what eight waves' walk costs more than slices do grows with M and N: up to K = 7168 1.03 ... 1.29x below N = 2304, and
-    // 0.88 ... 1.06x from there on (32 x 2944 x 6912 11.5 us, 14.0).  N = 4300 ... 8000, K = 1024 ... 1792 1.08 ... 1.34x.
+    // from there on what eight waves' walk costs more than slices do grows with M and N.  With B from HBM, up to K = 7168: 1.03 ... 1.29x
+    // below N = 2304, 0.77 ... 1.05x from there on (32 x 2944 x 6912 11.5 us, 14.0; with B in the Infinity Cache the ring is 1.08 ... 1.28x up to
+    // K = 7040), M = 17 ... 24 against N from 3264 on 0.94 ... 1.08x (and 1.0 ... 1.27x: 20 x 3915 x 6400 11.8 -> 9.6): this kernel.
+    // N = 4300 ... 8000, K = 1024 ... 1792 1.08 ... 1.34x.
     {17, 32, 1536, 2303, 2049, 7168, 0, ANY, 0, KERNEL_DECODE_RING},
     {17, 32, 2304, 4095, 2049, 6143, 0, ANY, 0, KERNEL_DECODE_RING},
+    {17, 24, 3264, 4095, 6144, 7168, 0, ANY, 0, KERNEL_DECODE_RING},
     {17, 32, 4097, 8192, 1024, 1792, 0, ANY, 0, KERNEL_DECODE_RING},
     // --- M = 65 ... 128 (eight row tiles): the ring kernel for K <= 512 up to N = 8192, K <= 1024 up to N = 4096
     // (median 1.45x).

@@ -127,6 +127,8 @@ def test_rows_of_the_persistent_kernel_hold_at_its_k_only(hgemm_lib, shape, kern
 # M = 9 ... 32 against N up to 8192 (microseconds on the split-K tile, on the ring kernel)
 @pytest.mark.parametrize("shape,kernel", [
     ((32, 2944, 6912), "split-K 32x64"),                       # 11.5, 14.0
+    ((20, 3915, 6400), "streaming decode"),                    # 13.4, 12.8; 11.8, 9.6 with B in the Infinity Cache
+    ((24, 3648, 6144), "streaming decode"),                    # 13.0, 13.5; 11.1, 9.2
     ((30, 1536, 6976), "streaming decode"),                    # the longer K below N = 2304
     ((24, 2560, 6080), "streaming decode"),
     ((20, 2624, 7000), "split-K 32x64"),                       # 11.4, 16.6: K ends inside a chunk
