@@ -31,7 +31,8 @@ ARCH = "gfx950"
 # pick by itself are not trusted on this hardware pool.
 # Kernel arguments are preloaded: the dispatcher writes the first 14 to 16 dwords of them into scalar registers before a wave
 # starts, where it would otherwise begin with a load and its latency.  0.25 us of every launch that is short enough to show
-# it: 256^3 3.07 -> 2.80 us, 512^3 4.01 -> 3.72, 1 x 4096 x 4096 7.08 -> 6.86; level from about 15 us on.
+# it: 256^3 3.07 -> 2.80 us, 512^3 4.01 -> 3.72, 1 x 4096 x 4096 7.08 -> 6.86; level from about 15 us on
+# (the persistent decode kernel lost 0.8 % by it until its first copies were held back again, mfma_decode_resident.h).
 DEVICE_FLAGS = ["--offload-arch=" + ARCH, "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
                 "-Xarch_device", "-mllvm=-amdgpu-kernarg-preload-count=16"]
 CXXFLAGS = ["-O3", "-std=c++17", "-fPIC", "-Wall", "-Wextra", "-Wno-unused-parameter", "-I" + INCLUDE]

@@ -45,7 +45,7 @@ __global__ void __launch_bounds__(Cfg::THREADS)
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave / Cfg::WAVES_N, wn = wave % Cfg::WAVES_N;
 
-    // One-dimensional grid, slice-major.  Up to two workgroups of a look-ahead tile to a CU are dealt so that those an XCD runs
+    // One-dimensional grid, slice-major.  Up to two workgroups of a look-ahead tile to each of the 256 CUs are dealt so that those an XCD runs
     // together are neighbours in a slice (32x64, M = 9 ... 16: 1.01 ... 1.05x).  More of them go round the XCDs, and so do the wider
     // tiles (0.94 ... 1.0x the other way).
     // K of one chunk against a large C lives by what a workgroup does beside its loads and stores: no division for what is not sliced or
@@ -148,7 +148,7 @@ __global__ void __launch_bounds__(Cfg::THREADS)
     // and the barrier confirm chunk kt+1 and retire every wave's reads of chunk kt-1, whose buffer the new copy refills; then
     // the wave issues all operand reads of chunk kt+1, the copy, and only then the MFMAs of chunk kt.  Against a loop that reads a
     // chunk's operands behind its own barrier, at the best slice counts of both: 32x64 1.02 ... 1.05x, 64x64 1.05x (14 ... 18 shapes a
-    // class of M; 64 x 4096 x 4096 11.2 -> 10.1 us, unsliced 19.9 -> 14.6).  That loop (!LOOKAHEAD) stays for a few
+    // class of M; 64 x 4096 x 4096 11.2 -> 10.3 us, unsliced 19.9 -> 14.6).  That loop (!LOOKAHEAD) stays for a few
     // chunks, where it is 0.2 ... 0.3 us ahead (38 x 40 x 136 3.0 us, 3.4), and on the wider tiles, whose waves have more
     // than one MFMA to a k-step (128x64 0.87 ... 1.0x, 64x128 0.89 ... 1.0x, 128x128 1.01x by ring depth).
 #pragma unroll

@@ -3,10 +3,11 @@
 //
 // Direct-to-LDS copies want an aligned source, so these rows travel through registers: 16-byte loads at the rows' own
 // alignment, one chunk ahead, then 16-byte LDS writes, a share of each in front of every MFMA step so that neither blocks
-// the other.  A chunk is 128 of K, twice the other kernels': what an unaligned row costs is the cache line that a piece of
-// it straddles into, and of 256-byte pieces a CU loads 32 bytes a cycle where of 128-byte pieces it loads 22 (aligned rows:
-// 35 either way).  That load path is the bound (64x64: 0.55 us a chunk, of which 0.44 are its 32 KB at that rate); with
-// one wave on a SIMD its latency too, which is why the wider tiles have eight waves.
+// the other.  What a row on a 2-byte boundary costs is the load path: a CU takes 30 bytes a clock of such rows, in pieces of 256 bytes as
+// in pieces of 128, where it takes 53 of rows on 16-byte boundaries and 63 of rows of whole lines (operands in the L2s,
+// profiles/l2_load_rates_by_row_alignment.txt).  64x64: 0.55 us a chunk, of which 0.46 are its 32 KB at that rate.  A chunk is 128 of K, twice
+// the other kernels', for half as many barriers and twice the loads in flight; with one wave on a SIMD the loads' latency counts too, which
+// is why the wider tiles have eight waves.
 // Two chunks ahead in registers measured 0 ... 10 % slower.
 #pragma once
 

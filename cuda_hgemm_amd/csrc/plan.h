@@ -35,7 +35,7 @@ enum KernelId {
     KERNEL_T160x256,
     KERNEL_T192x256,
     KERNEL_T224x256,
-    KERNEL_UNALIGNED64,  // K % 8 != 0: rows read where they lie, through registers; 64x64x128, 96x96x128, 128x64x128, 128x128x128
+    KERNEL_UNALIGNED64,  // K % 8 != 0, and some of K % 64 != 0: rows read where they lie, through registers; 64x64x128, 96x96x128, 128x64x128, 128x128x128
     KERNEL_UNALIGNED96,
     KERNEL_UNALIGNED128x64,
     KERNEL_UNALIGNED128,
