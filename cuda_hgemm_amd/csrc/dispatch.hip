@@ -413,6 +413,9 @@ double predict_subtile_us(const Candidate &big, const Candidate &small, size_t M
 // scaled by the balance too, 8 and 1 us, which this replaced there, chose too many slices since the tiles' loop is faster
 // (6 ... 10 % behind: 12 x 8448 x 1280 in three slices 1.42x the time of one).  The wider and the pipelined tiles keep the older
 // form (`scaled`), fitted to 91 shapes.
+//   From 48 MB of B on, which 64x64 tiles stream past the caches, partial sums weigh less there: 11.  At 16 a B of 130 ... 170 or 257 ... 290 tiles
+// was left in one slice (42 x 8896 x 4864 24.9 us, in three 22.1; 59 x 16576 x 4032 41.8, 38.0); at 8 five slices take the place of three, which are
+// ahead (35 x 8770 x 6592 0.89x).  220 shapes whose count changed: geomean 1.069, one more than 5 % slower.
 // A slice is a whole number of 64-wide chunks, at least
 // two (`min_chunks`: the pipelined tiles need as many as their ring has stages); slices differ by at most one chunk.
 // `slice_bytes`: fp32 partial sums of one slice; the slices together stay within `limit`.
@@ -420,7 +423,7 @@ struct SliceModel {
     double weight, overhead;
     bool scaled;  // partial sums scaled by the balance
 };
-constexpr SliceModel SLICES{16.0, 4.0, false}, SLICES_WIDE_TILE{8.0, 1.0, true};
+constexpr SliceModel SLICES{16.0, 4.0, false}, SLICES_LARGE_B{11.0, 4.0, false}, SLICES_WIDE_TILE{8.0, 1.0, true};
 int choose_splits(const SliceModel &model, size_t tiles, size_t M, size_t N, size_t cus, size_t K, size_t slice_bytes, size_t limit,
                   size_t min_chunks = 2) {
     int best = 1;
@@ -870,7 +873,8 @@ Plan plan_for(size_t M, size_t N, size_t K, const PlanLimits &limits) {
                     (two_rows <= cus ? K < 2500 || N < 2048 || N * K < (size_t)10000000 || 3 * tiles > cus : (K < 192 && M >= 96) || tiles > cus))
                     p.kernel = KERNEL_SPLIT_2x64x64, tiles = two_rows;
                 const bool wide = p.kernel != KERNEL_SPLIT_32x64 && p.kernel != KERNEL_SPLIT_64x64;
-                p.splits = choose_splits(wide ? SLICES_WIDE_TILE : SLICES, tiles, M, columns, cus, K, slice_bytes, limits.partial_bytes);
+                const SliceModel &model = wide ? SLICES_WIDE_TILE : p.kernel == KERNEL_SPLIT_64x64 && N * K >= ((size_t)24 << 20) ? SLICES_LARGE_B : SLICES;
+                p.splits = choose_splits(model, tiles, M, columns, cus, K, slice_bytes, limits.partial_bytes);
                 if (p.splits > 1) p.partial_bytes = (size_t)p.splits * slice_bytes;
             }
         }

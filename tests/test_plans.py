@@ -202,3 +202,16 @@ def test_copies_of_unaligned_rows_where_they_pay(hgemm_lib, shape, copied):
 ])
 def test_two_rows_of_split_k_tiles_where_they_pay(hgemm_lib, shape, two_rows):
     assert hgemm_lib.auto_plan(*shape)["kernel"].startswith("split-K 2x64x64x64" if two_rows else "split-K 128x64")
+
+
+# 64x64 split-K tiles against a B of 48 MB and more
+@pytest.mark.parametrize("shape,splits", [
+    ((64, 10432, 6528), 3),          # 1.14x of one slice
+    ((56, 10335, 5440), 3),          # 1.17
+    ((59, 16576, 4032), 3),          # 1.09
+    ((43, 8832, 5824), 3),           # five slices 0.92 of three
+    ((46, 11328, 6848), 1),          # four slices 0.97 of one
+])
+def test_slice_counts_for_a_large_b(hgemm_lib, shape, splits):
+    plan = hgemm_lib.auto_plan(*shape)
+    assert plan["kernel"].startswith("split-K 64x64") and plan["splits"] == splits, plan
